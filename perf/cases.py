@@ -1,0 +1,369 @@
+"""Measured cases of the mesh data path: what its users' programs have it do, through the public entry points.
+
+A case is a dict of plain values; its ``kind`` names the program it stands for:
+
+* ``parameter_server``  workers push their chunk into the server's registered buffers, the server adds the chunks to its
+                        weights, the workers pull the weights (RDMABuffer.write_from / all_reduce in place / read_into)
+* ``slice_pipeline``    each member packs a strided view of its tensor, the packed chunks are summed, the sum is scattered
+                        back through the view (staging.pack / all_reduce / staging.unpack)
+* ``reduce``            one GPU's share of a gradient bucket: the members' chunks in the slots of a staging area are summed
+                        or averaged into one tensor (reduce.stream_reduce)
+* ``bucket_sync``       data-parallel step over ragged gradients: flatten them into this member's slot, average the slots,
+                        write the average back into the gradients (FlatBucket.pack / all_reduce / FlatBucket.unpack)
+* ``reshard``           column blocks of one tensor are packed for their receivers, moved, and unpacked on the other side
+                        (staging.pack_many / transfer_many / unpack_many)
+* ``stage``             one non-contiguous tensor is sent and received: TensorBuffer.stage() before the transfer and
+                        TensorBuffer.commit() after it; ``layout`` says which view of the tensor is sent
+* ``mesh_scatter``      Reduce over one mesh dimension with the last tensor dimension scattered, then the blocks stacked
+                        again, which is how the result is gathered (reduce_scatter_views / stream_reduce with Stack)
+* ``fp8_exchange``      compressed gradient exchange: quantise the local bucket, then add it and the peers' payloads into
+                        the fp32 accumulators (fp8.quantize_bucket / dequant_accumulate_bucket_many)
+
+Everything a program allocates once (staging buffers, tables, block indexes, outputs) is allocated in ``prepare``.
+"""
+import math
+import random
+
+import torch
+
+from monarch_amd import Slice, fp8, staging
+from monarch_amd import reduce as R
+from monarch_amd.staging import RDMABuffer, StagingArea, TensorBuffer
+
+DEV = "cuda:0"
+DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32, "f64": torch.float64, "u8": torch.uint8}
+BYTES = {"bf16": 2, "f16": 2, "f32": 4, "f64": 8, "u8": 1}
+
+
+def listed():
+    return [
+        # the parameter-server example at the larger of the two sizes its test runs: nine small calls, launches and host work
+        dict(name="parameter_server_1mib", kind="parameter_server", workers=4, nbytes=(1 << 20) + 5),
+        # every other row of an fp32 [4, 256, 256] tensor, eight members: the reference's own CPU-sized configuration
+        dict(name="slice_pipeline_1mib", kind="slice_pipeline", members=8, planes=4, rows=128, cols=256),
+        # one member's share of a ring step over a bf16 gradient bucket, averaged: the headline configuration
+        dict(name="reduce_bucket_bf16", kind="reduce", members=8, numel=25165824, dtype="bf16", op="avg"),
+        # data-parallel step over the ragged gradients of a few layers, about 20 million elements
+        dict(name="bucket_sync_bf16", kind="bucket_sync", members=8, tensors=40, largest=1 << 22, layout=3, dtype="bf16"),
+        # column-parallel reshard of a bf16 weight [4096, 14336] over eight receivers
+        dict(name="reshard_columns_bf16", kind="reshard", rows=4096, cols=14336, blocks=8, dtype="bf16"),
+        # a column block that fits no 16-byte grid: rows of an odd number of bf16 elements that start at an odd column
+        dict(name="stage_odd_columns_bf16", kind="stage", layout="columns", a=4096, b=14336, lo=1, n=7165, dtype="bf16"),
+        # a weight kept transposed, extents that are no multiple of a tile, as a column-major view
+        dict(name="stage_transposed_bf16", kind="stage", layout="transposed", a=5000, b=7000, lo=0, n=0, dtype="bf16"),
+        # the keys of an attention layer sent as [batch, heads, head dim, sequence]: many narrow transposes
+        dict(name="stage_keys_bf16", kind="stage", layout="keys", a=4096, b=64, lo=0, n=64, dtype="bf16"),
+        # interleaved data, every second element of a row kept (x[:, ::2])
+        dict(name="stage_every_other_f32", kind="stage", layout="strided", a=4096, b=8192, lo=0, n=2, dtype="f32"),
+        # [2 hosts, 8 gpus] x [2048, 4096] fp32: summed over gpus, the last dimension scattered over eight ranks
+        dict(name="mesh_scatter_f32", kind="mesh_scatter", hosts=2, gpus=8, rows=2048, cols=4096, dtype="f32"),
+        # compressed exchange of a small model's gradients with seven peers: a few million elements
+        dict(name="fp8_exchange_small", kind="fp8_exchange", tensors=24, largest=1 << 20, peers=7, layout=5),
+        # 1500 tensors of 1K to 4M elements with one peer: the whole gradient of a large layer group
+        dict(name="fp8_exchange_large", kind="fp8_exchange", tensors=1500, largest=1 << 22, peers=1, layout=7),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["parameter_server", "slice_pipeline", "reduce", "bucket_sync", "reshard", "stage", "stage", "stage",
+                       "mesh_scatter", "fp8_exchange"])
+    if kind == "parameter_server":
+        return dict(kind=kind, workers=rng.randint(2, 8), nbytes=_log(rng, 1 << 12, 1 << 24) | 1)
+    if kind == "slice_pipeline":
+        return dict(kind=kind, members=rng.randint(2, 8), planes=rng.randint(1, 8), rows=_log(rng, 16, 1024), cols=_log(rng, 32, 2048))
+    if kind == "reduce":
+        dtype = rng.choice(["bf16", "bf16", "f16", "f32", "f64"])
+        return dict(kind=kind, members=rng.randint(2, 16), numel=_log(rng, 1 << 14, (1 << 26) // BYTES[dtype]), dtype=dtype,
+                    op=rng.choice(["sum", "avg"]))
+    if kind == "bucket_sync":
+        return dict(kind=kind, members=rng.randint(2, 8), tensors=_log(rng, 4, 160), largest=1 << rng.randint(16, 22),
+                    layout=rng.randrange(1 << 20), dtype=rng.choice(["bf16", "f16", "f32"]))
+    if kind == "reshard":
+        dtype, blocks = rng.choice(["bf16", "f32"]), rng.choice([2, 4, 8])
+        return dict(kind=kind, rows=_log(rng, 64, 8192), cols=blocks * _log(rng, 64, 2048), blocks=blocks, dtype=dtype)
+    if kind == "mesh_scatter":
+        gpus = rng.choice([2, 4, 8])
+        return dict(kind=kind, hosts=rng.randint(1, 2), gpus=gpus, rows=_log(rng, 32, 2048), cols=gpus * _log(rng, 16, 512),
+                    dtype=rng.choice(["f32", "bf16"]))
+    if kind == "fp8_exchange":
+        return dict(kind=kind, tensors=_log(rng, 4, 320), largest=1 << rng.randint(16, 22), peers=rng.randint(1, 7),
+                    layout=rng.randrange(1 << 20))
+    layout = rng.choice(["columns", "transposed", "keys", "heads", "strided"])
+    dtype = rng.choice(["bf16", "bf16", "f32", "f16", "u8"])
+    width = 28672 // BYTES[dtype]  # rows of up to 28 KiB
+    if layout == "columns":
+        b = _log(rng, 128, width)
+        n = _log(rng, 32, b - 1)
+        return dict(kind=kind, layout=layout, a=_log(rng, 64, 16384), b=b, lo=rng.randint(0, b - n), n=n, dtype=dtype)
+    if layout == "transposed":
+        return dict(kind=kind, layout=layout, a=_log(rng, 16, 16384), b=_log(rng, 64, 8192), lo=0, n=0, dtype=dtype)
+    if layout == "strided":
+        return dict(kind=kind, layout=layout, a=_log(rng, 64, 8192), b=_log(rng, 128, 8192), lo=0, n=rng.randint(2, 4), dtype=dtype)
+    # attention layouts: sequence length, batch x heads, head dimension
+    return dict(kind=kind, layout=layout, a=_log(rng, 64, 4096), b=_log(rng, 4, 64), lo=0, n=rng.choice([32, 64, 80, 96, 128]),
+                dtype=rng.choice(["bf16", "f16", "f32"]))
+
+
+# ---- what the cases have in common ----
+
+def _values(shape, dtype, g):
+    """Gradient- or weight-like values: normal(0, 0.02); bytes are uniform."""
+    shape = (shape,) if isinstance(shape, int) else shape
+    if dtype == torch.uint8:
+        return torch.randint(0, 256, shape, dtype=dtype, device=DEV, generator=g)
+    if dtype == torch.float64:
+        return torch.randn(shape, dtype=dtype, device=DEV, generator=g) * 0.02
+    return (torch.randn(shape, device=DEV, generator=g) * 0.02).to(dtype)
+
+
+def _ragged_sizes(case):
+    """Element counts of a ragged bucket, log-uniform from 1K up: part of the case, the same for every seed."""
+    rng = random.Random(case["layout"])
+    return [_log(rng, 1 << 10, case["largest"]) for _ in range(case["tensors"])]
+
+
+def _stage_view(x, case):
+    layout = case["layout"]
+    if layout == "columns":
+        return x[:, case["lo"]: case["lo"] + case["n"]]
+    if layout == "transposed":
+        return x.t()
+    if layout == "keys":       # [batch x heads, sequence, head dim] -> [batch x heads, head dim, sequence]
+        return x.transpose(1, 2)
+    if layout == "heads":      # [sequence, batch x heads, head dim] -> [batch x heads, sequence, head dim]
+        return x.permute(1, 0, 2)
+    return x[:, ::case["n"]]   # strided
+
+
+def _stage_shape(case):
+    a, b, n = case["a"], case["b"], case["n"]
+    return {"keys": (b, a, n), "heads": (a, b, n)}.get(case["layout"], (a, b))
+
+
+def _stage_numel(case):
+    a, b, n = case["a"], case["b"], case["n"]
+    if case["layout"] in ("keys", "heads"):
+        return a * b * n
+    return a * {"columns": n, "transposed": b}.get(case["layout"], -(-b // max(1, n)))
+
+
+# ---- prepare ----
+
+def prepare(case, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return dict(_PREPARE[case["kind"]](case, g), kind=case["kind"])
+
+
+def _prepare_parameter_server(case, g):
+    n, size = case["workers"], case["nbytes"]
+    weights = _values(size, torch.uint8, g)
+    chunks = [torch.zeros(size, dtype=torch.uint8, device=DEV) for _ in range(n)]
+    return dict(weights=weights, chunks=chunks, weights_handle=RDMABuffer(weights), grad_handles=[RDMABuffer(c) for c in chunks],
+                grads=[_values(size, torch.uint8, g) for _ in range(n)],
+                pulled=[torch.zeros(size, dtype=torch.uint8, device=DEV) for _ in range(n)])
+
+
+def _prepare_slice_pipeline(case, g):
+    p, r, c = case["planes"], case["rows"], case["cols"]
+    view = Slice(offset=0, sizes=[p, r, c], strides=[2 * r * c, 2 * c, 1])   # every other row of [planes, 2 rows, cols]
+    xs = [torch.rand(p, 2 * r, c, device=DEV, generator=g) * 2 - 1 for _ in range(case["members"])]
+    return dict(view=view, xs=xs, packed=[torch.empty(p * r * c, device=DEV) for _ in xs], total=torch.empty(p * r * c, device=DEV),
+                back=torch.zeros(p, 2 * r, c, device=DEV))
+
+
+def _prepare_reduce(case, g):
+    dtype = DTYPES[case["dtype"]]
+    area = StagingArea(case["members"], case["numel"] * BYTES[case["dtype"]], DEV)
+    group = area.slots(dtype)
+    for t in group:
+        t.copy_(_values(case["numel"], dtype, g))
+    out = torch.empty(case["numel"], dtype=dtype, device=DEV)
+    return dict(area=area, group=group, out=out, factory=R.Factory.of(out), reduction=R.Reduction.from_str(case["op"]))
+
+
+def _prepare_bucket_sync(case, g):
+    dtype = DTYPES[case["dtype"]]
+    bucket = fp8.FlatBucket([_values(n, dtype, g) for n in _ragged_sizes(case)])
+    bucket.block_index()
+    area = StagingArea(case["members"], bucket.total * BYTES[case["dtype"]], DEV)
+    group = area.slots(dtype)
+    for t in group[1:]:
+        t.copy_(_values(bucket.total, dtype, g))
+    # the synchronised gradients: tensors of one allocation, each on a 256-byte boundary
+    sizes, step = bucket.sizes, 256 // BYTES[case["dtype"]]
+    starts, at = [], 0
+    for n in sizes:
+        starts.append(at)
+        at += -(-n // step) * step
+    synced = torch.zeros(at, dtype=dtype, device=DEV)
+    return dict(bucket=bucket, area=area, group=group, mean=torch.empty(bucket.total, dtype=dtype, device=DEV), synced=synced,
+                outs=[synced[s: s + n] for s, n in zip(starts, sizes)])
+
+
+def _prepare_reshard(case, g):
+    dtype, k = DTYPES[case["dtype"]], case["blocks"]
+    w = case["cols"] // k
+    x = _values((case["rows"], case["cols"]), dtype, g)
+    views = [Slice(offset=i * w, sizes=[case["rows"], w], strides=[case["cols"], 1]) for i in range(k)]
+    send = [torch.empty(case["rows"] * w, dtype=dtype, device=DEV) for _ in range(k)]
+    recv = [torch.empty_like(t) for t in send]
+    return dict(x=x, back=torch.zeros_like(x), views=views, send=send, recv=recv, nbytes=[t.numel() * t.element_size() for t in send])
+
+
+def _prepare_stage(case, g):
+    x = _values(_stage_shape(case), DTYPES[case["dtype"]], g)
+    received = torch.zeros_like(x)
+    send = TensorBuffer(_stage_view(x, case))
+    return dict(x=x, received=received, send=send, recv=TensorBuffer(_stage_view(received, case), staging=send.buffer.data))
+
+
+def _prepare_mesh_scatter(case, g):
+    h, n, r, c = case["hosts"], case["gpus"], case["rows"], case["cols"]
+    dtype, w = DTYPES[case["dtype"]], c // n
+    x = _values((h, n, r, c), dtype, g)
+    flat = x.view(-1)
+    outs = [torch.empty(h, r, w, dtype=dtype, device=DEV) for _ in range(n)]
+    return dict(x=x, group=[flat[i * r * c:] for i in range(n)], in_view=Slice(offset=0, sizes=[h, r, c], strides=[n * r * c, c, 1]),
+                out_views=[Slice(offset=k * w, sizes=[h, r, w], strides=[r * c, c, 1]) for k in range(n)], outs=outs,
+                gathered=torch.empty(n, h, r, w, dtype=dtype, device=DEV), factory=R.Factory.of(outs[0]))
+
+
+def _prepare_fp8_exchange(case, g):
+    sizes = _ragged_sizes(case)
+    total = sum(sizes)
+
+    def gradients():   # normal(0, 1) with 0.1 % outliers at 50 x
+        x = torch.randn(total, device=DEV, generator=g)
+        x[torch.randint(0, total, (max(1, total // 1000),), device=DEV, generator=g)] *= 50.0
+        return x.bfloat16()
+
+    def cut(x):
+        return list(torch.split(x, sizes))
+
+    bucket = fp8.FlatBucket([t.clone() for t in cut(gradients())])
+    bucket.block_index()
+    payloads = [fp8.quantize(gradients()) for _ in range(case["peers"])]
+    sums = torch.zeros(total, device=DEV)   # the contiguous fp32 gradient buffer an optimizer keeps
+    acc = fp8.FlatBucket(cut(sums))
+    acc.block_index()
+    q = torch.empty(total, dtype=torch.uint8, device=DEV)
+    scales = torch.empty((total + fp8.BLOCK - 1) // fp8.BLOCK, device=DEV)
+    return dict(bucket=bucket, acc=acc, sums=sums, q=q, scales=scales, qs=[q] + [p[0] for p in payloads],
+                all_scales=[scales] + [p[1] for p in payloads])
+
+
+_PREPARE = dict(parameter_server=_prepare_parameter_server, slice_pipeline=_prepare_slice_pipeline, reduce=_prepare_reduce,
+                bucket_sync=_prepare_bucket_sync, reshard=_prepare_reshard, stage=_prepare_stage,
+                mesh_scatter=_prepare_mesh_scatter, fp8_exchange=_prepare_fp8_exchange)
+
+
+# ---- run ----
+
+def run(state):
+    return _RUN[state["kind"]](state)
+
+
+def _run_parameter_server(s):
+    for handle, grads in zip(s["grad_handles"], s["grads"]):
+        handle.write_from(grads)
+    R.all_reduce(s["weights"], [s["weights"]] + s["chunks"], R.ReduceOp.Sum)
+    for pulled in s["pulled"]:
+        s["weights_handle"].read_into(pulled)
+    return [s["weights"]] + s["pulled"] + s["chunks"]
+
+
+def _run_slice_pipeline(s):
+    for x, packed in zip(s["xs"], s["packed"]):
+        staging.pack(x, s["view"], out=packed)
+    R.all_reduce(s["total"], s["packed"], R.ReduceOp.Sum)
+    staging.unpack(s["back"], s["view"], s["total"])
+    return [s["back"], s["total"]] + s["packed"]
+
+
+def _run_reduce(s):
+    return R.stream_reduce(s["group"], 0, s["factory"], s["reduction"], scatter=False, in_place=False, out=s["out"])
+
+
+def _run_bucket_sync(s):
+    s["bucket"].pack(flat=s["group"][0])
+    R.all_reduce(s["mean"], s["group"], R.ReduceOp.Avg)
+    s["bucket"].unpack(s["mean"], s["outs"])
+    return [s["synced"], s["mean"], s["group"][0]]
+
+
+def _run_reshard(s):
+    staging.pack_many(s["x"], s["views"], s["send"])
+    staging.transfer_many([t.data_ptr() for t in s["recv"]], [t.data_ptr() for t in s["send"]], s["nbytes"])
+    staging.unpack_many(s["back"], s["views"], s["recv"])
+    return [s["back"]] + s["send"] + s["recv"]
+
+
+def _run_stage(s):
+    s["send"].stage()
+    s["recv"].commit()
+    return [s["received"], s["send"].buffer.data]
+
+
+def _run_mesh_scatter(s):
+    R.reduce_scatter_views(s["outs"], s["out_views"], s["group"], s["in_view"], R.ReduceOp.Sum)
+    gathered = R.stream_reduce(s["outs"], 0, s["factory"], R.Reduction(None), scatter=False, in_place=False, out=s["gathered"])
+    return [gathered] + s["outs"]
+
+
+def _run_fp8_exchange(s):
+    fp8.quantize_bucket(s["bucket"], s["q"], s["scales"])
+    fp8.dequant_accumulate_bucket_many(s["acc"], s["qs"], s["all_scales"])
+    return [s["q"], s["scales"], s["sums"]]
+
+
+_RUN = dict(parameter_server=_run_parameter_server, slice_pipeline=_run_slice_pipeline, reduce=_run_reduce,
+            bucket_sync=_run_bucket_sync, reshard=_run_reshard, stage=_run_stage, mesh_scatter=_run_mesh_scatter,
+            fp8_exchange=_run_fp8_exchange)
+
+
+# ---- work and tolerance ----
+
+def work(case):
+    """Bytes: each call of the path reads its inputs once and writes its outputs once; what one call hands to the next
+    crosses a buffer that the program owns (staging memory, a wire payload), so it is written by the one and read by the other."""
+    kind = case["kind"]
+    flops = 0
+    if kind == "parameter_server":
+        n, size = case["workers"], case["nbytes"]
+        nbytes, flops = (2 * n + n + 2 + 2 * n) * size, n * size
+    elif kind == "slice_pipeline":
+        n, v = case["members"], 4 * case["planes"] * case["rows"] * case["cols"]
+        nbytes, flops = (2 * n + n + 1 + 2) * v, n * v // 4
+    elif kind == "reduce":
+        nbytes, flops = (case["members"] + 1) * case["numel"] * BYTES[case["dtype"]], case["members"] * case["numel"]
+    elif kind == "bucket_sync":
+        total = sum(_ragged_sizes(case))
+        nbytes, flops = (2 + case["members"] + 1 + 2) * total * BYTES[case["dtype"]], case["members"] * total
+    elif kind == "reshard":
+        nbytes = 6 * case["rows"] * case["cols"] * BYTES[case["dtype"]]
+    elif kind == "stage":
+        nbytes = 4 * _stage_numel(case) * BYTES[case["dtype"]]
+    elif kind == "mesh_scatter":
+        v = case["hosts"] * case["rows"] * case["cols"]
+        nbytes, flops = (case["gpus"] + 1 + 2) * v * BYTES[case["dtype"]], case["gpus"] * v
+    else:
+        total = sum(_ragged_sizes(case))
+        n = case["peers"] + 1
+        nbytes, flops = (3 + n + 8) * total + 4 * (1 + n) * (total // fp8.BLOCK + 1), (2 + 2 * n) * total
+    return {"bytes": nbytes, "flops": flops}
+
+
+def tolerance(case):
+    """Bytes that are only moved, and sums of bytes, are exact.  Sums: measured against the same path in 64 bits, times four."""
+    kind = case["kind"]
+    if kind in ("parameter_server", "reshard", "stage"):
+        return "exact"
+    if kind == "fp8_exchange":
+        # codes computed in 64 bits fall the other way at a tie for 3.5e-4 of the elements, which moves a sum by one code step
+        return {"rel": 3e-3, "max": 0.4, "differ": 1.5e-3}
+    dtype = case.get("dtype", "f32")
+    return {"rel": {"bf16": 7e-3, "f16": 9e-4, "f32": 3e-7, "f64": 8e-16}[dtype]}
