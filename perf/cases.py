@@ -102,7 +102,8 @@ def draw(rng):
     if layout == "transposed":
         return dict(kind=kind, layout=layout, a=_log(rng, 16, 16384), b=_log(rng, 64, 8192), lo=0, n=0, dtype=dtype)
     if layout == "strided":
-        return dict(kind=kind, layout=layout, a=_log(rng, 64, 8192), b=_log(rng, 128, 8192), lo=0, n=rng.randint(2, 4), dtype=dtype)
+        step = rng.randint(2, 4)   # a Slice has strides that are multiples of one another: rows of whole steps
+        return dict(kind=kind, layout=layout, a=_log(rng, 64, 8192), b=step * _log(rng, 64, 4096), lo=0, n=step, dtype=dtype)
     # attention layouts: sequence length, batch x heads, head dimension
     return dict(kind=kind, layout=layout, a=_log(rng, 64, 4096), b=_log(rng, 4, 64), lo=0, n=rng.choice([32, 64, 80, 96, 128]),
                 dtype=rng.choice(["bf16", "f16", "f32"]))
@@ -148,7 +149,7 @@ def _stage_numel(case):
     a, b, n = case["a"], case["b"], case["n"]
     if case["layout"] in ("keys", "heads"):
         return a * b * n
-    return a * {"columns": n, "transposed": b}.get(case["layout"], -(-b // max(1, n)))
+    return a * {"columns": n, "transposed": b}.get(case["layout"], b // max(1, n))
 
 
 # ---- prepare ----
