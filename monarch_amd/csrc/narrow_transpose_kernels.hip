@@ -1,0 +1,305 @@
+// Transposing pack / unpack of views with a short side, and of small views.
+//
+// The tiles of transpose_kernels.hip are 256 or 512 bytes long on both sides, so a view whose memory-contiguous extent
+// or whose packed rows are shorter than that (the keys of an attention layer sent as [.., head dim, sequence], a tall
+// matrix of a few columns) fills only part of them, and a small view makes too few of them for 256 CUs.  Here the two
+// sides of a tile have lengths of their own: 64 to 512 bytes along the short side, what a tile of 8 to 64 KiB leaves
+// along the other.
+//
+// A tile is read as rows i of consecutive elements j and written as rows j of consecutive elements i: packing, i runs
+// over q and j over the memory-contiguous dimension c; unpacking, the other way round.  HBM-bound: 2 bytes of traffic
+// per byte moved.  Both sides move 16-byte vectors whatever the extents: the last vector of a row is moved back so that it
+// ends where the row ends.  bf16 [64, 4096, 64] -> [64, 64, 4096] (33.6 MB), pack / unpack: 95.8 / 104 us with the tiles
+// that fill a quarter of their lanes, 14.8 / 14.1 us here (4.5 / 4.8 TB/s); head dim 80: 98 / 82 -> 17.3 / 19.2,
+// 32: 94 / 81 -> 7.5 / 7.6; u8 head dim 128: 222 / 303 -> 12.4 / 13.2; bf16 1024^2: 3.3 / 3.4 -> 2.6 / 2.6.
+#include "mhip_device.h"
+#include "pack_internal.h"
+
+namespace mhip {
+
+struct NarrowArgs {
+    char* base;                   // address of the view's first element
+    char* packed;
+    uint32_t Sc, Q;               // extents along c and along q
+    uint32_t vi, vj;              // read rows and columns a tile holds: the tile's own, or the extent where that is shorter
+    uint32_t ti_count, tj_count;  // tiles along i and along j
+    uint32_t nv;                  // vectors per read row
+    uint32_t write_through;       // how written vectors are stored, see try_narrow_transpose
+    FastDiv32 nv_div;
+    uint64_t ntiles, per_xcd;     // each XCD takes a contiguous share of the tiles
+    uint64_t wg0;                 // workgroups of this copy launched before this grid
+    int n_inner, n_outer;         // dimensions after c (q -> memory offset) and before c (batch -> memory offset)
+    FastDiv32 inner_div[kMaxCanonDims];
+    uint64_t inner_stride[kMaxCanonDims];  // bytes
+    uint32_t outer_size[kMaxCanonDims];
+    uint64_t outer_stride[kMaxCanonDims];  // bytes
+};
+
+// v shifted down by `bytes` < 16
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, uint32_t bytes) {
+    if (bytes & 8u) { v.x = v.z; v.y = v.w; }
+    if (bytes & 4u) { v.x = v.y; v.y = v.z; v.z = v.w; }
+    const uint32_t r = bytes & 3u;
+    return u32x4{__builtin_amdgcn_alignbyte(v.y, v.x, r), __builtin_amdgcn_alignbyte(v.z, v.y, r),
+                 __builtin_amdgcn_alignbyte(v.w, v.z, r), v.w >> (8 * r)};
+}
+
+// TI x TJ elements.  In LDS the 16-byte groups of the read rows are numbered through, f = i * GJ + group, and permuted by
+// XOR of the low four bits of f with a key of i / E.  Sixteen consecutive groups lie in one block of E read rows, so the
+// key is the same for all of them and the permutation stays inside their 256 bytes, i.e. inside one turn of the banks:
+//   * a lane stores its vector as one group, sixteen lanes a whole turn, whatever the key;
+//   * on the way out a lane collects E elements of one column from E consecutive read rows, as 32-bit words (narrower
+//     elements: 2 or 4 columns at once, sorted out in registers).  The NIV lanes that take different blocks of one column
+//     see different keys (M apart), the 64 / NIV word columns beside them fill the rest of the turn: no two of the 64
+//     lanes meet in a bank at different addresses.
+template <typename T, int THREADS, bool PACK, int TI, int TJ>
+__global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowArgs a) {
+    constexpr uint32_t ES = sizeof(T), E = 16 / ES;
+    constexpr uint32_t GJ = TJ / E, GI = TI / E;
+    constexpr uint32_t W = ES >= 4 ? 1 : 4 / ES;  // columns per LDS word
+    constexpr uint32_t NIV = GI >= 16 ? 16 : GI, M = 16 / NIV;
+    static_assert(TI % E == 0 && TJ % E == 0 && TJ >= 16 && (TI * GJ) % 16 == 0, "whole turns of the permutation");
+    constexpr uint32_t RP = TI * GJ / THREADS;             // load passes
+    constexpr uint32_t WP = GI * (TJ / W) / THREADS;       // store passes
+    static_assert(RP * THREADS == TI * GJ && WP * THREADS == GI * (TJ / W) && GI % NIV == 0, "whole passes");
+    using Word = typename UnitType<(ES >= 4 ? ES : 4)>::type;
+    __shared__ __attribute__((aligned(16))) char tile[TI * TJ * ES];
+
+    const uint64_t wg = a.wg0 + blockIdx.x;
+    const uint64_t id = (wg & 7) * a.per_xcd + (wg >> 3);
+    if (id >= a.ntiles) return;
+    const uint32_t per_batch = a.ti_count * a.tj_count;
+    const uint64_t b = id / per_batch;
+    const uint32_t in_batch = (uint32_t)(id - b * per_batch);
+    // the side with fewer tiles is the fast one: neighbouring workgroups share whole rows of it
+    uint32_t it, jt;
+    if (a.ti_count < a.tj_count) { jt = in_batch / a.ti_count; it = in_batch - jt * a.ti_count; }
+    else { it = in_batch / a.tj_count; jt = in_batch - it * a.tj_count; }
+    // a tile that would hang over the edge is moved back inside; the overlap is written twice, same bytes
+    const uint32_t I = PACK ? a.Q : a.Sc, J = PACK ? a.Sc : a.Q;
+    uint32_t i0 = it * TI, j0 = jt * TJ;
+    if (i0 + a.vi > I) i0 = I - a.vi;
+    if (j0 + a.vj > J) j0 = J - a.vj;
+    char* __restrict__ mem = a.base;
+    {
+        uint64_t rem = b;
+        for (int k = a.n_outer - 1; k >= 0; --k) {
+            const uint64_t qd = rem / a.outer_size[k];
+            mem += (rem - qd * a.outer_size[k]) * a.outer_stride[k];
+            rem = qd;
+        }
+    }
+    char* __restrict__ packed = a.packed + b * a.Sc * (uint64_t)a.Q * ES;
+    auto q_offset = [&](uint32_t q) -> uint64_t {
+        uint64_t off = 0;
+        for (int k = a.n_inner - 1; k > 0; --k) {
+            uint32_t qd, r;
+            a.inner_div[k].divmod(q, qd, r);
+            off += (uint64_t)r * a.inner_stride[k];
+            q = qd;
+        }
+        return off + (uint64_t)q * a.inner_stride[0];
+    };
+
+    // ---- read side -> LDS: the tile's vectors numbered through, so that short rows leave no lane idle ----
+    const uint32_t total = a.vi * a.nv;
+    u32x4 d[RP];
+#pragma unroll
+    for (uint32_t p = 0; p < RP; ++p) {
+        if (p * THREADS < total) {
+            uint32_t x = threadIdx.x + p * THREADS;
+            x = x < total ? x : total - 1;  // no load is predicated
+            uint32_t r, g;
+            a.nv_div.divmod(x, r, g);
+            const uint32_t col = g * E + E <= a.vj ? g * E : a.vj - E;
+            const char* src;
+            if constexpr (PACK) src = mem + q_offset(i0 + r) + (uint64_t)(j0 + col) * ES;
+            else src = packed + ((uint64_t)(i0 + r) * a.Q + j0 + col) * ES;
+            const uint4 v = load16_unaligned(src);
+            d[p] = u32x4{v.x, v.y, v.z, v.w};
+        }
+    }
+    const bool ragged_j = a.vj % E != 0;
+#pragma unroll
+    for (uint32_t p = 0; p < RP; ++p) {
+        const uint32_t x = threadIdx.x + p * THREADS;
+        if (x < total) {
+            uint32_t r, g;
+            a.nv_div.divmod(x, r, g);
+            u32x4 v = d[p];
+            if (ragged_j) v = shift_down(v, g * E + E <= a.vj ? 0u : (g * E + E - a.vj) * ES);  // a vector that was moved back
+            const uint32_t f = (r * GJ + g) ^ (((r / E) * M) & 15u);
+            *reinterpret_cast<u32x4*>(tile + f * 16) = v;
+        }
+    }
+    __syncthreads();
+
+    // ---- LDS -> written side ----
+    const bool ragged_i = a.vi % E != 0;
+#pragma unroll
+    for (uint32_t p = 0; p < WP; ++p) {
+        const uint32_t u = threadIdx.x + p * THREADS;
+        const uint32_t rest = u / 64;
+        const uint32_t iv = u % NIV + NIV * (rest % (GI / NIV));                               // block of E read rows
+        const uint32_t j = ((rest / (GI / NIV)) * (64 / NIV) + (u % 64) / NIV) * W;            // first column of the word
+        if (j < a.vj && iv * E < a.vi) {
+            const uint32_t g = j / E, byte = (j % E) * ES;
+            Word w[E];
+            uint32_t i = iv * E;
+            if (!ragged_i) {
+                // within a block the rows' groups differ from the first row's by XOR with a constant
+                const uint32_t first = (((E * iv * GJ + g) ^ ((iv * M) & 15u)) * 16) + byte;
+#pragma unroll
+                for (uint32_t k = 0; k < E; ++k)
+                    w[k] = *reinterpret_cast<const Word*>(tile + (GJ >= 16 ? first + k * GJ * 16 : first ^ (k * GJ * 16)));
+            } else {
+                if (i + E > a.vi) i = a.vi - E;  // the last vector of a written row, moved back
+#pragma unroll
+                for (uint32_t k = 0; k < E; ++k) {
+                    const uint32_t r = i + k;
+                    w[k] = *reinterpret_cast<const Word*>(tile + ((r * GJ + g) ^ (((r / E) * M) & 15u)) * 16 + byte);
+                }
+            }
+            u32x4 out[W];
+            if constexpr (ES == 8) {
+                out[0] = u32x4{(uint32_t)w[0], (uint32_t)(w[0] >> 32), (uint32_t)w[1], (uint32_t)(w[1] >> 32)};
+            } else if constexpr (ES == 4) {
+                out[0] = u32x4{w[0], w[1], w[2], w[3]};
+            } else if constexpr (ES == 2) {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    out[0][k] = __builtin_amdgcn_perm(w[2 * k + 1], w[2 * k], 0x05040100u);
+                    out[1][k] = __builtin_amdgcn_perm(w[2 * k + 1], w[2 * k], 0x07060302u);
+                }
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {  // four rows of four bytes, transposed
+                    const uint32_t ab_lo = __builtin_amdgcn_perm(w[4 * k + 1], w[4 * k], 0x05010400u);
+                    const uint32_t ab_hi = __builtin_amdgcn_perm(w[4 * k + 1], w[4 * k], 0x07030602u);
+                    const uint32_t cd_lo = __builtin_amdgcn_perm(w[4 * k + 3], w[4 * k + 2], 0x05010400u);
+                    const uint32_t cd_hi = __builtin_amdgcn_perm(w[4 * k + 3], w[4 * k + 2], 0x07030602u);
+                    out[0][k] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x05040100u);
+                    out[1][k] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x07060302u);
+                    out[2][k] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x05040100u);
+                    out[3][k] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x07060302u);
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < W; ++k) {
+                if (k == 0 || j + k < a.vj) {
+                    char* dst;
+                    if constexpr (PACK) dst = packed + ((uint64_t)(j0 + j + k) * a.Q + i0 + i) * ES;
+                    else dst = mem + q_offset(j0 + j + k) + (uint64_t)(i0 + i) * ES;
+                    if (a.write_through) store16_writethrough_raw(dst, out[k]);  // wave-uniform
+                    else *reinterpret_cast<u32x4_unaligned*>(dst) = out[k];
+                }
+            }
+        }
+    }
+}
+
+// WB and RB: bytes of a written and of a read row of the tile
+template <typename T, bool PACK, int WB, int RB>
+static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
+    constexpr uint32_t ES = sizeof(T), E = 16 / ES, TI = WB / ES, TJ = RB / ES;
+    constexpr int kBytes = TI * TJ * ES, kLanes = kBytes >= 32768 ? 512 : kBytes >= 8192 ? 256 : 128;
+    const uint32_t I = PACK ? a.Q : a.Sc, J = PACK ? a.Sc : a.Q;
+    a.vi = I < TI ? I : TI;
+    a.vj = J < TJ ? J : TJ;
+    a.ti_count = (I + TI - 1) / TI;
+    a.tj_count = (J + TJ - 1) / TJ;
+    a.nv = (a.vj + E - 1) / E;
+    a.nv_div = FastDiv32(a.nv);
+    a.ntiles = nbatch * a.ti_count * a.tj_count;
+    a.per_xcd = (a.ntiles + 7) / 8;
+    return launch_in_pieces(a.per_xcd * 8, kLanes, 8, [&](uint64_t wg0, uint32_t count) {
+        a.wg0 = wg0;
+        MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ>), dim3(count), dim3(kLanes), 0, stream, a);
+    });
+}
+
+// Tile length along a side of `bytes` <= 512: pieces of 128 bytes where they cover the side with little overlap (the last
+// one is moved back), else the next power of two (272 bytes, 67 MB, pack / unpack: one tile of 512 26 / 27 us, three
+// of 128 47 / 29; 384 bytes: 27.8 / 25 against 27.5 / 24.5).
+static uint32_t narrow_tile_bytes(uint64_t bytes) {
+    if (bytes <= 64) return 64;
+    if (bytes <= 128) return 128;
+    const uint64_t pieces = (bytes + 127) / 128 * 128;
+    return pieces * 10 <= bytes * 11 ? 128 : bytes <= 256 ? 256 : 512;
+}
+
+// Which tile: from 16 MiB on, the short side's length from narrow_tile_bytes and the other side's so that the two lengths
+// multiply to 64 KiB (tiles of 64, 32, 16, 8 KiB of 1-, 2-, 4-, 8-byte elements); below that 128 x 128 bytes, which makes
+// more workgroups (bf16 16384 x 20: 2.4 us against 3.0, 65536 x 64 (8.4 MB) 3.6 against 3.8; 16.8 MB of keys of 64 bytes
+// 8.6 against 7.5, of u8 keys of 64 bytes 8.6 against 7.5).
+template <typename T, bool PACK>
+static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
+    constexpr uint32_t ES = sizeof(T);
+    const uint64_t ib = (uint64_t)(PACK ? a.Q : a.Sc) * ES, jb = (uint64_t)(PACK ? a.Sc : a.Q) * ES;
+    if (nbatch * ib * jb / ES >= (16ull << 20)) {  // one of the sides is at most 512 bytes then
+        const bool short_j = jb <= ib;
+        uint32_t n = narrow_tile_bytes(short_j ? jb : ib);
+        if (ES == 8 && n == 64) n = 128;  // a read row of 64 bytes would be fewer than 16 elements
+        if (short_j) {
+            if constexpr (ES < 8)
+                if (n == 64) return launch_narrow<T, PACK, 1024, 64>(a, nbatch, stream);
+            if (n == 128) return launch_narrow<T, PACK, 512, 128>(a, nbatch, stream);
+            if (n == 256) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+            return launch_narrow<T, PACK, 128, 512>(a, nbatch, stream);
+        }
+        if constexpr (ES < 8)
+            if (n == 64) return launch_narrow<T, PACK, 64, 1024>(a, nbatch, stream);
+        if (n == 128) return launch_narrow<T, PACK, 128, 512>(a, nbatch, stream);
+        if (n == 256) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+        return launch_narrow<T, PACK, 512, 128>(a, nbatch, stream);
+    }
+    return launch_narrow<T, PACK, 128, 128>(a, nbatch, stream);
+}
+
+// Takes the view when one of its sides is at most 512 bytes long (bf16 67 MB, sides of 512 / 768 bytes, pack: 23.8 / 27 us
+// here against 24.0 / 25.4 with the long tiles; rows that are not whole lines 26.6 against 34.3, and 27 against 25.4) or
+// when it has at most 12 MiB (bf16 2048^2 3.6 us against 4.0, 2000 x 3000 6.9 against 8.4, u8 2000 x 3000 4.4 against
+// 6.2; fp32 2000 x 3000, 24 MB, 11 against 10.4), both sides holding at least one vector.
+template <bool PACK>
+bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd, uint64_t nbatch, uint32_t Q, uint32_t unit,
+                          hipStream_t stream, int* rc) {
+    const uint64_t Sc = c.dims[cd].size, bytes = nbatch * Sc * Q * unit;
+    const uint64_t short_side = (Sc < Q ? Sc : Q) * unit;
+    if (unit > 8 || short_side < 16) return false;
+    if (short_side > 512 && bytes > (12ull << 20)) return false;
+    NarrowArgs a{};
+    uint64_t written = PACK ? (uint64_t)(uintptr_t)packed | (uint64_t)Q * unit : (uint64_t)(uintptr_t)(base + c.offset * unit);
+    for (int k = 0; k < c.ndim; ++k) {
+        if (k == cd) continue;
+        const uint64_t stride = c.dims[k].stride * unit;
+        if (k > cd) {
+            a.inner_div[a.n_inner] = FastDiv32((uint32_t)c.dims[k].size);
+            a.inner_stride[a.n_inner++] = stride;
+        } else {
+            a.outer_size[a.n_outer] = (uint32_t)c.dims[k].size;
+            a.outer_stride[a.n_outer++] = stride;
+        }
+        if (!PACK) written |= stride;
+    }
+    a.base = base + c.offset * unit;
+    a.packed = packed;
+    a.Sc = (uint32_t)Sc;
+    a.Q = Q;
+    // Written rows that start on half cache lines are stored write-through (33.6 MB of keys 14.8 us against 16.5 through
+    // the cache, unpacked rows of 64 bytes 7.6 against 8.5); others go through the cache, which combines what neighbouring
+    // tiles share (rows of 4001 bf16 15.9 against 18.9, unpacked rows of 160 bytes 19.2 against 19.9), unless the launch
+    // is small enough to be bound by latency (bf16 1500^2 3.5 against 3.7).
+    a.write_through = (written & 63u) == 0 || bytes <= (8ull << 20);
+    switch (unit) {
+        case 1: *rc = launch_narrow_tile<uint8_t, PACK>(a, nbatch, stream); break;
+        case 2: *rc = launch_narrow_tile<uint16_t, PACK>(a, nbatch, stream); break;
+        case 4: *rc = launch_narrow_tile<uint32_t, PACK>(a, nbatch, stream); break;
+        default: *rc = launch_narrow_tile<uint64_t, PACK>(a, nbatch, stream); break;
+    }
+    return true;
+}
+
+template bool try_narrow_transpose<true>(char*, char*, const CanonSlice&, int, uint64_t, uint32_t, uint32_t, hipStream_t, int*);
+template bool try_narrow_transpose<false>(char*, char*, const CanonSlice&, int, uint64_t, uint32_t, uint32_t, hipStream_t, int*);
+
+}  // namespace mhip

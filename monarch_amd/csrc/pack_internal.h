@@ -12,4 +12,10 @@ namespace mhip {
 template <bool PACK>
 bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t unit, hipStream_t stream, int* rc);
 
+// The same for views with a side of at most 512 bytes and for small views; `cd` is the memory-contiguous dimension of
+// `c`, nbatch the product of the dimensions before it and Q of those after it.  Returns false for other views.
+template <bool PACK>
+bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd, uint64_t nbatch, uint32_t Q, uint32_t unit,
+                          hipStream_t stream, int* rc);
+
 }  // namespace mhip

@@ -265,11 +265,11 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
     uint64_t b;
     uint32_t qt, ct;
     if (!walk_tile(a, &b, &qt, &ct)) return;
-    // A tile that would hang over the edge is moved back inside when the extent allows it: it
-    // then overlaps its neighbour, and both write the same bytes to the overlap.
+    // A tile that would hang over the edge is moved back inside (both extents are at least a tile): it then overlaps
+    // its neighbour, and both write the same bytes to the overlap.
     uint32_t q0 = qt * TQ, c0 = ct * TC;
-    if (q0 + TQ > a.Q && a.Q >= (uint32_t)TQ) q0 = a.Q - TQ;
-    if (c0 + TC > a.Sc && a.Sc >= (uint32_t)TC) c0 = a.Sc - TC;
+    if (q0 + TQ > a.Q) q0 = a.Q - TQ;
+    if (c0 + TC > a.Sc) c0 = a.Sc - TC;
     uint64_t batch_off = 0;
     {
         uint64_t rem = b;
@@ -282,21 +282,18 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
     if (threadIdx.x < TQ) {
         uint32_t q = q0 + threadIdx.x;
         uint64_t off = 0;
-        if (q < a.Q) {
-            for (int k = a.n_inner - 1; k > 0; --k) {
-                uint32_t qd, r;
-                a.inner_div[k].divmod(q, qd, r);
-                off += (uint64_t)r * a.inner_stride[k];
-                q = qd;
-            }
-            off += (uint64_t)q * a.inner_stride[0];
+        for (int k = a.n_inner - 1; k > 0; --k) {
+            uint32_t qd, r;
+            a.inner_div[k].divmod(q, qd, r);
+            off += (uint64_t)r * a.inner_stride[k];
+            q = qd;
         }
+        off += (uint64_t)q * a.inner_stride[0];
         s_off[threadIdx.x] = off;
     }
     __syncthreads();
     T* mem_tile = mem + batch_off + c0;                                        // + s_off[q] + c
     T* packed_tile = packed + (b * a.Sc + c0) * (uint64_t)a.Q + q0;            // + c * Q + q
-    const bool full = q0 + TQ <= a.Q && c0 + TC <= a.Sc;
     const int v16 = threadIdx.x % G;  // which 16-byte vector of a row
     const int r16 = threadIdx.x / G;  // which row of a pass of ROWS rows
     constexpr int ROWS = THREADS / G;
@@ -308,139 +305,90 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
     const int qv = G == 16 ? v16 : (threadIdx.x % 16) + 16 * ((threadIdx.x / 64) % 2);
     const int cc0 = G == 16 ? r16 : 4 * (threadIdx.x / 128) + (threadIdx.x % 64) / 16;
     constexpr int CSTEP = G == 16 ? ROWS : 4 * (THREADS / 128);  // columns per pass
-    if (full) {
-        constexpr int PASSES = TQ / ROWS;
-        Vec d[PASSES];
-        if constexpr (PACK) {
+    constexpr int PASSES = TQ / ROWS;
+    Vec d[PASSES];
+    if constexpr (PACK) {
 #pragma unroll
-            for (int p = 0; p < PASSES; ++p) {
-                const int q = r16 + ROWS * p;
-                d[p].v = tload<STREAM>(mem_tile + s_off[q] + v16 * E);
-            }
+        for (int p = 0; p < PASSES; ++p) {
+            const int q = r16 + ROWS * p;
+            d[p].v = tload<STREAM>(mem_tile + s_off[q] + v16 * E);
+        }
 #pragma unroll
-            for (int p = 0; p < PASSES; ++p) {
-                const int q = r16 + ROWS * p;
-                *reinterpret_cast<u32x4*>(&tile[at(q, v16 * E)]) = d[p].v;
-            }
-            __syncthreads();
-            if constexpr (sizeof(T) == 2) {
-                // Two neighbouring columns at once: eight 32-bit LDS reads fetch (q, c) and (q, c+1) for
-                // eight rows, and a 2x2 transpose in registers turns them into the two output vectors.
-                // Half the LDS instructions of the element-wise form, and no sub-dword accesses.
+        for (int p = 0; p < PASSES; ++p) {
+            const int q = r16 + ROWS * p;
+            *reinterpret_cast<u32x4*>(&tile[at(q, v16 * E)]) = d[p].v;
+        }
+        __syncthreads();
+        if constexpr (sizeof(T) == 2) {
+            // Two neighbouring columns at once: eight 32-bit LDS reads fetch (q, c) and (q, c+1) for
+            // eight rows, and a 2x2 transpose in registers turns them into the two output vectors.
+            // Half the LDS instructions of the element-wise form, and no sub-dword accesses.
 #pragma unroll
-                for (int p = 0; p < PASSES / 2; ++p) {
-                    const int c = 2 * (cc0 + CSTEP * p);
-                    uint32_t w[E];
+            for (int p = 0; p < PASSES / 2; ++p) {
+                const int c = 2 * (cc0 + CSTEP * p);
+                uint32_t w[E];
 #pragma unroll
-                    for (int j = 0; j < E; ++j) w[j] = *reinterpret_cast<const uint32_t*>(&tile[at(qv * E + j, c)]);
-                    u32x4 lo, hi;
+                for (int j = 0; j < E; ++j) w[j] = *reinterpret_cast<const uint32_t*>(&tile[at(qv * E + j, c)]);
+                u32x4 lo, hi;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        lo[k] = (w[2 * k] & 0xffffu) | (w[2 * k + 1] << 16);
-                        hi[k] = (w[2 * k] >> 16) | (w[2 * k + 1] & 0xffff0000u);
-                    }
-                    tstore(packed_tile + (uint64_t)c * a.Q + qv * E, lo, a.aligned_stores);
-                    tstore(packed_tile + (uint64_t)(c + 1) * a.Q + qv * E, hi, a.aligned_stores);
+                for (int k = 0; k < 4; ++k) {
+                    lo[k] = (w[2 * k] & 0xffffu) | (w[2 * k + 1] << 16);
+                    hi[k] = (w[2 * k] >> 16) | (w[2 * k + 1] & 0xffff0000u);
                 }
-            } else {
+                tstore(packed_tile + (uint64_t)c * a.Q + qv * E, lo, a.aligned_stores);
+                tstore(packed_tile + (uint64_t)(c + 1) * a.Q + qv * E, hi, a.aligned_stores);
+            }
+        } else {
 #pragma unroll
-                for (int p = 0; p < PASSES; ++p) {
-                    const int cc = cc0 + CSTEP * p;
-                    Vec o;
+            for (int p = 0; p < PASSES; ++p) {
+                const int cc = cc0 + CSTEP * p;
+                Vec o;
 #pragma unroll
-                    for (int j = 0; j < E; ++j) o.e[j] = tile[at(qv * E + j, cc)];
-                    tstore(packed_tile + (uint64_t)cc * a.Q + qv * E, o.v, a.aligned_stores);
+                for (int j = 0; j < E; ++j) o.e[j] = tile[at(qv * E + j, cc)];
+                tstore(packed_tile + (uint64_t)cc * a.Q + qv * E, o.v, a.aligned_stores);
+            }
+        }
+    } else {
+        if constexpr (sizeof(T) == 2) {
+            // the mirror image: rows c and c+1 of the packed side are loaded together and their
+            // halves interleaved into eight 32-bit LDS writes
+#pragma unroll
+            for (int p = 0; p < PASSES / 2; ++p) {
+                const int c = 2 * (cc0 + CSTEP * p);
+                d[2 * p].v = tload<STREAM>(packed_tile + (uint64_t)c * a.Q + qv * E);
+                d[2 * p + 1].v = tload<STREAM>(packed_tile + (uint64_t)(c + 1) * a.Q + qv * E);
+            }
+#pragma unroll
+            for (int p = 0; p < PASSES / 2; ++p) {
+                const int c = 2 * (cc0 + CSTEP * p);
+                const u32x4 lo = d[2 * p].v, hi = d[2 * p + 1].v;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t w0 = (lo[k] & 0xffffu) | (hi[k] << 16);
+                    const uint32_t w1 = (lo[k] >> 16) | (hi[k] & 0xffff0000u);
+                    *reinterpret_cast<uint32_t*>(&tile[at(qv * E + 2 * k, c)]) = w0;
+                    *reinterpret_cast<uint32_t*>(&tile[at(qv * E + 2 * k + 1, c)]) = w1;
                 }
             }
         } else {
-            if constexpr (sizeof(T) == 2) {
-                // the mirror image: rows c and c+1 of the packed side are loaded together and their
-                // halves interleaved into eight 32-bit LDS writes
-#pragma unroll
-                for (int p = 0; p < PASSES / 2; ++p) {
-                    const int c = 2 * (cc0 + CSTEP * p);
-                    d[2 * p].v = tload<STREAM>(packed_tile + (uint64_t)c * a.Q + qv * E);
-                    d[2 * p + 1].v = tload<STREAM>(packed_tile + (uint64_t)(c + 1) * a.Q + qv * E);
-                }
-#pragma unroll
-                for (int p = 0; p < PASSES / 2; ++p) {
-                    const int c = 2 * (cc0 + CSTEP * p);
-                    const u32x4 lo = d[2 * p].v, hi = d[2 * p + 1].v;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t w0 = (lo[k] & 0xffffu) | (hi[k] << 16);
-                        const uint32_t w1 = (lo[k] >> 16) | (hi[k] & 0xffff0000u);
-                        *reinterpret_cast<uint32_t*>(&tile[at(qv * E + 2 * k, c)]) = w0;
-                        *reinterpret_cast<uint32_t*>(&tile[at(qv * E + 2 * k + 1, c)]) = w1;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int p = 0; p < PASSES; ++p) {
-                    const int cc = cc0 + CSTEP * p;
-                    d[p].v = tload<STREAM>(packed_tile + (uint64_t)cc * a.Q + qv * E);
-                }
-#pragma unroll
-                for (int p = 0; p < PASSES; ++p) {
-                    const int cc = cc0 + CSTEP * p;
-#pragma unroll
-                    for (int j = 0; j < E; ++j) tile[at(qv * E + j, cc)] = d[p].e[j];
-                }
-            }
-            __syncthreads();
 #pragma unroll
             for (int p = 0; p < PASSES; ++p) {
-                const int q = r16 + ROWS * p;
-                const u32x4 o = *reinterpret_cast<const u32x4*>(&tile[at(q, v16 * E)]);
-                tstore(mem_tile + s_off[q] + v16 * E, o, a.aligned_stores);
-            }
-        }
-        return;
-    }
-    // Narrow extent (fewer than a tile's worth of q or of c): element by element through the same
-    // LDS layout.  Loads are unconditional, from a clamped address, so that a batch of them is
-    // in flight at once; only the stores are predicated.
-    constexpr int BATCH = TQ * TC / THREADS < 8 ? TQ * TC / THREADS : 8;
-    static_assert((TQ * TC) % (THREADS * BATCH) == 0, "whole batches");
-    if constexpr (PACK) {
-        for (int i0 = threadIdx.x; i0 < TQ * TC; i0 += THREADS * BATCH) {
-            T v[BATCH];
-#pragma unroll
-            for (int k = 0; k < BATCH; ++k) {
-                const int i = i0 + k * THREADS, q = i / TC, c = i % TC;
-                const bool ok = q0 + q < a.Q && c0 + c < a.Sc;
-                v[k] = mem_tile[ok ? s_off[q] + c : s_off[0]];
+                const int cc = cc0 + CSTEP * p;
+                d[p].v = tload<STREAM>(packed_tile + (uint64_t)cc * a.Q + qv * E);
             }
 #pragma unroll
-            for (int k = 0; k < BATCH; ++k) {
-                const int i = i0 + k * THREADS;
-                tile[at(i / TC, i % TC)] = v[k];
+            for (int p = 0; p < PASSES; ++p) {
+                const int cc = cc0 + CSTEP * p;
+#pragma unroll
+                for (int j = 0; j < E; ++j) tile[at(qv * E + j, cc)] = d[p].e[j];
             }
         }
         __syncthreads();
-        for (int i = threadIdx.x; i < TQ * TC; i += THREADS) {
-            const int c = i / TQ, q = i % TQ;
-            if (q0 + q < a.Q && c0 + c < a.Sc) packed_tile[(uint64_t)c * a.Q + q] = tile[at(q, c)];
-        }
-    } else {
-        for (int i0 = threadIdx.x; i0 < TQ * TC; i0 += THREADS * BATCH) {
-            T v[BATCH];
 #pragma unroll
-            for (int k = 0; k < BATCH; ++k) {
-                const int i = i0 + k * THREADS, c = i / TQ, q = i % TQ;
-                const bool ok = q0 + q < a.Q && c0 + c < a.Sc;
-                v[k] = packed_tile[ok ? (uint64_t)c * a.Q + q : 0];
-            }
-#pragma unroll
-            for (int k = 0; k < BATCH; ++k) {
-                const int i = i0 + k * THREADS;
-                tile[at(i % TQ, i / TQ)] = v[k];
-            }
-        }
-        __syncthreads();
-        for (int i = threadIdx.x; i < TQ * TC; i += THREADS) {
-            const int q = i / TC, c = i % TC;
-            if (q0 + q < a.Q && c0 + c < a.Sc) mem_tile[s_off[q] + c] = tile[at(q, c)];
+        for (int p = 0; p < PASSES; ++p) {
+            const int q = r16 + ROWS * p;
+            const u32x4 o = *reinterpret_cast<const u32x4*>(&tile[at(q, v16 * E)]);
+            tstore(mem_tile + s_off[q] + v16 * E, o, a.aligned_stores);
         }
     }
 }
@@ -816,6 +764,15 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // worth it only when both sides have something to coalesce
     if (Sc < 8 || Q < 8 || Sc >= kFastDivLimit) return false;
     const bool vec = unit <= 8;  // 16-byte elements already move 16 bytes per lane in the scalar kernel
+    // Short sides and small views have tiles of their own (narrow_transpose_kernels.hip).  A variant forced through the
+    // tuning aids applies to every view the kernels of this file can take, i.e. from one tile on along both sides.
+    const bool whole_tiles = Sc * unit >= 256 && Q * unit >= 256;
+    const bool forced = tuning_env("MONARCH_HIP_TRANSPOSE_LINES") || tuning_env("MONARCH_HIP_TRANSPOSE_WALK") ||
+                        tuning_env("MONARCH_HIP_TRANSPOSE_POLICY");
+    if (vec && !(forced && whole_tiles) &&
+        try_narrow_transpose<PACK>(base, packed, c, cd, nbatch, (uint32_t)Q, unit, stream, rc))
+        return true;
+    if (vec && !whole_tiles) return false;  // sides of fewer than 16 bytes
     // 4-byte elements whose rows are 512-byte aligned on both sides and whose extents are whole tiles get 128 x 128
     // tiles (512-byte runs, 64 KiB of LDS, 1024 lanes): 8192^2 fp32 0.65 -> 0.70 of peak.  Rows that are not aligned
     // that way do better with the 64 x 64 tile (8200^2: 0.61 against 0.57).

@@ -799,3 +799,34 @@ def test_stream_send_tensor_semantics():
         stream_send_tensor(world, 0, None, None, f)
     fr, to = Slice(offset=0, sizes=[2], strides=[1]), Slice(offset=2, sizes=[2], strides=[1])
     assert route(fr, to, 3) == (1, None)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.int16, torch.int32, torch.int64])
+def test_transposes_with_a_short_side_and_small_ones(dtype):
+    # the tiles of narrow_transpose_kernels.hip: sides of one vector, a vector and a bit, and the edges of every tile length
+    # (64, 128, 256, 512 bytes) on either side, long sides that are no whole tiles, batches, a packed side spanning two
+    # dimensions, views that start inside a row; the larger ones take the tiles used when there are many
+    es = torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator().manual_seed(33)
+    info = torch.iinfo(dtype)
+    short = sorted({max(16 // es, 8) + 1, 16} | {b // es + d for b in (64, 128, 160, 256, 272, 384, 512) for d in (-1, 0, 1)})
+    cases = [((2 * 128 // es + 5, n), lambda x: x.t()) for n in short] + [((n, 2 * 128 // es + 5), lambda x: x.t()) for n in short]
+    cases += [((3, 70, 40), lambda x: x.transpose(1, 2)), ((2, 5, 33, 24), lambda x: x.permute(0, 3, 1, 2)[:, 1:]),
+              ((4, 65, 300), lambda x: x[:, 1:, 7:40].transpose(1, 2)), ((1029, 700), lambda x: x[:, 3:].t())]
+    many = 70_000_000 // es
+    cases += [((many // (n * es) // es, n), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
+    cases += [((n, many // (n * es) // es + 1), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
+    for shape, view_of in cases:
+        host = torch.randint(info.min, info.max, shape, dtype=dtype, generator=g)
+        dev = host.to(DEV)
+        view, hview = view_of(dev), view_of(host)
+        s = Slice.of_tensor(view)
+        out = staging.pack(view, s)
+        sync()
+        assert torch.equal(out.cpu(), hview.contiguous().flatten()), (shape, dtype)
+        back = torch.full_like(dev, 7)
+        staging.unpack(back, s, out)
+        sync()
+        ref = torch.full_like(host, 7)
+        view_of(ref).copy_(hview)
+        assert torch.equal(back.cpu(), ref), (shape, dtype)
