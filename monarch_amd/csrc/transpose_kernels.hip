@@ -881,6 +881,13 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // the kernel with line-aligned windows re-reads rows of the tile before it along the written rows, and finds them
     // in L2 sooner with smaller blocks: 4-byte elements 8200^2 0.66 / 0.65 -> 0.68 / 0.67, 8-byte 0.67 -> 0.69
     if (lines && unit >= 4) a.group = 4;
+    // Where few tiles lie along one side, whole blocks are mostly padding, workgroups that are launched and retired without a
+    // tile: blocks are halved while those are more than 0.7 of the tiles (fp32 [65536, 256], 4 tiles by 1024, blocks of
+    // 16 / 4: 32.3 / 21.5 us, f64 [65536, 128] 37.5 / 21.4).  Less padding costs less than smaller blocks do (fp32 [144, 116508],
+    // 3 tiles, blocks of 4 / 1: 24.3 / 31.3 us; bf16 [640, 52428], 5 tiles, blocks of 8 / 2: 22.4 / 24.7).
+    const uint64_t ntiles2d = (uint64_t)a.ctiles * a.qtiles;
+    auto walked = [&](uint32_t g) { return (uint64_t)((a.ctiles + g - 1) / g) * ((a.qtiles + g - 1) / g) * g * g; };
+    while (a.group > 1 && 10 * walked(a.group) > 17 * ntiles2d) a.group /= 2;
     a.cgroups = (a.ctiles + a.group - 1) / a.group;
     bool stream_loads = false;
     if (vec) {
