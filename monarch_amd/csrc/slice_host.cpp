@@ -16,11 +16,11 @@ namespace mhip {
 int validate_slice(const uint64_t* sizes, uint32_t nsizes, const uint64_t* strides, uint32_t nstrides) {
     if (nsizes != nstrides) return MHIP_ERR_INVALID_DIMS;
     if (nsizes > MHIP_MAX_DIMS) return MHIP_ERR_INVALID_ARGUMENT;
-    std::vector<std::pair<uint64_t, uint64_t>> dims(nsizes);  // (stride, size)
+    std::pair<uint64_t, uint64_t> dims[MHIP_MAX_DIMS];  // (stride, size)
     for (uint32_t k = 0; k < nsizes; ++k) dims[k] = {strides[k], sizes[k]};
-    std::sort(dims.begin(), dims.end());
+    std::sort(dims, dims + nsizes);
     uint64_t space = 1;  // stride * size of the previous (smaller-stride) dimension
-    for (size_t k = 0; k < dims.size(); ++k) {
+    for (uint32_t k = 0; k < nsizes; ++k) {
         const auto [stride, size] = dims[k];
         if (k > 0) {
             const auto [pstride, psize] = dims[k - 1];

@@ -132,12 +132,13 @@ class FlatBucket:
         _torch.require_contiguous(flat)
         if flat.numel() != self.total or flat.device != self.device:
             raise ValueError(f"flat buffer must hold {self.total} elements on {self.device}")
+        size, device = flat.element_size(), self.device
         for t in outs:
             _torch.require_contiguous(t)
-            if t.element_size() != flat.element_size():
+            if t.element_size() != size:
                 raise ValueError("element size mismatch")
-            if t.device != self.device:
-                raise ValueError(f"output is on {t.device}, the bucket on {self.device}")
+            if t.device != device:
+                raise ValueError(f"output is on {t.device}, the bucket on {device}")
         ptrs = self.pointer_table(outs)
         check(lib().mhip_flat_unpack(ptrs.data_ptr(), flat.data_ptr(), self.d_offsets.data_ptr(), len(self.sizes),
                                      self.total, flat.element_size(), self._index_ptr(indexed, stream),

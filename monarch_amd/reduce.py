@@ -136,15 +136,15 @@ def check_reduce_args(mesh_names: Sequence[str], mesh_sizes: Dict[str, int], sha
 def all_reduce(out: torch.Tensor, group: Sequence[torch.Tensor], op: ReduceOp, stream=None) -> None:
     """Local combine of ``Communicator::all_reduce`` (torch-sys-cuda/src/nccl.rs:464-489):
     ``out = op(group)``; ``out`` may be one of the group's tensors (the in-place form)."""
-    for t in (out, *group):
-        _torch.require_contiguous(t)
-    code = _torch.dtype_code(out.dtype)
+    _torch.require_all_contiguous((out, *group))
+    dtype, numel = out.dtype, out.numel()
+    code = _torch.dtype_code(dtype)
     for t in group:
-        if t.dtype != out.dtype:
+        if t.dtype != dtype:
             raise MhipError(_lib.ERR_TYPE_MISMATCH, "output tensor must have the same type as input tensor")
-        if t.numel() != out.numel():
+        if t.numel() != numel:
             raise MhipError(_lib.ERR_INPUT_SIZE_MISMATCH, "all group members must hold the same number of elements")
-    check(lib().mhip_reduce(out.data_ptr(), ptr_array([t.data_ptr() for t in group]), len(group), out.numel(),
+    check(lib().mhip_reduce(out.data_ptr(), ptr_array([t.data_ptr() for t in group]), len(group), numel,
                             code, int(op), _torch.stream_handle(stream)))
 
 
@@ -152,9 +152,7 @@ def reduce_scatter_tensor(out: torch.Tensor, group: Sequence[torch.Tensor], rank
                           stream=None) -> None:
     """Local combine of ``Communicator::reduce_scatter_tensor`` (nccl.rs:661-703) for member
     ``rank``: ``out = op_g group[g].flat[rank*c : (rank+1)*c]`` with ``c = out.numel()``."""
-    _torch.require_contiguous(out)
-    for t in group:
-        _torch.require_contiguous(t)
+    _torch.require_all_contiguous((out, *group))
     n = len(group)
     for t in group:
         if t.dtype != out.dtype:
@@ -174,8 +172,7 @@ def reduce_scatter_views(outs: Sequence[torch.Tensor], out_views: Sequence[Slice
                          in_view: Optional[Slice], op: ReduceOp, stream=None) -> None:
     """Reduce ``group`` (each read through ``in_view``) and scatter the result through
     ``out_views`` (Slices of the reduced tensor) into contiguous ``outs`` in one pass."""
-    for t in outs:
-        _torch.require_contiguous(t)
+    _torch.require_all_contiguous(outs)
     for t in group:
         _torch.require_device(t)
     code = _torch.dtype_code(outs[0].dtype)
