@@ -8,8 +8,8 @@
 //   slice_copy_ragged_kernel  rows of at least a chunk that are not whole chunks: a chunk
 //                             straddling a row boundary moves as two overlapping vectors
 //   slice_unpack_lines_kernel unpacks of such rows from 256 bytes on: whole cache lines of the written side
-//   slice_gather_kernel       runs shorter than (a few) chunks: the chunk's units are
-//                             gathered / scattered one by one
+//   slice_units_kernel        runs shorter than (a few) chunks: the strided side unit by unit, consecutive lanes on
+//                             consecutive units (slice_gather_kernel from 2^31 units on)
 //   contiguous_copy_kernel    one run of any alignment: rows on the destination's 1 KiB boundaries
 // (views whose memory-contiguous dimension is not the innermost one go to the LDS-tiled
 // transposing kernels instead).  The host picks the form per launch from the canonical slice.
@@ -43,6 +43,7 @@ struct PackArgs {
     uint64_t nrows;              //   rows per view
     uint64_t per_xcd;            // copies whose pieces share cache lines: workgroups in each XCD's contiguous
     uint64_t nwg;                //   share of the nwg workgroups (0: workgroup i takes tile i)
+    uint32_t stream_units;       // slice_units_kernel: non-temporal accesses to the strided side
     uint32_t stream_stores;      // slice_copy_kernel unpacking 16-byte units, slice_unpack_lines_kernel: non-temporal
                                  //   instead of write-through stores
     DimsArg dims;
@@ -340,17 +341,96 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
     }
 }
 
-// Views whose contiguous runs are shorter than a chunk (element-strided selections such as
-// x[:, ::2], rows of a few bytes): a lane still owns whole 16-byte chunks of the packed side,
-// which it moves with one aligned 128-bit access, and gathers (pack) or scatters (unpack) the
-// chunk's units one by one on the strided side.  All unit loads of a lane are issued before
-// the first use and none is predicated.  Unit addresses come from one full decode per chunk
-// followed by an odometer over the run and the innermost dimension outside it; a full decode
-// is repeated only when that dimension wraps.  Strided-side accesses are NOT non-temporal:
-// the lanes of a wavefront return to the same cache lines for every unit of their chunks.
+// Views whose contiguous runs are shorter than (a few) chunks: element-strided selections such as x[:, ::2], rows of a
+// few bytes.  The packed side moves as aligned 16-byte vectors, the strided side unit by unit, and consecutive lanes take
+// CONSECUTIVE units there: one access of a wavefront touches the 64 * stride bytes that lie side by side in memory, each
+// line once.  The two sides' orders meet in 1 KiB of LDS (a single-wavefront workgroup; both LDS orders are linear).
+//
+// Bound by the lines of the strided side: all of them cross HBM, and an unpack, which fills them in part, has them read
+// as well as written.  In the order of the kernel this one replaces a lane owned the 16 bytes of one packed vector on the
+// strided side as well, so that every access of a wavefront touched 16 times (1-byte units) to 4 times the lines.  Pack /
+// unpack of x[:, ::k] over [8192, k * 4096], before -> now, us (in brackets what the lines need at 5.5 TB/s): u8 k=2
+// 59.8 / 84.9 -> 26.6 / 31.9 [18 / 31], k=4 60.5 / 154 -> 31.1 / 56.5 [30 / 55]; bf16 k=2 60.6 / 87.1 -> 36.0 / 60.0
+// [37 / 61], k=4 61.2 / 156 -> 54 / 110 [61 / 110]; f32 k=2 68.0 / 126 -> 60.7 / 118, k=4 111 / 237 -> 108 / 222; f64 k=8
+// 209 / 460 -> 199 / 451.
+// Element-strided views that span 32 MiB or more stream (non-temporal accesses: u8 k=2 packing 27.2 -> 26.6, f32 66 ->
+// 61, unpacking 33.9 -> 31.9 and 123 -> 118); smaller ones (u8 [3001, 7108] k=4, 21 MB: 6.3 / 9.4 us, 7.7 / 11.7 streamed)
+// and rows of several units, whose lines several accesses share (rows of 33 floats unpacking 6.7, 10.8 streamed), keep
+// to the cache.  Rows of several units of a single view also take XCD-contiguous shares (rows of 33 floats unpacking
+// 6.7 -> 6.1); element-strided ones do not (u8 k=2 26.6 -> 28.5).
+template <int U, bool PACK, int NDIM, bool STREAM>
+__global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
+    using T = typename UnitType<U>::type;
+    using M = typename UnitType<U>::mem;  // the strided side may be less aligned than the unit
+    constexpr int VU = 16 / U;
+    __shared__ __attribute__((aligned(16))) T buf[kPackThreads * VU];
+    uint64_t wg = a.wg0 + blockIdx.x;
+    if (a.per_xcd != 0) {  // each XCD on a contiguous share: see the note above copy_views
+        wg = (wg & 7) * a.per_xcd + (wg >> 3);
+        if (wg >= a.nwg) return;
+    }
+    const uint64_t tile = wg / a.nviews;
+    const uint32_t v = (uint32_t)(wg % a.nviews);
+    char* __restrict__ packed = a.packed[v];
+    M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
+    const uint32_t total = (uint32_t)a.total;
+    const uint32_t pos0 = (uint32_t)tile * (kPackThreads * VU);  // position of the tile, counted from the aligned-down start
+    const uint32_t mine = pos0 + threadIdx.x * VU;               // and of this lane's vector of the packed side
+    const bool full = mine >= a.shift && mine + VU - a.shift <= total;
+    uint64_t loc[VU];
+    bool live[VU];
+#pragma unroll
+    for (int k = 0; k < VU; ++k) {
+        const uint32_t pos = pos0 + k * kPackThreads + threadIdx.x;
+        live[k] = pos >= a.shift && pos - a.shift < total;
+        uint64_t col;
+        loc[k] = decode<false, NDIM>(a.dims, live[k] ? pos - a.shift : 0u, &col);
+    }
+    if constexpr (PACK) {
+        T d[VU];
+#pragma unroll
+        for (int k = 0; k < VU; ++k) {
+            if constexpr (STREAM) d[k] = __builtin_nontemporal_load(strided + loc[k]);
+            else d[k] = strided[loc[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < VU; ++k) buf[k * kPackThreads + threadIdx.x] = d[k];
+        __syncthreads();
+        if (full) {
+            store16_aligned(packed + (uint64_t)(mine - a.shift) * U, *reinterpret_cast<const uint4*>(buf + threadIdx.x * VU));
+        } else {
+            for (int j = 0; j < VU; ++j)
+                if (mine + j >= a.shift && mine + j - a.shift < total)
+                    *reinterpret_cast<T*>(packed + (uint64_t)(mine + j - a.shift) * U) = buf[threadIdx.x * VU + j];
+        }
+    } else {
+        if (full) {
+            *reinterpret_cast<uint4*>(buf + threadIdx.x * VU) = load16_aligned(packed + (uint64_t)(mine - a.shift) * U);
+        } else {
+            for (int j = 0; j < VU; ++j)
+                if (mine + j >= a.shift && mine + j - a.shift < total)
+                    buf[threadIdx.x * VU + j] = *reinterpret_cast<const T*>(packed + (uint64_t)(mine + j - a.shift) * U);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < VU; ++k) {
+            if (live[k]) {
+                if constexpr (STREAM) __builtin_nontemporal_store(buf[k * kPackThreads + threadIdx.x], strided + loc[k]);
+                else strided[loc[k]] = buf[k * kPackThreads + threadIdx.x];
+            }
+        }
+    }
+}
+
+// The same views from 2^31 units on, where an index takes 64-bit divisions: too many for one per unit.  A lane owns whole
+// 16-byte chunks of the packed side and gathers (pack) or scatters (unpack) the chunk's units one by one on the strided
+// side.  All unit loads of a lane are issued before the first use and none is predicated.  Unit addresses come from one
+// full decode per chunk followed by an odometer over the run and the innermost dimension outside it; a full decode is
+// repeated only when that dimension wraps.  Strided-side accesses are NOT non-temporal: the lanes of a wavefront return
+// to the same cache lines for every unit of their chunks.
 constexpr int kGatherUnroll = 1;
 
-template <int U, bool PACK, bool WIDE, int NDIM>
+template <int U, bool PACK>
 __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) {
     using T = typename UnitType<U>::type;
     constexpr int VU = 16 / U;
@@ -362,7 +442,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
     using M = typename UnitType<U>::mem;  // the strided side may be less aligned than the unit
     M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
     const uint64_t c0 = tile * (kPackThreads * UN) + threadIdx.x;
-    const int nd = NDIM >= 0 ? NDIM : a.dims.ndim;
+    const int nd = a.dims.ndim;
     const uint64_t run = a.dims.run;
     const uint64_t size_last = a.dims.size[nd - 1];
     const uint64_t step_last = a.dims.stride[nd - 1] - run;  // from one past a run's end to the start of the next run
@@ -379,16 +459,8 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
         edge[i] = c < a.nchunks && !full[i];
         if (full[i]) {
             uint64_t col;
-            uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
-            uint64_t ilast;  // index along the innermost dimension outside the run
-            if constexpr (WIDE) {
-                ilast = ((first - col) / run) % size_last;
-            } else {
-                uint32_t r32, c32, q32, i32;
-                a.dims.run_div.divmod((uint32_t)first, r32, c32);
-                a.dims.size_div[nd - 1].divmod(r32, q32, i32);
-                ilast = i32;
-            }
+            uint64_t loc = decode<true, -1>(a.dims, first, &col);
+            uint64_t ilast = ((first - col) / run) % size_last;  // index along the innermost dimension outside the run
             off[i][0] = loc;
 #pragma unroll
             for (int j = 1; j < VU; ++j) {
@@ -399,7 +471,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
                     ++ilast;
                     loc += step_last;
                     if (ilast == size_last) {
-                        loc = decode<WIDE, NDIM>(a.dims, first + j, &col);
+                        loc = decode<true, -1>(a.dims, first + j, &col);
                         ilast = 0;
                     }
                 }
@@ -439,7 +511,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
     // ragged first and last chunk of the view: unit by unit
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
-        if (edge[i]) move_chunk_by_units<U, PACK, WIDE, NDIM>(a, reinterpret_cast<char*>(strided), packed, c0 + (uint64_t)i * kPackThreads);
+        if (edge[i]) move_chunk_by_units<U, PACK, true, -1>(a, reinterpret_cast<char*>(strided), packed, c0 + (uint64_t)i * kPackThreads);
     }
 }
 
@@ -724,6 +796,16 @@ static void launch_whole_chunks(bool wide, bool large, int ndim, dim3 grid, hipS
     else launch_whole_chunks_u<U, PACK, kUnrollSmall>(wide, ndim, grid, stream, a);
 }
 
+template <int U, bool PACK, bool STREAM>
+static void launch_units(int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
+    const dim3 block(kPackThreads);
+    switch (ndim) {
+        case 1: MHIP_LAUNCH((slice_units_kernel<U, PACK, 1, STREAM>), grid, block, 0, stream, a); break;
+        case 2: MHIP_LAUNCH((slice_units_kernel<U, PACK, 2, STREAM>), grid, block, 0, stream, a); break;
+        default: MHIP_LAUNCH((slice_units_kernel<U, PACK, -1, STREAM>), grid, block, 0, stream, a); break;
+    }
+}
+
 template <int U, bool PACK>
 static void launch_slice_copy_u(bool wide, bool large, CopyForm form, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
     const dim3 block(kPackThreads);
@@ -744,14 +826,11 @@ static void launch_slice_copy_u(bool wide, bool large, CopyForm form, int ndim, 
     if constexpr (U < 16) {
         if (form == kShortRuns) {
             if (wide) {
-                MHIP_LAUNCH((slice_gather_kernel<U, PACK, true, -1>), grid, block, 0, stream, a);
+                MHIP_LAUNCH((slice_gather_kernel<U, PACK>), grid, block, 0, stream, a);
                 return;
             }
-            switch (ndim) {
-                case 1: MHIP_LAUNCH((slice_gather_kernel<U, PACK, false, 1>), grid, block, 0, stream, a); break;
-                case 2: MHIP_LAUNCH((slice_gather_kernel<U, PACK, false, 2>), grid, block, 0, stream, a); break;
-                default: MHIP_LAUNCH((slice_gather_kernel<U, PACK, false, -1>), grid, block, 0, stream, a); break;
-            }
+            if (a.stream_units) launch_units<U, PACK, true>(ndim, grid, stream, a);
+            else launch_units<U, PACK, false>(ndim, grid, stream, a);
             return;
         }
         if (form == kRaggedRows) {
@@ -808,8 +887,7 @@ static int copy_deep_view(char* base, char* packed, const mhip_slice_t& s, uint3
 // 0:1784 0.69 -> 0.73, pitch 14335 0.68 -> 0.73, fp32 rows of 1024 at pitch 8191 0.70 -> 0.75.  Rows of whole lines
 // measure the same either way or better (64 of 256 fp32 columns 0.57 -> 0.63; bf16 columns 0:1792 0.746 both ways), so
 // every single-view pack of whole chunks takes the shares (the eight column blocks of one tensor in one launch, where
-// the view index already pins each view to one XCD, lose with them: 0.78 -> 0.68).  The gathering form does not (bf16 rows of 1790: 0.69 -> 0.59,
-// though fp32 rows of 255 gain 0.03).  The two-vector form and the line-by-line unpack take them for rows of 6 KiB and
+// the view index already pins each view to one XCD, lose with them: 0.78 -> 0.68).  For short runs see slice_units_kernel.  The two-vector form and the line-by-line unpack take them for rows of 6 KiB and
 // more (bf16 [16384, 14336], columns c:c+7166, packing 0.75 -> 0.78, unpacking 0.72 -> 0.755; rows of 7160 bytes +0.02 /
 // +0.03 to +0.10; rows of 3580 bytes -0.02 either way, so shorter rows keep the plain mapping).
 //
@@ -825,6 +903,7 @@ static int copy_deep_view(char* base, char* packed, const mhip_slice_t& s, uint3
 // of a 117 MB tensor: 0.794 against 0.777).
 constexpr uint64_t kSharesFromRowBytes = 6144;
 constexpr uint64_t kStreamUnpackFromBytes = 96ull << 20;
+constexpr uint64_t kStreamUnitsFromSpan = 32ull << 20;  // see slice_units_kernel
 template <bool PACK>
 static int copy_views(char* base, char* const* packed, const mhip_slice_t* views, uint32_t nviews,
                       uint32_t elem_size, hipStream_t stream) {
@@ -901,15 +980,17 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
         }
         CopyForm form = kWholeChunks;
         if (unit < 16 && first.ndim >= 1 && (first.run % vu != 0 || a.shift != 0)) {
-            // Rows that are not whole chunks.  Measured on 8192^2 matrices with rows of r-1 of r elements:
-            // gathering 4-byte units into a chunk streams at 0.77 of peak whatever the row length (the
-            // two-vector form reaches 0.64-0.75), gathering 2-byte units at 0.50 (two-vector form: 0.50 at
-            // 254-byte rows, 0.58 at 510, 0.69 at 2046); scattering units is slower than either beyond
-            // 256-byte rows (fp32: 0.46-0.49 against 0.61-0.73).
-            uint64_t gather_below = 16 * vu;                 // row length in units
-            if (unit == 1) gather_below = 4 * vu;
-            if (PACK && unit >= 4) gather_below = 256 * vu;  // rows under 4 KiB; longer ones: 0.72-0.75 two-vector vs 0.69-0.74
-            if (first.run < gather_below && first.total >= 2 * vu) form = kShortRuns;
+            // Rows that are not whole chunks: unit by unit below a length, above it as two vectors or line by line.  Where
+            // the line lies (rows at twice their length, 35 to 126 MB moved; unit by unit / the other form, us).  Packing:
+            // 1-byte units 263 B 10.1 / 12.6, 519 B 18.5 / 19.1, 1031 B 32.3 / 30.9; 2-byte units 262 B 8.8 / 12.1, 1030 B
+            // 25.4 / 26.4, 1544 B 25.6 / 24.9, 3080 B 26.2 / 24.2, but two or eight views in one launch of 1222 B 8.4 / 10.4
+            // and 29 / 32, of 1790 B 11.2 / 13.1 and 42 / 42.7; 4-byte units 260 B 8.5 / 11.8, 2052 B 23.6 / 24.4, 4104 B
+            // 24.6 / 24.4.  Unpacking: 1-byte units 199 B 11.6 / 12.4, 263 B 13.4 / 10.9; 2-byte units 198 B 9.1 / 12.5, 262 B 10.6 / 10.8, 398 B 14.1 / 13.0; 4-byte units 260 B 9.1 /
+            // 9.3, 516 B 17.1 / 15.5.  From 2^31 units on slice_gather_kernel takes the short rows, which loses earlier.
+            uint64_t units_below = (PACK ? (unit == 1 ? 512 : unit > 2 ? 4096 : nbatch == 1 ? 1280 : 2048) : 256) / unit;  // row length in units
+            if (!fits32 && unit == 1) units_below = 64;
+            if (!fits32 && unit == 2) units_below = 128;
+            if (first.run < units_below && first.total >= 2 * vu) form = kShortRuns;
             else if (first.run >= vu) form = kRaggedRows;
         }
         // Unpacking ragged rows of 256 bytes and more line by line of the written side (see slice_unpack_lines_kernel).
@@ -953,18 +1034,23 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
             }
         }
         const bool large = a.nchunks >= kLargeCopyChunks;
-        const uint64_t per_block = (uint64_t)kPackThreads * (form == kRaggedRows ? kRaggedUnroll : form == kShortRuns ? kGatherUnroll : large ? kUnrollLarge : kUnrollSmall);
+        const uint64_t per_block = (uint64_t)kPackThreads * (form == kRaggedRows ? kRaggedUnroll : form == kShortRuns ? 1 : large ? kUnrollLarge : kUnrollSmall);
         uint64_t blocks = (a.nchunks + per_block - 1) / per_block;
         if (form == kUnpackLines) blocks = line_blocks;  // eight lanes per line of every row
         a.nviews = nbatch;
         uint64_t nwg = blocks * nbatch;
+        if (form == kShortRuns && first.run == 1)
+            a.stream_units = nbatch * first.total * first.dims[first.ndim - 1].stride * unit >= kStreamUnitsFromSpan;
         // which single-view copies take XCD-contiguous shares, and how an unpack of 16-byte units stores: see the
         // note above copy_views
         bool shares = false;
         if (nbatch == 1) {
             const uint64_t run_bytes = first.run * unit;
+            const bool short_rows = form == kShortRuns && !wide && first.run > 1;
             if (PACK) {
-                shares = form == kWholeChunks || (form == kRaggedRows && run_bytes >= kSharesFromRowBytes);
+                shares = form == kWholeChunks || (form == kRaggedRows && run_bytes >= kSharesFromRowBytes) || short_rows;
+            } else if (form == kShortRuns) {
+                shares = short_rows;
             } else if (form == kUnpackLines) {
                 shares = run_bytes >= kSharesFromRowBytes;
             } else if (form == kWholeChunks) {
