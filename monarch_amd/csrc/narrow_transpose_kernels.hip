@@ -236,7 +236,9 @@ template <typename T, bool PACK>
 static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     constexpr uint32_t ES = sizeof(T);
     const uint64_t ib = (uint64_t)(PACK ? a.Q : a.Sc) * ES, jb = (uint64_t)(PACK ? a.Sc : a.Q) * ES;
-    if (nbatch * ib * jb / ES >= (16ull << 20)) {  // one of the sides is at most 512 bytes then
+    if (nbatch * ib * jb / ES >= (16ull << 20)) {  // one of the sides is at most 512 bytes then, or elements are bytes
+        if constexpr (ES == 1)
+            if (ib > 512 && jb > 512) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
         const bool short_j = jb <= ib;
         uint32_t n = narrow_tile_bytes(short_j ? jb : ib);
         if (ES == 8 && n == 64) n = 128;  // a read row of 64 bytes would be fewer than 16 elements
@@ -259,14 +261,18 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
 // Takes the view when one of its sides is at most 512 bytes long (bf16 67 MB, sides of 512 / 768 bytes, pack: 23.8 / 27 us
 // here against 24.0 / 25.4 with the long tiles; rows that are not whole lines 26.6 against 34.3, and 27 against 25.4) or
 // when it has at most 12 MiB (bf16 2048^2 3.6 us against 4.0, 2000 x 3000 6.9 against 8.4, u8 2000 x 3000 4.4 against
-// 6.2; fp32 2000 x 3000, 24 MB, 11 against 10.4), both sides holding at least one vector.
+// 6.2; fp32 2000 x 3000, 24 MB, 11 against 10.4), both sides holding at least one vector.  Byte matrices whose rows are not
+// whole cache lines are taken up to 40 MiB, in tiles of 256 x 256: the strips of the other file need more of them to fill
+// the part, its fixed tiles share lines (3001 x 7001, pack / unpack, 16.2 / 15.2 us -> 13.6 / 14.0; 5000^2 17.0 / 15.9 ->
+// 14.9 / 14.3; 5600^2 18.3 / 17.8 -> 13.7 / 13.9; 6001 x 6403 26.2 / 25.6 -> 22.2 / 23.1; but 7000^2, 47 MiB, 30.3 / 28.3
+// -> 31.5 / 31.1, and 4096^2, whole lines, 7.2 -> 7.7).
 template <bool PACK>
 bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd, uint64_t nbatch, uint32_t Q, uint32_t unit,
                           hipStream_t stream, int* rc) {
     const uint64_t Sc = c.dims[cd].size, bytes = nbatch * Sc * Q * unit;
     const uint64_t short_side = (Sc < Q ? Sc : Q) * unit;
     if (unit > 8 || short_side < 16) return false;
-    if (short_side > 512 && bytes > (12ull << 20)) return false;
+    if (short_side > 512 && bytes > (unit == 1 ? 40ull << 20 : 12ull << 20)) return false;
     NarrowArgs a{};
     uint64_t written = PACK ? (uint64_t)(uintptr_t)packed | (uint64_t)Q * unit : (uint64_t)(uintptr_t)(base + c.offset * unit);
     for (int k = 0; k < c.ndim; ++k) {
@@ -280,6 +286,12 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
             a.outer_stride[a.n_outer++] = stride;
         }
         if (!PACK) written |= stride;
+    }
+    if (short_side > 512 && bytes > (12ull << 20)) {  // bytes, see above
+        uint64_t rows = (uint64_t)(uintptr_t)packed | Q | (uint64_t)(uintptr_t)(base + c.offset);
+        for (int k = 0; k < c.ndim; ++k)
+            if (k != cd) rows |= c.dims[k].stride;
+        if ((rows & 127u) == 0) return false;
     }
     a.base = base + c.offset * unit;
     a.packed = packed;
