@@ -509,6 +509,13 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
 // The same with n peers' payloads in one pass: every accumulator element crosses HBM once
 // (n + 8 bytes per element instead of 9n).  Peers are added in order, product rounded before
 // each add, so the result has the bits of n single-peer passes.
+// Large buckets are bound by HBM, small ones (one round of wavefronts) by how long a wavefront lives: three dependent
+// table reads, then the data.  So only the codes of peers that exist are loaded (they were loaded four peers at a time,
+// the surplus a repeated peer's), and the first four peers' are on their way before the tables are read.  The registers
+// that takes, 96, are worth more than wavefronts: 5 per SIMD 1122 us, 6 and 7 (which spill) 1199, on 717 M elements and 2
+// peers; half blocks per wavefront 1127 to 1148, quarter blocks 1371 to 1559.  Elements and peers, before -> now, us:
+// 717 M, 2: 1230 -> 1122 (6.4 TB/s); 172 M, 2: 283 -> 261, 8: 451 -> 441; 30 M, 3: 56.3 -> 54.5; 11 M, 8: 33.0 -> 31.8;
+// 4.5 M, 8: 16.4 -> 15.7, 2: 11.8 -> 11.0.
 constexpr int kMaxBucketPeers = 64;
 
 struct BucketPeersArgs {
@@ -518,28 +525,21 @@ struct BucketPeersArgs {
     uint32_t n;
 };
 
-// One full block of all peers: accumulator vectors through load(j) / store(j, r), peers four at a time with all
-// their codes loaded before the first add.
-template <typename Load, typename Store>
-__device__ __forceinline__ void dequant_accumulate_block_peers(const BucketPeersArgs& p, uint64_t b, int lane, Load&& load, Store&& store) {
-    const uint64_t begin = b * kBlock;
-    float v[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint4 r = load(j);
-        v[j][0] = __uint_as_float(r.x); v[j][1] = __uint_as_float(r.y);
-        v[j][2] = __uint_as_float(r.z); v[j][3] = __uint_as_float(r.w);
-    }
-    for (uint32_t r0 = 0; r0 < p.n; r0 += 4) {
-        uint32_t codes[4][4];
-        float s[4];
+// Up to four peers' codes of one full block: step j of a lane is the elements j * 256 + lane * 4 .. + 3.
+struct PeerCodes {
+    uint32_t codes[4][4];
+    float s[4];
+    __device__ __forceinline__ void load(const BucketPeersArgs& p, uint32_t r0, uint64_t b, int lane) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const uint32_t r = r0 + g < p.n ? r0 + g : p.n - 1;  // clamped: surplus loads are unused
-            s[g] = p.scales[r][b];
+            if (r0 + g < p.n) {  // wave-uniform
+                s[g] = p.scales[r0 + g][b];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) codes[g][j] = load4_unaligned(p.q[r] + begin + j * 256 + lane * 4);
+                for (int j = 0; j < 4; ++j) codes[g][j] = load4_unaligned(p.q[r0 + g] + b * kBlock + j * 256 + lane * 4);
+            }
         }
+    }
+    __device__ __forceinline__ void add_to(float (&v)[4][4], const BucketPeersArgs& p, uint32_t r0) const {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             if (r0 + g < p.n) {
@@ -555,31 +555,54 @@ __device__ __forceinline__ void dequant_accumulate_block_peers(const BucketPeers
             }
         }
     }
+};
+
+// One full block of all peers: `c` holds the first four peers' codes, accumulator vectors go through load(j) / store(j, r),
+// the other peers four at a time with all their codes loaded before the first add.
+template <typename Load, typename Store>
+__device__ __forceinline__ void dequant_accumulate_block_peers(const BucketPeersArgs& p, PeerCodes& c, uint64_t b, int lane, Load&& load,
+                                                               Store&& store) {
+    float v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint4 r = load(j);
+        v[j][0] = __uint_as_float(r.x); v[j][1] = __uint_as_float(r.y);
+        v[j][2] = __uint_as_float(r.z); v[j][3] = __uint_as_float(r.w);
+    }
+    c.add_to(v, p, 0);
+    for (uint32_t r0 = 4; r0 < p.n; r0 += 4) {
+        c.load(p, r0, b, lane);
+        c.add_to(v, p, r0);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
         store(j, make_uint4(__float_as_uint(v[j][0]), __float_as_uint(v[j][1]), __float_as_uint(v[j][2]), __float_as_uint(v[j][3])));
 }
 
-__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(7))) void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
+__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(5))) void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
     const BucketArgs& a = p.b;
     const int lane = threadIdx.x & 63;
     const uint64_t wave = (uint64_t)blockIdx.x * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // see fp8_quantize_bucket_kernel
     const uint64_t nwaves = (uint64_t)gridDim.x * (kBucketThreads / 64);
     for (uint64_t b = wave; b < a.nblocks; b += nwaves) {
         const uint64_t begin = b * kBlock;
-        const uint64_t end = begin + kBlock < a.total ? begin + kBlock : a.total;
+        const bool full = begin + kBlock <= a.total;
+        const uint64_t end = full ? begin + kBlock : a.total;
+        // The codes' addresses do not wait for the tables: they are on their way while the block's tensor is looked up.
+        PeerCodes c;
+        if (full) c.load(p, 0, b, lane);
         uint32_t t_lo, t_hi;
         span_tensors(a, begin, end, &t_lo, &t_hi);
-        if (t_lo == t_hi && end - begin == kBlock) {
+        if (full && t_lo == t_hi) {
             float* dst = reinterpret_cast<float*>(a.tensors[t_lo]) + (begin - a.offsets[t_lo]);
-            dequant_accumulate_block_peers(p, b, lane, [&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
+            dequant_accumulate_block_peers(p, c, b, lane, [&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
                                            [&](int j, const uint4& r) { store16_unaligned(dst + j * 256 + lane * 4, r); });
             continue;
         }
-        if (end - begin == kBlock && block_cut_once(a, t_lo, begin)) {
-            const CutBlock c(a, t_lo, begin);
-            dequant_accumulate_block_peers(p, b, lane, [&](int j) { return c.load(j, lane); },
-                                           [&](int j, const uint4& r) { c.store(j, lane, r); });
+        if (full && block_cut_once(a, t_lo, begin)) {
+            const CutBlock cut(a, t_lo, begin);
+            dequant_accumulate_block_peers(p, c, b, lane, [&](int j) { return cut.load(j, lane); },
+                                           [&](int j, const uint4& r) { cut.store(j, lane, r); });
             continue;
         }
         // more than two tensors, or the short last block
