@@ -23,12 +23,6 @@ constexpr int kMaxViews = 16;
 // Lanes per workgroup of the slice copy kernels: single wavefronts stream best (column-block pack 0.767 -> 0.775 of
 // peak, unpack 0.757 -> 0.792 against 256 lanes; ragged and short-run forms equal or better).
 constexpr int kPackThreads = 64;
-// Chunks per lane of slice_copy_kernel, all loads issued before the first store.  Large copies stream
-// fastest with one chunk per lane and many workgroups (8 column blocks of 14 MiB: 0.76 of peak against
-// 0.73 with eight chunks); copies of a few MiB finish sooner with fewer, fatter workgroups.
-constexpr int kUnrollSmall = 4, kUnrollLarge = 1;
-constexpr uint64_t kLargeCopyChunks = 1ull << 19;  // 8 MiB
-
 struct PackArgs {
     char* base;                  // strided tensor
     char* packed[kMaxViews];     // staging buffers, one per view
@@ -37,6 +31,7 @@ struct PackArgs {
     uint64_t nchunks;            // 16-byte chunks per view, including a ragged first one
     uint32_t shift;              // units missing from chunk 0 so that chunk c starts 16-byte aligned
     uint32_t nviews;             // views handled by this launch
+    FastDiv32 nviews_div;
     uint64_t wg0;                // workgroups of this copy launched before this grid
     uint32_t pieces;             // slice_unpack_lines_kernel: cache lines a row can overlap
     FastDiv32 pieces_div;        //   division by it, valid in 32-bit mode
@@ -48,6 +43,24 @@ struct PackArgs {
                                  //   instead of write-through stores
     DimsArg dims;
 };
+
+// The view index is the fastest-varying part of the workgroup id, so that workgroups running side by side work on the
+// same rows of neighbouring views (for column blocks of one tensor: neighbouring segments of the same rows).  No 64-bit
+// division on the way (0.05 us of a small copy's 3).
+__device__ __forceinline__ void tile_and_view(const PackArgs& a, uint64_t wg, uint64_t* tile, uint32_t* v) {
+    if (a.nviews == 1) {
+        *tile = wg;
+        *v = 0;
+    } else if (wg < kFastDivLimit) {
+        uint32_t q, r;
+        a.nviews_div.divmod((uint32_t)wg, q, r);
+        *tile = q;
+        *v = r;
+    } else {
+        *tile = wg / a.nviews;
+        *v = (uint32_t)(wg % a.nviews);
+    }
+}
 
 template <int U, bool PACK>
 __device__ __forceinline__ void move_unit(char* strided, char* packed) {
@@ -75,116 +88,50 @@ __device__ __forceinline__ void move_chunk_by_units(const PackArgs& a, char* str
     }
 }
 
-template <int U, bool PACK, bool WIDE, int NDIM, int kUnroll>
+// One chunk per lane at every size: copies of a few MiB took four before, which leaves most of the 256 CUs without a
+// workgroup (back to back, pack / unpack: 0.5 MiB in rows of 1 KiB 3.04 / 2.92 us -> 2.65 / 2.66, 4 MiB 3.25 / 3.21 -> 2.75 /
+// 2.84, 2 MiB of attention heads 3.17 / 3.10 -> 2.47 / 2.61, 7 MiB in rows of 1200 bytes 4.02 / 4.59 -> 3.55 / 3.66), and at
+// 117 MiB eight chunks per lane reach 0.73 of peak where one reaches 0.76.
+template <int U, bool PACK, bool WIDE, int NDIM>
 __global__ __launch_bounds__(kPackThreads) void slice_copy_kernel(PackArgs a) {
     constexpr int VU = 16 / U;  // units per chunk
-    // The view index is the fastest-varying part of the workgroup id, so that workgroups
-    // running side by side work on the same rows of neighbouring views (for column blocks
-    // of one tensor: neighbouring segments of the same rows).
     uint64_t wg = a.wg0 + blockIdx.x;
     if (a.per_xcd != 0) {  // each XCD on a contiguous share: see the note above copy_views
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    const uint64_t tile = wg / a.nviews;
-    const uint32_t v = (uint32_t)(wg % a.nviews);
+    uint64_t tile;
+    uint32_t v;
+    tile_and_view(a, wg, &tile, &v);
     char* __restrict__ packed = a.packed[v];
     char* __restrict__ strided = a.base + a.offset[v] * U;
-    const uint64_t c0 = tile * (kPackThreads * kUnroll) + threadIdx.x;
-
-    if constexpr (NDIM == 0) {
-        // Contiguous view: when the whole tile of this workgroup lies inside the
-        // buffer (decided on the scalar unit), no per-chunk tests are needed at all.
-        const uint64_t tile_first = tile * (kPackThreads * kUnroll) * VU;
-        const uint64_t tile_end = tile_first + (uint64_t)(kPackThreads * kUnroll) * VU;
-        if (tile_first >= a.shift && tile_end - a.shift <= a.total) {
-            char* __restrict__ p = packed + (c0 * VU - a.shift) * U;
-            char* __restrict__ s = strided + (c0 * VU - a.shift) * U;
-            uint4 d[kUnroll];
-#pragma unroll
-            for (int i = 0; i < kUnroll; ++i) {
-                if constexpr (PACK) d[i] = load16_unaligned(s + (size_t)i * kPackThreads * 16);
-                else d[i] = load16_aligned(p + (size_t)i * kPackThreads * 16);
-            }
-#pragma unroll
-            for (int i = 0; i < kUnroll; ++i) {
-                if constexpr (PACK) store16_writethrough(p + (size_t)i * kPackThreads * 16, d[i]);
-                else store16_unaligned(s + (size_t)i * kPackThreads * 16, d[i]);
+    const uint64_t c = tile * kPackThreads + threadIdx.x;
+    if (c >= a.nchunks) return;
+    const uint64_t tb = c * VU;           // position counted from the aligned-down start
+    const uint64_t first = tb - a.shift;  // first packed unit of the chunk; wraps for a ragged chunk 0, which is not a vector
+    if (tb >= a.shift && first + VU <= a.total) {
+        uint64_t col;
+        const uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
+        if (col + VU <= a.dims.run) {
+            // Stores to 16-byte aligned addresses go out write-through (column blocks of 3584-byte runs: pack 0.77 -> 0.79 of
+            // peak; 128-byte runs of a [B,H,S,D] -> [B,S,H,D] permute: 0.69 -> 0.77); unaligned ones do not
+            // (a row pitch that is only 2-byte aligned: unpack 0.74 -> 0.71), nor do the
+            // flat bucket pack and the fp8 accumulate, which all lose 1-2 points with it.
+            if constexpr (PACK) {
+                store16_writethrough(packed + first * U, load16_unaligned(strided + loc * U));
+            } else {
+                const uint4 data = load16_aligned(packed + first * U);
+                if constexpr (U == 16) {
+                    if (a.stream_stores) store16_unaligned(strided + loc * U, data);  // wave-uniform
+                    else store16_writethrough(strided + loc * U, data);
+                } else {
+                    store16_unaligned(strided + loc * U, data);
+                }
             }
             return;
         }
     }
-
-    uint64_t loc[kUnroll];
-    uint64_t first[kUnroll];  // first packed unit of the chunk (may be "negative": see below)
-    bool vec[kUnroll];
-    bool live[kUnroll];
-#pragma unroll
-    for (int i = 0; i < kUnroll; ++i) {
-        const uint64_t c = c0 + (uint64_t)i * kPackThreads;
-        live[i] = c < a.nchunks;
-        const uint64_t tb = c * VU;  // position counted from the aligned-down start
-        vec[i] = false;
-        first[i] = tb - a.shift;     // wraps for a ragged chunk 0; only used when tb >= shift
-        if (live[i] && tb >= a.shift && first[i] + VU <= a.total) {
-            uint64_t col;
-            loc[i] = decode<WIDE, NDIM>(a.dims, first[i], &col);
-            vec[i] = col + VU <= a.dims.run;
-        }
-    }
-    bool all_vec = true;
-#pragma unroll
-    for (int i = 0; i < kUnroll; ++i) all_vec = all_vec && vec[i];
-    uint4 data[kUnroll];
-    if (all_vec) {
-        // The common case, free of per-chunk predicates: all loads in flight, then all stores.  Stores to
-        // 16-byte aligned addresses go out write-through (column blocks of 3584-byte runs: pack 0.77 -> 0.79 of
-        // peak; 128-byte runs of a [B,H,S,D] -> [B,S,H,D] permute: 0.69 -> 0.77); unaligned ones do not
-        // (a row pitch that is only 2-byte aligned: unpack 0.74 -> 0.71), nor do the gathering form, the
-        // flat bucket pack and the fp8 accumulate, which all lose 1-2 points with it.
-#pragma unroll
-        for (int i = 0; i < kUnroll; ++i) {
-            if constexpr (PACK)
-                data[i] = load16_unaligned(strided + loc[i] * U);
-            else
-                data[i] = load16_aligned(packed + first[i] * U);
-        }
-#pragma unroll
-        for (int i = 0; i < kUnroll; ++i) {
-            if constexpr (PACK)
-                store16_writethrough(packed + first[i] * U, data[i]);
-            else if constexpr (U == 16) {
-                if (a.stream_stores) store16_unaligned(strided + loc[i] * U, data[i]);  // wave-uniform
-                else store16_writethrough(strided + loc[i] * U, data[i]);
-            } else
-                store16_unaligned(strided + loc[i] * U, data[i]);
-        }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < kUnroll; ++i) {
-        if (vec[i]) {
-            if constexpr (PACK)
-                data[i] = load16_unaligned(strided + loc[i] * U);
-            else
-                data[i] = load16_aligned(packed + first[i] * U);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kUnroll; ++i) {
-        if (vec[i]) {
-            if constexpr (PACK)
-                store16_aligned(packed + first[i] * U, data[i]);
-            else
-                store16_unaligned(strided + loc[i] * U, data[i]);
-        }
-    }
-    if constexpr (VU > 1) {
-#pragma unroll
-        for (int i = 0; i < kUnroll; ++i) {
-            if (live[i] && !vec[i]) move_chunk_by_units<U, PACK, WIDE, NDIM>(a, strided, packed, c0 + (uint64_t)i * kPackThreads);
-        }
-    }
+    if constexpr (VU > 1) move_chunk_by_units<U, PACK, WIDE, NDIM>(a, strided, packed, c);
 }
 
 // The same copy for views whose rows are not whole chunks (row length not a multiple of 16
@@ -213,8 +160,9 @@ __global__ __launch_bounds__(kPackThreads) void slice_copy_ragged_kernel(PackArg
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    const uint64_t tile = wg / a.nviews;
-    const uint32_t v = (uint32_t)(wg % a.nviews);
+    uint64_t tile;
+    uint32_t v;
+    tile_and_view(a, wg, &tile, &v);
     char* __restrict__ packed = a.packed[v];
     char* __restrict__ strided = a.base + a.offset[v] * U;
     const uint64_t c0 = tile * (kPackThreads * UN) + threadIdx.x;
@@ -308,8 +256,9 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    const uint64_t tile = wg / a.nviews;
-    const uint32_t v = (uint32_t)(wg % a.nviews);
+    uint64_t tile;
+    uint32_t v;
+    tile_and_view(a, wg, &tile, &v);
     const uint64_t task = tile * (kPackThreads / 8) + (threadIdx.x >> 3);  // one line of one row
     uint64_t r;                                                             // row of the view, in iteration order
     uint32_t line;
@@ -369,8 +318,9 @@ __global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    const uint64_t tile = wg / a.nviews;
-    const uint32_t v = (uint32_t)(wg % a.nviews);
+    uint64_t tile;
+    uint32_t v;
+    tile_and_view(a, wg, &tile, &v);
     char* __restrict__ packed = a.packed[v];
     M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
     const uint32_t total = (uint32_t)a.total;
@@ -436,8 +386,9 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
     constexpr int VU = 16 / U;
     constexpr int UN = kGatherUnroll;
     const uint64_t wg = a.wg0 + blockIdx.x;
-    const uint64_t tile = wg / a.nviews;
-    const uint32_t v = (uint32_t)(wg % a.nviews);
+    uint64_t tile;
+    uint32_t v;
+    tile_and_view(a, wg, &tile, &v);
     char* __restrict__ packed = a.packed[v];
     using M = typename UnitType<U>::mem;  // the strided side may be less aligned than the unit
     M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
@@ -775,25 +726,18 @@ __global__ __launch_bounds__(THREADS) void flat_copy_kernel(FlatArgs a) {
 
 enum CopyForm { kWholeChunks, kRaggedRows, kShortRuns, kUnpackLines };
 
-template <int U, bool PACK, int UNROLL>
-static void launch_whole_chunks_u(bool wide, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
+template <int U, bool PACK>
+static void launch_whole_chunks(bool wide, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
     const dim3 block(kPackThreads);
     if (wide) {
-        MHIP_LAUNCH((slice_copy_kernel<U, PACK, true, -1, UNROLL>), grid, block, 0, stream, a);
+        MHIP_LAUNCH((slice_copy_kernel<U, PACK, true, -1>), grid, block, 0, stream, a);
         return;
     }
     switch (ndim) {  // the common shapes get a decode without loops
-        case 0: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 0, UNROLL>), grid, block, 0, stream, a); break;
-        case 1: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 1, UNROLL>), grid, block, 0, stream, a); break;
-        case 2: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 2, UNROLL>), grid, block, 0, stream, a); break;
-        default: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, -1, UNROLL>), grid, block, 0, stream, a); break;
+        case 1: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 1>), grid, block, 0, stream, a); break;
+        case 2: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 2>), grid, block, 0, stream, a); break;
+        default: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, -1>), grid, block, 0, stream, a); break;
     }
-}
-
-template <int U, bool PACK>
-static void launch_whole_chunks(bool wide, bool large, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
-    if (large) launch_whole_chunks_u<U, PACK, kUnrollLarge>(wide, ndim, grid, stream, a);
-    else launch_whole_chunks_u<U, PACK, kUnrollSmall>(wide, ndim, grid, stream, a);
 }
 
 template <int U, bool PACK, bool STREAM>
@@ -807,7 +751,7 @@ static void launch_units(int ndim, dim3 grid, hipStream_t stream, const PackArgs
 }
 
 template <int U, bool PACK>
-static void launch_slice_copy_u(bool wide, bool large, CopyForm form, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
+static void launch_slice_copy_u(bool wide, CopyForm form, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
     const dim3 block(kPackThreads);
     if (form == kUnpackLines) {
         if constexpr (!PACK) {
@@ -846,17 +790,17 @@ static void launch_slice_copy_u(bool wide, bool large, CopyForm form, int ndim, 
             return;
         }
     }
-    launch_whole_chunks<U, PACK>(wide, large, ndim, grid, stream, a);
+    launch_whole_chunks<U, PACK>(wide, ndim, grid, stream, a);
 }
 
 template <bool PACK>
-static void launch_slice_copy(uint32_t unit, bool wide, bool large, CopyForm form, dim3 grid, hipStream_t stream, const PackArgs& a) {
+static void launch_slice_copy(uint32_t unit, bool wide, CopyForm form, dim3 grid, hipStream_t stream, const PackArgs& a) {
     switch (unit) {
-        case 1: launch_slice_copy_u<1, PACK>(wide, large, form, a.dims.ndim, grid, stream, a); break;
-        case 2: launch_slice_copy_u<2, PACK>(wide, large, form, a.dims.ndim, grid, stream, a); break;
-        case 4: launch_slice_copy_u<4, PACK>(wide, large, form, a.dims.ndim, grid, stream, a); break;
-        case 8: launch_slice_copy_u<8, PACK>(wide, large, form, a.dims.ndim, grid, stream, a); break;
-        default: launch_slice_copy_u<16, PACK>(wide, large, form == kUnpackLines ? kUnpackLines : kWholeChunks, a.dims.ndim, grid, stream, a); break;
+        case 1: launch_slice_copy_u<1, PACK>(wide, form, a.dims.ndim, grid, stream, a); break;
+        case 2: launch_slice_copy_u<2, PACK>(wide, form, a.dims.ndim, grid, stream, a); break;
+        case 4: launch_slice_copy_u<4, PACK>(wide, form, a.dims.ndim, grid, stream, a); break;
+        case 8: launch_slice_copy_u<8, PACK>(wide, form, a.dims.ndim, grid, stream, a); break;
+        default: launch_slice_copy_u<16, PACK>(wide, form == kUnpackLines ? kUnpackLines : kWholeChunks, a.dims.ndim, grid, stream, a); break;
     }
 }
 
@@ -1033,11 +977,11 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
                 a.stream_stores = nbatch * first.total * unit >= kStreamUnpackFromBytes;  // by the bytes the launch writes
             }
         }
-        const bool large = a.nchunks >= kLargeCopyChunks;
-        const uint64_t per_block = (uint64_t)kPackThreads * (form == kRaggedRows ? kRaggedUnroll : form == kShortRuns ? 1 : large ? kUnrollLarge : kUnrollSmall);
+        const uint64_t per_block = (uint64_t)kPackThreads * (form == kRaggedRows ? kRaggedUnroll : 1);
         uint64_t blocks = (a.nchunks + per_block - 1) / per_block;
         if (form == kUnpackLines) blocks = line_blocks;  // eight lanes per line of every row
         a.nviews = nbatch;
+        a.nviews_div = FastDiv32(nbatch);
         uint64_t nwg = blocks * nbatch;
         if (form == kShortRuns && first.run == 1)
             a.stream_units = nbatch * first.total * first.dims[first.ndim - 1].stride * unit >= kStreamUnitsFromSpan;
@@ -1071,7 +1015,7 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
         }
         if (int rc = launch_in_pieces(nwg, kPackThreads, 8, [&](uint64_t wg0, uint32_t count) {
                 a.wg0 = wg0;
-                launch_slice_copy<PACK>(unit, wide, large, form, dim3(count), stream, a);
+                launch_slice_copy<PACK>(unit, wide, form, dim3(count), stream, a);
             }))
             return rc;
         k += nbatch;
