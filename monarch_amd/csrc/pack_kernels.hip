@@ -587,8 +587,10 @@ __global__ __launch_bounds__(THREADS) void flat_copy_kernel(FlatArgs a) {
         if (lo >= a.ntensors) lo = a.ntensors - 1;  // an index built for another bucket must not send loads out of the tables
         while (lo + 1 < a.ntensors && a.offsets[lo + 1] * a.units_per_elem <= u_first) ++lo;
         uint32_t hi = lo;
-        if (lo + 1 < a.ntensors && a.offsets[lo + 1] * a.units_per_elem <= u_last)
-            hi = wave_find_tensor(a.offsets, a.units_per_elem, lo, a.ntensors, u_last);
+        if (lo + 1 < a.ntensors && a.offsets[lo + 1] * a.units_per_elem <= u_last) {
+            if (a.offsets[lo + 2] * a.units_per_elem > u_last) hi = lo + 1;  // ends in the next tensor (offsets has ntensors + 1 entries)
+            else hi = wave_find_tensor(a.offsets, a.units_per_elem, lo, a.ntensors, u_last);
+        }
         r_lo = lo;
         r_hi = hi;
     } else if (threadIdx.x < 64) {
@@ -664,6 +666,53 @@ __global__ __launch_bounds__(THREADS) void flat_copy_kernel(FlatArgs a) {
             }
             return;
         }
+    }
+
+    // A tile that one tensor boundary cuts (every tile across a boundary, where tensors are longer than a tile): the chunk
+    // the cut goes through moves unit by unit, all its loads in flight together with the others, and nothing is searched.
+    // A launch ends with its slowest wavefront, so this shows at every size: through the general path below, which looks up
+    // the tensor of each of those units in turn, 40 ragged bf16 tensors of 84 MB moved pack / unpack in 18.3 / 18.1 us
+    // against 15.9 / 16.4 here, 160 of 31 MB pack in 11.2 against 7.7, 20 of 11 MB 7.5 against 4.7.  (The ends of the buffer
+    // in this path as well: 16.1, 8.5, 5.1.)
+    const uint64_t tile_first = block_c0 * VU, tile_end = tile_first + (uint64_t)(kFlatThreads * kUnroll) * VU;
+    if (r_hi == r_lo + 1 && tile_first >= a.shift && tile_end - a.shift <= a.total) {
+        using T = typename UnitType<U>::type;
+        using M = typename UnitType<U>::mem;
+        const uint64_t cut = a.offsets[r_hi] * upe;
+        // where unit 0 of the flat buffer would lie, counted back from either tensor
+        const uintptr_t head = reinterpret_cast<uintptr_t>(a.tensors[r_lo]) - a.offsets[r_lo] * upe * U;
+        const uintptr_t rest = reinterpret_cast<uintptr_t>(a.tensors[r_hi]) - cut * U;
+        auto on_tensor = [&](uint64_t unit) { return reinterpret_cast<M*>((unit < cut ? head : rest) + unit * U); };
+        union Chunk {
+            uint4 v;
+            T e[VU];
+        };
+        Chunk d[kUnroll];
+#pragma unroll
+        for (int i = 0; i < kUnroll; ++i) {
+            const uint64_t first = (block_c0 + (uint64_t)i * kFlatThreads + threadIdx.x) * VU - a.shift;
+            if constexpr (!PACK) {
+                d[i].v = load16_aligned(a.flat + first * U);
+            } else if (first < cut && first + VU > cut) {
+#pragma unroll
+                for (int j = 0; j < VU; ++j) d[i].e[j] = *on_tensor(first + j);
+            } else {
+                d[i].v = load16_unaligned(on_tensor(first));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kUnroll; ++i) {
+            const uint64_t first = (block_c0 + (uint64_t)i * kFlatThreads + threadIdx.x) * VU - a.shift;
+            if constexpr (PACK) {
+                store16_aligned(a.flat + first * U, d[i].v);
+            } else if (first < cut && first + VU > cut) {
+#pragma unroll
+                for (int j = 0; j < VU; ++j) *on_tensor(first + j) = d[i].e[j];
+            } else {
+                store16_unaligned(on_tensor(first), d[i].v);
+            }
+        }
+        return;
     }
 
     // phase 1: resolve every chunk of this lane to (tensor address, flat address)

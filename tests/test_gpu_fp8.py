@@ -475,3 +475,35 @@ def test_block_index_forms_match_table_search(ntensors):
     for hq_r, hs_r in ((hq, ws), (hq, ws), (hq & 0xF7, ws * np.float32(0.5)), (hq, ws)):  # clearing a bit never makes a NaN code
         oracle.fp8_dequant_accumulate(acc_h, hq_r, hs_r, 1024)
     assert np.array_equal(results[1].cpu().numpy().view(np.uint32), acc_h.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.float64])
+@pytest.mark.parametrize("indexed", [False, True])
+def test_flat_tiles_cut_by_one_boundary(dtype, indexed):
+    # tiles are 1 KiB (indexed) or 8 / 16 KiB of the flat buffer: boundaries at, one before and one after the ends of a tile and
+    # of a 16-byte chunk, tensors just longer and just shorter than a tile, flat buffers that start inside a chunk
+    es = torch.empty(0, dtype=dtype).element_size()
+    tile = 1024 // es
+    for sizes in ([tile, 5 * tile], [tile - 1, 9 * tile], [tile + 1, 9 * tile + 1], [tile + 16 // es, 3 * tile, 17 * tile - 1],
+                  [16 * tile + 3, 16 * tile + 5, 8 * tile], [tile + 1, tile - 1, tile + 1, 20 * tile + 7], [40 * tile + 1, 1, 1, 30 * tile]):
+        total = sum(sizes)
+        raw = torch.randint(0, 120, (total * es,), dtype=torch.uint8, generator=torch.Generator().manual_seed(total))
+        host = raw.view(dtype)
+        dev = []
+        for i, part in enumerate(torch.split(host, sizes)):
+            store = torch.zeros(part.numel() + 3, dtype=dtype, device=DEV)
+            dev.append(store[i % 3: i % 3 + part.numel()])
+            dev[-1].copy_(part)
+        bucket = fp8.FlatBucket(dev)
+        for lead in (0, 1):
+            store = torch.zeros(total + 40, dtype=dtype, device=DEV)
+            flat = store[lead: lead + total]
+            bucket.pack(flat, indexed=indexed)
+            outs = [torch.zeros(n + 2, dtype=dtype, device=DEV) for n in sizes]
+            bucket.unpack(flat, [o[1:-1] for o in outs], indexed=indexed)
+            sync()
+            assert torch.equal(flat.cpu().view(torch.uint8), raw), (sizes, lead)
+            rest = torch.cat([store[:lead], store[lead + total:]] + [o[[0, -1]] for o in outs])
+            assert int(torch.count_nonzero(rest.view(torch.uint8))) == 0, (sizes, lead)
+            for o, part in zip(outs, torch.split(host, sizes)):
+                assert torch.equal(o[1:-1].cpu().view(torch.uint8), part.view(torch.uint8)), (sizes, lead)
