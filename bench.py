@@ -1209,8 +1209,8 @@ Every cell is the fraction of the 8 TB/s HBM peak that `mhip_slice_pack` / `mhip
 `x[:, c0:c0 + cols]` of a `[16384, pitch]` matrix whose rows are 28 KiB apart (algorithmic bytes = 2 x elements x
 element size); median of 3 runs of {launches} launches, 3 rotating buffer sets.  Rows of a multiple of 16 bytes take the
 whole-chunk form (line by line when a view of 96 MiB and more does not start and end its rows on cache lines), other
-rows the two-vector form when packed (the gathering form under 4 KiB where shape and pitch are 4-byte granular) and the
-line-by-line form when unpacked; a view that starts off the unit of its shape (c0 = 1) is moved in that unit from a
+rows the two-vector form when packed (unit by unit under 512 bytes, 1280 bytes or 4 KiB where shape and pitch are 1-, 2- or
+4-byte granular) and the line-by-line form when unpacked; a view that starts off the unit of its shape (c0 = 1) is moved in that unit from a
 skewed base.  Views of 59 MB and less (rows of 1792 bytes and less) partly live in the 256 MB Infinity Cache across the
 three buffer sets; the larger ones do not.
 """
