@@ -306,7 +306,8 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
 // 61, unpacking 33.9 -> 31.9 and 123 -> 118); smaller ones (u8 [3001, 7108] k=4, 21 MB: 6.3 / 9.4 us, 7.7 / 11.7 streamed)
 // and rows of several units, whose lines several accesses share (rows of 33 floats unpacking 6.7, 10.8 streamed), keep
 // to the cache.  Rows of several units of a single view also take XCD-contiguous shares (rows of 33 floats unpacking
-// 6.7 -> 6.1); element-strided ones do not (u8 k=2 26.6 -> 28.5).
+// 6.7 -> 6.1); element-strided ones do not (u8 k=2 26.6 -> 28.5), nor do 8-byte units (bf16 rows of 1400 bytes packing 10.4 ->
+// 11.0, of 3080 bytes 19.1 -> 20.1).
 template <int U, bool PACK, int NDIM, bool STREAM>
 __global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
     using T = typename UnitType<U>::type;
@@ -1039,7 +1040,7 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
         bool shares = false;
         if (nbatch == 1) {
             const uint64_t run_bytes = first.run * unit;
-            const bool short_rows = form == kShortRuns && !wide && first.run > 1;
+            const bool short_rows = form == kShortRuns && !wide && first.run > 1 && unit < 8;
             if (PACK) {
                 shares = form == kWholeChunks || (form == kRaggedRows && run_bytes >= kSharesFromRowBytes) || short_rows;
             } else if (form == kShortRuns) {
