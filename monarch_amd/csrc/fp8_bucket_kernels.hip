@@ -39,17 +39,26 @@ __global__ __launch_bounds__(kThreads) void bucket_index_kernel(uint32_t* __rest
         index[b] = b < nblocks ? find_tensor(offsets, 1, 0, ntensors, b * kBlock) : ntensors - 1;
 }
 
+// An entry of a bucket's tables at a wave-uniform address.  SCALAR: as a scalar load (the tables do not change while a
+// kernel runs), which vector loads that are still in flight do not hold up.
+template <bool SCALAR, typename T>
+__device__ __forceinline__ T table_entry(const T* p) {
+    if constexpr (SCALAR) return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+    else return *p;
+}
+
 // Tensors of the first and the last element of [begin, end), begin a block start.  With an index, *t_hi is exact
 // when it equals *t_lo and an upper bound otherwise (the tensor-by-tensor walks skip the empty segments).
 // All 64 lanes call it with the same arguments.
+template <bool SCALAR = false>
 __device__ __forceinline__ void span_tensors(const BucketArgs& a, uint64_t begin, uint64_t end, uint32_t* t_lo, uint32_t* t_hi) {
     if (a.index != nullptr) {
         // clamped: an index that was built for another bucket, or that another call on this GPU is rewriting (the
         // library's static index is shared), must not send the table reads out of bounds
         const uint32_t last = a.ntensors - 1;
-        uint32_t lo = a.index[begin / kBlock];
+        uint32_t lo = table_entry<SCALAR>(a.index + begin / kBlock);
         lo = lo < last ? lo : last;
-        uint32_t hi = a.offsets[lo + 1] >= end ? lo : a.index[(end + kBlock - 1) / kBlock];
+        uint32_t hi = table_entry<SCALAR>(a.offsets + lo + 1) >= end ? lo : table_entry<SCALAR>(a.index + (end + kBlock - 1) / kBlock);
         *t_lo = lo;
         *t_hi = hi < last ? hi : last;
     } else {
@@ -407,6 +416,12 @@ __device__ __forceinline__ void dequant_bucket_block_careful(const BucketArgs& a
     }
 }
 
+// flat element `begin`, which tensor t holds, of a bucket of fp32 tensors
+template <bool SCALAR = false>
+__device__ __forceinline__ float* tensor_at(const BucketArgs& a, uint32_t t, uint64_t begin) {
+    return reinterpret_cast<float*>(table_entry<SCALAR>(a.tensors + t)) + (begin - table_entry<SCALAR>(a.offsets + t));
+}
+
 // Accumulator elements of a full block that one tensor boundary cuts (every block that straddles tensors of 1024
 // elements and more): element i of the block is head[i] for i < cut and rest[i] from there on.  Step j of a lane is
 // elements j * 256 + lane * 4 .. + 3: a 128-bit access to one of the two tensors, except in the step that holds the
@@ -417,10 +432,11 @@ struct CutBlock {
     float* head;
     float* rest;
     uint32_t cut;  // 0 < cut < kBlock
-    __device__ __forceinline__ CutBlock(const BucketArgs& a, uint32_t t, uint64_t begin) {
-        cut = (uint32_t)(a.offsets[t + 1] - begin);
-        head = reinterpret_cast<float*>(a.tensors[t]) + (begin - a.offsets[t]);
-        rest = reinterpret_cast<float*>(reinterpret_cast<uintptr_t>(a.tensors[t + 1]) - (uintptr_t)cut * 4);
+    template <bool SCALAR>
+    static __device__ __forceinline__ CutBlock of(const BucketArgs& a, uint32_t t, uint64_t begin) {
+        const uint32_t cut = (uint32_t)(table_entry<SCALAR>(a.offsets + t + 1) - begin);
+        char* const rest = table_entry<SCALAR>(a.tensors + t + 1);
+        return {tensor_at<SCALAR>(a, t, begin), reinterpret_cast<float*>(reinterpret_cast<uintptr_t>(rest) - (uintptr_t)cut * 4), cut};
     }
     __device__ __forceinline__ bool by_elements(int j) const { return cut % 4 != 0 && cut / 256 == (uint32_t)j; }
     __device__ __forceinline__ float* at(uint32_t i) const { return (i < cut ? head : rest) + i; }
@@ -445,8 +461,10 @@ struct CutBlock {
 };
 
 // whether the full block [begin, begin + kBlock), whose first element tensor t holds, ends in tensor t + 1
+template <bool SCALAR = false>
 __device__ __forceinline__ bool block_cut_once(const BucketArgs& a, uint32_t t, uint64_t begin) {
-    return t + 2 <= a.ntensors && a.offsets[t + 1] < begin + kBlock && a.offsets[t + 2] >= begin + kBlock;
+    return t + 2 <= a.ntensors && table_entry<SCALAR>(a.offsets + t + 1) < begin + kBlock &&
+           table_entry<SCALAR>(a.offsets + t + 2) >= begin + kBlock;
 }
 
 // One block of one peer: codes at q + begin, accumulator vectors through load(j) / store(j, r), 4 steps of 256
@@ -490,13 +508,13 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
         const float s = scales[b];
         if (t_lo == t_hi && end - begin == kBlock) {
             // the whole block lies in one tensor
-            float* dst = reinterpret_cast<float*>(a.tensors[t_lo]) + (begin - a.offsets[t_lo]);
+            float* dst = tensor_at(a, t_lo, begin);
             dequant_accumulate_block(q, s, begin, lane, [&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
                                      [&](int j, const uint4& r) { store16_unaligned(dst + j * 256 + lane * 4, r); });
             continue;
         }
         if (end - begin == kBlock && block_cut_once(a, t_lo, begin)) {
-            const CutBlock c(a, t_lo, begin);
+            const CutBlock c = CutBlock::of<false>(a, t_lo, begin);
             dequant_accumulate_block(q, s, begin, lane, [&](int j) { return c.load(j, lane); },
                                      [&](int j, const uint4& r) { c.store(j, lane, r); });
             continue;
@@ -509,13 +527,17 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
 // The same with n peers' payloads in one pass: every accumulator element crosses HBM once
 // (n + 8 bytes per element instead of 9n).  Peers are added in order, product rounded before
 // each add, so the result has the bits of n single-peer passes.
-// Large buckets are bound by HBM, small ones (one round of wavefronts) by how long a wavefront lives: three dependent
-// table reads, then the data.  So only the codes of peers that exist are loaded (they were loaded four peers at a time,
-// the surplus a repeated peer's), and the first four peers' are on their way before the tables are read.  The registers
-// that takes, 96, are worth more than wavefronts: 5 per SIMD 1122 us, 6 and 7 (which spill) 1199, on 717 M elements and 2
-// peers; half blocks per wavefront 1127 to 1148, quarter blocks 1371 to 1559.  Elements and peers, before -> now, us:
-// 717 M, 2: 1230 -> 1122 (6.4 TB/s); 172 M, 2: 283 -> 261, 8: 451 -> 441; 30 M, 3: 56.3 -> 54.5; 11 M, 8: 33.0 -> 31.8;
-// 4.5 M, 8: 16.4 -> 15.7, 2: 11.8 -> 11.0.
+// Only the codes of peers that exist are loaded.  Large buckets are bound by HBM, small ones (one round of wavefronts) by how
+// long a wavefront lives: three dependent table reads, then the data.  Two forms (kSmallBucketBlocks):
+//   * small buckets read the tables with scalar loads (5.9 M elements, 1 / 8 peers: 10.9 / 18.6 us, with the vector loads that
+//     the compiler makes of them in a kernel that stores through their results 11.9 / 19.2);
+//   * large buckets lose with scalar loads (163 M elements, 5 / 7 peers: 366 / 422 us against 350 / 416) and gain from five
+//     wavefronts per SIMD instead of six (345 / 411).
+// The codes do not go ahead of the tables: the wait for a table entry is then one for the codes as well, since vector loads
+// return in order.  One form for all sizes, with the first codes ahead of the tables, against the two forms: 24 tensors of 0.8 M elements, 4 peers 6.2 us ->
+// 6.5, now 6.0; 5.9 M elements 1 / 8 / 16 peers 12.1 / 20.4 / 30.5, now 10.9 / 19.1 / 29.3; 40 blocks, 4 peers 5.6, now 5.3;
+// 2000 tensors of 10 to 600 elements, 8 peers 20.8, now 19.6; 163 M elements 1 / 2 / 5 peers 233 / 265 / 351, now 238 / 264 /
+// 345 (4 peers at a time with repeated loads for those that do not exist: 242 / 283 / 348).
 constexpr int kMaxBucketPeers = 64;
 
 struct BucketPeersArgs {
@@ -525,11 +547,20 @@ struct BucketPeersArgs {
     uint32_t n;
 };
 
-// Up to four peers' codes of one full block: step j of a lane is the elements j * 256 + lane * 4 .. + 3.
-struct PeerCodes {
-    uint32_t codes[4][4];
-    float s[4];
-    __device__ __forceinline__ void load(const BucketPeersArgs& p, uint32_t r0, uint64_t b, int lane) {
+// One full block of all peers: accumulator vectors through load(j) / store(j, r), peers four at a time with all their codes
+// loaded before the first add.  Step j of a lane is the elements j * 256 + lane * 4 .. + 3.
+template <typename Load, typename Store>
+__device__ __forceinline__ void dequant_accumulate_block_peers(const BucketPeersArgs& p, uint64_t b, int lane, Load&& load, Store&& store) {
+    float v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint4 r = load(j);
+        v[j][0] = __uint_as_float(r.x); v[j][1] = __uint_as_float(r.y);
+        v[j][2] = __uint_as_float(r.z); v[j][3] = __uint_as_float(r.w);
+    }
+    for (uint32_t r0 = 0; r0 < p.n; r0 += 4) {
+        uint32_t codes[4][4];
+        float s[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             if (r0 + g < p.n) {  // wave-uniform
@@ -538,8 +569,6 @@ struct PeerCodes {
                 for (int j = 0; j < 4; ++j) codes[g][j] = load4_unaligned(p.q[r0 + g] + b * kBlock + j * 256 + lane * 4);
             }
         }
-    }
-    __device__ __forceinline__ void add_to(float (&v)[4][4], const BucketPeersArgs& p, uint32_t r0) const {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             if (r0 + g < p.n) {
@@ -555,31 +584,14 @@ struct PeerCodes {
             }
         }
     }
-};
-
-// One full block of all peers: `c` holds the first four peers' codes, accumulator vectors go through load(j) / store(j, r),
-// the other peers four at a time with all their codes loaded before the first add.
-template <typename Load, typename Store>
-__device__ __forceinline__ void dequant_accumulate_block_peers(const BucketPeersArgs& p, PeerCodes& c, uint64_t b, int lane, Load&& load,
-                                                               Store&& store) {
-    float v[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint4 r = load(j);
-        v[j][0] = __uint_as_float(r.x); v[j][1] = __uint_as_float(r.y);
-        v[j][2] = __uint_as_float(r.z); v[j][3] = __uint_as_float(r.w);
-    }
-    c.add_to(v, p, 0);
-    for (uint32_t r0 = 4; r0 < p.n; r0 += 4) {
-        c.load(p, r0, b, lane);
-        c.add_to(v, p, r0);
-    }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
         store(j, make_uint4(__float_as_uint(v[j][0]), __float_as_uint(v[j][1]), __float_as_uint(v[j][2]), __float_as_uint(v[j][3])));
 }
 
-__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(5))) void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
+template <bool SMALL>
+__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(SMALL ? 6 : 5, SMALL ? 8 : 5)))
+void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
     const BucketArgs& a = p.b;
     const int lane = threadIdx.x & 63;
     const uint64_t wave = (uint64_t)blockIdx.x * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // see fp8_quantize_bucket_kernel
@@ -588,21 +600,18 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
         const uint64_t begin = b * kBlock;
         const bool full = begin + kBlock <= a.total;
         const uint64_t end = full ? begin + kBlock : a.total;
-        // The codes' addresses do not wait for the tables: they are on their way while the block's tensor is looked up.
-        PeerCodes c;
-        if (full) c.load(p, 0, b, lane);
         uint32_t t_lo, t_hi;
-        span_tensors(a, begin, end, &t_lo, &t_hi);
+        span_tensors<SMALL>(a, begin, end, &t_lo, &t_hi);
         if (full && t_lo == t_hi) {
-            float* dst = reinterpret_cast<float*>(a.tensors[t_lo]) + (begin - a.offsets[t_lo]);
-            dequant_accumulate_block_peers(p, c, b, lane, [&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
+            float* dst = tensor_at<SMALL>(a, t_lo, begin);
+            dequant_accumulate_block_peers(p, b, lane, [&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
                                            [&](int j, const uint4& r) { store16_unaligned(dst + j * 256 + lane * 4, r); });
             continue;
         }
-        if (full && block_cut_once(a, t_lo, begin)) {
-            const CutBlock cut(a, t_lo, begin);
-            dequant_accumulate_block_peers(p, c, b, lane, [&](int j) { return cut.load(j, lane); },
-                                           [&](int j, const uint4& r) { cut.store(j, lane, r); });
+        if (full && block_cut_once<SMALL>(a, t_lo, begin)) {
+            const CutBlock c = CutBlock::of<SMALL>(a, t_lo, begin);
+            dequant_accumulate_block_peers(p, b, lane, [&](int j) { return c.load(j, lane); },
+                                           [&](int j, const uint4& r) { c.store(j, lane, r); });
             continue;
         }
         // more than two tensors, or the short last block
@@ -796,8 +805,9 @@ int mhip_fp8_dequant_accumulate_bucket_many(void* const* d_acc_tensors, const ui
     const uint64_t cap = max_workgroups(kBucketThreads);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     DeviceGuard guard(hs);
-    MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel, dim3((uint32_t)(wgs > cap ? cap : wgs)), dim3(kBucketThreads),
-                       0, hs, p);
+    const dim3 grid((uint32_t)(wgs > cap ? cap : wgs));
+    if (p.b.nblocks <= kSmallBucketBlocks) MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel<true>, grid, dim3(kBucketThreads), 0, hs, p);
+    else MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel<false>, grid, dim3(kBucketThreads), 0, hs, p);
     return launch_status();
 }
 

@@ -163,6 +163,29 @@ def test_dequant_accumulate_bucket_from_many_peers(npeers):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), npeers
 
 
+@pytest.mark.parametrize("blocks", [32768, 32769])
+@pytest.mark.parametrize("npeers", [1, 3, 6])
+def test_dequant_accumulate_bucket_many_of_large_buckets(blocks, npeers):
+    # up to 32768 blocks and more of them take different forms of the kernel: the same bits as one pass per peer, on tensors
+    # whose boundaries fall inside blocks, on blocks and around tiny and empty tensors, with a short last block
+    g = torch.Generator(device=DEV).manual_seed(blocks + npeers)
+    total = blocks * 1024 - 5
+    sizes = [5_000_001, 1, 0, 1000, 23, 1024 * 7, 9_999_999, 2048]
+    sizes.append(total - sum(sizes))
+    acc = torch.randn(total, device=DEV, generator=g)
+    want, got = acc.clone(), torch.empty_like(acc)
+    one, many = (fp8.FlatBucket(list(torch.split(x, sizes))) for x in (want, got))
+    qs = [torch.randint(0, 120, (total,), dtype=torch.uint8, device=DEV, generator=g) for _ in range(npeers)]
+    ss = [torch.rand(blocks, device=DEV, generator=g) for _ in range(npeers)]
+    for q, s in zip(qs, ss):
+        fp8.dequant_accumulate_bucket(one, q, s)
+    for indexed in (False, True):
+        got.copy_(acc)
+        fp8.dequant_accumulate_bucket_many(many, qs, ss, indexed=indexed)
+        sync()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), indexed
+
+
 def test_fused_bucket_forms_equal_two_step_pipeline():
     # ragged sizes around block boundaries, empty tensors, odd element alignment, NaN/Inf blocks
     g = torch.Generator().manual_seed(77)
