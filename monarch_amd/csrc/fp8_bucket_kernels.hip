@@ -125,7 +125,7 @@ __device__ __forceinline__ void quantize_bucket_block_careful(uint8_t* __restric
 // cooperative search pair locates the tensors of the first and the last element of the
 // whole span; when they coincide (the common case) all 2 * kBucketBlocks loads of a lane
 // are issued back to back from one base pointer.
-constexpr uint64_t kSmallBucketBlocks = 32768;  // buckets of up to 33.5 M elements take one block per wavefront step (see quantize_bucket)
+constexpr uint64_t kSmallBucketBlocks = 32768;  // buckets of up to 33.5 M elements have forms of their own (see quantize_bucket, BucketPeersArgs)
 constexpr int kBucketBlocks = 4;       // blocks per wavefront step of the quantiser on large buckets (template parameter NB)
 // Lanes per workgroup.  Unlike the plain copy and the tensor-less quantiser, which stream best as single
 // wavefronts, the bucket kernels want 4 wavefronts: quantise / dequantise / dequantise 8 peers reach
@@ -534,10 +534,9 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
 //   * large buckets lose with scalar loads (163 M elements, 5 / 7 peers: 366 / 422 us against 350 / 416) and gain from five
 //     wavefronts per SIMD instead of six (345 / 411).
 // The codes do not go ahead of the tables: the wait for a table entry is then one for the codes as well, since vector loads
-// return in order.  One form for all sizes, with the first codes ahead of the tables, against the two forms: 24 tensors of 0.8 M elements, 4 peers 6.2 us ->
-// 6.5, now 6.0; 5.9 M elements 1 / 8 / 16 peers 12.1 / 20.4 / 30.5, now 10.9 / 19.1 / 29.3; 40 blocks, 4 peers 5.6, now 5.3;
-// 2000 tensors of 10 to 600 elements, 8 peers 20.8, now 19.6; 163 M elements 1 / 2 / 5 peers 233 / 265 / 351, now 238 / 264 /
-// 345 (4 peers at a time with repeated loads for those that do not exist: 242 / 283 / 348).
+// return in order.  That form for all sizes / the two forms here: 0.8 M elements in 24 tensors, 4 peers 6.5 / 6.0 us; 5.9 M,
+// 1, 8 and 16 peers 12.1 / 10.9, 20.4 / 19.1, 30.5 / 29.3; 40 blocks, 4 peers 5.6 / 5.3; 2000 tensors of 10 to 600 elements, 8
+// peers 20.8 / 19.6; 163 M elements, 1, 2 and 5 peers 233 / 238, 265 / 264, 351 / 345.
 constexpr int kMaxBucketPeers = 64;
 
 struct BucketPeersArgs {
