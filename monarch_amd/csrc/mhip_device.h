@@ -46,6 +46,29 @@ inline bool make_dims_arg(const CanonSlice& c, DimsArg* d, bool* fits32, int pad
     return true;
 }
 
+// Unit offset of row `row` of a slice in 32-bit mode; NDIM as in decode.
+template <int NDIM = -1>
+__device__ __forceinline__ uint64_t row_offset(const DimsArg& d, uint32_t row) {
+    uint64_t off = 0;
+    if constexpr (NDIM >= 0) {
+#pragma unroll
+        for (int k = NDIM - 1; k > 0; --k) {
+            uint32_t q, r;
+            d.size_div[k].divmod(row, q, r);
+            off += (uint64_t)r * d.stride[k];
+            row = q;
+        }
+    } else {
+        for (int k = d.ndim - 1; k > 0; --k) {
+            uint32_t q, r;
+            d.size_div[k].divmod(row, q, r);
+            off += (uint64_t)r * d.stride[k];
+            row = q;
+        }
+    }
+    return off + (uint64_t)row * d.stride[0];
+}
+
 // Unit offset of packed unit t, and its column within the row (for run-boundary tests).
 // NDIM >= 0 fixes the number of dimensions outside the run at compile time (no loop, no
 // kernel-argument loads inside the decode); NDIM < 0 reads it from the arguments.
@@ -73,23 +96,7 @@ __device__ __forceinline__ uint64_t decode(const DimsArg& d, uint64_t t, uint64_
         d.run_div.divmod((uint32_t)t, row, col);
         *col_out = col;
         off = col;
-        if constexpr (NDIM >= 0) {
-#pragma unroll
-            for (int k = NDIM - 1; k > 0; --k) {
-                uint32_t q, r;
-                d.size_div[k].divmod(row, q, r);
-                off += (uint64_t)r * d.stride[k];
-                row = q;
-            }
-        } else {
-            for (int k = ndim - 1; k > 0; --k) {
-                uint32_t q, r;
-                d.size_div[k].divmod(row, q, r);
-                off += (uint64_t)r * d.stride[k];
-                row = q;
-            }
-        }
-        off += (uint64_t)row * d.stride[0];
+        off += row_offset<NDIM>(d, row);
     }
     return off;
 }
