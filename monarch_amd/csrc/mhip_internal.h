@@ -41,6 +41,10 @@ struct CanonSlice {
 bool canonicalize(const mhip_slice_t& s, uint32_t elem_size, uint64_t align_mask, uint32_t max_unit,
                   CanonSlice* out, uint32_t* unit, uint64_t* skew = nullptr);
 
+// Whether a copy of this view unit by unit streams past the caches: a view of single units (run == 1) that touches many
+// lines, and each of them with one access only (no unit of another dimension lies between those of the innermost one).
+bool streams_units(const CanonSlice& c, uint32_t unit);
+
 // Same dimension list for two canonical slices (offsets may differ).
 bool same_shape(const CanonSlice& a, const CanonSlice& b);
 

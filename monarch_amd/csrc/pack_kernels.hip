@@ -306,10 +306,13 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
 // three, and views of single units (RUN1) are spared the division by the run: channels of images packed side by side, u8
 // [13, 50176, 3] -> [13, 3, 50176] 6.7 / 7.8 -> 3.5 / 4.6 us (in the order of the kernel this one replaces 4.8 / 10.9), bf16
 // [6, 50176, 3] 4.4 / 5.4 -> 3.0 / 3.8 (3.5 / 6.6).
-// Element-strided views that span 32 MiB or more stream (non-temporal accesses: u8 k=2 packing 27.2 -> 26.6, f32 66 ->
-// 61, unpacking 33.9 -> 31.9 and 123 -> 118); smaller ones (u8 [3001, 7108] k=4, 21 MB: 6.3 / 9.4 us, 7.7 / 11.7 streamed)
-// and rows of several units, whose lines several accesses share (rows of 33 floats unpacking 6.7, 10.8 streamed), keep
-// to the cache.  Rows of several units of a single view also take XCD-contiguous shares (rows of 33 floats unpacking
+// Views whose lines are touched by one access each stream (non-temporal accesses, streams_units) from 92 MiB of lines on, where
+// they no longer fit the Infinity Cache between passes: f32 [:, ::2] over 88 MiB packing / unpacking 22.2 / 31.9 us, streamed
+// 22.0 / 40.7; over 96 MiB 26.1 / 45.9, streamed 24.0 / 44.4.  Where the units of another dimension lie in between (the columns of
+// a tall matrix, channels packed side by side) every line is touched again and again, and at no size is streaming better:
+// f32 [2 M, 3].t() 15.1 / 21.4, streamed 16.5 / 31.1; [3.6 M, 7].t() 118 / 168, streamed 134 / 303; nor is it for several views
+// of one tensor in one launch (f32 x[:, i::4] over 60 MiB 44.4 / 63.3, streamed 50.2 / 101.9).
+// Rows of several units of a single view also take XCD-contiguous shares (rows of 33 floats unpacking
 // 6.7 -> 6.1); element-strided ones do not (u8 k=2 26.6 -> 28.5), nor do 8-byte units (bf16 rows of 1400 bytes packing 10.4 ->
 // 11.0, of 3080 bytes 19.1 -> 20.1).
 template <int U, bool PACK, int NDIM, bool RUN1, bool STREAM>
@@ -914,7 +917,6 @@ static int copy_deep_view(char* base, char* packed, const mhip_slice_t& s, uint3
 // of a 117 MB tensor: 0.794 against 0.777).
 constexpr uint64_t kSharesFromRowBytes = 6144;
 constexpr uint64_t kStreamUnpackFromBytes = 96ull << 20;
-constexpr uint64_t kStreamUnitsFromSpan = 32ull << 20;  // see slice_units_kernel
 template <bool PACK>
 static int copy_views(char* base, char* const* packed, const mhip_slice_t* views, uint32_t nviews,
                       uint32_t elem_size, hipStream_t stream) {
@@ -1050,8 +1052,7 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
         a.nviews = nbatch;
         a.nviews_div = FastDiv32(nbatch);
         uint64_t nwg = blocks * nbatch;
-        if (form == kShortRuns && first.run == 1)
-            a.stream_units = nbatch * first.total * first.dims[first.ndim - 1].stride * unit >= kStreamUnitsFromSpan;
+        a.stream_units = form == kShortRuns && nbatch == 1 && streams_units(first, unit);
         // which single-view copies take XCD-contiguous shares, and how an unpack of 16-byte units stores: see the
         // note above copy_views
         bool shares = false;

@@ -50,6 +50,19 @@ bool canonicalize(const mhip_slice_t& s, uint32_t elem_size, uint64_t align_mask
     return true;
 }
 
+// Bytes of lines from which the strided side of a copy unit by unit is streamed: from there on the lines do not stay in
+// the Infinity Cache between one pass over them and the next.
+constexpr uint64_t kStreamUnitsFromBytes = 92ull << 20;
+
+bool streams_units(const CanonSlice& c, uint32_t unit) {
+    if (c.ndim == 0 || c.run != 1) return false;
+    const uint64_t step = c.dims[c.ndim - 1].stride;
+    for (int k = 0; k < c.ndim; ++k)
+        if (c.dims[k].stride < step) return false;  // its units lie between the innermost dimension's: shared lines
+    const uint64_t line = 128 / unit;
+    return c.total >= kStreamUnitsFromBytes / unit / (step < line ? step : line);
+}
+
 bool same_shape(const CanonSlice& a, const CanonSlice& b) {
     if (a.ndim != b.ndim || a.run != b.run || a.total != b.total) return false;
     for (int k = 0; k < a.ndim; ++k)

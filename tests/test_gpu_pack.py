@@ -837,19 +837,20 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.int16, torch.int32, torch.int64])
 def test_short_runs_unit_by_unit(dtype):
     # slice_units_kernel: 1 KiB of the packed side per workgroup, so lengths round one and several of those, rows up to the
-    # lengths at which the other forms take over, staging addresses inside a 16-byte vector, one launch of several views,
-    # and element-strided views on both sides of the 32 MiB from which they stream
+    # lengths at which the other forms take over, staging addresses inside a 16-byte vector, views of up to four dimensions,
+    # one launch of several views, and element-strided views on both sides of the 92 MiB from which one of them streams
     es = torch.empty(0, dtype=dtype).element_size()
     tile = 1024 // es
     cases = [(0, [n], [k]) for k in (2, 3, 5) for n in (2 * 16 // es, tile - 1, tile, tile + 1, 3 * tile + 7)]
     cases += [(1, [77, n], [2 * n + 1, 1]) for n in (1, 3, 255 // es, 257 // es, 511 // es, 513 // es, 2047 // es, 4095 // es, 4097 // es) if n]
-    cases += [(0, [3, 40, 50], [40 * 50 * 4, 50 * 4, 2])]
+    cases += [(0, [3, 40, 50], [40 * 50 * 4, 50 * 4, 2]), (5, [3, 5, 41, 50], [40 * 50 * 64, 40 * 50 * 8, 50 * 4, 2]),
+              (0, [3, 5, 7, 50, 3], [7 * 800 * 5, 7 * 800, 800, 4, 1]), (0, [2, 3, 1000], [3000, 1, 3]), (0, [2, 1000, 3], [3000, 1, 1000])]
     for i, (offset, sizes, strides) in enumerate(cases):
         s = Slice(offset=offset, sizes=sizes, strides=strides)
         for mis in (0, es, 16 - es):
             _roundtrip(s, es, seed=70 + i, misalign=mis % 8, dst_misalign=mis)
     g = torch.Generator(device=DEV).manual_seed(7)
-    for nbytes in ((32 << 20) - 64, (32 << 20) + 64 + 3 * es):
+    for nbytes in ((92 << 20) - 64, (92 << 20) + 64 + 2 * es):
         x = torch.randint(0, 127, (nbytes // es // 2, 2), dtype=torch.int32, device=DEV, generator=g).to(dtype)
         views = [Slice.of_tensor(x[:, 0]), Slice.of_tensor(x[:-1, 1])]
         outs = staging.pack_many(x, views)
