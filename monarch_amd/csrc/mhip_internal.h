@@ -45,6 +45,10 @@ bool canonicalize(const mhip_slice_t& s, uint32_t elem_size, uint64_t align_mask
 // lines, and each of them with one access only (no unit of another dimension lies between those of the innermost one).
 bool streams_units(const CanonSlice& c, uint32_t unit);
 
+// Whether consecutive units of the packed side come from four to seven places far apart (the planes of an image whose
+// channels are packed side by side) in a view large enough to be bound by memory.
+bool gathers_units(const CanonSlice& c, uint32_t unit);
+
 // Same dimension list for two canonical slices (offsets may differ).
 bool same_shape(const CanonSlice& a, const CanonSlice& b);
 

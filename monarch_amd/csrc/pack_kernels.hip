@@ -382,15 +382,21 @@ __global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
     }
 }
 
-// The same views from 2^31 units on, where an index takes 64-bit divisions: too many for one per unit.  A lane owns whole
-// 16-byte chunks of the packed side and gathers (pack) or scatters (unpack) the chunk's units one by one on the strided
-// side.  All unit loads of a lane are issued before the first use and none is predicated.  Unit addresses come from one
-// full decode per chunk followed by an odometer over the run and the innermost dimension outside it; a full decode is
-// repeated only when that dimension wraps.  Strided-side accesses are NOT non-temporal: the lanes of a wavefront return
-// to the same cache lines for every unit of their chunks.
+// The same views where that loses: from 2^31 units on, since an index takes 64-bit divisions there, too many for one per unit;
+// and bytes and 2-byte units from four to seven planes side by side (gathers_units), where each access of a wavefront in that
+// order touches a short piece of every plane.  Units side by side / this kernel, pack / unpack: u8 [930, 6, 12544] ->
+// [930, 12544, 6] 92 / 105 us, 68 / 82; bf16 [697, 4, 12544] 27.5 / 35.6, 25.9 / 30.9; bf16 [7, 5 M].t() 55 / 73, 47 / 68.  Small
+// views stay with the units (bf16 [11, 7, 12544], 4 MB moved, 3.9 / 4.0, here 5.2 / 5.9), and so do two and three planes (bf16
+// [3, 17 M].t() 54 / 62, here 56 / 82).
+//
+// A lane owns whole 16-byte chunks of the packed side and gathers (pack) or scatters (unpack) the chunk's units one by one
+// on the strided side.  All unit loads of a lane are issued before the first use and none is predicated.  Unit addresses
+// come from one full decode per chunk followed by an odometer over the run and the innermost dimension outside it; a full
+// decode is repeated only when that dimension wraps.  Strided-side accesses are NOT non-temporal: the lanes of a wavefront
+// return to the same cache lines for every unit of their chunks.
 constexpr int kGatherUnroll = 1;
 
-template <int U, bool PACK>
+template <int U, bool PACK, bool WIDE, int NDIM>
 __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) {
     using T = typename UnitType<U>::type;
     constexpr int VU = 16 / U;
@@ -403,7 +409,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
     using M = typename UnitType<U>::mem;  // the strided side may be less aligned than the unit
     M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
     const uint64_t c0 = tile * (kPackThreads * UN) + threadIdx.x;
-    const int nd = a.dims.ndim;
+    const int nd = NDIM >= 0 ? NDIM : a.dims.ndim;
     const uint64_t run = a.dims.run;
     const uint64_t size_last = a.dims.size[nd - 1];
     const uint64_t step_last = a.dims.stride[nd - 1] - run;  // from one past a run's end to the start of the next run
@@ -420,8 +426,16 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
         edge[i] = c < a.nchunks && !full[i];
         if (full[i]) {
             uint64_t col;
-            uint64_t loc = decode<true, -1>(a.dims, first, &col);
-            uint64_t ilast = ((first - col) / run) % size_last;  // index along the innermost dimension outside the run
+            uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
+            uint64_t ilast;  // index along the innermost dimension outside the run
+            if constexpr (WIDE) {
+                ilast = ((first - col) / run) % size_last;
+            } else {
+                uint32_t row, c32, q, i;
+                a.dims.run_div.divmod((uint32_t)first, row, c32);
+                a.dims.size_div[nd - 1].divmod(row, q, i);
+                ilast = i;
+            }
             off[i][0] = loc;
 #pragma unroll
             for (int j = 1; j < VU; ++j) {
@@ -432,7 +446,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
                     ++ilast;
                     loc += step_last;
                     if (ilast == size_last) {
-                        loc = decode<true, -1>(a.dims, first + j, &col);
+                        loc = decode<WIDE, NDIM>(a.dims, first + j, &col);
                         ilast = 0;
                     }
                 }
@@ -472,7 +486,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
     // ragged first and last chunk of the view: unit by unit
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
-        if (edge[i]) move_chunk_by_units<U, PACK, true, -1>(a, reinterpret_cast<char*>(strided), packed, c0 + (uint64_t)i * kPackThreads);
+        if (edge[i]) move_chunk_by_units<U, PACK, WIDE, NDIM>(a, reinterpret_cast<char*>(strided), packed, c0 + (uint64_t)i * kPackThreads);
     }
 }
 
@@ -792,7 +806,7 @@ __global__ __launch_bounds__(THREADS) void flat_copy_kernel(FlatArgs a) {
 
 // ---------------- host side ----------------
 
-enum CopyForm { kWholeChunks, kRaggedRows, kShortRuns, kUnpackLines };
+enum CopyForm { kWholeChunks, kRaggedRows, kShortRuns, kGatherUnits, kUnpackLines };
 
 template <int U, bool PACK>
 static void launch_whole_chunks(bool wide, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
@@ -837,11 +851,16 @@ static void launch_slice_copy_u(bool wide, CopyForm form, int ndim, dim3 grid, h
         return;
     }
     if constexpr (U < 16) {
-        if (form == kShortRuns) {
+        if (form == kGatherUnits) {
             if (wide) {
-                MHIP_LAUNCH((slice_gather_kernel<U, PACK>), grid, block, 0, stream, a);
-                return;
+                MHIP_LAUNCH((slice_gather_kernel<U, PACK, true, -1>), grid, block, 0, stream, a);
+            } else if constexpr (U <= 2) {
+                if (ndim == 2) MHIP_LAUNCH((slice_gather_kernel<U, PACK, false, 2>), grid, block, 0, stream, a);
+                else MHIP_LAUNCH((slice_gather_kernel<U, PACK, false, -1>), grid, block, 0, stream, a);
             }
+            return;
+        }
+        if (form == kShortRuns) {
             if (a.dims.run != 1) launch_units<U, PACK, false, false>(ndim, grid, stream, a);
             else if (a.stream_units) launch_units<U, PACK, true, true>(ndim, grid, stream, a);
             else launch_units<U, PACK, true, false>(ndim, grid, stream, a);
@@ -1003,7 +1022,8 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
             uint64_t units_below = (PACK ? (unit == 1 ? 512 : unit > 2 ? 4096 : nbatch == 1 ? 1280 : 2048) : 256) / unit;  // row length in units
             if (!fits32 && unit == 1) units_below = 64;
             if (!fits32 && unit == 2) units_below = 128;
-            if (first.run < units_below && first.total >= 2 * vu) form = kShortRuns;
+            if (first.run < units_below && first.total >= 2 * vu)
+                form = fits32 && !(unit <= 2 && gathers_units(first, unit)) ? kShortRuns : kGatherUnits;
             else if (first.run >= vu) form = kRaggedRows;
         }
         // Unpacking ragged rows of 256 bytes and more line by line of the written side (see slice_unpack_lines_kernel).
@@ -1058,7 +1078,7 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
         bool shares = false;
         if (nbatch == 1) {
             const uint64_t run_bytes = first.run * unit;
-            const bool short_rows = form == kShortRuns && !wide && first.run > 1 && unit < 8;
+            const bool short_rows = form == kShortRuns && first.run > 1 && unit < 8;
             if (PACK) {
                 shares = form == kWholeChunks || (form == kRaggedRows && run_bytes >= kSharesFromRowBytes) || short_rows;
             } else if (form == kShortRuns) {

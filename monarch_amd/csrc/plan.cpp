@@ -63,6 +63,15 @@ bool streams_units(const CanonSlice& c, uint32_t unit) {
     return c.total >= kStreamUnitsFromBytes / unit / (step < line ? step : line);
 }
 
+bool gathers_units(const CanonSlice& c, uint32_t unit) {
+    if (c.ndim < 2 || c.run != 1 || c.total < (6ull << 20) / unit) return false;
+    const CanonDim& last = c.dims[c.ndim - 1];
+    if (last.size < 4 || last.size > 7) return false;
+    for (int k = 0; k < c.ndim - 1; ++k)
+        if (c.dims[k].stride < last.stride) return true;
+    return false;
+}
+
 bool same_shape(const CanonSlice& a, const CanonSlice& b) {
     if (a.ndim != b.ndim || a.run != b.run || a.total != b.total) return false;
     for (int k = 0; k < a.ndim; ++k)

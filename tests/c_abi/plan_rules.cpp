@@ -1,6 +1,6 @@
 // Prints what the copy planner (plan.cpp) decides about a view copied unit by unit.  Input, one view per line:
 //   element_size offset ndim sizes... strides...     (elements)
-// Output, one line per view: unit in bytes, streams_units.  No GPU, no HIP headers.
+// Output, one line per view: unit in bytes, streams_units, gathers_units.  No GPU, no HIP headers.
 #include <cstdio>
 #include <iostream>
 
@@ -16,7 +16,7 @@ int main() {
         mhip::CanonSlice c;
         uint32_t unit = 0;
         if (!mhip::canonicalize(s, elem_size, 0, 16, &c, &unit)) return 1;
-        std::printf("%u %d\n", unit, mhip::streams_units(c, unit));
+        std::printf("%u %d %d\n", unit, mhip::streams_units(c, unit), mhip::gathers_units(c, unit));
     }
     return 0;
 }

@@ -862,3 +862,28 @@ def test_short_runs_unit_by_unit(dtype):
             assert torch.equal(o, want) and torch.equal(one, want)
         x[-1, 1] = 0
         assert torch.equal(back, x)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.int16])
+@pytest.mark.parametrize("planes", [3, 4, 5, 7])
+def test_interleaving_planes(dtype, planes):
+    # consecutive units of the packed side come from planes far apart: 4 to 7 planes are gathered by chunks from 6 MiB on
+    # (slice_gather_kernel), fewer planes and smaller views go unit by unit; sizes on both sides of that, with and without
+    # a batch, staging addresses off the 16-byte grid
+    es = torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=DEV).manual_seed(planes)
+    n = (6 << 20) // (planes * es)
+    for shape in ((1, planes, (n - 64) | 1), (1, planes, (n + 64) | 1), (4, planes, ((n + 64) // 4) | 1)):
+        x = torch.randint(0, 120, shape, device=DEV, generator=g, dtype=torch.int32).to(dtype)
+        view = x.transpose(1, 2)
+        s = Slice.of_tensor(view)
+        for lead in (0, 1, 3):
+            store = torch.full((len(s) + 16,), 9, dtype=dtype, device=DEV)
+            out = store[lead: lead + len(s)]
+            staging.pack(x, s, out=out)
+            back = torch.full_like(x, 7)
+            staging.unpack(back, s, out)
+            sync()
+            assert torch.equal(out.view(view.shape), view), (shape, lead)
+            assert torch.equal(back, x), (shape, lead)
+            assert int((store[:lead] != 9).sum()) + int((store[lead + len(s):] != 9).sum()) == 0, (shape, lead)

@@ -1,5 +1,5 @@
-"""The copy planner's rules on views that move unit by unit (plan.cpp, plain C++): which of them stream past the caches.
-Compiled with the host compiler, no GPU."""
+"""The copy planner's rules on views that move unit by unit (plan.cpp, plain C++): which of them stream past the caches
+and which are gathered chunk by chunk.  Compiled with the host compiler, no GPU."""
 import os
 import shutil
 import subprocess
@@ -31,12 +31,12 @@ def decide(tmp_path_factory):
 def test_every_kth_element_streams_from_92_mib_of_lines_on(decide, es, k):
     cols = 4096
     rows = 92 * MIB // (cols * k * es)
-    assert decide(es, [rows, cols], [cols * k, k]) == (es, 1)
-    assert decide(es, [rows - 1, cols], [cols * k, k]) == (es, 0)
-    assert decide(es, [32 * MIB // (cols * k * es), cols], [cols * k, k]) == (es, 0)
+    assert decide(es, [rows, cols], [cols * k, k]) == (es, 1, 0)
+    assert decide(es, [rows - 1, cols], [cols * k, k]) == (es, 0, 0)
+    assert decide(es, [32 * MIB // (cols * k * es), cols], [cols * k, k]) == (es, 0, 0)
     # every other row as well: the lines in between are not touched
-    assert decide(es, [rows, cols], [2 * cols * k, k]) == (es, 1)
-    assert decide(es, [rows // 2, cols], [2 * cols * k, k]) == (es, 0)
+    assert decide(es, [rows, cols], [2 * cols * k, k]) == (es, 1, 0)
+    assert decide(es, [rows // 2, cols], [2 * cols * k, k]) == (es, 0, 0)
 
 
 @pytest.mark.parametrize("nbytes", [8_000_000, 24_000_000, 400_000_000])
@@ -53,5 +53,16 @@ def test_interleaved_views_keep_to_the_cache(decide, nbytes):
 
 def test_units_far_apart_count_one_line_each(decide):
     # a stride of 1 KiB touches one line of 128 bytes per element, not 1 KiB
-    assert decide(4, [92 * MIB // 128], [256]) == (4, 1)
-    assert decide(4, [92 * MIB // 128 - 1], [256]) == (4, 0)
+    assert decide(4, [92 * MIB // 128], [256]) == (4, 1, 0)
+    assert decide(4, [92 * MIB // 128 - 1], [256]) == (4, 0, 0)
+
+
+@pytest.mark.parametrize("es", [1, 2])
+def test_four_to_seven_planes_are_gathered_from_6_mib_on(decide, es):
+    for k in (4, 5, 6, 7):
+        n = -(-6 * MIB // (k * es)) | 1   # odd, so that the unit stays the element
+        assert decide(es, [n, k], [1, n]) == (es, 0, 1)
+        assert decide(es, [n - 2 * k, k], [1, n - 2 * k])[2] == 0
+        assert decide(es, [k, n], [1, k])[2] == 0      # the other way round
+    for k in (2, 3):
+        assert decide(es, [8 * MIB, k], [1, 8 * MIB + 1])[2] == 0
