@@ -312,9 +312,10 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
 // a tall matrix, channels packed side by side) every line is touched again and again, and at no size is streaming better:
 // f32 [2 M, 3].t() 15.1 / 21.4, streamed 16.5 / 31.1; [3.6 M, 7].t() 118 / 168, streamed 134 / 303; nor is it for several views
 // of one tensor in one launch (f32 x[:, i::4] over 60 MiB 44.4 / 63.3, streamed 50.2 / 101.9).
-// Rows of several units of a single view also take XCD-contiguous shares (rows of 33 floats unpacking
-// 6.7 -> 6.1); element-strided ones do not (u8 k=2 26.6 -> 28.5), nor do 8-byte units (bf16 rows of 1400 bytes packing 10.4 ->
-// 11.0, of 3080 bytes 19.1 -> 20.1).
+// Rows of several units of a single view also take XCD-contiguous shares (rows of 33 floats unpacking 6.7 -> 6.1); element-strided
+// ones do not (u8 k=2 26.6 -> 28.5), nor do 8-byte units (bf16 rows of 1400 bytes packing 10.4 -> 11.0, of 3080 bytes 19.1 ->
+// 20.1), nor do rows under 256 bytes of 2- and 4-byte units packing 32 MiB and more (60 MB in rows of 20 / 44 / 136 bytes 35.4 /
+// 32.8 / 30.2, plain mapping 33.2 / 31.5 / 29.1; 16 MB in rows of 72 bytes 8.7, plain 9.9).
 template <int U, bool PACK, int NDIM, bool RUN1, bool STREAM>
 __global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
     using T = typename UnitType<U>::type;
@@ -1078,7 +1079,8 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
         bool shares = false;
         if (nbatch == 1) {
             const uint64_t run_bytes = first.run * unit;
-            const bool short_rows = form == kShortRuns && first.run > 1 && unit < 8;
+            const bool short_rows = form == kShortRuns && first.run > 1 && unit < 8 &&
+                                    !(PACK && unit > 1 && run_bytes < 256 && first.total * unit >= (32ull << 20));
             if (PACK) {
                 shares = form == kWholeChunks || (form == kRaggedRows && run_bytes >= kSharesFromRowBytes) || short_rows;
             } else if (form == kShortRuns) {
