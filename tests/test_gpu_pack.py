@@ -818,6 +818,9 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
     cases += [((n, many // (n * es) // es + 1), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
     if es == 1:  # 16 to 40 MiB with rows that are not whole lines
         cases += [((4099, 4100), lambda x: x.t()), ((5001, 8191), lambda x: x.t()), ((4100, 4224), lambda x: x[:, 1:4097].t())]
+    if es == 8:  # both sides of the 2 MiB at which the tile of small matrices changes
+        cases += [((511, 512), lambda x: x.t()), ((513, 512), lambda x: x.t()), ((3, 300, 305), lambda x: x.transpose(1, 2)),
+                  ((1000, 1555), lambda x: x[:, 3:].t())]
     for shape, view_of in cases:
         host = torch.randint(info.min, info.max, shape, dtype=dtype, generator=g)
         dev = host.to(DEV)
