@@ -240,9 +240,9 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
     constexpr uint32_t ES = sizeof(T);
     const uint64_t ib = (uint64_t)(PACK ? a.Q : a.Sc) * ES, jb = (uint64_t)(PACK ? a.Sc : a.Q) * ES;
     const uint64_t bytes = nbatch * ib * jb / ES;
-    if (bytes >= (16ull << 20)) {  // one of the sides is at most 512 bytes then, or elements are bytes
-        if constexpr (ES == 1)
-            if (ib > 512 && jb > 512) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+    if constexpr (ES == 1)
+        if (ib > 512 && jb > 512 && bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+    if (bytes >= (16ull << 20) && (ib <= 512 || jb <= 512)) {
         const bool short_j = jb <= ib;
         uint32_t n = narrow_tile_bytes(short_j ? jb : ib);
         if (ES == 8 && n == 64) n = 128;  // a read row of 64 bytes would be fewer than 16 elements
@@ -268,10 +268,12 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
 // here against 24.0 / 25.4 with the long tiles; rows that are not whole lines 26.6 against 34.3, and 27 against 25.4) or
 // when it has at most 12 MiB (bf16 2048^2 3.6 us against 4.0, 2000 x 3000 6.9 against 8.4, u8 2000 x 3000 4.4 against
 // 6.2; fp32 2000 x 3000, 24 MB, 11 against 10.4), both sides holding at least one vector.  Byte matrices whose rows are not
-// whole cache lines are taken up to 40 MiB, in tiles of 256 x 256: the strips of the other file need more of them to fill
-// the part, its fixed tiles share lines (3001 x 7001, pack / unpack, 16.2 / 15.2 us -> 13.6 / 14.0; 5000^2 17.0 / 15.9 ->
-// 14.9 / 14.3; 5600^2 18.3 / 17.8 -> 13.7 / 13.9; 6001 x 6403 26.2 / 25.6 -> 22.2 / 23.1; but 7000^2, 47 MiB, 30.3 / 28.3
-// -> 31.5 / 31.1, and 4096^2, whole lines, 7.2 -> 7.7).
+// whole cache lines are taken up to 40 MiB, in tiles of 128 x 128 up to 23 MiB and of 256 x 256 above: the strips of the other
+// file need more of them to fill the part, its fixed tiles share lines.  Fixed tiles / 128 x 128 / 256 x 256, packing, over
+// 700 MB of buffers: 4097^2 16.2 / 11.8 / 15.2 us, 4803^2 17.5 / 13.6 / 16.2, 5017^2 18.2 / 15.9 / 16.3, 5616^2 21.3 / 17.3 / 15.3,
+// 6395^2 28.7 / 26.1 / 24.0 (7000^2, 47 MiB, 30.3 with the fixed tiles and 31.5 with 256 x 256; 4096^2, whole lines, 7.2 and 7.7).
+// Over three sets of buffers, which the Infinity Cache holds: 11.3 / 10.4 / 13.6, 12.1 / 13.0 / 15.1, 12.4 / 15.7 / 15.9, 18.0 / 17.1 /
+// 13.7, 20.7 / 25.4 / 23.0, so above 23 MiB copies between cached buffers lose up to a third and the others gain as much.
 template <bool PACK>
 bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd, uint64_t nbatch, uint32_t Q, uint32_t unit,
                           hipStream_t stream, int* rc) {

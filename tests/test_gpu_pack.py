@@ -816,8 +816,9 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
     many = 70_000_000 // es
     cases += [((many // (n * es) // es, n), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
     cases += [((n, many // (n * es) // es + 1), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
-    if es == 1:  # 16 to 40 MiB with rows that are not whole lines
-        cases += [((4099, 4100), lambda x: x.t()), ((5001, 8191), lambda x: x.t()), ((4100, 4224), lambda x: x[:, 1:4097].t())]
+    if es == 1:  # 12 to 40 MiB with rows that are not whole lines, on both sides of the 23 MiB at which the tile changes
+        cases += [((4099, 4100), lambda x: x.t()), ((4909, 4911), lambda x: x.t()), ((4913, 4915), lambda x: x.t()),
+                  ((5001, 8191), lambda x: x.t()), ((4100, 4224), lambda x: x[:, 1:4097].t())]
     if es == 8:  # both sides of the 2 MiB at which the tile of small matrices changes
         cases += [((511, 512), lambda x: x.t()), ((513, 512), lambda x: x.t()), ((3, 300, 305), lambda x: x.transpose(1, 2)),
                   ((1000, 1555), lambda x: x[:, 3:].t())]
