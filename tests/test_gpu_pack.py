@@ -805,7 +805,7 @@ def test_stream_send_tensor_semantics():
 def test_transposes_with_a_short_side_and_small_ones(dtype):
     # the tiles of narrow_transpose_kernels.hip: sides of one vector, a vector and a bit, and the edges of every tile length
     # (64, 128, 256, 512 bytes) on either side, long sides that are no whole tiles, batches, a packed side spanning two
-    # dimensions, views that start inside a row; the larger ones take the tiles used when there are many
+    # dimensions, views that start inside a row
     es = torch.empty(0, dtype=dtype).element_size()
     g = torch.Generator().manual_seed(33)
     info = torch.iinfo(dtype)
@@ -813,9 +813,13 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
     cases = [((2 * 128 // es + 5, n), lambda x: x.t()) for n in short] + [((n, 2 * 128 // es + 5), lambda x: x.t()) for n in short]
     cases += [((3, 70, 40), lambda x: x.transpose(1, 2)), ((2, 5, 33, 24), lambda x: x.permute(0, 3, 1, 2)[:, 1:]),
               ((4, 65, 300), lambda x: x[:, 1:, 7:40].transpose(1, 2)), ((1029, 700), lambda x: x[:, 3:].t())]
-    many = 70_000_000 // es
-    cases += [((many // (n * es) // es, n), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
-    cases += [((n, many // (n * es) // es + 1), lambda x: x.t()) for n in (24, 64 // es + 16, 128 // es, 272 // es, 384 // es)]
+    # 16 MiB and more take a tile length of 64, 128, 256 or 512 bytes for the short side: sides that get each of them
+    # (8-byte elements: 128 for the first), on either side of the matrix, the long side no whole tiles
+    for side in (48 if es < 8 else 64, 64, 128, 160, 200, 272, 300, 384, 512):
+        n = side // es
+        rows = (17 << 20) // (n * es) | 1
+        assert rows * n * es >= 16 << 20 and n * es <= 512
+        cases += [((rows, n), lambda x: x.t()), ((n, rows), lambda x: x.t())]
     if es == 1:  # 12 to 40 MiB with rows that are not whole lines, on both sides of the 23 MiB at which the tile changes
         cases += [((4099, 4100), lambda x: x.t()), ((4909, 4911), lambda x: x.t()), ((4913, 4915), lambda x: x.t()),
                   ((5001, 8191), lambda x: x.t()), ((4100, 4224), lambda x: x[:, 1:4097].t())]
