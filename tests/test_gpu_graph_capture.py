@@ -156,7 +156,8 @@ def test_strided_copy_forms_replay():
     g = torch.Generator(device=DEV).manual_seed(9)
     cases = [(torch.int16, (300, 4096), lambda x: x[:, 1:3581]),          # ragged rows of 7160 bytes at an odd column
              (torch.int16, (300, 4096), lambda x: x[:, 1:3585]),          # whole chunks from a skewed base
-             (torch.int32, (257, 1031), lambda x: x[:, 3:].t()),          # transposing, written rows off the cache lines
+             (torch.int32, (257, 1031), lambda x: x[:, 3:].t()),          # transposing, the tiles of small views
+             (torch.int32, (1801, 1831), lambda x: x[:, 3:].t()),         # transposing, windows that start on cache lines
              (torch.uint8, (600, 1000), lambda x: x[5:, 7:900])]          # one-byte units
     views, outs, backs, xs = [], [], [], []
     for dt, shape, view_of in cases:

@@ -647,15 +647,55 @@ def test_transposing_views_interior_and_edge_tiles(dtype):
 
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.int16, torch.int32, torch.int64])
 def test_transposes_whose_written_rows_start_inside_cache_lines(dtype):
-    # written rows that start anywhere in a cache line, with the kernel the library picks for them (both kernels, forced
-    # in turn, run in tests/tuning_variants.py): extents of exactly one tile, of a tile and a bit, shorter than the early start of a
-    # window, batches, offsets, a packed side spanning two dimensions
+    # written rows that start anywhere in a cache line, with the kernel the library picks for them (the kernels with windows
+    # that start on lines are forced on such sizes in tests/tuning_variants.py; views of up to 12 MiB take the small tiles of
+    # narrow_transpose_kernels.hip, see the next test for larger ones): extents of exactly one tile, of a tile and a bit, a few
+    # elements, batches, offsets, a packed side spanning two dimensions
     g = torch.Generator().manual_seed(18)
     info = torch.iinfo(dtype)
     t = 256 // torch.empty(0, dtype=dtype).element_size()
     cases = [((t, t + 1), lambda x: x.t()), ((t + 3, t), lambda x: x.t()), ((2 * t + 5, 3 * t + 7), lambda x: x[1:, 2:].t()),
              ((7, t + 9), lambda x: x.t()), ((t + 9, 7), lambda x: x.t()), ((3, t + 2, t + 1), lambda x: x.transpose(1, 2)),
              ((2, t + 1, 2, 300 // (t // 32 + 1) + t), lambda x: x.permute(0, 3, 2, 1)[:, 1:]), ((1100, 1031), lambda x: x[:, 5:].t())]
+    for shape, view_of in cases:
+        host = torch.randint(info.min, info.max, shape, dtype=dtype, generator=g)
+        dev = host.to(DEV)
+        view, hview = view_of(dev), view_of(host)
+        s = Slice.of_tensor(view)
+        out = staging.pack(view, s)
+        sync()
+        assert torch.equal(out.cpu(), hview.contiguous().flatten()), (shape, dtype)
+        back = torch.full_like(dev, 7)
+        staging.unpack(back, s, out)
+        sync()
+        ref = torch.full_like(host, 7)
+        view_of(ref).copy_(hview)
+        assert torch.equal(back.cpu(), ref), (shape, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.int16, torch.int32, torch.int64])
+def test_large_transposes_whose_written_rows_start_inside_cache_lines(dtype):
+    # the sizes from which the library takes the kernels whose windows start on cache lines: 2-, 4- and 8-byte elements above
+    # 12 MiB (a window per tile), bytes from 1024 segments of 256 x 256 on (strips); bytes between 40 MiB and that take fixed
+    # tiles.  Extents just past the 512 bytes of a short side, whole tiles and tiles and a bit on either side, a batch, a
+    # packed side that spans two dimensions, views that start inside a row, matrices of just under and over 12 MiB
+    es = torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator().manual_seed(19)
+    info = torch.iinfo(dtype)
+    if es == 1:
+        cases = [((8200, 8195), lambda x: x.t()), ((2, 5801, 5803), lambda x: x.transpose(1, 2)), ((8193, 8201), lambda x: x[1:, 5:].t()),
+                 ((7001, 6501), lambda x: x.t())]
+    else:
+        t = 256 // es
+        cases = []
+        for side in (2 * t + 1, 3 * t, 3 * t + 7, 5 * t - 1):
+            other = (13 << 20) // (side * es) | 1
+            cases += [((side, other), lambda x: x.t()), ((other, side), lambda x: x.t())]
+        n = int(((12 << 20) // es) ** 0.5)
+        cases += [((n - 1, n), lambda x: x.t()), ((n + 2, n + 1), lambda x: x.t())]
+        m = int(((5 << 20) // es) ** 0.5) | 1
+        cases += [((3, m, m + 2), lambda x: x.transpose(1, 2)), ((m, 3, m + 2), lambda x: x.permute(2, 0, 1)),
+                  ((2 * m, 2 * m + 9), lambda x: x[3:, 5:].t())]
     for shape, view_of in cases:
         host = torch.randint(info.min, info.max, shape, dtype=dtype, generator=g)
         dev = host.to(DEV)
