@@ -3,7 +3,7 @@
 // The tiles of transpose_kernels.hip are 256 or 512 bytes long on both sides, so a view whose memory-contiguous extent
 // or whose packed rows are shorter than that (the keys of an attention layer sent as [.., head dim, sequence], a tall
 // matrix of a few columns) fills only part of them, and a small view makes too few of them for 256 CUs.  Here the two
-// sides of a tile have lengths of their own: 64 to 512 bytes along the short side, what a tile of 8 to 64 KiB leaves
+// sides of a tile have lengths of their own: 64 to 512 bytes along the short side, what a tile of 2 to 64 KiB leaves
 // along the other.
 //
 // A tile is read as rows i of consecutive elements j and written as rows j of consecutive elements i: packing, i runs
@@ -50,8 +50,10 @@ __device__ __forceinline__ u32x4 shift_down(u32x4 v, uint32_t bytes) {
 //   * a lane stores its vector as one group, sixteen lanes a whole turn, whatever the key;
 //   * on the way out a lane collects E elements of one column from E consecutive read rows, as 32-bit words (narrower
 //     elements: 2 or 4 columns at once, sorted out in registers).  The NIV lanes that take different blocks of one column
-//     see different keys (M apart), the 64 / NIV word columns beside them fill the rest of the turn: no two of the 64
-//     lanes meet in a bank at different addresses.
+//     see different keys (M apart), the 64 / NIV word columns beside them fill the rest of the turn: while the read rows
+//     are whole blocks, no two of the 64 lanes meet in a bank at different addresses.  The last vector of a ragged row
+//     starts inside a block and sees two keys, i.e. up to two addresses in a bank; words of 8 bytes take two turns anyway,
+//     three when ragged.
 template <typename T, int THREADS, bool PACK, int TI, int TJ>
 __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowArgs a) {
     constexpr uint32_t ES = sizeof(T), E = 16 / ES;

@@ -9,7 +9,7 @@
 //                             straddling a row boundary moves as two overlapping vectors
 //   slice_unpack_lines_kernel unpacks of such rows from 256 bytes on: whole cache lines of the written side
 //   slice_units_kernel        runs shorter than (a few) chunks: the strided side unit by unit, consecutive lanes on
-//                             consecutive units (slice_gather_kernel from 2^31 units on)
+//                             consecutive units (slice_gather_kernel from 2^31 units on and for a few planes side by side)
 //   contiguous_copy_kernel    one run of any alignment: rows on the destination's 1 KiB boundaries
 // (views whose memory-contiguous dimension is not the innermost one go to the LDS-tiled
 // transposing kernels instead).  The host picks the form per launch from the canonical slice.
@@ -395,13 +395,10 @@ __global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
 // come from one full decode per chunk followed by an odometer over the run and the innermost dimension outside it; a full
 // decode is repeated only when that dimension wraps.  Strided-side accesses are NOT non-temporal: the lanes of a wavefront
 // return to the same cache lines for every unit of their chunks.
-constexpr int kGatherUnroll = 1;
-
 template <int U, bool PACK, bool WIDE, int NDIM>
 __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) {
     using T = typename UnitType<U>::type;
     constexpr int VU = 16 / U;
-    constexpr int UN = kGatherUnroll;
     const uint64_t wg = a.wg0 + blockIdx.x;
     uint64_t tile;
     uint32_t v;
@@ -409,86 +406,68 @@ __global__ __launch_bounds__(kPackThreads) void slice_gather_kernel(PackArgs a) 
     char* __restrict__ packed = a.packed[v];
     using M = typename UnitType<U>::mem;  // the strided side may be less aligned than the unit
     M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
-    const uint64_t c0 = tile * (kPackThreads * UN) + threadIdx.x;
+    const uint64_t c = tile * kPackThreads + threadIdx.x;
     const int nd = NDIM >= 0 ? NDIM : a.dims.ndim;
     const uint64_t run = a.dims.run;
     const uint64_t size_last = a.dims.size[nd - 1];
     const uint64_t step_last = a.dims.stride[nd - 1] - run;  // from one past a run's end to the start of the next run
-    const uint64_t safe_first = a.shift ? VU - a.shift : 0;  // first unit of the view's first whole chunk (the host checks there is one)
+    // first unit of the view's first whole chunk (the host checks there is one)
+    const uint64_t safe_first = a.shift ? VU - a.shift : 0;
+    const uint64_t tb = c * VU;
+    const uint64_t first = tb - a.shift;
+    const bool full = c < a.nchunks && tb >= a.shift && first + VU <= a.total;
 
-    uint64_t off[UN][VU];
-    bool full[UN], edge[UN];
-#pragma unroll
-    for (int i = 0; i < UN; ++i) {
-        const uint64_t c = c0 + (uint64_t)i * kPackThreads;
-        const uint64_t tb = c * VU;
-        const uint64_t first = tb - a.shift;
-        full[i] = c < a.nchunks && tb >= a.shift && first + VU <= a.total;
-        edge[i] = c < a.nchunks && !full[i];
-        if (full[i]) {
-            uint64_t col;
-            uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
-            uint64_t ilast;  // index along the innermost dimension outside the run
-            if constexpr (WIDE) {
-                ilast = ((first - col) / run) % size_last;
-            } else {
-                uint32_t row, c32, q, i;
-                a.dims.run_div.divmod((uint32_t)first, row, c32);
-                a.dims.size_div[nd - 1].divmod(row, q, i);
-                ilast = i;
-            }
-            off[i][0] = loc;
-#pragma unroll
-            for (int j = 1; j < VU; ++j) {
-                ++col;
-                ++loc;
-                if (col == run) {
-                    col = 0;
-                    ++ilast;
-                    loc += step_last;
-                    if (ilast == size_last) {
-                        loc = decode<WIDE, NDIM>(a.dims, first + j, &col);
-                        ilast = 0;
-                    }
-                }
-                off[i][j] = loc;
-            }
+    uint64_t off[VU];
+    if (full) {
+        uint64_t col;
+        uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
+        uint64_t ilast;  // index along the innermost dimension outside the run
+        if constexpr (WIDE) {
+            ilast = ((first - col) / run) % size_last;
         } else {
-#pragma unroll
-            for (int j = 0; j < VU; ++j) off[i][j] = 0;  // a valid unit: the view is not empty
+            uint32_t row, in_row, q, i;
+            a.dims.run_div.divmod((uint32_t)first, row, in_row);
+            a.dims.size_div[nd - 1].divmod(row, q, i);
+            ilast = i;
         }
+        off[0] = loc;
+#pragma unroll
+        for (int j = 1; j < VU; ++j) {
+            ++col;
+            ++loc;
+            if (col == run) {
+                col = 0;
+                ++ilast;
+                loc += step_last;
+                if (ilast == size_last) {
+                    loc = decode<WIDE, NDIM>(a.dims, first + j, &col);
+                    ilast = 0;
+                }
+            }
+            off[j] = loc;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < VU; ++j) off[j] = 0;  // a valid unit: the view is not empty
     }
     union Chunk {
         uint4 v;
         T e[VU];
     };
-    Chunk d[UN];
+    Chunk d;
     if constexpr (PACK) {
 #pragma unroll
-        for (int i = 0; i < UN; ++i)
-#pragma unroll
-            for (int j = 0; j < VU; ++j) d[i].e[j] = strided[off[i][j]];
-#pragma unroll
-        for (int i = 0; i < UN; ++i)
-            if (full[i]) store16_aligned(packed + ((c0 + (uint64_t)i * kPackThreads) * VU - a.shift) * U, d[i].v);
+        for (int j = 0; j < VU; ++j) d.e[j] = strided[off[j]];
+        if (full) store16_aligned(packed + first * U, d.v);
     } else {
+        d.v = load16_aligned(packed + (full ? first : safe_first) * U);
+        if (full) {
 #pragma unroll
-        for (int i = 0; i < UN; ++i) {
-            const uint64_t first = (c0 + (uint64_t)i * kPackThreads) * VU - a.shift;
-            d[i].v = load16_aligned(packed + (full[i] ? first : safe_first) * U);
+            for (int j = 0; j < VU; ++j) strided[off[j]] = d.e[j];
         }
-#pragma unroll
-        for (int i = 0; i < UN; ++i)
-            if (full[i]) {
-#pragma unroll
-                for (int j = 0; j < VU; ++j) strided[off[i][j]] = d[i].e[j];
-            }
     }
     // ragged first and last chunk of the view: unit by unit
-#pragma unroll
-    for (int i = 0; i < UN; ++i) {
-        if (edge[i]) move_chunk_by_units<U, PACK, WIDE, NDIM>(a, reinterpret_cast<char*>(strided), packed, c0 + (uint64_t)i * kPackThreads);
-    }
+    if (c < a.nchunks && !full) move_chunk_by_units<U, PACK, WIDE, NDIM>(a, reinterpret_cast<char*>(strided), packed, c);
 }
 
 // Contiguous copy between byte ranges of any alignment (a contiguous view, the "transfer" of a staging buffer):
@@ -921,9 +900,10 @@ static int copy_deep_view(char* base, char* packed, const mhip_slice_t& s, uint3
 // 0:1784 0.69 -> 0.73, pitch 14335 0.68 -> 0.73, fp32 rows of 1024 at pitch 8191 0.70 -> 0.75.  Rows of whole lines
 // measure the same either way or better (64 of 256 fp32 columns 0.57 -> 0.63; bf16 columns 0:1792 0.746 both ways), so
 // every single-view pack of whole chunks takes the shares (the eight column blocks of one tensor in one launch, where
-// the view index already pins each view to one XCD, lose with them: 0.78 -> 0.68).  For short runs see slice_units_kernel.  The two-vector form and the line-by-line unpack take them for rows of 6 KiB and
-// more (bf16 [16384, 14336], columns c:c+7166, packing 0.75 -> 0.78, unpacking 0.72 -> 0.755; rows of 7160 bytes +0.02 /
-// +0.03 to +0.10; rows of 3580 bytes -0.02 either way, so shorter rows keep the plain mapping).
+// the view index already pins each view to one XCD, lose with them: 0.78 -> 0.68).  For short runs see slice_units_kernel.
+// The two-vector form and the line-by-line unpack take them for rows of 6 KiB and more (bf16 [16384, 14336], columns
+// c:c+7166, packing 0.75 -> 0.78, unpacking 0.72 -> 0.755; rows of 7160 bytes +0.02 / +0.03 to +0.10; rows of 3580 bytes
+// -0.02 either way, so shorter rows keep the plain mapping).
 //
 // Unpacks of whole chunks write the strided side in 1 KiB pieces cut on the packed side's grid.  With units under 16
 // bytes (a view that starts 2-8 bytes past a 16-byte boundary, a pitch that is not a multiple of 16) every piece
@@ -1018,9 +998,11 @@ static int copy_views(char* base, char* const* packed, const mhip_slice_t* views
             // 1-byte units 263 B 10.1 / 12.6, 519 B 18.5 / 19.1, 1031 B 32.3 / 30.9; 2-byte units 262 B 8.8 / 12.1, 1030 B
             // 25.4 / 26.4, 1544 B 25.6 / 24.9, 3080 B 26.2 / 24.2, but two or eight views in one launch of 1222 B 8.4 / 10.4
             // and 29 / 32, of 1790 B 11.2 / 13.1 and 42 / 42.7; 4-byte units 260 B 8.5 / 11.8, 2052 B 23.6 / 24.4, 4104 B
-            // 24.6 / 24.4.  Unpacking: 1-byte units 199 B 11.6 / 12.4, 263 B 13.4 / 10.9; 2-byte units 198 B 9.1 / 12.5, 262 B 10.6 / 10.8, 398 B 14.1 / 13.0; 4-byte units 260 B 9.1 /
-            // 9.3, 516 B 17.1 / 15.5.  From 2^31 units on slice_gather_kernel takes the short rows, which loses earlier.
-            uint64_t units_below = (PACK ? (unit == 1 ? 512 : unit > 2 ? 4096 : nbatch == 1 ? 1280 : 2048) : 256) / unit;  // row length in units
+            // 24.6 / 24.4.  Unpacking: 1-byte units 199 B 11.6 / 12.4, 263 B 13.4 / 10.9; 2-byte units 198 B 9.1 / 12.5,
+            // 262 B 10.6 / 10.8, 398 B 14.1 / 13.0; 4-byte units 260 B 9.1 / 9.3, 516 B 17.1 / 15.5.  From 2^31 units on
+            // slice_gather_kernel takes the short rows, which loses earlier.
+            const uint64_t bytes_below = !PACK ? 256 : unit == 1 ? 512 : unit > 2 ? 4096 : nbatch == 1 ? 1280 : 2048;
+            uint64_t units_below = bytes_below / unit;  // row length in units
             if (!fits32 && unit == 1) units_below = 64;
             if (!fits32 && unit == 2) units_below = 128;
             if (first.run < units_below && first.total >= 2 * vu)

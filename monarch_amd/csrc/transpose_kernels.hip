@@ -818,7 +818,7 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // tile, 2 strips (1- and 2-byte elements).
     bool lines = false, strips = false;
     uint32_t seg_chunks = 2;
-    if (vec && !big && (PACK ? Sc : Q) >= tile) {
+    if (vec && !big) {
         uint64_t written = PACK ? ((uint64_t)(uintptr_t)packed | Q * unit) : ((uint64_t)(uintptr_t)base + c.offset * unit);
         if (!PACK)
             for (int k = 0; k < c.ndim; ++k)

@@ -1,8 +1,9 @@
 """Random cases for the differential tests of the GPU entry points (tests/test_gpu_fuzz.py): Slice pack / unpack against
 numpy indexing, reduces and fp8 buckets against the CPU oracle.  Shapes are drawn around the sizes at which the library
-switches kernels (tile, chunk, block and vector widths and their neighbours; the sizes of 2 MiB and more from which it takes other
-tiles or streams have tests of their own in tests/test_gpu_pack.py), buffers start at odd alignments, and guard zones either side of every buffer catch stray writes.  Each `*_case` function runs one case and raises AssertionError
-naming it; run as a program it repeats them for a number of seconds: python tests/fuzz_cases.py SECONDS SEED [pack|many|reduce|scatter|fp8 ...]."""
+switches kernels (tile, chunk, block and vector widths and their neighbours; the sizes of 2 MiB and more from which it takes
+other tiles or streams have tests of their own in tests/test_gpu_pack.py), buffers start at odd alignments, and guard zones
+either side of every buffer catch stray writes.  Each `*_case` function runs one case and raises AssertionError naming it; run
+as a program it repeats them for a number of seconds: python tests/fuzz_cases.py SECONDS SEED [pack|many|reduce|scatter|fp8 ...]."""
 import ctypes as C
 import math
 import os
