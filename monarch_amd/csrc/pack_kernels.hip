@@ -296,12 +296,11 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
 // line once.  The two sides' orders meet in 1 KiB of LDS (a single-wavefront workgroup; both LDS orders are linear).
 //
 // Bound by the lines of the strided side: all of them cross HBM, and an unpack, which fills them in part, has them read
-// as well as written.  In the order of the kernel this one replaces a lane owned the 16 bytes of one packed vector on the
-// strided side as well, so that every access of a wavefront touched 16 times (1-byte units) to 4 times the lines.  Pack /
-// unpack of x[:, ::k] over [8192, k * 4096], before -> now, us (in brackets what the lines need at 5.5 TB/s): u8 k=2
-// 59.8 / 84.9 -> 26.6 / 31.9 [18 / 31], k=4 60.5 / 154 -> 31.1 / 56.5 [30 / 55]; bf16 k=2 60.6 / 87.1 -> 36.0 / 60.0
-// [37 / 61], k=4 61.2 / 156 -> 54 / 110 [61 / 110]; f32 k=2 68.0 / 126 -> 60.7 / 118, k=4 111 / 237 -> 108 / 222; f64 k=8
-// 209 / 460 -> 199 / 451.
+// as well as written.  In the order of slice_gather_kernel a lane owns the 16 bytes of one packed vector on the strided side
+// as well, so that every access of a wavefront touches 16 times (1-byte units) to 4 times the lines.  Pack / unpack of
+// x[:, ::k] over [8192, k * 4096], that order -> this one, us: u8 k=2 59.5 / 82.8 -> 19.7 / 24.9, k=4 61.3 / 154 -> 30.1 / 54.7;
+// bf16 k=2 61.1 / 87.1 -> 34.4 / 58.6, k=4 61.9 / 157 -> 54.7 / 108; f32 k=2 67.2 / 120 -> 61.3 / 118, k=4 112 / 232 -> 108 / 220; f64
+// k=8 433 / 910 -> 412 / 901.
 // A lane decodes up to 16 units, so the arithmetic counts as well: the number of dimensions is known at compile time up to
 // three, and views of single units (RUN1) are spared the division by the run: channels of images packed side by side, u8
 // [13, 50176, 3] -> [13, 3, 50176] 6.7 / 7.8 -> 3.5 / 4.6 us (in the order of the kernel this one replaces 4.8 / 10.9), bf16
