@@ -233,10 +233,10 @@ static uint32_t narrow_tile_bytes(uint64_t bytes) {
 // Which tile: from 16 MiB on, the short side's length from narrow_tile_bytes and the other side's so that the two lengths
 // multiply to 64 KiB (tiles of 64, 32, 16, 8 KiB of 1-, 2-, 4-, 8-byte elements); below that 128 x 128 bytes, which makes
 // more workgroups (bf16 16384 x 20: 2.4 us against 3.0, 65536 x 64 (8.4 MB) 3.6 against 3.8; 16.8 MB of keys of 64 bytes
-// 8.6 against 7.5, of u8 keys of 64 bytes 8.6 against 7.5).  Of 8-byte elements that tile is 16 x 16 in 2 KiB, good for the
-// smallest only; from 2 MiB on they take 256 x 256 bytes (f64 pack / unpack, 128 x 128 and 256 x 256: 443^2 2.5 / 2.7 and 2.6 /
-// 2.9, 627^2 3.1 / 3.3 and 2.9 / 2.9, 887^2 4.8 / 5.1 and 4.0 / 3.9, 1145^2 6.7 / 6.5 and 5.8 / 5.7, the tiles of
-// transpose_kernels.hip 6.0 / 6.0).
+// 8.6 against 7.5, of u8 keys of 64 bytes 8.6 against 7.5).  Of 8-byte elements that tile is 16 x 16 in 2 KiB: matrices of
+// 4 MiB and more whose sides are both longer than 512 bytes take 256 x 256 bytes (f64 pack / unpack, 128 x 128 and 256 x 256: 627^2
+// 3.1 / 3.3 and 2.9 / 2.9, 640^2 3.1 / 3.2 and 3.3 / 3.1, 887^2 4.8 / 5.1 and 4.0 / 3.9, 1145^2 6.7 / 6.5 and 5.8 / 5.7, where the
+// tiles of transpose_kernels.hip take 6.0 / 6.0; [3584, 16, 16] 4.5 / 4.4 and 6.5 / 6.4).
 template <typename T, bool PACK>
 static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     constexpr uint32_t ES = sizeof(T);
@@ -262,7 +262,7 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
         return launch_narrow<T, PACK, 512, 128>(a, nbatch, stream);
     }
     if constexpr (ES == 8)
-        if (bytes >= (2ull << 20)) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+        if (bytes >= (4ull << 20) && ib > 512 && jb > 512) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
     return launch_narrow<T, PACK, 128, 128>(a, nbatch, stream);
 }
 

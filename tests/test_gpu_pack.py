@@ -863,8 +863,8 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
     if es == 1:  # 12 to 40 MiB with rows that are not whole lines, on both sides of the 23 MiB at which the tile changes
         cases += [((4099, 4100), lambda x: x.t()), ((4909, 4911), lambda x: x.t()), ((4913, 4915), lambda x: x.t()),
                   ((5001, 8191), lambda x: x.t()), ((4100, 4224), lambda x: x[:, 1:4097].t())]
-    if es == 8:  # both sides of the 2 MiB at which the tile of small matrices changes
-        cases += [((511, 512), lambda x: x.t()), ((513, 512), lambda x: x.t()), ((3, 300, 305), lambda x: x.transpose(1, 2)),
+    if es == 8:  # both sides of the 4 MiB at which the tile of small matrices changes
+        cases += [((723, 725), lambda x: x.t()), ((725, 727), lambda x: x.t()), ((3, 419, 421), lambda x: x.transpose(1, 2)),
                   ((1000, 1555), lambda x: x[:, 3:].t())]
     for shape, view_of in cases:
         host = torch.randint(info.min, info.max, shape, dtype=dtype, generator=g)
