@@ -237,6 +237,8 @@ static uint32_t narrow_tile_bytes(uint64_t bytes) {
 // 4 MiB and more whose sides are both longer than 512 bytes take 256 x 256 bytes (f64 pack / unpack, 128 x 128 and 256 x 256: 627^2
 // 3.1 / 3.3 and 2.9 / 2.9, 640^2 3.1 / 3.2 and 3.3 / 3.1, 887^2 4.8 / 5.1 and 4.0 / 3.9, 1145^2 6.7 / 6.5 and 5.8 / 5.7, where the
 // tiles of transpose_kernels.hip take 6.0 / 6.0; [3584, 16, 16] 4.5 / 4.4 and 6.5 / 6.4).
+// Batches of matrices that fit 128 x 128 bytes keep that tile at any size: u8 [78125, 16, 16] 94 / 95 us, in tiles of 1024 x 64 of
+// which one matrix fills little 335 / 333; bf16 [39062, 16, 16] 45 / 46 and 97 / 98, [8544, 64, 64] 23.2 / 23.3 and 30.2 / 31.3.
 template <typename T, bool PACK>
 static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     constexpr uint32_t ES = sizeof(T);
@@ -244,7 +246,7 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
     const uint64_t bytes = nbatch * ib * jb / ES;
     if constexpr (ES == 1)
         if (ib > 512 && jb > 512 && bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
-    if (bytes >= (16ull << 20) && (ib <= 512 || jb <= 512)) {
+    if (bytes >= (16ull << 20) && (ib <= 512 || jb <= 512) && (ib > 128 || jb > 128)) {  // a long side to fill the tile with
         const bool short_j = jb <= ib;
         uint32_t n = narrow_tile_bytes(short_j ? jb : ib);
         if (ES == 8 && n == 64) n = 128;  // a read row of 64 bytes would be fewer than 16 elements

@@ -860,6 +860,9 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
         rows = (17 << 20) // (n * es) | 1
         assert rows * n * es >= 16 << 20 and n * es <= 512
         cases += [((rows, n), lambda x: x.t()), ((n, rows), lambda x: x.t())]
+    # batches of matrices that fit the smallest tile, which they keep from 16 MiB on, and of some that just do not
+    for a, b in ((max(16 // es, 8), 128 // es), (128 // es, 128 // es), (16, 128 // es + 1)):
+        cases += [(((17 << 20) // (a * b * es), a, b), lambda x: x.transpose(1, 2))]
     if es == 1:  # 12 to 40 MiB with rows that are not whole lines, on both sides of the 23 MiB at which the tile changes
         cases += [((4099, 4100), lambda x: x.t()), ((4909, 4911), lambda x: x.t()), ((4913, 4915), lambda x: x.t()),
                   ((5001, 8191), lambda x: x.t()), ((4100, 4224), lambda x: x[:, 1:4097].t())]
