@@ -527,16 +527,18 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
 // The same with n peers' payloads in one pass: every accumulator element crosses HBM once
 // (n + 8 bytes per element instead of 9n).  Peers are added in order, product rounded before
 // each add, so the result has the bits of n single-peer passes.
-// Only the codes of peers that exist are loaded.  Large buckets are bound by HBM, small ones (one round of wavefronts) by how
-// long a wavefront lives: three dependent table reads, then the data.  Two forms (kSmallBucketBlocks):
-//   * small buckets read the tables with scalar loads (5.9 M elements, 1 / 8 peers: 10.9 / 18.6 us, with the vector loads that
-//     the compiler makes of them in a kernel that stores through their results 11.9 / 19.2);
+// Only the codes of peers that exist are loaded.  Large buckets are bound by HBM, small ones (one to a few rounds of
+// wavefronts) by how long a wavefront lives: three dependent table reads, then the data.  Two kernels (kSmallBucketBlocks):
+//   * small buckets read the tables with scalar loads, beside the codes of up to eight peers, which are in flight first
+//     (fp8_dequant_accumulate_small_bucket_kernel);
 //   * large buckets lose with scalar loads (163 M elements, 5 / 7 peers: 366 / 422 us against 350 / 416) and gain from five
-//     wavefronts per SIMD instead of six (345 / 411).
-// The codes do not go ahead of the tables: the wait for a table entry is then one for the codes as well, since vector loads
-// return in order.  That form for all sizes / the two forms here: 0.8 M elements in 24 tensors, 4 peers 6.5 / 6.0 us; 5.9 M,
-// 1, 8 and 16 peers 12.1 / 10.9, 20.4 / 19.1, 30.5 / 29.3; 40 blocks, 4 peers 5.6 / 5.3; 2000 tensors of 10 to 600 elements, 8
-// peers 20.8 / 19.6; 163 M elements, 1, 2 and 5 peers 233 / 238, 265 / 264, 351 / 345.
+//     wavefronts per SIMD instead of six (345 / 411).  Their codes do not go ahead of the tables: the wait for a table entry
+//     is then one for the codes as well, since vector loads return in order (163 M elements, 1 and 5 peers 233 / 351 us; here
+//     238 / 345).
+// Small buckets in the large form with scalar tables / now, us: 0.82 M elements in 31 tensors, 2, 4 and 6 peers 4.28 / 3.76,
+// 4.59 / 4.06, 5.42 / 4.49; 4.6 M in 24 tensors, 1, 2, 4 and 8 peers 8.94 / 7.96, 9.64 / 8.67, 11.25 / 10.57, 14.37 / 13.73 (4.7 ->
+// 5.3 TB/s); 8.4 M in 61 tensors, 2 and 8 peers 15.9 / 15.0, 24.5 / 23.5; 23 M +-1 % (both at 5.9 TB/s), so the line stays where
+// the quantiser's is.  Codes behind the tables: 4.6 M elements, 2, 4 and 8 peers 9.18 / 10.91 / 14.09.
 constexpr int kMaxBucketPeers = 64;
 
 struct BucketPeersArgs {
@@ -588,8 +590,7 @@ __device__ __forceinline__ void dequant_accumulate_block_peers(const BucketPeers
         store(j, make_uint4(__float_as_uint(v[j][0]), __float_as_uint(v[j][1]), __float_as_uint(v[j][2]), __float_as_uint(v[j][3])));
 }
 
-template <bool SMALL>
-__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(SMALL ? 6 : 5, SMALL ? 8 : 5)))
+__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(5, 5)))
 void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
     const BucketArgs& a = p.b;
     const int lane = threadIdx.x & 63;
@@ -600,15 +601,15 @@ void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
         const bool full = begin + kBlock <= a.total;
         const uint64_t end = full ? begin + kBlock : a.total;
         uint32_t t_lo, t_hi;
-        span_tensors<SMALL>(a, begin, end, &t_lo, &t_hi);
+        span_tensors(a, begin, end, &t_lo, &t_hi);
         if (full && t_lo == t_hi) {
-            float* dst = tensor_at<SMALL>(a, t_lo, begin);
+            float* dst = tensor_at(a, t_lo, begin);
             dequant_accumulate_block_peers(p, b, lane, [&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
                                            [&](int j, const uint4& r) { store16_unaligned(dst + j * 256 + lane * 4, r); });
             continue;
         }
-        if (full && block_cut_once<SMALL>(a, t_lo, begin)) {
-            const CutBlock c = CutBlock::of<SMALL>(a, t_lo, begin);
+        if (full && block_cut_once(a, t_lo, begin)) {
+            const CutBlock c = CutBlock::of<false>(a, t_lo, begin);
             dequant_accumulate_block_peers(p, b, lane, [&](int j) { return c.load(j, lane); },
                                            [&](int j, const uint4& r) { c.store(j, lane, r); });
             continue;
@@ -617,6 +618,107 @@ void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
         dequant_bucket_block_careful(a, t_lo, t_hi, begin, end, lane, p.n, [&](uint32_t r) { return p.q[r]; },
                                      [&](uint32_t r) { return p.scales[r][b]; });
     }
+}
+
+// Small buckets, N peers (N == 8: eight and more), one block per wavefront.  The codes of the first N peers go first and the
+// look-up of the block's tensors runs beside them: the tables come through scalar loads, which do not wait for vector loads
+// in flight.  With the number of peers known all N * 4 code loads of a lane are in flight together (the form of large buckets
+// loads four peers at a time, and branches on each).
+template <int N>
+struct PeerCodes {
+    uint32_t codes[N][4];
+    float s[N];
+};
+
+template <int N>
+__device__ __forceinline__ void load_peers(PeerCodes<N>& c, const BucketPeersArgs& p, uint32_t r0, uint64_t b, int lane) {
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+        const uint8_t* q = p.q[r0 + g] + b * kBlock;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c.codes[g][j] = load4_unaligned(q + (uint32_t)(j * 256 + lane * 4));
+        c.s[g] = table_entry<true>(p.scales[r0 + g] + b);
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void add_peers(float (&v)[4][4], const PeerCodes<N>& c) {
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const auto p01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)c.codes[g][j], false);
+            const auto p23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)c.codes[g][j], true);
+            v[j][0] = v[j][0] + p01[0] * c.s[g];  // product rounded, then added
+            v[j][1] = v[j][1] + p01[1] * c.s[g];
+            v[j][2] = v[j][2] + p23[0] * c.s[g];
+            v[j][3] = v[j][3] + p23[1] * c.s[g];
+        }
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void load_and_add_peers(float (&v)[4][4], const BucketPeersArgs& p, uint32_t r0, uint64_t b, int lane) {
+    PeerCodes<N> c;
+    load_peers<N>(c, p, r0, b, lane);
+    add_peers<N>(v, c);
+}
+
+template <int N>
+__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(5, 8)))
+void fp8_dequant_accumulate_small_bucket_kernel(BucketPeersArgs p, uint64_t wg0) {
+    const BucketArgs& a = p.b;
+    const int lane = threadIdx.x & 63;
+    const uint64_t b = (wg0 + blockIdx.x) * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // see fp8_quantize_bucket_kernel
+    if (b >= a.nblocks) return;
+    const uint64_t begin = b * kBlock;
+    const bool full = begin + kBlock <= a.total;
+    const uint64_t end = full ? begin + kBlock : a.total;
+    PeerCodes<N> first;
+    if (full) load_peers<N>(first, p, 0, b, lane);
+    asm volatile("" ::: "memory");  // the loads above stay above the look-up
+    uint32_t t_lo, t_hi;
+    span_tensors<true>(a, begin, end, &t_lo, &t_hi);
+    auto whole_block = [&](auto&& load, auto&& store) {
+        float v[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint4 r = load(j);
+            v[j][0] = __uint_as_float(r.x); v[j][1] = __uint_as_float(r.y);
+            v[j][2] = __uint_as_float(r.z); v[j][3] = __uint_as_float(r.w);
+        }
+        add_peers<N>(v, first);
+        if constexpr (N == 8) {
+            uint32_t r = 8;
+            for (; r + 4 <= p.n; r += 4) load_and_add_peers<4>(v, p, r, b, lane);
+            if (r + 3 == p.n) load_and_add_peers<3>(v, p, r, b, lane);
+            else if (r + 2 == p.n) load_and_add_peers<2>(v, p, r, b, lane);
+            else if (r + 1 == p.n) load_and_add_peers<1>(v, p, r, b, lane);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            store(j, make_uint4(__float_as_uint(v[j][0]), __float_as_uint(v[j][1]), __float_as_uint(v[j][2]), __float_as_uint(v[j][3])));
+    };
+    if (full && t_lo == t_hi) {
+        float* dst = tensor_at<true>(a, t_lo, begin);
+        whole_block([&](int j) { return load16_unaligned(dst + j * 256 + lane * 4); },
+                    [&](int j, const uint4& r) { store16_unaligned(dst + j * 256 + lane * 4, r); });
+    } else if (full && block_cut_once<true>(a, t_lo, begin)) {
+        const CutBlock c = CutBlock::of<true>(a, t_lo, begin);
+        whole_block([&](int j) { return c.load(j, lane); }, [&](int j, const uint4& r) { c.store(j, lane, r); });
+    } else {
+        // more than two tensors, or the short last block
+        dequant_bucket_block_careful(a, t_lo, t_hi, begin, end, lane, p.n, [&](uint32_t r) { return p.q[r]; },
+                                     [&](uint32_t r) { return p.scales[r][b]; });
+    }
+}
+
+template <int N>
+static int launch_small_bucket(const BucketPeersArgs& p, hipStream_t stream) {
+    constexpr uint64_t per_wg = kBucketThreads / 64;
+    return launch_in_pieces((p.b.nblocks + per_wg - 1) / per_wg, kBucketThreads, 1, [&](uint64_t wg0, uint32_t count) {
+        MHIP_LAUNCH(fp8_dequant_accumulate_small_bucket_kernel<N>, dim3(count), dim3(kBucketThreads), 0, stream, p, wg0);
+    });
 }
 
 // shared by the entry points that quantise a bucket: `index` is a device pointer or null
@@ -800,13 +902,24 @@ int mhip_fp8_dequant_accumulate_bucket_many(void* const* d_acc_tensors, const ui
     p.b.total = total;
     p.b.nblocks = (total + kBlock - 1) / kBlock;
     p.b.ntensors = ntensors;
-    const uint64_t wgs = (p.b.nblocks + 3) / 4;
-    const uint64_t cap = max_workgroups(kBucketThreads);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     DeviceGuard guard(hs);
+    if (p.b.nblocks <= kSmallBucketBlocks) {
+        switch (n) {
+            case 1: return launch_small_bucket<1>(p, hs);
+            case 2: return launch_small_bucket<2>(p, hs);
+            case 3: return launch_small_bucket<3>(p, hs);
+            case 4: return launch_small_bucket<4>(p, hs);
+            case 5: return launch_small_bucket<5>(p, hs);
+            case 6: return launch_small_bucket<6>(p, hs);
+            case 7: return launch_small_bucket<7>(p, hs);
+            default: return launch_small_bucket<8>(p, hs);
+        }
+    }
+    const uint64_t wgs = (p.b.nblocks + 3) / 4;
+    const uint64_t cap = max_workgroups(kBucketThreads);
     const dim3 grid((uint32_t)(wgs > cap ? cap : wgs));
-    if (p.b.nblocks <= kSmallBucketBlocks) MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel<true>, grid, dim3(kBucketThreads), 0, hs, p);
-    else MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel<false>, grid, dim3(kBucketThreads), 0, hs, p);
+    MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel, grid, dim3(kBucketThreads), 0, hs, p);
     return launch_status();
 }
 

@@ -186,6 +186,29 @@ def test_dequant_accumulate_bucket_many_of_large_buckets(blocks, npeers):
         assert torch.equal(got.view(torch.int32), want.view(torch.int32)), indexed
 
 
+@pytest.mark.parametrize("npeers", [2, 5, 6, 7, 8, 10, 11, 12, 13])
+@pytest.mark.parametrize("total", [1023, 1024, 5 * 1024, 37 * 1024 + 1])
+def test_dequant_accumulate_bucket_many_of_small_buckets(total, npeers):
+    # every number of peers has a kernel of its own up to eight, and tails of one to three peers after that: the same bits as
+    # one pass per peer, on one tensor, on boundaries inside and between blocks, with codes that start at odd addresses
+    g = torch.Generator(device=DEV).manual_seed(total + npeers)
+    sizes = [total] if total <= 1024 else [1500, 548, 1, 0, 1024 - 7, total - 3066]
+    assert sum(sizes) == total
+    acc = torch.randn(total, device=DEV, generator=g)
+    want, store = acc.clone(), torch.full((total + 2,), 7.0, device=DEV)
+    one, many = (fp8.FlatBucket(list(torch.split(x, sizes))) for x in (want, store[1:-1]))
+    qs = [torch.randint(0, 120, (total + 1,), dtype=torch.uint8, device=DEV, generator=g)[r % 2: r % 2 + total] for r in range(npeers)]
+    ss = [torch.rand((total + 1023) // 1024, device=DEV, generator=g) for _ in range(npeers)]
+    for q, s in zip(qs, ss):
+        fp8.dequant_accumulate_bucket(one, q, s)
+    for indexed in (False, True):
+        store[1:-1] = acc
+        fp8.dequant_accumulate_bucket_many(many, qs, ss, indexed=indexed)
+        sync()
+        assert torch.equal(store[1:-1].view(torch.int32), want.view(torch.int32)), indexed
+        assert store[0].item() == 7.0 and store[-1].item() == 7.0
+
+
 def test_fused_bucket_forms_equal_two_step_pipeline():
     # ragged sizes around block boundaries, empty tensors, odd element alignment, NaN/Inf blocks
     g = torch.Generator().manual_seed(77)
