@@ -22,11 +22,9 @@ struct FastDiv32 {
     FastDiv32() = default;
     explicit FastDiv32(uint32_t divisor) {
         d = divisor ? divisor : 1;
-        uint32_t l = 0;
-        while ((1ull << l) < d) ++l;
-        shift = 31 + l;
-        const unsigned __int128 one = 1;
-        mul = (uint32_t)(((one << shift) + d - 1) / d);
+        const uint32_t l = d > 1 ? 32 - (uint32_t)__builtin_clz(d - 1) : 0;
+        shift = 31 + l;  // at most 62
+        mul = (uint32_t)(((1ull << shift) + d - 1) / d);
     }
     MHIP_HD uint32_t div(uint32_t n) const { return (uint32_t)(((uint64_t)n * mul) >> shift); }
     MHIP_HD void divmod(uint32_t n, uint32_t& q, uint32_t& r) const {

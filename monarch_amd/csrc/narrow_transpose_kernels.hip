@@ -10,8 +10,15 @@
 // over q and j over the memory-contiguous dimension c; unpacking, the other way round.  HBM-bound: 2 bytes of traffic
 // per byte moved.  Both sides move 16-byte vectors whatever the extents: the last vector of a row is moved back so that it
 // ends where the row ends.  bf16 [64, 4096, 64] -> [64, 64, 4096] (33.6 MB), pack / unpack: 95.8 / 104 us with the tiles
-// that fill a quarter of their lanes, 14.8 / 14.1 us here (4.5 / 4.8 TB/s); head dim 80: 98 / 82 -> 17.3 / 19.2,
-// 32: 94 / 81 -> 7.5 / 7.6; u8 head dim 128: 222 / 303 -> 12.4 / 13.2; bf16 1024^2: 3.3 / 3.4 -> 2.6 / 2.6.
+// that fill a quarter of their lanes, 15.6 / 14.9 us here (4.3 / 4.5 TB/s); head dim 80: 98 / 82 -> 16.9 / 19.2,
+// 32: 94 / 81 -> 8.0 / 7.6; u8 head dim 128: 222 / 303 -> 12.9 / 13.8; bf16 1024^2: 3.3 / 3.4 -> 2.4 / 2.4.
+//
+// Most launches are one or two rounds of workgroups, so what a wavefront issues before its first load and between its loads
+// and its stores is not hidden: tile numbers are decoded by multiplication (FastDiv32; the compiler's 64-bit divisions were
+// some 120 of 185 scalar instructions a wavefront), an address is one 32 x 32-bit multiply-add (ONE), rows and vectors of a
+// pass follow from those of the pass before.  With divisions and 64-bit multiplications / now, us: f32 512^2 2.77 / 2.58,
+// 1216^2 3.47 / 2.96, u8 [68359, 32, 32] 86 / 69, f32 [68359, 16, 16] 45.9 / 37, f32 [40, 2000, 128] 18.7 / 17.0, 1000 calls of all
+// types and sizes 0.92 x on average.
 #include "mhip_device.h"
 #include "pack_internal.h"
 
@@ -24,14 +31,19 @@ struct NarrowArgs {
     uint32_t vi, vj;              // read rows and columns a tile holds: the tile's own, or the extent where that is shorter
     uint32_t ti_count, tj_count;  // tiles along i and along j
     uint32_t nv;                  // vectors per read row
+    uint32_t row_step, vec_step;  // a pass of all lanes over the vectors of the read rows: lanes / nv and lanes % nv
     uint32_t write_through;       // how written vectors are stored, see try_narrow_transpose
     FastDiv32 nv_div;
-    uint64_t ntiles, per_xcd;     // each XCD takes a contiguous share of the tiles
-    uint64_t wg0;                 // workgroups of this copy launched before this grid
+    uint32_t ntiles, per_xcd;     // each XCD takes a contiguous share of the tiles
+    uint32_t wg0;                 // workgroups of this copy launched before this grid
+    FastDiv32 per_batch_div;      // tiles per matrix
+    FastDiv32 fast_div;           // tiles along the side that has fewer of them
+    uint32_t one_inner;           // consecutive q lie mem_pitch elements apart: one dimension after c
+    uint32_t mem_pitch;
     int n_inner, n_outer;         // dimensions after c (q -> memory offset) and before c (batch -> memory offset)
     FastDiv32 inner_div[kMaxCanonDims];
     uint64_t inner_stride[kMaxCanonDims];  // bytes
-    uint32_t outer_size[kMaxCanonDims];
+    FastDiv32 outer_div[kMaxCanonDims];
     uint64_t outer_stride[kMaxCanonDims];  // bytes
 };
 
@@ -54,7 +66,7 @@ __device__ __forceinline__ u32x4 shift_down(u32x4 v, uint32_t bytes) {
 //     are whole blocks, no two of the 64 lanes meet in a bank at different addresses.  The last vector of a ragged row
 //     starts inside a block and sees two keys, i.e. up to two addresses in a bank; words of 8 bytes take two turns anyway,
 //     three when ragged.
-template <typename T, int THREADS, bool PACK, int TI, int TJ>
+template <typename T, int THREADS, bool PACK, int TI, int TJ, bool ONE>
 __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowArgs a) {
     constexpr uint32_t ES = sizeof(T), E = 16 / ES;
     constexpr uint32_t GJ = TJ / E, GI = TI / E;
@@ -67,67 +79,75 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowA
     using Word = typename UnitType<(ES >= 4 ? ES : 4)>::type;
     __shared__ __attribute__((aligned(16))) char tile[TI * TJ * ES];
 
-    const uint64_t wg = a.wg0 + blockIdx.x;
-    const uint64_t id = (wg & 7) * a.per_xcd + (wg >> 3);
+    const uint32_t wg = a.wg0 + blockIdx.x;
+    const uint32_t id = (wg & 7) * a.per_xcd + (wg >> 3);
     if (id >= a.ntiles) return;
-    const uint32_t per_batch = a.ti_count * a.tj_count;
-    const uint64_t b = id / per_batch;
-    const uint32_t in_batch = (uint32_t)(id - b * per_batch);
+    uint32_t b, in_batch, slow, fast;
+    a.per_batch_div.divmod(id, b, in_batch);
     // the side with fewer tiles is the fast one: neighbouring workgroups share whole rows of it
-    uint32_t it, jt;
-    if (a.ti_count < a.tj_count) { jt = in_batch / a.ti_count; it = in_batch - jt * a.ti_count; }
-    else { it = in_batch / a.tj_count; jt = in_batch - it * a.tj_count; }
+    a.fast_div.divmod(in_batch, slow, fast);
+    const bool i_fast = a.ti_count < a.tj_count;
     // a tile that would hang over the edge is moved back inside; the overlap is written twice, same bytes
     const uint32_t I = PACK ? a.Q : a.Sc, J = PACK ? a.Sc : a.Q;
-    uint32_t i0 = it * TI, j0 = jt * TJ;
+    uint32_t i0 = (i_fast ? fast : slow) * TI, j0 = (i_fast ? slow : fast) * TJ;
     if (i0 + a.vi > I) i0 = I - a.vi;
     if (j0 + a.vj > J) j0 = J - a.vj;
-    char* __restrict__ mem = a.base;
-    {
-        uint64_t rem = b;
-        for (int k = a.n_outer - 1; k >= 0; --k) {
-            const uint64_t qd = rem / a.outer_size[k];
-            mem += (rem - qd * a.outer_size[k]) * a.outer_stride[k];
-            rem = qd;
-        }
+    const uint32_t q0 = PACK ? i0 : j0, c0 = PACK ? j0 : i0;
+    char* __restrict__ packed = a.packed + (((uint64_t)b * a.Sc + c0) * a.Q + q0) * ES;  // the tile's first element, on both sides
+    char* __restrict__ mem = a.base + (uint64_t)c0 * ES;
+    for (int k = a.n_outer - 1; k >= 0; --k) {
+        uint32_t rest, index;
+        a.outer_div[k].divmod(b, rest, index);
+        mem += index * a.outer_stride[k];
+        b = rest;
     }
-    char* __restrict__ packed = a.packed + b * a.Sc * (uint64_t)a.Q * ES;
-    auto q_offset = [&](uint32_t q) -> uint64_t {
-        uint64_t off = 0;
-        for (int k = a.n_inner - 1; k > 0; --k) {
-            uint32_t qd, r;
-            a.inner_div[k].divmod(q, qd, r);
-            off += (uint64_t)r * a.inner_stride[k];
-            q = qd;
+    if constexpr (ONE) mem += (uint64_t)q0 * a.mem_pitch * ES;
+    // addresses inside the tile: q and c counted from its first element
+    auto packed_at = [&](uint32_t q, uint32_t c) { return packed + ((uint64_t)c * a.Q + q) * ES; };
+    auto mem_at = [&](uint32_t q, uint32_t c) {
+        if constexpr (ONE) {
+            return mem + ((uint64_t)q * a.mem_pitch + c) * ES;
+        } else {
+            uint64_t off = 0;
+            uint32_t rest = q0 + q;
+            for (int k = a.n_inner - 1; k > 0; --k) {
+                uint32_t qd, r;
+                a.inner_div[k].divmod(rest, qd, r);
+                off += (uint64_t)r * a.inner_stride[k];
+                rest = qd;
+            }
+            return mem + (off + (uint64_t)rest * a.inner_stride[0] + (uint64_t)c * ES);
         }
-        return off + (uint64_t)q * a.inner_stride[0];
     };
 
     // ---- read side -> LDS: the tile's vectors numbered through, so that short rows leave no lane idle ----
     const uint32_t total = a.vi * a.nv;
+    const bool ragged_j = a.vj % E != 0;
     u32x4 d[RP];
+    uint32_t row[RP], vec[RP];
+    a.nv_div.divmod(threadIdx.x, row[0], vec[0]);
 #pragma unroll
     for (uint32_t p = 0; p < RP; ++p) {
+        if (p > 0) {  // every pass moves on by the same number of vectors
+            row[p] = row[p - 1] + a.row_step;
+            vec[p] = vec[p - 1] + a.vec_step;
+            if (vec[p] >= a.nv) {
+                vec[p] -= a.nv;
+                ++row[p];
+            }
+        }
         if (p * THREADS < total) {
-            uint32_t x = threadIdx.x + p * THREADS;
-            x = x < total ? x : total - 1;  // no load is predicated
-            uint32_t r, g;
-            a.nv_div.divmod(x, r, g);
-            const uint32_t col = g * E + E <= a.vj ? g * E : a.vj - E;
-            const char* src;
-            if constexpr (PACK) src = mem + q_offset(i0 + r) + (uint64_t)(j0 + col) * ES;
-            else src = packed + ((uint64_t)(i0 + r) * a.Q + j0 + col) * ES;
-            const uint4 v = load16_unaligned(src);
+            const uint32_t r = row[p] < a.vi ? row[p] : a.vi - 1;  // no load is predicated
+            uint32_t col = vec[p] * E;
+            if (ragged_j) col = col + E <= a.vj ? col : a.vj - E;
+            const uint4 v = load16_unaligned(PACK ? mem_at(r, col) : packed_at(col, r));
             d[p] = u32x4{v.x, v.y, v.z, v.w};
         }
     }
-    const bool ragged_j = a.vj % E != 0;
 #pragma unroll
     for (uint32_t p = 0; p < RP; ++p) {
-        const uint32_t x = threadIdx.x + p * THREADS;
-        if (x < total) {
-            uint32_t r, g;
-            a.nv_div.divmod(x, r, g);
+        const uint32_t r = row[p], g = vec[p];
+        if (r < a.vi) {
             u32x4 v = d[p];
             if (ragged_j) v = shift_down(v, g * E + E <= a.vj ? 0u : (g * E + E - a.vj) * ES);  // a vector that was moved back
             const uint32_t f = (r * GJ + g) ^ (((r / E) * M) & 15u);
@@ -189,9 +209,7 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowA
 #pragma unroll
             for (uint32_t k = 0; k < W; ++k) {
                 if (k == 0 || j + k < a.vj) {
-                    char* dst;
-                    if constexpr (PACK) dst = packed + ((uint64_t)(j0 + j + k) * a.Q + i0 + i) * ES;
-                    else dst = mem + q_offset(j0 + j + k) + (uint64_t)(i0 + i) * ES;
+                    char* dst = PACK ? packed_at(i, j + k) : mem_at(j + k, i);
                     if (a.write_through) store16_writethrough_raw(dst, out[k]);  // wave-uniform
                     else *reinterpret_cast<u32x4_unaligned*>(dst) = out[k];
                 }
@@ -212,11 +230,17 @@ static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     a.tj_count = (J + TJ - 1) / TJ;
     a.nv = (a.vj + E - 1) / E;
     a.nv_div = FastDiv32(a.nv);
-    a.ntiles = nbatch * a.ti_count * a.tj_count;
+    a.row_step = kLanes / a.nv;
+    a.vec_step = kLanes % a.nv;
+    // fewer than kFastDivLimit: a tile moves 256 bytes at least, and no GPU holds 2^31 times that (see try_narrow_transpose)
+    a.ntiles = (uint32_t)(nbatch * a.ti_count * a.tj_count);
     a.per_xcd = (a.ntiles + 7) / 8;
-    return launch_in_pieces(a.per_xcd * 8, kLanes, 8, [&](uint64_t wg0, uint32_t count) {
-        a.wg0 = wg0;
-        MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ>), dim3(count), dim3(kLanes), 0, stream, a);
+    a.per_batch_div = FastDiv32(a.ti_count * a.tj_count);
+    a.fast_div = FastDiv32(a.ti_count < a.tj_count ? a.ti_count : a.tj_count);
+    return launch_in_pieces((uint64_t)a.per_xcd * 8, kLanes, 8, [&](uint64_t wg0, uint32_t count) {
+        a.wg0 = (uint32_t)wg0;
+        if (a.one_inner) MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, true>), dim3(count), dim3(kLanes), 0, stream, a);
+        else MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, false>), dim3(count), dim3(kLanes), 0, stream, a);
     });
 }
 
@@ -284,6 +308,7 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
     const uint64_t Sc = c.dims[cd].size, bytes = nbatch * Sc * Q * unit;
     const uint64_t short_side = (Sc < Q ? Sc : Q) * unit;
     if (unit > 8 || short_side < 16) return false;
+    if (bytes / 256 >= kFastDivLimit) return false;  // every tile holds at least 16 x 16 bytes: tile numbers stay below 2^31
     if (short_side > 512 && bytes > (unit == 1 ? 40ull << 20 : 12ull << 20)) return false;
     NarrowArgs a{};
     uint64_t written = PACK ? (uint64_t)(uintptr_t)packed | (uint64_t)Q * unit : (uint64_t)(uintptr_t)(base + c.offset * unit);
@@ -294,7 +319,7 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
             a.inner_div[a.n_inner] = FastDiv32((uint32_t)c.dims[k].size);
             a.inner_stride[a.n_inner++] = stride;
         } else {
-            a.outer_size[a.n_outer] = (uint32_t)c.dims[k].size;
+            a.outer_div[a.n_outer] = FastDiv32((uint32_t)c.dims[k].size);
             a.outer_stride[a.n_outer++] = stride;
         }
         if (!PACK) written |= stride;
@@ -309,6 +334,9 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
     a.packed = packed;
     a.Sc = (uint32_t)Sc;
     a.Q = Q;
+    const uint64_t pitch = a.inner_stride[0] / unit;
+    a.one_inner = a.n_inner == 1 && pitch <= UINT32_MAX;
+    a.mem_pitch = (uint32_t)pitch;
     // Written rows that start on half cache lines are stored write-through (33.6 MB of keys 14.8 us against 16.5 through
     // the cache, unpacked rows of 64 bytes 7.6 against 8.5); others go through the cache, which combines what neighbouring
     // tiles share (rows of 4001 bf16 15.9 against 18.9, unpacked rows of 160 bytes 19.2 against 19.9), unless the launch

@@ -45,6 +45,10 @@ struct TransArgs {
     uint32_t outer_size[kMaxCanonDims];
     FastDiv32 outer_div[kMaxCanonDims];
     uint64_t outer_stride[kMaxCanonDims];
+    uint32_t one_inner;       // consecutive q lie mem_pitch elements apart: one dimension after c
+    uint32_t mem_pitch;
+    // the walk (walk_tile): tiles per batch, tiles per block, c-groups, tiles along a block's side, tiles along q and along c
+    FastDiv32 per_batch_div, block_div, cgroups_div, group_div, qtiles_div, ctiles_div;
 };
 
 // Loads and stores of the 16-byte-element kernel (one element per lane, 512-byte runs).  It unpacks with streaming (nt) loads and stores - sixteen shapes of complex128,
@@ -180,53 +184,73 @@ __global__ __launch_bounds__(kThreads) void slice_transpose_kernel(TransArgs a) 
 }
 
 // The tile (batch b, q-tile qt, c-tile ct) this workgroup takes, in the order the host chose (see choose_walk); false when
-// the workgroup is padding of the walk.  Uniform over the workgroup.
-__device__ __forceinline__ bool walk_tile(const TransArgs& a, uint64_t* b_out, uint32_t* qt_out, uint32_t* ct_out) {
-    const uint64_t per_batch = (uint64_t)a.cgroups * ((a.qtiles + a.group - 1) / a.group) * a.group * a.group;
-
+// the workgroup is padding of the walk.  Uniform over the workgroup.  Tile numbers stay below 2^31 (try_transpose_copy), so
+// every division is a multiplication: with the compiler's 64-bit divisions a wavefront issued 190 scalar instructions, most of
+// them before its first load.  With this and with addresses of one 32 x 32-bit multiply-add (ONE) in the kernels below, packing /
+// unpacking, us: bf16 5000 x 7000 33.4 / 34.0 -> 32.5 / 32.9, 8200^2 60.1 / 59.5 -> 57.1 / 57.6, [8, 2000, 3001] 47.6 / 43.5 -> 43.9 /
+// 42.2, f32 8200^2 101.4 / 101.2 -> 98.5 / 98.2; rows of whole lines +-1 %.
+__device__ __forceinline__ bool walk_tile(const TransArgs& a, uint32_t* b_out, uint32_t* qt_out, uint32_t* ct_out) {
     // workgroup w runs on XCD w % 8
-    const uint64_t per_xcd = (a.ntiles + 7) / 8;
-    const uint64_t wg = a.wg0 + blockIdx.x;
-    const uint64_t tile_id = a.xcd_ranges ? (wg % 8) * per_xcd + wg / 8 : wg;
-    if (tile_id >= a.ntiles) return false;
+    const uint32_t ntiles = (uint32_t)a.ntiles;
+    const uint32_t wg = (uint32_t)a.wg0 + blockIdx.x;
+    const uint32_t tile_id = a.xcd_ranges ? (wg % 8) * ((ntiles + 7) / 8) + wg / 8 : wg;
+    if (tile_id >= ntiles) return false;
 
-    uint64_t b;
-    uint32_t qt, ct;
+    uint32_t b, t, qt, ct;
+    a.per_batch_div.divmod(tile_id, b, t);
     if (a.walk == kWalkBlocked) {
-        b = tile_id / per_batch;
-        const uint32_t in_batch = (uint32_t)(tile_id - b * per_batch);
-        const uint32_t gsz = a.group * a.group;
-        const uint32_t grp = in_batch / gsz, within = in_batch - grp * gsz;
-        const uint32_t gq = grp / a.cgroups;
-        uint32_t gc = grp - gq * a.cgroups;
+        uint32_t grp, within, gq, gc, wq, wc;
+        a.block_div.divmod(t, grp, within);
+        a.cgroups_div.divmod(grp, gq, gc);
+        a.group_div.divmod(within, wq, wc);
         if (a.rotate) {
             // a function of the row of groups alone, so that every row still visits each of its c-groups once
-            const uint32_t eighth = (uint32_t)((b * a.qgroups + gq) / a.rows_per_eighth);  // 0..7: the XCD, when ranges hold whole rows
-            gc = (gc + eighth * a.cgroups / 8) % a.cgroups;
+            const uint32_t eighth = (b * a.qgroups + gq) / (uint32_t)a.rows_per_eighth;  // 0..7: the XCD, when ranges hold whole rows
+            gc += eighth * a.cgroups / 8;
+            if (gc >= a.cgroups) gc -= a.cgroups;
         }
-        qt = gq * a.group + within / a.group;
-        ct = gc * a.group + within % a.group;
+        qt = gq * a.group + wq;
+        ct = gc * a.group + wc;
         if (qt >= a.qtiles || ct >= a.ctiles) return false;  // padding of the blocked walk (uniform per workgroup)
+    } else if (a.walk == kWalkMemoryFastest) {   // neighbours read neighbouring pieces of the same memory rows
+        a.ctiles_div.divmod(t, qt, ct);
     } else {
-        const uint64_t plain = (uint64_t)a.qtiles * a.ctiles;
-        b = tile_id / plain;
-        const uint32_t t = (uint32_t)(tile_id - b * plain);
-        if (a.walk == kWalkPackedFastest) {          // neighbours write neighbouring pieces of the same packed rows
-            ct = t / a.qtiles;
-            qt = t - ct * a.qtiles;
-        } else if (a.walk == kWalkMemoryFastest) {   // neighbours read neighbouring pieces of the same memory rows
-            qt = t / a.ctiles;
-            ct = t - qt * a.ctiles;
-        } else {                                     // kWalkDiagonal: neighbours differ in both coordinates
-            const uint32_t d = t / a.qtiles;
-            qt = t - d * a.qtiles;
-            ct = (d + qt) % a.ctiles;
+        a.qtiles_div.divmod(t, ct, qt);          // kWalkPackedFastest: neighbours write neighbouring pieces of the same packed rows
+        if (a.walk == kWalkDiagonal) {           // neighbours differ in both coordinates
+            uint32_t whole;
+            a.ctiles_div.divmod(ct + qt, whole, ct);
         }
     }
     *b_out = b;
     *qt_out = qt;
     *ct_out = ct;
     return true;
+}
+
+// Memory offset of batch b of a transposing copy, in elements.
+__device__ __forceinline__ uint64_t batch_offset(const TransArgs& a, uint32_t b) {
+    uint64_t off = 0;
+    for (int k = a.n_outer - 1; k >= 0; --k) {
+        uint32_t rest, index;
+        a.outer_div[k].divmod(b, rest, index);
+        off += index * a.outer_stride[k];
+        b = rest;
+    }
+    return off;
+}
+
+// Memory offset of row q of a batch, in elements; ONE: its rows lie mem_pitch elements apart.
+template <bool ONE>
+__device__ __forceinline__ uint64_t q_offset(const TransArgs& a, uint32_t q) {
+    if constexpr (ONE) return (uint64_t)q * a.mem_pitch;
+    uint64_t off = 0;
+    for (int k = a.n_inner - 1; k > 0; --k) {
+        uint32_t qd, r;
+        a.inner_div[k].divmod(q, qd, r);
+        off += (uint64_t)r * a.inner_stride[k];
+        q = qd;
+    }
+    return off + (uint64_t)q * a.inner_stride[0];
 }
 
 // ---- 16-byte-per-lane variant for elements of 1, 2, 4 and 8 bytes ----
@@ -245,14 +269,14 @@ __device__ __forceinline__ bool walk_tile(const TransArgs& a, uint64_t* b_out, u
 // range of the blocked walk: tiles whose 256-byte rows share a cache line when rows are not
 // 256-byte aligned are then combined in one L2 instead of being written as partial lines from
 // eight of them.
-template <typename T, int THREADS, bool PACK, int ROWB = 256, bool STREAM = false>
+template <typename T, int THREADS, bool PACK, bool ONE, int ROWB = 256, bool STREAM = false>
 __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs a) {
     constexpr int E = 16 / sizeof(T);
     constexpr int TQ = ROWB / sizeof(T), TC = TQ;
     constexpr int G = TC / E;  // groups of 16 bytes per LDS row (16 for 256-byte rows)
     static_assert(G == ROWB / 16 && (G == 16 || G == 32), "a tile row is 256 or 512 bytes");
     __shared__ __attribute__((aligned(16))) T tile[TQ * TC];
-    __shared__ uint64_t s_off[TQ];
+    __shared__ uint64_t s_off[ONE ? 1 : TQ];
     union Vec {
         u32x4 v;
         T e[E];
@@ -262,38 +286,25 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
 
     T* __restrict__ mem = reinterpret_cast<T*>(a.base) + a.offset;
     T* __restrict__ packed = reinterpret_cast<T*>(a.packed);
-    uint64_t b;
-    uint32_t qt, ct;
+    uint32_t b, qt, ct;
     if (!walk_tile(a, &b, &qt, &ct)) return;
     // A tile that would hang over the edge is moved back inside (both extents are at least a tile): it then overlaps
     // its neighbour, and both write the same bytes to the overlap.
     uint32_t q0 = qt * TQ, c0 = ct * TC;
     if (q0 + TQ > a.Q) q0 = a.Q - TQ;
     if (c0 + TC > a.Sc) c0 = a.Sc - TC;
-    uint64_t batch_off = 0;
-    {
-        uint64_t rem = b;
-        for (int k = a.n_outer - 1; k >= 0; --k) {
-            const uint64_t qd = rem / a.outer_size[k];
-            batch_off += (rem - qd * a.outer_size[k]) * a.outer_stride[k];
-            rem = qd;
-        }
+    const uint64_t batch_off = batch_offset(a, b);
+    // offsets of the tile's memory rows, looked up once per row where they take more than a multiplication
+    if constexpr (!ONE) {
+        if (threadIdx.x < TQ) s_off[threadIdx.x] = q_offset<false>(a, q0 + threadIdx.x);
+        __syncthreads();
     }
-    if (threadIdx.x < TQ) {
-        uint32_t q = q0 + threadIdx.x;
-        uint64_t off = 0;
-        for (int k = a.n_inner - 1; k > 0; --k) {
-            uint32_t qd, r;
-            a.inner_div[k].divmod(q, qd, r);
-            off += (uint64_t)r * a.inner_stride[k];
-            q = qd;
-        }
-        off += (uint64_t)q * a.inner_stride[0];
-        s_off[threadIdx.x] = off;
-    }
-    __syncthreads();
-    T* mem_tile = mem + batch_off + c0;                                        // + s_off[q] + c
-    T* packed_tile = packed + (b * a.Sc + c0) * (uint64_t)a.Q + q0;            // + c * Q + q
+    T* mem_tile = mem + batch_off + (ONE ? (uint64_t)q0 * a.mem_pitch : 0) + c0;  // + row(q) + c
+    auto mem_row = [&](uint32_t q) -> uint64_t {
+        if constexpr (ONE) return (uint64_t)q * a.mem_pitch;
+        else return s_off[q];
+    };
+    T* packed_tile = packed + ((uint64_t)b * a.Sc + c0) * a.Q + q0;            // + c * Q + q
     const int v16 = threadIdx.x % G;  // which 16-byte vector of a row
     const int r16 = threadIdx.x / G;  // which row of a pass of ROWS rows
     constexpr int ROWS = THREADS / G;
@@ -311,7 +322,7 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
             const int q = r16 + ROWS * p;
-            d[p].v = tload<STREAM>(mem_tile + s_off[q] + v16 * E);
+            d[p].v = tload<STREAM>(mem_tile + (mem_row(q) + (uint32_t)(v16 * E)));
         }
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
@@ -388,7 +399,7 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
         for (int p = 0; p < PASSES; ++p) {
             const int q = r16 + ROWS * p;
             const u32x4 o = *reinterpret_cast<const u32x4*>(&tile[at(q, v16 * E)]);
-            tstore(mem_tile + s_off[q] + v16 * E, o, a.aligned_stores);
+            tstore(mem_tile + (mem_row(q) + (uint32_t)(v16 * E)), o, a.aligned_stores);
         }
     }
 }
@@ -407,57 +418,42 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_vec_kernel(TransArgs 
 // 0.67 / 0.67 and 0.60 / 0.58 -> 0.63 / 0.62.  Rows that do start on lines keep the kernel above.  Loads go through
 // the cache at every size: streaming (nt) loads lose what the neighbouring tile left in L2 (bf16 5000 x 7000 0.70 -> 0.49).
 // W is the index of a written row (c when packing, q when unpacking), X the position along it.
-template <typename T, int THREADS, bool PACK>
+template <typename T, int THREADS, bool PACK, bool ONE>
 __global__ __launch_bounds__(THREADS) void slice_transpose_lines_kernel(TransArgs a) {
     constexpr int ES = sizeof(T), E = 16 / ES;
     constexpr int TW = 256 / ES, TX = 256 / ES, D = 128 / ES, XR = TX + D;
     constexpr int ROWS = THREADS / 16;
     static_assert(XR <= THREADS && TW <= THREADS, "one lane per decoded row");
     __shared__ __attribute__((aligned(16))) T tile[XR * TW];  // [read row][written row]
-    __shared__ uint64_t s_off[PACK ? XR : TW];
+    __shared__ uint64_t s_off[ONE ? 1 : PACK ? XR : TW];
     union Vec {
         u32x4 v;
         T e[E];
     };
     // LDS position of (read row xr, written row wc): xr * TW + (wc ^ (E * ((xr / E) % 16)))
 
-    uint64_t b;
-    uint32_t qt, ct;
+    uint32_t b, qt, ct;
     if (!walk_tile(a, &b, &qt, &ct)) return;
     const uint32_t Wn = PACK ? a.Sc : a.Q, Xn = PACK ? a.Q : a.Sc;
     uint32_t w0 = (PACK ? ct : qt) * TW;
     if (w0 + TW > Wn) w0 = Wn - TW;  // the host sends extents of at least a tile; the overlap is written twice, same bytes
-    const int64_t x0 = (int64_t)(PACK ? qt : ct) * TX;
+    const uint32_t x0 = (PACK ? qt : ct) * TX;
 
-    T* __restrict__ mem = reinterpret_cast<T*>(a.base) + a.offset;
-    T* __restrict__ packed = reinterpret_cast<T*>(a.packed);
-    uint64_t batch_off = 0;
-    {
-        uint64_t rem = b;
-        for (int k = a.n_outer - 1; k >= 0; --k) {
-            const uint64_t qd = rem / a.outer_size[k];
-            batch_off += (rem - qd * a.outer_size[k]) * a.outer_stride[k];
-            rem = qd;
-        }
+    // the first element of the tile's written rows (packing) / of what it reads of every row (unpacking), at position 0
+    T* __restrict__ mem = reinterpret_cast<T*>(a.base) + a.offset + batch_offset(a, b) + (PACK ? w0 : 0);
+    T* __restrict__ packed = reinterpret_cast<T*>(a.packed) + (uint64_t)b * a.Sc * a.Q + (PACK ? (uint64_t)w0 * a.Q : w0);
+    // read row xr of the tile is row x0 - D + xr of the other side, clamped into the extent: what a clamped row holds is
+    // never written
+    auto read_row = [&](uint32_t xr) {
+        uint32_t x = x0 + xr < D ? 0 : x0 + xr - D;
+        return x < Xn ? x : Xn - 1;
+    };
+    // memory offsets of the q rows this tile touches: the read rows when packing, the written rows when unpacking; looked up
+    // once per row where they take more than a multiplication
+    if constexpr (!ONE) {
+        if (threadIdx.x < (PACK ? XR : TW)) s_off[threadIdx.x] = q_offset<false>(a, PACK ? read_row(threadIdx.x) : w0 + threadIdx.x);
+        __syncthreads();
     }
-    // memory offsets of the q rows this tile touches: the read rows when packing (clamped into the extent: what a
-    // clamped row holds is never written), the written rows when unpacking
-    if (threadIdx.x < (PACK ? XR : TW)) {
-        int64_t qi = PACK ? x0 - D + (int64_t)threadIdx.x : (int64_t)w0 + threadIdx.x;
-        if (qi < 0) qi = 0;
-        if (qi > (int64_t)a.Q - 1) qi = (int64_t)a.Q - 1;
-        uint32_t q = (uint32_t)qi;
-        uint64_t off = 0;
-        for (int k = a.n_inner - 1; k > 0; --k) {
-            uint32_t qd, r;
-            a.inner_div[k].divmod(q, qd, r);
-            off += (uint64_t)r * a.inner_stride[k];
-            q = qd;
-        }
-        off += (uint64_t)q * a.inner_stride[0];
-        s_off[threadIdx.x] = off;
-    }
-    __syncthreads();
 
     // ---- read side -> LDS: rows x0 - D .. x0 + TX - 1, TW consecutive written-row indices of each ----
     const int v16 = threadIdx.x % 16, r16 = threadIdx.x / 16;
@@ -468,14 +464,8 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_lines_kernel(TransArg
         int xr = r16 + ROWS * p;
         if (xr > XR - 1) xr = XR - 1;  // surplus lanes of the last pass repeat its last row
         const T* src;
-        if constexpr (PACK) {
-            src = mem + batch_off + s_off[xr] + w0 + v16 * E;
-        } else {
-            int64_t c = x0 - D + xr;
-            if (c < 0) c = 0;
-            if (c > (int64_t)a.Sc - 1) c = (int64_t)a.Sc - 1;
-            src = packed + (b * a.Sc + (uint64_t)c) * (uint64_t)a.Q + w0 + v16 * E;
-        }
+        if constexpr (PACK) src = mem + ((ONE ? (uint64_t)read_row(xr) * a.mem_pitch : s_off[ONE ? 0 : xr]) + (uint32_t)(v16 * E));
+        else src = packed + ((uint64_t)read_row(xr) * a.Q + (uint32_t)(v16 * E));
         d[p].v = tload<false>(src);
     }
 #pragma unroll
@@ -497,11 +487,11 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_lines_kernel(TransArg
         const int logical = r16 + ROWS * p;
         const int in_block = logical % (4 * S);
         const int wr = logical - in_block + (in_block % 4) * S + in_block / 4;
-        T* row;  // position 0 of the written row
-        if constexpr (PACK) row = packed + (b * a.Sc + w0 + wr) * (uint64_t)a.Q;
-        else row = mem + batch_off + s_off[wr];
-        const int dw = (int)((((uintptr_t)row + (uint64_t)x0 * ES) & 127u) / ES);
-        const int64_t xs = x0 - dw + v16 * E;  // first position of this lane's vector
+        T* row;  // position x0 of the written row
+        if constexpr (PACK) row = packed + ((uint64_t)(uint32_t)wr * a.Q + x0);
+        else row = mem + ((ONE ? (uint64_t)(w0 + wr) * a.mem_pitch : s_off[ONE ? 0 : wr]) + x0);
+        const int dw = (int)(((uintptr_t)row & 127u) / ES);
+        const int xs = v16 * E - dw;           // first position of this lane's vector, counted from x0
         const int xr0 = D - dw + v16 * E;      // and the LDS row that holds it
         // The E rows xr0 .. xr0 + E - 1 lie in at most two groups of E rows, i.e. see two XOR permutations: one base
         // address for each, and a compare per element instead of the permutation's arithmetic (which is what made the
@@ -513,12 +503,13 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_lines_kernel(TransArg
         Vec o;
 #pragma unroll
         for (int j = 0; j < E; ++j) o.e[j] = (j < first ? p0 : p1)[j * TW];
-        if (xs >= 0 && xs + E <= (int64_t)Xn) {
+        const uint32_t x = x0 + (uint32_t)xs;  // wraps below position 0
+        if (x < Xn && x + E <= Xn) {
             tstore(row + xs, o.v, kStoreStreaming);
         } else {
 #pragma unroll
             for (int j = 0; j < E; ++j)
-                if (xs + j >= 0 && xs + j < (int64_t)Xn) row[xs + j] = o.e[j];
+                if (x + j < Xn) row[xs + j] = o.e[j];
         }
     }
 }
@@ -541,7 +532,7 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_lines_kernel(TransArg
 // whole lines, bare 256-byte reads run at 4.9 TB/s and line-by-line writes of rows a pitch apart at 5.4 TB/s, against
 // 6.4 and 5.6 for aligned rows.)
 // W is the index of a written row (c when packing, q when unpacking), X the position along it.
-template <typename T, int THREADS, bool PACK>
+template <typename T, int THREADS, bool PACK, bool ONE>
 __global__ __launch_bounds__(THREADS) void slice_transpose_strip_kernel(TransArgs a) {
     constexpr int ES = sizeof(T), E = 16 / ES;
     constexpr int TW = 256 / ES, CH = 128 / ES, RING = 2 * CH;
@@ -557,13 +548,13 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_strip_kernel(TransArg
 
     // workgroup i runs on XCD i % 8: each XCD takes a contiguous eighth of the (batch, segment, strip) list, strips
     // fastest, so that the strips that read neighbouring pieces of the same rows run side by side in one L2
-    const uint64_t wg = a.wg0 + blockIdx.x;
-    const uint64_t id = (wg % 8) * ((a.ntiles + 7) / 8) + wg / 8;
-    if (id >= a.ntiles) return;
-    const uint64_t per_batch = (uint64_t)a.nseg * a.nstrips;
-    const uint64_t b = id / per_batch;
-    const uint32_t in_batch = (uint32_t)(id - b * per_batch);
-    const uint32_t seg = in_batch / a.nstrips, sw = in_batch - seg * a.nstrips;
+    const uint32_t ntiles = (uint32_t)a.ntiles;
+    const uint32_t wg = (uint32_t)a.wg0 + blockIdx.x;
+    const uint32_t id = (wg % 8) * ((ntiles + 7) / 8) + wg / 8;
+    if (id >= ntiles) return;
+    uint32_t b, in_batch, seg, sw;
+    a.per_batch_div.divmod(id, b, in_batch);  // nseg * nstrips
+    a.qtiles_div.divmod(in_batch, seg, sw);   // nstrips
     const uint32_t Wn = PACK ? a.Sc : a.Q, Xn = PACK ? a.Q : a.Sc;
     uint32_t w0 = sw * TW;
     if (w0 + TW > Wn) w0 = Wn - TW;  // the host sends extents of at least a strip; the overlap is written twice, same bytes
@@ -575,25 +566,7 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_strip_kernel(TransArg
 
     T* __restrict__ mem = reinterpret_cast<T*>(a.base) + a.offset;
     T* __restrict__ packed = reinterpret_cast<T*>(a.packed);
-    uint64_t batch_off = 0;
-    {
-        uint64_t rem = b;
-        for (int k = a.n_outer - 1; k >= 0; --k) {
-            const uint64_t qd = rem / a.outer_size[k];
-            batch_off += (rem - qd * a.outer_size[k]) * a.outer_stride[k];
-            rem = qd;
-        }
-    }
-    auto q_offset = [&](uint32_t q) {  // memory offset of row q of the batch
-        uint64_t off = 0;
-        for (int k = a.n_inner - 1; k > 0; --k) {
-            uint32_t qd, r;
-            a.inner_div[k].divmod(q, qd, r);
-            off += (uint64_t)r * a.inner_stride[k];
-            q = qd;
-        }
-        return off + (uint64_t)q * a.inner_stride[0];
-    };
+    const uint64_t batch_off = batch_offset(a, b);
 
     const int v16 = threadIdx.x % 16, r16 = threadIdx.x / 16;
     const int v8 = threadIdx.x % 8, r8 = threadIdx.x / 8;
@@ -604,8 +577,8 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_strip_kernel(TransArg
             int64_t x = (int64_t)xs + (int64_t)c * CH + r16 + LROWS * p;
             x = x < 0 ? 0 : (x > (int64_t)Xn - 1 ? (int64_t)Xn - 1 : x);
             const T* src;
-            if constexpr (PACK) src = mem + batch_off + q_offset((uint32_t)x) + w0 + v16 * E;
-            else src = packed + (b * a.Sc + (uint64_t)x) * (uint64_t)a.Q + w0 + v16 * E;
+            if constexpr (PACK) src = mem + batch_off + q_offset<ONE>(a, (uint32_t)x) + w0 + v16 * E;
+            else src = packed + ((uint64_t)b * a.Sc + (uint64_t)x) * (uint64_t)a.Q + w0 + v16 * E;
             d[p].v = tload<false>(src);
         }
     };
@@ -628,8 +601,8 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_strip_kernel(TransArg
         const int logical = r8 + SROWS * p;
         const int in_block = logical % (8 * S);
         wr[p] = logical - in_block + (in_block % 8) * S + in_block / 8;
-        if constexpr (PACK) rowp[p] = packed + (b * a.Sc + w0 + wr[p]) * (uint64_t)a.Q;
-        else rowp[p] = mem + batch_off + q_offset(w0 + wr[p]);
+        if constexpr (PACK) rowp[p] = packed + ((uint64_t)b * a.Sc + w0 + wr[p]) * (uint64_t)a.Q;
+        else rowp[p] = mem + batch_off + q_offset<ONE>(a, w0 + wr[p]);
         dws[p] = (int)(((uintptr_t)rowp[p] & 127u) / ES);  // xs is a multiple of CH, i.e. of a line
     }
 
@@ -734,6 +707,66 @@ static void choose_walk(TransArgs* a, uint32_t unit, uint64_t nbatch) {
     }
 }
 
+struct TransForm {
+    uint32_t unit;
+    bool lines, big, stream_loads;
+    uint32_t lanes;
+};
+
+template <bool PACK, bool ONE>
+static void launch_tiles(const TransForm& f, dim3 grid, hipStream_t stream, const TransArgs& a) {
+    if (f.lines) {
+        switch (f.unit) {
+            case 1: MHIP_LAUNCH((slice_transpose_lines_kernel<uint8_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
+            case 2: MHIP_LAUNCH((slice_transpose_lines_kernel<uint16_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
+            case 4: MHIP_LAUNCH((slice_transpose_lines_kernel<uint32_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
+            default: MHIP_LAUNCH((slice_transpose_lines_kernel<uint64_t, 256, PACK, ONE>), grid, dim3(256), 0, stream, a); break;
+        }
+        return;
+    }
+    if (f.stream_loads) {
+        switch (f.unit) {
+            case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a); break;
+            case 2:
+                if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
+                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a);
+                break;
+            case 4:
+                if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
+                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a);
+                break;
+            default:
+                if (f.lanes == 1024) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
+                else if (f.lanes == 512) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 512, PACK, ONE, 512, true>), grid, dim3(512), 0, stream, a);
+                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 256, PACK, ONE, 256, true>), grid, dim3(256), 0, stream, a);
+                break;
+        }
+        return;
+    }
+    switch (f.unit) {
+        case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
+        case 2:
+            if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
+            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a);
+            break;
+        case 4:
+            if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
+            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a);
+            break;
+        default:
+            if (f.lanes == 1024) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
+            else if (f.lanes == 512) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 512, PACK, ONE, 512>), grid, dim3(512), 0, stream, a);
+            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 256, PACK, ONE>), grid, dim3(256), 0, stream, a);
+            break;
+    }
+}
+
+template <bool PACK, bool ONE>
+static void launch_strips(uint32_t unit, dim3 grid, hipStream_t stream, const TransArgs& a) {
+    if (unit == 1) MHIP_LAUNCH((slice_transpose_strip_kernel<uint8_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a);
+    else MHIP_LAUNCH((slice_transpose_strip_kernel<uint16_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a);
+}
+
 template <bool PACK>
 bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t unit, hipStream_t stream, int* rc) {
     if (c.run != 1 || c.ndim < 2 || c.ndim > kMaxCanonDims) return false;
@@ -761,6 +794,8 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
         a.outer_stride[j] = c.dims[k].stride;
     }
     const uint64_t Sc = c.dims[cd].size;
+    a.one_inner = a.n_inner == 1 && a.inner_stride[0] <= UINT32_MAX;
+    a.mem_pitch = (uint32_t)a.inner_stride[0];
     // worth it only when both sides have something to coalesce
     if (Sc < 8 || Q < 8 || Sc >= kFastDivLimit) return false;
     const bool vec = unit <= 8;  // 16-byte elements already move 16 bytes per lane in the scalar kernel
@@ -855,11 +890,14 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
         a.nseg = (uint32_t)((Xn + a.seg_len - 1) / a.seg_len);
         a.nstrips = (uint32_t)((Wn + rows_per_strip - 1) / rows_per_strip);
         a.ntiles = nbatch * a.nseg * a.nstrips;
+        if (a.ntiles >= kFastDivLimit - 8) return false;
+        a.per_batch_div = FastDiv32(a.nseg * a.nstrips);
+        a.qtiles_div = FastDiv32(a.nstrips);
         const uint64_t nblocks = 8 * ((a.ntiles + 7) / 8);
         *rc = launch_in_pieces(nblocks, 512, 8, [&](uint64_t wg0, uint32_t count) {
             a.wg0 = wg0;
-            if (unit == 1) MHIP_LAUNCH((slice_transpose_strip_kernel<uint8_t, 512, PACK>), dim3(count), dim3(512), 0, stream, a);
-            else MHIP_LAUNCH((slice_transpose_strip_kernel<uint16_t, 512, PACK>), dim3(count), dim3(512), 0, stream, a);
+            if (a.one_inner) launch_strips<PACK, true>(unit, dim3(count), stream, a);
+            else launch_strips<PACK, false>(unit, dim3(count), stream, a);
         });
         return true;
     }
@@ -925,55 +963,21 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     if (vec) choose_walk(&a, unit, nbatch);
     a.ntiles = a.walk == kWalkBlocked ? nbatch * a.cgroups * a.qgroups * a.group * a.group : nbatch * (uint64_t)a.qtiles * a.ctiles;
     if (vec) {
+        // tile numbers fit the 32-bit divisions of walk_tile: 2^31 tiles of 16 KiB and more would be 32 TiB
+        if (a.ntiles >= kFastDivLimit - 8) return false;
+        a.per_batch_div = FastDiv32(a.walk == kWalkBlocked ? a.cgroups * a.qgroups * a.group * a.group : a.qtiles * a.ctiles);
+        a.block_div = FastDiv32(a.group * a.group);
+        a.cgroups_div = FastDiv32(a.cgroups);
+        a.group_div = FastDiv32(a.group);
+        a.qtiles_div = FastDiv32(a.qtiles);
+        a.ctiles_div = FastDiv32(a.ctiles);
         const uint64_t nblocks = 8 * ((a.ntiles + 7) / 8);  // one tile per workgroup, eight XCD ranges
         const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big ? 1024 : 512;
         *rc = launch_in_pieces(nblocks, lanes, 8, [&](uint64_t wg0, uint32_t count) {
             a.wg0 = wg0;
-            const dim3 grid(count);
-            if (lines) {
-                switch (unit) {
-                    case 1: MHIP_LAUNCH((slice_transpose_lines_kernel<uint8_t, 512, PACK>), grid, dim3(512), 0, stream, a); break;
-                    case 2: MHIP_LAUNCH((slice_transpose_lines_kernel<uint16_t, 512, PACK>), grid, dim3(512), 0, stream, a); break;
-                    case 4: MHIP_LAUNCH((slice_transpose_lines_kernel<uint32_t, 512, PACK>), grid, dim3(512), 0, stream, a); break;
-                    default: MHIP_LAUNCH((slice_transpose_lines_kernel<uint64_t, 256, PACK>), grid, dim3(256), 0, stream, a); break;
-                }
-                return;
-            }
-            if (stream_loads) {
-                switch (unit) {
-                    case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, 256, true>), grid, dim3(512), 0, stream, a); break;
-                    case 2:
-                        if (big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, 512, true>), grid, dim3(1024), 0, stream, a);
-                        else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, 256, true>), grid, dim3(512), 0, stream, a);
-                        break;
-                    case 4:
-                        if (big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, 512, true>), grid, dim3(1024), 0, stream, a);
-                        else MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 512, PACK, 256, true>), grid, dim3(512), 0, stream, a);
-                        break;
-                    default:
-                        if (big8_lanes == 1024) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 1024, PACK, 512, true>), grid, dim3(1024), 0, stream, a);
-                        else if (big8_lanes == 512) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 512, PACK, 512, true>), grid, dim3(512), 0, stream, a);
-                        else MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 256, PACK, 256, true>), grid, dim3(256), 0, stream, a);
-                        break;
-                }
-                return;
-            }
-            switch (unit) {
-                case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK>), grid, dim3(512), 0, stream, a); break;
-                case 2:
-                    if (big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, 512>), grid, dim3(1024), 0, stream, a);
-                    else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK>), grid, dim3(512), 0, stream, a);
-                    break;
-                case 4:
-                    if (big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, 512>), grid, dim3(1024), 0, stream, a);
-                    else MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 512, PACK>), grid, dim3(512), 0, stream, a);
-                    break;
-                default:
-                    if (big8_lanes == 1024) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 1024, PACK, 512>), grid, dim3(1024), 0, stream, a);
-                    else if (big8_lanes == 512) MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 512, PACK, 512>), grid, dim3(512), 0, stream, a);
-                    else MHIP_LAUNCH((slice_transpose_vec_kernel<uint64_t, 256, PACK>), grid, dim3(256), 0, stream, a);
-                    break;
-            }
+            const TransForm form{unit, lines, big, stream_loads, lanes};
+            if (a.one_inner) launch_tiles<PACK, true>(form, dim3(count), stream, a);
+            else launch_tiles<PACK, false>(form, dim3(count), stream, a);
         });
         return true;
     }
