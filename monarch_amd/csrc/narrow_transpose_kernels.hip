@@ -10,7 +10,7 @@
 // over q and j over the memory-contiguous dimension c; unpacking, the other way round.  HBM-bound: 2 bytes of traffic
 // per byte moved.  Both sides move 16-byte vectors whatever the extents: the last vector of a row is moved back so that it
 // ends where the row ends.  bf16 [64, 4096, 64] -> [64, 64, 4096] (33.6 MB), pack / unpack: 95.8 / 104 us with the tiles
-// that fill a quarter of their lanes, 15.6 / 14.9 us here (4.3 / 4.5 TB/s); head dim 80: 98 / 82 -> 16.9 / 19.2,
+// that fill a quarter of their lanes, 13.1 / 13.0 us here (5.1 / 5.2 TB/s); head dim 80: 98 / 82 -> 16.9 / 19.2,
 // 32: 94 / 81 -> 8.0 / 7.6; u8 head dim 128: 222 / 303 -> 12.9 / 13.8; bf16 1024^2: 3.3 / 3.4 -> 2.4 / 2.4.
 //
 // Most launches are one or two rounds of workgroups, so what a wavefront issues before its first load and between its loads
@@ -244,6 +244,35 @@ static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     });
 }
 
+// The same with tiles that are longer along the long side (the written rows where LONG_I, else the read rows), where that
+// pays.  It does in two cases:
+//   * 400 to 512 tiles of 64 KiB (two fit a CU's LDS): all of them are resident at once, so the part first reads everything and
+//     then writes everything, in pieces of 1 KiB and more, and no write gets between the reads.  2- and 4-byte elements, packing /
+//     unpacking, one tile of 32 or 16 KiB -> 64 KiB, us: bf16 [64, 4096, 64] 15.6 / 14.9 -> 13.1 / 13.1, [56, 4096, 64] 13.9 / 13.7 ->
+//     12.1 / 11.2, [256, 1024, 64] 16.0 / 14.9 -> 13.1 / 15.0, f32 [262144, 32] 16.2 / 12.3 -> 11.1 / 10.8.  With fewer or more of them
+//     the part runs out of step again and large tiles lose: [32, 4096, 64] 8.1 / 7.5 -> 8.8 / 8.4, [96, 4001, 64] 21.7 / 20.2 ->
+//     22.4 / 22.1.
+//   * 4-byte elements from 28 MiB on: tiles of 32 KiB instead of 16 (f32 [64, 4096, 32] 18.0 / 14.3 -> 15.2 / 14.5, [1 M, 16] 28.0 /
+//     25.8 -> 24.7 / 23.2; sides of 64 to 256 bytes, 33 to 100 MiB, 0.89 to 0.99 x; 17 MiB up to 1.1 x).
+constexpr uint64_t kResidentTilesMin = 400, kResidentTilesMax = 512;
+template <typename T, bool PACK, int WB, int RB, bool LONG_I>
+static int launch_narrow_long(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
+    constexpr int ES = sizeof(T), K = 65536 / (WB * RB / ES);  // times as long: a tile of 64 KiB
+    const uint32_t I = PACK ? a.Q : a.Sc, J = PACK ? a.Sc : a.Q;
+    // whether the long side fills most of a tile that is `k` times as long
+    auto fills = [&](int k) { return (uint64_t)(LONG_I ? I : J) * ES * 4 >= (uint64_t)(LONG_I ? WB : RB) * k * 3; };
+    if constexpr (ES == 2 || ES == 4) {
+        constexpr uint32_t TI = WB / ES * (LONG_I ? K : 1), TJ = RB / ES * (LONG_I ? 1 : K);
+        const uint64_t tiles = nbatch * ((I + TI - 1) / TI) * ((J + TJ - 1) / TJ);
+        if (fills(K) && tiles >= kResidentTilesMin && tiles <= kResidentTilesMax)
+            return launch_narrow<T, PACK, WB * (LONG_I ? K : 1), RB * (LONG_I ? 1 : K)>(a, nbatch, stream);
+    }
+    if constexpr (ES == 4)
+        if (fills(2) && nbatch * I * J * ES >= (28ull << 20))
+            return launch_narrow<T, PACK, WB * (LONG_I ? 2 : 1), RB * (LONG_I ? 1 : 2)>(a, nbatch, stream);
+    return launch_narrow<T, PACK, WB, RB>(a, nbatch, stream);
+}
+
 // Tile length along a side of `bytes` <= 512: pieces of 128 bytes where they cover the side with little overlap (the last
 // one is moved back), else the next power of two (272 bytes, 67 MB, pack / unpack: one tile of 512 26 / 27 us, three
 // of 128 47 / 29; 384 bytes: 27.8 / 25 against 27.5 / 24.5).
@@ -276,15 +305,15 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
         if (ES == 8 && n == 64) n = 128;  // a read row of 64 bytes would be fewer than 16 elements
         if (short_j) {
             if constexpr (ES < 8)
-                if (n == 64) return launch_narrow<T, PACK, 1024, 64>(a, nbatch, stream);
-            if (n == 128) return launch_narrow<T, PACK, 512, 128>(a, nbatch, stream);
-            if (n == 256) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+                if (n == 64) return launch_narrow_long<T, PACK, 1024, 64, true>(a, nbatch, stream);
+            if (n == 128) return launch_narrow_long<T, PACK, 512, 128, true>(a, nbatch, stream);
+            if (n == 256) return launch_narrow_long<T, PACK, 256, 256, true>(a, nbatch, stream);
             return launch_narrow<T, PACK, 128, 512>(a, nbatch, stream);
         }
         if constexpr (ES < 8)
-            if (n == 64) return launch_narrow<T, PACK, 64, 1024>(a, nbatch, stream);
-        if (n == 128) return launch_narrow<T, PACK, 128, 512>(a, nbatch, stream);
-        if (n == 256) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+            if (n == 64) return launch_narrow_long<T, PACK, 64, 1024, false>(a, nbatch, stream);
+        if (n == 128) return launch_narrow_long<T, PACK, 128, 512, false>(a, nbatch, stream);
+        if (n == 256) return launch_narrow_long<T, PACK, 256, 256, false>(a, nbatch, stream);
         return launch_narrow<T, PACK, 512, 128>(a, nbatch, stream);
     }
     if constexpr (ES == 8)

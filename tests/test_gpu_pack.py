@@ -885,6 +885,39 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
         assert torch.equal(back.cpu(), ref), (shape, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
+@pytest.mark.parametrize("tiles", [399, 400, 512, 513])
+def test_transposes_with_a_short_side_in_tiles_that_are_resident_at_once(dtype, tiles):
+    # 2- and 4-byte elements of 400 to 512 tiles of 64 KiB take that tile, 4-byte elements of 28 MiB and more twice the small
+    # one, on either side of the matrix: short sides that need every tile length, long sides of whole tiles and one element
+    # less, batches whose matrices fill the tile or do not, views whose rows span two dimensions
+    es = torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=DEV).manual_seed(tiles)
+    info = torch.iinfo(dtype)
+    cases = []
+    for side in (48, 64, 104, 128, 250, 256):
+        n, length = side // es, 65536 // (64 if side <= 64 else 128 if side <= 128 or side == 256 else 256)  # bytes of a tile's long side
+        pieces = 2 if side == 256 else 1
+        for less in (0, 1):
+            m = tiles // pieces * (length // es) - less
+            cases += [((m, n), lambda x: x.t()), ((n, m), lambda x: x.t())]
+    cases += [((tiles // 4, 4 * 512 // es, 128 // es), lambda x: x.transpose(1, 2)), ((tiles * 4, 128 // es, 128 // es), lambda x: x.transpose(1, 2)),
+              ((tiles // 2, 2 * 512 // es + 6, 128 // es), lambda x: x[:, 3:-3].permute(2, 0, 1))]
+    for shape, view_of in cases:
+        x = torch.randint(info.min, info.max, shape, dtype=dtype, device=DEV, generator=g)
+        view = view_of(x)
+        s = Slice.of_tensor(view)
+        out = staging.pack(view, s)
+        want = view.contiguous().flatten()
+        sync()
+        assert torch.equal(out, want), (shape, dtype)
+        back, ref = torch.full_like(x, 7), torch.full_like(x, 7)
+        staging.unpack(back, s, out)
+        view_of(ref).copy_(view)
+        sync()
+        assert torch.equal(back, ref), (shape, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.int16, torch.int32, torch.int64])
 def test_short_runs_unit_by_unit(dtype):
     # slice_units_kernel: 1 KiB of the packed side per workgroup, so lengths round one and several of those, rows up to the
