@@ -16,6 +16,7 @@ import torch
 
 from . import _torch
 from ._lib import check, lib, ptr_array
+from ._native import host
 
 BLOCK = 1024
 FP8_MAX = 448.0
@@ -58,6 +59,7 @@ class FlatBucket:
         self.total = self.offsets[-1]
         # device-resident tables, uploaded once and reused by every pack / unpack
         self.d_offsets = torch.tensor(self.offsets, dtype=torch.int64, device=self.device)
+        self._sizes64 = b"".join(n.to_bytes(8, "little") for n in self.sizes)
         self._tables = {}
         self._index = None
         self.d_ptrs = self.pointer_table(tensors)
@@ -71,13 +73,17 @@ class FlatBucket:
     def pointer_table(self, tensors: Sequence[torch.Tensor]) -> torch.Tensor:
         if [t.numel() for t in tensors] != self.sizes:
             raise ValueError("tensor sizes do not match the bucket")
-        key = tuple(t.data_ptr() for t in tensors)
+        return self._table_of(b"".join(t.data_ptr().to_bytes(8, "little") for t in tensors), tensors)
+
+    def _table_of(self, key: bytes, tensors: Sequence[torch.Tensor]) -> torch.Tensor:
+        """The table of these tensors, whose addresses are the 64-bit integers in ``key``."""
         hit = self._tables.get(key)
         if hit is None:
             if len(self._tables) >= self._MAX_TABLES:   # retire the oldest once everything queued so far has run
                 torch.cuda.synchronize(self.device)
                 self._tables.pop(next(iter(self._tables)))
-            hit = (torch.tensor(key, dtype=torch.int64, device=self.device), list(tensors))
+            addresses = [int.from_bytes(key[i: i + 8], "little") for i in range(0, len(key), 8)]
+            hit = (torch.tensor(addresses, dtype=torch.int64, device=self.device), list(tensors))
             self._tables[key] = hit
         return hit[0]
 
@@ -107,6 +113,12 @@ class FlatBucket:
 
     def pack(self, flat: torch.Tensor = None, d_ptrs: torch.Tensor = None, stream=None, indexed: bool = None) -> torch.Tensor:
         """flat[offsets[t] + j] = tensors[t][j]; ``indexed`` as in ``_index_ptr``."""
+        if stream is None and indexed is None and flat is not None:
+            status = host.flat_copy(True, flat, self.d_ptrs if d_ptrs is None else d_ptrs, self.d_offsets, self.total, self._index,
+                                    self.tensors[0])
+            if status >= 0:
+                check(status)
+                return flat
         if flat is None:
             flat = torch.empty(self.total, dtype=self.dtype, device=self.device)
         else:
@@ -129,6 +141,12 @@ class FlatBucket:
     def unpack(self, flat: torch.Tensor, outs: Sequence[torch.Tensor], stream=None, indexed: bool = None) -> None:
         """outs[t][j] = flat[offsets[t] + j]; ``flat`` may have any dtype of the outs' element size;
         ``indexed`` as in ``_index_ptr``."""
+        if stream is None and indexed is None:
+            key = host.tensor_addresses(outs, self._sizes64, flat)
+            if key is not None and flat.device == self.device:
+                status = host.flat_copy(False, flat, self._table_of(key, outs), self.d_offsets, self.total, self._index, None)
+                if status >= 0:
+                    return check(status)
         _torch.require_contiguous(flat)
         if flat.numel() != self.total or flat.device != self.device:
             raise ValueError(f"flat buffer must hold {self.total} elements on {self.device}")
@@ -157,6 +175,11 @@ def quantize_bucket(bucket: FlatBucket, q: torch.Tensor = None, scales: torch.Te
         q = torch.empty(n, dtype=torch.uint8, device=bucket.device)
     if scales is None:
         scales = torch.empty(_nblocks(n), dtype=torch.float32, device=bucket.device)
+    if stream is None and indexed is None:
+        status = host.quantize_bucket(bucket.d_ptrs, bucket.d_offsets, n, bucket._index, q, scales)
+        if status >= 0:
+            check(status)
+            return q, scales
     _check_payload(q, scales, n, bucket.device)
     check(lib().mhip_fp8_quantize_bucket(q.data_ptr(), scales.data_ptr(), bucket.d_ptrs.data_ptr(),
                                          bucket.d_offsets.data_ptr(), len(bucket.sizes), n, BLOCK,
@@ -224,6 +247,10 @@ def dequant_accumulate_bucket_many(bucket: FlatBucket, qs: Sequence[torch.Tensor
     """``dequant_accumulate_bucket`` for all peers' payloads in one pass (peers added in order)."""
     if bucket.dtype != torch.float32:
         raise ValueError("dequant_accumulate_bucket_many expects a bucket of fp32 accumulators")
+    if stream is None and indexed is None:
+        status = host.dequant_accumulate_bucket(bucket.d_ptrs, bucket.d_offsets, bucket.total, bucket._index, qs, scales)
+        if status >= 0:
+            return check(status)
     if len(qs) == 0 or len(qs) != len(scales):
         raise ValueError("one scales tensor per code tensor, at least one peer")
     for q, s in zip(qs, scales):

@@ -20,7 +20,7 @@ _ITER_CHUNK = 1 << 16
 
 
 class Slice:
-    __slots__ = ("_offset", "_sizes", "_strides", "_c", "_keep", "_len", "_bounds")
+    __slots__ = ("_offset", "_sizes", "_strides", "_c", "_keep", "_len", "_bounds", "_addr")
 
     def __init__(self, *, offset: int, sizes: Sequence[int], strides: Sequence[int], _validate: bool = True):
         sizes, strides = [int(x) for x in sizes], [int(x) for x in strides]
@@ -33,6 +33,7 @@ class Slice:
         self._offset, self._sizes, self._strides = int(offset), sizes, strides
         self._keep = (u64_array(sizes), u64_array(strides))
         self._c = SliceC(self._offset, len(sizes), self._keep[0], self._keep[1])
+        self._addr = C.addressof(self._c)  # where the native host path reads it
         # a Slice never changes: the library is asked once for what every pack and unpack call checks (a pack call
         # through Python 9.2 us -> 5.1 together with the cheaper stream look-up)
         self._len = self._bounds = None

@@ -26,6 +26,7 @@ import torch
 
 from . import _lib, _torch
 from ._lib import MhipError, check, lib, ptr_array
+from ._native import host
 from .device_mesh import DeviceMesh
 from .ndslice import Slice, slice_array
 
@@ -136,6 +137,10 @@ def check_reduce_args(mesh_names: Sequence[str], mesh_sizes: Dict[str, int], sha
 def all_reduce(out: torch.Tensor, group: Sequence[torch.Tensor], op: ReduceOp, stream=None) -> None:
     """Local combine of ``Communicator::all_reduce`` (torch-sys-cuda/src/nccl.rs:464-489):
     ``out = op(group)``; ``out`` may be one of the group's tensors (the in-place form)."""
+    if stream is None:
+        status = host.reduce(out, group, op)
+        if status >= 0:
+            return check(status)
     _torch.require_all_contiguous((out, *group))
     dtype, numel = out.dtype, out.numel()
     code = _torch.dtype_code(dtype)
@@ -172,6 +177,10 @@ def reduce_scatter_views(outs: Sequence[torch.Tensor], out_views: Sequence[Slice
                          in_view: Optional[Slice], op: ReduceOp, stream=None) -> None:
     """Reduce ``group`` (each read through ``in_view``) and scatter the result through
     ``out_views`` (Slices of the reduced tensor) into contiguous ``outs`` in one pass."""
+    if stream is None and in_view is not None:
+        status = host.reduce_scatter(outs, out_views, group, in_view, op)
+        if status >= 0:
+            return check(status)
     _torch.require_all_contiguous(outs)
     for t in group:
         _torch.require_device(t)
@@ -194,6 +203,11 @@ def stream_reduce(group: Sequence[Optional[torch.Tensor]], rank: int, factory: F
     upstream and is replaced by zeros of ``factory`` (stream.rs:976-989).
     """
     n = len(group)
+    if stream is None and out is not None and not scatter and not in_place and 0 <= rank < n:
+        status = host.stack(out, group) if reduction.op is None else host.reduce(out, group, reduction.op)
+        if status >= 0:
+            check(status)
+            return out
     group = [factory.zeros() if t is None else t for t in group]
     local = group[rank]
     if reduction.is_stack:

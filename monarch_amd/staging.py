@@ -16,6 +16,7 @@ import torch
 
 from . import _torch
 from ._lib import RdmaBufferC, check, lib, ptr_array
+from ._native import host
 from .ndslice import Slice, slice_array
 
 
@@ -49,6 +50,11 @@ def _check_staging(buf: torch.Tensor, nbytes: int, device: torch.device) -> None
 
 def pack(base: torch.Tensor, s: Slice, out: Optional[torch.Tensor] = None, stream=None) -> torch.Tensor:
     """``out[i] = storage(base)[s.get(i)]``; returns a 1-D tensor of ``base.dtype``."""
+    if stream is None and out is not None:
+        status = host.slice_copy(True, base, s, out)
+        if status >= 0:
+            check(status)
+            return out
     _torch.require_device(base)
     _check_view_fits(base, s)
     n = len(s)
@@ -63,6 +69,10 @@ def pack(base: torch.Tensor, s: Slice, out: Optional[torch.Tensor] = None, strea
 
 def unpack(base: torch.Tensor, s: Slice, src: torch.Tensor, stream=None) -> None:
     """``storage(base)[s.get(i)] = src[i]``; elements outside the view keep their values."""
+    if stream is None:
+        status = host.slice_copy(False, base, s, src)
+        if status >= 0:
+            return check(status)
     _torch.require_device(base)
     _check_view_fits(base, s)
     _check_staging(src, len(s) * base.element_size(), base.device)
@@ -73,6 +83,11 @@ def unpack(base: torch.Tensor, s: Slice, src: torch.Tensor, stream=None) -> None
 def pack_many(base: torch.Tensor, views: Sequence[Slice], outs: Optional[List[torch.Tensor]] = None,
               stream=None) -> List[torch.Tensor]:
     """Packs several views of one tensor (a reshard's column blocks) in as few launches as possible."""
+    if stream is None and outs is not None:
+        status = host.slice_copy_many(True, base, views, outs)
+        if status >= 0:
+            check(status)
+            return outs
     _torch.require_device(base)
     for s in views:
         _check_view_fits(base, s)
@@ -89,6 +104,10 @@ def pack_many(base: torch.Tensor, views: Sequence[Slice], outs: Optional[List[to
 
 
 def unpack_many(base: torch.Tensor, views: Sequence[Slice], srcs: Sequence[torch.Tensor], stream=None) -> None:
+    if stream is None:
+        status = host.slice_copy_many(False, base, views, srcs)
+        if status >= 0:
+            return check(status)
     _torch.require_device(base)
     if len(srcs) != len(views):
         raise ValueError(f"{len(views)} views need {len(views)} staging buffers, got {len(srcs)}")
@@ -117,6 +136,12 @@ def transfer(dst_ptr: int, src_ptr: int, nbytes: int, max_segment_bytes: int = 0
 def transfer_many(dst_ptrs, src_ptrs, nbytes, max_segment_bytes: int = 0, stream=None) -> int:
     """The same for several buffers at once, the requests of all of them in one launch (64 per launch); returns
     the number of requests posted."""
+    if stream is None:
+        posted = host.transfer_many(dst_ptrs, src_ptrs, nbytes, max_segment_bytes)
+        if posted >= 0:
+            return posted
+        if posted != host.NOT_TAKEN:
+            check(-posted)
     n = len(nbytes)
     if len(dst_ptrs) != n or len(src_ptrs) != n:
         raise ValueError("transfer_many needs one destination, one source and one length per buffer")
@@ -156,6 +181,11 @@ class RDMABuffer:
         ``offset`` is added to the local address and then checked against ``dst.numel()``
         (python/monarch/_src/tensor_engine/rdma.py:160-165), which only ``offset == 0`` passes; every call that succeeds
         there means the same here, and a non-zero offset addresses the registered range instead of raising.)"""
+        if stream is None:
+            status = host.rdma_copy(True, self.addr, self.size, dst, offset)
+            if status >= 0:
+                check(status)
+                return dst.numel()
         _assert_tensor_is_1d_contiguous_uint8(dst)
         _torch.require_device(dst)
         size = dst.numel()
@@ -167,6 +197,10 @@ class RDMABuffer:
 
     def write_from(self, src: torch.Tensor, offset: int = 0, stream=None) -> None:
         """Copies ``src`` into the buffer at byte ``offset`` of it (rdma.py:187-214; ``offset`` as in ``read_into``)."""
+        if stream is None:
+            status = host.rdma_copy(False, self.addr, self.size, src, offset)
+            if status >= 0:
+                return check(status)
         _assert_tensor_is_1d_contiguous_uint8(src)
         _torch.require_device(src)
         size = src.numel()
@@ -193,12 +227,13 @@ class TensorBuffer:
 
     def stage(self, stream=None) -> RDMABuffer:
         """Gather the view into the staging bytes (call before ``buffer.read_into``)."""
-        pack(self.view, self.slice, out=self.buffer.data, stream=stream)
-        return self.buffer
+        buffer = self.buffer
+        pack(self.view, self.slice, buffer._data, stream)
+        return buffer
 
     def commit(self, stream=None) -> None:
         """Scatter the staging bytes back into the view (call after ``buffer.write_from``)."""
-        unpack(self.view, self.slice, self.buffer.data, stream=stream)
+        unpack(self.view, self.slice, self.buffer._data, stream)
 
 
 def slot_pitch(slot_bytes: int) -> int:
