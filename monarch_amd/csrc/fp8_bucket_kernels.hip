@@ -27,14 +27,15 @@ struct BucketArgs {
     uint64_t total;           // elements in the bucket
     uint64_t nblocks;
     uint32_t ntensors;
+    uint32_t grid;            // workgroups of the launch
 };
 
 // Block index of a bucket: index[b] = the tensor that holds flat element b * 1024 for b < nblocks, and
 // index[nblocks] = ntensors - 1.  Built once per bucket (the offsets do not change between steps), it replaces the
 // table search every wavefront otherwise does per span: one load instead of two dependent probe rounds.
 __global__ __launch_bounds__(kThreads) void bucket_index_kernel(uint32_t* __restrict__ index, const uint64_t* __restrict__ offsets,
-                                                                uint32_t ntensors, uint64_t nblocks) {
-    const uint64_t stride = (uint64_t)gridDim.x * kThreads;
+                                                                uint32_t ntensors, uint32_t grid, uint64_t nblocks) {
+    const uint64_t stride = (uint64_t)grid * kThreads;
     for (uint64_t b = (uint64_t)blockIdx.x * kThreads + threadIdx.x; b <= nblocks; b += stride)
         index[b] = b < nblocks ? find_tensor(offsets, 1, 0, ntensors, b * kBlock) : ntensors - 1;
 }
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
     // reads; forcing scalar loads there (reads through the constant address space) was measured and loses: single-peer
     // 0.746 -> 0.703, eight peers 0.716 -> 0.703, although buckets of a few MB gain 0.8 us.
     const uint64_t wave = (uint64_t)blockIdx.x * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint64_t nwaves = (uint64_t)gridDim.x * (kBucketThreads / 64);
+    const uint64_t nwaves = (uint64_t)a.grid * (kBucketThreads / 64);
     for (uint64_t b0 = wave * NB; b0 < a.nblocks; b0 += nwaves * NB) {
         const uint64_t span_begin = b0 * kBlock;
         const uint64_t span_end = span_begin + (uint64_t)NB * kBlock < a.total
@@ -499,7 +500,7 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
                                                                                  BucketArgs a) {
     const int lane = threadIdx.x & 63;
     const uint64_t wave = (uint64_t)blockIdx.x * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // see fp8_quantize_bucket_kernel
-    const uint64_t nwaves = (uint64_t)gridDim.x * (kBucketThreads / 64);
+    const uint64_t nwaves = (uint64_t)a.grid * (kBucketThreads / 64);
     for (uint64_t b = wave; b < a.nblocks; b += nwaves) {
         const uint64_t begin = b * kBlock;
         const uint64_t end = begin + kBlock < a.total ? begin + kBlock : a.total;
@@ -541,12 +542,14 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
 // the quantiser's is.  Codes behind the tables: 4.6 M elements, 2, 4 and 8 peers 9.18 / 10.91 / 14.09.
 constexpr int kMaxBucketPeers = 64;
 
-struct BucketPeersArgs {
+template <int N>
+struct BucketPeersArgsOf {
     BucketArgs b;
-    const uint8_t* q[kMaxBucketPeers];
-    const float* scales[kMaxBucketPeers];
+    const uint8_t* q[N];
+    const float* scales[N];
     uint32_t n;
 };
+using BucketPeersArgs = BucketPeersArgsOf<kMaxBucketPeers>;
 
 // One full block of all peers: accumulator vectors through load(j) / store(j, r), peers four at a time with all their codes
 // loaded before the first add.  Step j of a lane is the elements j * 256 + lane * 4 .. + 3.
@@ -595,7 +598,7 @@ void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
     const BucketArgs& a = p.b;
     const int lane = threadIdx.x & 63;
     const uint64_t wave = (uint64_t)blockIdx.x * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // see fp8_quantize_bucket_kernel
-    const uint64_t nwaves = (uint64_t)gridDim.x * (kBucketThreads / 64);
+    const uint64_t nwaves = (uint64_t)a.grid * (kBucketThreads / 64);
     for (uint64_t b = wave; b < a.nblocks; b += nwaves) {
         const uint64_t begin = b * kBlock;
         const bool full = begin + kBlock <= a.total;
@@ -620,7 +623,7 @@ void fp8_dequant_accumulate_bucket_many_kernel(BucketPeersArgs p) {
     }
 }
 
-// Small buckets, N peers (N == 8: eight and more), one block per wavefront.  The codes of the first N peers go first and the
+// Small buckets, N peers (and those after them, if there is room for more in the arguments), one block per wavefront.  The codes of the first N peers go first and the
 // look-up of the block's tensors runs beside them: the tables come through scalar loads, which do not wait for vector loads
 // in flight.  With the number of peers known all N * 4 code loads of a lane are in flight together (the form of large buckets
 // loads four peers at a time, and branches on each).
@@ -630,8 +633,8 @@ struct PeerCodes {
     float s[N];
 };
 
-template <int N>
-__device__ __forceinline__ void load_peers(PeerCodes<N>& c, const BucketPeersArgs& p, uint32_t r0, uint64_t b, int lane) {
+template <int N, typename Args>
+__device__ __forceinline__ void load_peers(PeerCodes<N>& c, const Args& p, uint32_t r0, uint64_t b, int lane) {
 #pragma unroll
     for (int g = 0; g < N; ++g) {
         const uint8_t* q = p.q[r0 + g] + b * kBlock;
@@ -657,16 +660,16 @@ __device__ __forceinline__ void add_peers(float (&v)[4][4], const PeerCodes<N>& 
     }
 }
 
-template <int N>
-__device__ __forceinline__ void load_and_add_peers(float (&v)[4][4], const BucketPeersArgs& p, uint32_t r0, uint64_t b, int lane) {
+template <int N, typename Args>
+__device__ __forceinline__ void load_and_add_peers(float (&v)[4][4], const Args& p, uint32_t r0, uint64_t b, int lane) {
     PeerCodes<N> c;
     load_peers<N>(c, p, r0, b, lane);
     add_peers<N>(v, c);
 }
 
-template <int N>
+template <int N, int ARGS>
 __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(5, 8)))
-void fp8_dequant_accumulate_small_bucket_kernel(BucketPeersArgs p, uint64_t wg0) {
+void fp8_dequant_accumulate_small_bucket_kernel(BucketPeersArgsOf<ARGS> p, uint64_t wg0) {
     const BucketArgs& a = p.b;
     const int lane = threadIdx.x & 63;
     const uint64_t b = (wg0 + blockIdx.x) * (kBucketThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // see fp8_quantize_bucket_kernel
@@ -688,8 +691,8 @@ void fp8_dequant_accumulate_small_bucket_kernel(BucketPeersArgs p, uint64_t wg0)
             v[j][2] = __uint_as_float(r.z); v[j][3] = __uint_as_float(r.w);
         }
         add_peers<N>(v, first);
-        if constexpr (N == 8) {
-            uint32_t r = 8;
+        if constexpr (ARGS > N) {
+            uint32_t r = N;
             for (; r + 4 <= p.n; r += 4) load_and_add_peers<4>(v, p, r, b, lane);
             if (r + 3 == p.n) load_and_add_peers<3>(v, p, r, b, lane);
             else if (r + 2 == p.n) load_and_add_peers<2>(v, p, r, b, lane);
@@ -713,11 +716,18 @@ void fp8_dequant_accumulate_small_bucket_kernel(BucketPeersArgs p, uint64_t wg0)
     }
 }
 
-template <int N>
+template <int N, int ARGS = N>
 static int launch_small_bucket(const BucketPeersArgs& p, hipStream_t stream) {
     constexpr uint64_t per_wg = kBucketThreads / 64;
+    BucketPeersArgsOf<ARGS> args;  // no more pointers than peers: see SmallDims
+    args.b = p.b;
+    args.n = p.n;
+    for (int r = 0; r < ARGS; ++r) {
+        args.q[r] = p.q[r];
+        args.scales[r] = p.scales[r];
+    }
     return launch_in_pieces((p.b.nblocks + per_wg - 1) / per_wg, kBucketThreads, 1, [&](uint64_t wg0, uint32_t count) {
-        MHIP_LAUNCH(fp8_dequant_accumulate_small_bucket_kernel<N>, dim3(count), dim3(kBucketThreads), 0, stream, p, wg0);
+        MHIP_LAUNCH((fp8_dequant_accumulate_small_bucket_kernel<N, ARGS>), dim3(count), dim3(kBucketThreads), 0, stream, args, wg0);
     });
 }
 
@@ -742,7 +752,8 @@ static int quantize_bucket(uint8_t* q, float* scales, const void* const* d_tenso
     const uint64_t per_wg = (uint64_t)(kBucketThreads / 64) * nb;
     const uint64_t wgs = (a.nblocks + per_wg - 1) / per_wg;
     const uint64_t cap = max_workgroups(kBucketThreads);
-    const dim3 grid((uint32_t)(wgs > cap ? cap : wgs));
+    a.grid = (uint32_t)(wgs > cap ? cap : wgs);
+    const dim3 grid(a.grid);
     if (nb == 1) MHIP_LAUNCH(fp8_quantize_bucket_kernel<1>, grid, dim3(kBucketThreads), 0, hs, q, scales, a);
     else MHIP_LAUNCH(fp8_quantize_bucket_kernel<kBucketBlocks>, grid, dim3(kBucketThreads), 0, hs, q, scales, a);
     return launch_status();
@@ -752,8 +763,8 @@ static int build_bucket_index(uint32_t* index, const uint64_t* d_offsets, uint32
     const uint64_t nblocks = (total + kBlock - 1) / kBlock;
     const uint64_t wgs = (nblocks + 1 + kThreads - 1) / kThreads;
     const uint64_t cap = max_workgroups(kThreads);
-    MHIP_LAUNCH(bucket_index_kernel, dim3((uint32_t)(wgs > cap ? cap : wgs)), dim3(kThreads), 0, hs, index, d_offsets, ntensors,
-                nblocks);
+    const uint32_t grid = (uint32_t)(wgs > cap ? cap : wgs);
+    MHIP_LAUNCH(bucket_index_kernel, dim3(grid), dim3(kThreads), 0, hs, index, d_offsets, ntensors, grid, nblocks);
     return launch_status();
 }
 
@@ -873,8 +884,8 @@ int mhip_fp8_dequant_accumulate_bucket(void* const* d_acc_tensors, const uint8_t
     const uint64_t cap = max_workgroups(kBucketThreads);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     DeviceGuard guard(hs);
-    MHIP_LAUNCH(fp8_dequant_accumulate_bucket_kernel, dim3((uint32_t)(wgs > cap ? cap : wgs)), dim3(kBucketThreads), 0,
-                       hs, q, scales, a);
+    a.grid = (uint32_t)(wgs > cap ? cap : wgs);
+    MHIP_LAUNCH(fp8_dequant_accumulate_bucket_kernel, dim3(a.grid), dim3(kBucketThreads), 0, hs, q, scales, a);
     return launch_status();
 }
 
@@ -913,13 +924,14 @@ int mhip_fp8_dequant_accumulate_bucket_many(void* const* d_acc_tensors, const ui
             case 5: return launch_small_bucket<5>(p, hs);
             case 6: return launch_small_bucket<6>(p, hs);
             case 7: return launch_small_bucket<7>(p, hs);
-            default: return launch_small_bucket<8>(p, hs);
+            case 8: return launch_small_bucket<8>(p, hs);
+            default: return launch_small_bucket<8, kMaxBucketPeers>(p, hs);
         }
     }
     const uint64_t wgs = (p.b.nblocks + 3) / 4;
     const uint64_t cap = max_workgroups(kBucketThreads);
-    const dim3 grid((uint32_t)(wgs > cap ? cap : wgs));
-    MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel, grid, dim3(kBucketThreads), 0, hs, p);
+    p.b.grid = (uint32_t)(wgs > cap ? cap : wgs);
+    MHIP_LAUNCH(fp8_dequant_accumulate_bucket_many_kernel, dim3(p.b.grid), dim3(kBucketThreads), 0, hs, p);
     return launch_status();
 }
 

@@ -52,10 +52,10 @@ constexpr int kQuantThreads = 64;  // single-wavefront workgroups: 0.825 of peak
 
 __global__ __launch_bounds__(kQuantThreads) void fp8_quantize_kernel(uint8_t* __restrict__ q, float* __restrict__ scales,
                                                                 const uint16_t* __restrict__ x, uint64_t numel,
-                                                                uint64_t nblocks) {
+                                                                uint64_t nblocks, uint32_t grid) {
     const int lane = threadIdx.x & 63;
     const uint64_t wave = (uint64_t)blockIdx.x * (kQuantThreads / 64) + (threadIdx.x >> 6);
-    const uint64_t nwaves = (uint64_t)gridDim.x * (kQuantThreads / 64);
+    const uint64_t nwaves = (uint64_t)grid * (kQuantThreads / 64);
     for (uint64_t b0 = wave * kQuantBlocks; b0 < nblocks; b0 += nwaves * kQuantBlocks) {
         uint4 lo[kQuantBlocks], hi[kQuantBlocks];
         bool full[kQuantBlocks];
@@ -120,8 +120,8 @@ static_assert(kBlock % kDeqTile == 0, "a tile lies inside one block");
 __global__ __launch_bounds__(kDeqThreads) void fp8_dequant_accumulate_kernel(float* __restrict__ acc,
                                                                              const uint8_t* __restrict__ q,
                                                                              const float* __restrict__ scales,
-                                                                             uint64_t numel, uint64_t ntiles) {
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+                                                                             uint64_t numel, uint64_t ntiles, uint32_t grid) {
+    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += grid) {
         const uint64_t i0 = tile * kDeqTile + threadIdx.x * 4;
         if ((tile + 1) * kDeqTile <= numel) {  // interior tile (workgroup-uniform)
             const uint32_t c = load4_unaligned(q + i0);
@@ -160,6 +160,7 @@ struct DequantManyArgs {
     uint32_t n;
     uint32_t overwrite;
     uint32_t rotate;  // workgroup i takes tile i + i / 8 of its group of 8 tiles (see the entry point)
+    uint32_t grid;    // workgroups of the launch
 };
 
 // N > 0: peers known at compile time; N == 0: a.n peers, eight at a time.  THREADS lanes cover THREADS * 4
@@ -172,8 +173,8 @@ __global__ __launch_bounds__(THREADS) void fp8_dequant_accumulate_many_kernel(De
     float* __restrict__ acc = a.acc;
     const uint32_t n = N > 0 ? N : a.n;
     uint32_t first = blockIdx.x;
-    if (a.rotate && first < (gridDim.x & ~7u)) first = (first & ~7u) | ((first + (first >> 3)) & 7u);
-    for (uint64_t tile = first; tile < a.ntiles; tile += gridDim.x) {
+    if (a.rotate && first < (a.grid & ~7u)) first = (first & ~7u) | ((first + (first >> 3)) & 7u);
+    for (uint64_t tile = first; tile < a.ntiles; tile += a.grid) {
         const uint64_t i0 = tile * TILE + threadIdx.x * 4;
         if ((tile + 1) * TILE <= a.numel) {  // interior tile, workgroup-uniform
             const uint64_t b = tile * TILE / kBlock;
@@ -238,7 +239,8 @@ template <int THREADS>
 static void launch_dequant_many(DequantManyArgs& a, hipStream_t hs) {
     a.ntiles = (a.numel + THREADS * 4 - 1) / (THREADS * 4);
     const uint64_t cap = max_workgroups(THREADS);
-    const dim3 grid((uint32_t)(a.ntiles > cap ? cap : a.ntiles)), blockdim(THREADS);
+    a.grid = (uint32_t)(a.ntiles > cap ? cap : a.ntiles);
+    const dim3 grid(a.grid), blockdim(THREADS);
     switch (a.n) {
         case 2: MHIP_LAUNCH((fp8_dequant_accumulate_many_kernel<2, THREADS>), grid, blockdim, 0, hs, a); break;
         case 4: MHIP_LAUNCH((fp8_dequant_accumulate_many_kernel<4, THREADS>), grid, blockdim, 0, hs, a); break;
@@ -265,8 +267,9 @@ int mhip_fp8_quantize(uint8_t* q, float* scales, const void* x_bf16, uint64_t nu
     const uint64_t cap = max_workgroups(kQuantThreads);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     DeviceGuard guard(hs);
-    MHIP_LAUNCH(fp8_quantize_kernel, dim3((uint32_t)(wgs > cap ? cap : wgs)), dim3(kQuantThreads), 0, hs, q, scales,
-                       static_cast<const uint16_t*>(x_bf16), numel, nblocks);
+    const uint32_t grid = (uint32_t)(wgs > cap ? cap : wgs);
+    MHIP_LAUNCH(fp8_quantize_kernel, dim3(grid), dim3(kQuantThreads), 0, hs, q, scales, static_cast<const uint16_t*>(x_bf16), numel, nblocks,
+                grid);
     return launch_status();
 }
 
@@ -280,8 +283,8 @@ int mhip_fp8_dequant_accumulate(float* acc, const uint8_t* q, const float* scale
     const uint64_t cap = max_workgroups(kDeqThreads);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     DeviceGuard guard(hs);
-    MHIP_LAUNCH(fp8_dequant_accumulate_kernel, dim3((uint32_t)(ntiles > cap ? cap : ntiles)), dim3(kDeqThreads), 0,
-                       hs, acc, q, scales, numel, ntiles);
+    const uint32_t grid = (uint32_t)(ntiles > cap ? cap : ntiles);
+    MHIP_LAUNCH(fp8_dequant_accumulate_kernel, dim3(grid), dim3(kDeqThreads), 0, hs, acc, q, scales, numel, ntiles, grid);
     return launch_status();
 }
 

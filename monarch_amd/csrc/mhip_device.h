@@ -46,15 +46,38 @@ inline bool make_dims_arg(const CanonSlice& c, DimsArg* d, bool* fits32, int pad
     return true;
 }
 
+// The same for a slice of ND dimensions (1 to 3) in 32-bit mode and nothing a kernel does not read.
+//
+// Why kernels of small copies have argument structs of their own, and why no kernel asks for gridDim: a launch writes the
+// arguments into memory that the GPU reads, and depending on where the calling thread runs that is free or not.  hipLaunchKernel
+// took 2.2 us whatever the size in some processes, and in others 2.4 at 8 to 64 bytes, 2.6 at 96 and 3.1 to 3.5 from 128 bytes on
+// (the general structs have 280 to 640).  A kernel that reads gridDim gets 256 bytes of hidden arguments on top.  Host time of
+// a call in such a process, general arguments / these, us: a pack of 512 KiB 4.2 / 2.8, a small transposing pack 3.8 / 2.85, rows of
+// 66 bytes 4.1 / 2.9, a reduce of eight 4.0 / 2.85, of three 4.0 / 2.75; in the others 2.5 / 2.35 and 2.4 / 2.25.
+template <int ND>
+struct SmallDims {
+    FastDiv32 run_div;
+    FastDiv32 inner_div[ND - 1];  // sizes of dimensions 1, 2
+    uint64_t stride[ND];          // units
+    explicit SmallDims(const DimsArg& d) : run_div(d.run_div) {
+        for (int k = 0; k < ND; ++k) stride[k] = d.stride[k];
+        for (int k = 1; k < ND; ++k) inner_div[k - 1] = d.size_div[k];
+    }
+};
+__device__ __forceinline__ uint64_t run_of(const DimsArg& d) { return d.run; }
+template <int ND> __device__ __forceinline__ uint32_t run_of(const SmallDims<ND>& d) { return d.run_div.d; }
+__device__ __forceinline__ const FastDiv32& size_div_of(const DimsArg& d, int k) { return d.size_div[k]; }
+template <int ND> __device__ __forceinline__ const FastDiv32& size_div_of(const SmallDims<ND>& d, int k) { return d.inner_div[k - 1]; }
+
 // Unit offset of row `row` of a slice in 32-bit mode; NDIM as in decode.
-template <int NDIM = -1>
-__device__ __forceinline__ uint64_t row_offset(const DimsArg& d, uint32_t row) {
+template <int NDIM = -1, typename Dims>
+__device__ __forceinline__ uint64_t row_offset(const Dims& d, uint32_t row) {
     uint64_t off = 0;
     if constexpr (NDIM >= 0) {
 #pragma unroll
         for (int k = NDIM - 1; k > 0; --k) {
             uint32_t q, r;
-            d.size_div[k].divmod(row, q, r);
+            size_div_of(d, k).divmod(row, q, r);
             off += (uint64_t)r * d.stride[k];
             row = q;
         }
@@ -72,9 +95,10 @@ __device__ __forceinline__ uint64_t row_offset(const DimsArg& d, uint32_t row) {
 // Unit offset of packed unit t, and its column within the row (for run-boundary tests).
 // NDIM >= 0 fixes the number of dimensions outside the run at compile time (no loop, no
 // kernel-argument loads inside the decode); NDIM < 0 reads it from the arguments.
-template <bool WIDE, int NDIM = -1>
-__device__ __forceinline__ uint64_t decode(const DimsArg& d, uint64_t t, uint64_t* col_out) {
-    const int ndim = NDIM >= 0 ? NDIM : d.ndim;
+template <bool WIDE, int NDIM = -1, typename Dims>
+__device__ __forceinline__ uint64_t decode(const Dims& d, uint64_t t, uint64_t* col_out) {
+    int ndim = NDIM;
+    if constexpr (NDIM < 0) ndim = d.ndim;
     if (ndim == 0) {
         *col_out = t;  // one row: run == total
         return t;

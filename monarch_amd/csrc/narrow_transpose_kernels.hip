@@ -19,27 +19,32 @@
 // pass follow from those of the pass before.  With divisions and 64-bit multiplications / now, us: f32 512^2 2.77 / 2.58,
 // 1216^2 3.47 / 2.96, u8 [68359, 32, 32] 86 / 69, f32 [68359, 16, 16] 45.9 / 37, f32 [40, 2000, 128] 18.7 / 17.0, 1000 calls of all
 // types and sizes 0.92 x on average.
+#include <type_traits>
+
 #include "mhip_device.h"
 #include "pack_internal.h"
 
 namespace mhip {
 
-struct NarrowArgs {
+// What views of one dimension after c and at most one before it need (ONE), in 112 bytes: see SmallDims for why that counts.
+struct NarrowOneArgs {
     char* base;                   // address of the view's first element
     char* packed;
     uint32_t Sc, Q;               // extents along c and along q
     uint32_t vi, vj;              // read rows and columns a tile holds: the tile's own, or the extent where that is shorter
-    uint32_t ti_count, tj_count;  // tiles along i and along j
-    uint32_t nv;                  // vectors per read row
+    FastDiv32 nv_div;             // vectors per read row
     uint32_t row_step, vec_step;  // a pass of all lanes over the vectors of the read rows: lanes / nv and lanes % nv
-    uint32_t write_through;       // how written vectors are stored, see try_narrow_transpose
-    FastDiv32 nv_div;
     uint32_t ntiles, per_xcd;     // each XCD takes a contiguous share of the tiles
     uint32_t wg0;                 // workgroups of this copy launched before this grid
+    uint32_t mem_pitch;           // consecutive q lie that many elements apart
     FastDiv32 per_batch_div;      // tiles per matrix
     FastDiv32 fast_div;           // tiles along the side that has fewer of them
-    uint32_t one_inner;           // consecutive q lie mem_pitch elements apart: one dimension after c
-    uint32_t mem_pitch;
+    uint32_t i_fast;              // that side is i
+    uint32_t write_through;       // how written vectors are stored, see try_narrow_transpose
+    uint64_t batch_stride;        // bytes
+};
+
+struct NarrowArgs : NarrowOneArgs {
     int n_inner, n_outer;         // dimensions after c (q -> memory offset) and before c (batch -> memory offset)
     FastDiv32 inner_div[kMaxCanonDims];
     uint64_t inner_stride[kMaxCanonDims];  // bytes
@@ -66,8 +71,18 @@ __device__ __forceinline__ u32x4 shift_down(u32x4 v, uint32_t bytes) {
 //     are whole blocks, no two of the 64 lanes meet in a bank at different addresses.  The last vector of a ragged row
 //     starts inside a block and sees two keys, i.e. up to two addresses in a bank; words of 8 bytes take two turns anyway,
 //     three when ragged.
-template <typename T, int THREADS, bool PACK, int TI, int TJ, bool ONE>
-__global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowArgs a) {
+// As many wavefronts per SIMD as the tiles that fit the 160 KiB of LDS bring, eight at most: the registers must not allow fewer.
+// (Left alone, the compiler moves the LDS reads of all passes of a 64 KiB tile ahead, in 230 registers: one workgroup per CU
+// and 19 us where two take 11.)  Where LATE it is left alone: all columns are collected before the first is stored (see
+// launch_narrow_tile).
+constexpr int narrow_waves(int threads, int tile_bytes, bool late) {
+    const int waves = 163840 / tile_bytes * threads / 256;
+    return late ? 1 : waves > 8 ? 8 : waves;
+}
+
+template <typename T, int THREADS, bool PACK, int TI, int TJ, bool ONE, bool LATE>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(narrow_waves(THREADS, TI * TJ * sizeof(T), LATE), 8)))
+void slice_transpose_narrow_kernel(std::conditional_t<ONE, NarrowOneArgs, NarrowArgs> a) {
     constexpr uint32_t ES = sizeof(T), E = 16 / ES;
     constexpr uint32_t GJ = TJ / E, GI = TI / E;
     constexpr uint32_t W = ES >= 4 ? 1 : 4 / ES;  // columns per LDS word
@@ -86,22 +101,24 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowA
     a.per_batch_div.divmod(id, b, in_batch);
     // the side with fewer tiles is the fast one: neighbouring workgroups share whole rows of it
     a.fast_div.divmod(in_batch, slow, fast);
-    const bool i_fast = a.ti_count < a.tj_count;
     // a tile that would hang over the edge is moved back inside; the overlap is written twice, same bytes
     const uint32_t I = PACK ? a.Q : a.Sc, J = PACK ? a.Sc : a.Q;
-    uint32_t i0 = (i_fast ? fast : slow) * TI, j0 = (i_fast ? slow : fast) * TJ;
+    uint32_t i0 = (a.i_fast ? fast : slow) * TI, j0 = (a.i_fast ? slow : fast) * TJ;
     if (i0 + a.vi > I) i0 = I - a.vi;
     if (j0 + a.vj > J) j0 = J - a.vj;
     const uint32_t q0 = PACK ? i0 : j0, c0 = PACK ? j0 : i0;
     char* __restrict__ packed = a.packed + (((uint64_t)b * a.Sc + c0) * a.Q + q0) * ES;  // the tile's first element, on both sides
     char* __restrict__ mem = a.base + (uint64_t)c0 * ES;
-    for (int k = a.n_outer - 1; k >= 0; --k) {
-        uint32_t rest, index;
-        a.outer_div[k].divmod(b, rest, index);
-        mem += index * a.outer_stride[k];
-        b = rest;
+    if constexpr (ONE) {
+        mem += b * a.batch_stride + (uint64_t)q0 * a.mem_pitch * ES;
+    } else {
+        for (int k = a.n_outer - 1; k >= 0; --k) {
+            uint32_t rest, index;
+            a.outer_div[k].divmod(b, rest, index);
+            mem += index * a.outer_stride[k];
+            b = rest;
+        }
     }
-    if constexpr (ONE) mem += (uint64_t)q0 * a.mem_pitch * ES;
     // addresses inside the tile: q and c counted from its first element
     auto packed_at = [&](uint32_t q, uint32_t c) { return packed + ((uint64_t)c * a.Q + q) * ES; };
     auto mem_at = [&](uint32_t q, uint32_t c) {
@@ -121,7 +138,7 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowA
     };
 
     // ---- read side -> LDS: the tile's vectors numbered through, so that short rows leave no lane idle ----
-    const uint32_t total = a.vi * a.nv;
+    const uint32_t nv = a.nv_div.d, total = a.vi * nv;
     const bool ragged_j = a.vj % E != 0;
     u32x4 d[RP];
     uint32_t row[RP], vec[RP];
@@ -131,8 +148,8 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowA
         if (p > 0) {  // every pass moves on by the same number of vectors
             row[p] = row[p - 1] + a.row_step;
             vec[p] = vec[p - 1] + a.vec_step;
-            if (vec[p] >= a.nv) {
-                vec[p] -= a.nv;
+            if (vec[p] >= nv) {
+                vec[p] -= nv;
                 ++row[p];
             }
         }
@@ -219,28 +236,31 @@ __global__ __launch_bounds__(THREADS) void slice_transpose_narrow_kernel(NarrowA
 }
 
 // WB and RB: bytes of a written and of a read row of the tile
-template <typename T, bool PACK, int WB, int RB>
+template <typename T, bool PACK, int WB, int RB, bool LATE = false>
 static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     constexpr uint32_t ES = sizeof(T), E = 16 / ES, TI = WB / ES, TJ = RB / ES;
     constexpr int kBytes = TI * TJ * ES, kLanes = kBytes >= 32768 ? 512 : kBytes >= 8192 ? 256 : 128;
     const uint32_t I = PACK ? a.Q : a.Sc, J = PACK ? a.Sc : a.Q;
     a.vi = I < TI ? I : TI;
     a.vj = J < TJ ? J : TJ;
-    a.ti_count = (I + TI - 1) / TI;
-    a.tj_count = (J + TJ - 1) / TJ;
-    a.nv = (a.vj + E - 1) / E;
-    a.nv_div = FastDiv32(a.nv);
-    a.row_step = kLanes / a.nv;
-    a.vec_step = kLanes % a.nv;
+    const uint32_t ti_count = (I + TI - 1) / TI, tj_count = (J + TJ - 1) / TJ, nv = (a.vj + E - 1) / E;
+    a.nv_div = FastDiv32(nv);
+    a.row_step = kLanes / nv;
+    a.vec_step = kLanes % nv;
     // fewer than kFastDivLimit: a tile moves 256 bytes at least, and no GPU holds 2^31 times that (see try_narrow_transpose)
-    a.ntiles = (uint32_t)(nbatch * a.ti_count * a.tj_count);
+    a.ntiles = (uint32_t)(nbatch * ti_count * tj_count);
     a.per_xcd = (a.ntiles + 7) / 8;
-    a.per_batch_div = FastDiv32(a.ti_count * a.tj_count);
-    a.fast_div = FastDiv32(a.ti_count < a.tj_count ? a.ti_count : a.tj_count);
+    a.per_batch_div = FastDiv32(ti_count * tj_count);
+    a.i_fast = ti_count < tj_count;
+    a.fast_div = FastDiv32(a.i_fast ? ti_count : tj_count);
+    const bool one = a.n_inner == 1 && a.n_outer <= 1 && a.inner_stride[0] / ES <= UINT32_MAX;
+    a.mem_pitch = (uint32_t)(a.inner_stride[0] / ES);
+    a.batch_stride = a.n_outer == 1 ? a.outer_stride[0] : 0;
     return launch_in_pieces((uint64_t)a.per_xcd * 8, kLanes, 8, [&](uint64_t wg0, uint32_t count) {
         a.wg0 = (uint32_t)wg0;
-        if (a.one_inner) MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, true>), dim3(count), dim3(kLanes), 0, stream, a);
-        else MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, false>), dim3(count), dim3(kLanes), 0, stream, a);
+        const NarrowOneArgs& small = a;
+        if (one) MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, true, LATE>), dim3(count), dim3(kLanes), 0, stream, small);
+        else MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, false, LATE>), dim3(count), dim3(kLanes), 0, stream, a);
     });
 }
 
@@ -251,7 +271,7 @@ static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
 //     unpacking, one tile of 32 or 16 KiB -> 64 KiB, us: bf16 [64, 4096, 64] 15.6 / 14.9 -> 13.1 / 13.1, [56, 4096, 64] 13.9 / 13.7 ->
 //     12.1 / 11.2, [256, 1024, 64] 16.0 / 14.9 -> 13.1 / 15.0, f32 [262144, 32] 16.2 / 12.3 -> 11.1 / 10.8.  With fewer or more of them
 //     the part runs out of step again and large tiles lose: [32, 4096, 64] 8.1 / 7.5 -> 8.8 / 8.4, [96, 4001, 64] 21.7 / 20.2 ->
-//     22.4 / 22.1.
+//     22.4 / 22.1.  (Kernels with NarrowArgs; with NarrowOneArgs and registers for two tiles per CU the first is 12.3 / 12.6.)
 //   * 4-byte elements from 28 MiB on: tiles of 32 KiB instead of 16 (f32 [64, 4096, 32] 18.0 / 14.3 -> 15.2 / 14.5, [1 M, 16] 28.0 /
 //     25.8 -> 24.7 / 23.2; sides of 64 to 256 bytes, 33 to 100 MiB, 0.89 to 0.99 x; 17 MiB up to 1.1 x).
 constexpr uint64_t kResidentTilesMin = 400, kResidentTilesMax = 512;
@@ -290,6 +310,8 @@ static uint32_t narrow_tile_bytes(uint64_t bytes) {
 // 4 MiB and more whose sides are both longer than 512 bytes take 256 x 256 bytes (f64 pack / unpack, 128 x 128 and 256 x 256: 627^2
 // 3.1 / 3.3 and 2.9 / 2.9, 640^2 3.1 / 3.2 and 3.3 / 3.1, 887^2 4.8 / 5.1 and 4.0 / 3.9, 1145^2 6.7 / 6.5 and 5.8 / 5.7, where the
 // tiles of transpose_kernels.hip take 6.0 / 6.0; [3584, 16, 16] 4.5 / 4.4 and 6.5 / 6.4).
+// Byte matrices of 12 to 23 MiB collect all columns of a tile before they store the first (LATE): warm 0.95 of the time it took
+// with 64-bit tile numbers where the other order takes 1.05, cold 0.98 and 1.11; up to 12 MiB 0.92 and 0.82.
 // Batches of matrices that fit 128 x 128 bytes keep that tile at any size: u8 [78125, 16, 16] 94 / 95 us, in tiles of 1024 x 64 of
 // which one matrix fills little 335 / 333; bf16 [39062, 16, 16] 45 / 46 and 97 / 98, [8544, 64, 64] 23.2 / 23.3 and 30.2 / 31.3.
 template <typename T, bool PACK>
@@ -298,7 +320,10 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
     const uint64_t ib = (uint64_t)(PACK ? a.Q : a.Sc) * ES, jb = (uint64_t)(PACK ? a.Sc : a.Q) * ES;
     const uint64_t bytes = nbatch * ib * jb / ES;
     if constexpr (ES == 1)
-        if (ib > 512 && jb > 512 && bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+        if (ib > 512 && jb > 512 && bytes > (12ull << 20)) {
+            if (bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
+            return launch_narrow<T, PACK, 128, 128, true>(a, nbatch, stream);
+        }
     if (bytes >= (16ull << 20) && (ib <= 512 || jb <= 512) && (ib > 128 || jb > 128)) {  // a long side to fill the tile with
         const bool short_j = jb <= ib;
         uint32_t n = narrow_tile_bytes(short_j ? jb : ib);
@@ -363,9 +388,6 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
     a.packed = packed;
     a.Sc = (uint32_t)Sc;
     a.Q = Q;
-    const uint64_t pitch = a.inner_stride[0] / unit;
-    a.one_inner = a.n_inner == 1 && pitch <= UINT32_MAX;
-    a.mem_pitch = (uint32_t)pitch;
     // Written rows that start on half cache lines are stored write-through (33.6 MB of keys 14.8 us against 16.5 through
     // the cache, unpacked rows of 64 bytes 7.6 against 8.5); others go through the cache, which combines what neighbouring
     // tiles share (rows of 4001 bf16 15.9 against 18.9, unpacked rows of 160 bytes 19.2 against 19.9), unless the launch

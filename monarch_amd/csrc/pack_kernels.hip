@@ -13,6 +13,8 @@
 //   contiguous_copy_kernel    one run of any alignment: rows on the destination's 1 KiB boundaries
 // (views whose memory-contiguous dimension is not the innermost one go to the LDS-tiled
 // transposing kernels instead).  The host picks the form per launch from the canonical slice.
+#include <type_traits>
+
 #include "mhip_device.h"
 #include "fp8_common.h"
 #include "pack_internal.h"
@@ -42,7 +44,35 @@ struct PackArgs {
     uint32_t stream_stores;      // slice_copy_kernel unpacking 16-byte units, slice_unpack_lines_kernel: non-temporal
                                  //   instead of write-through stores
     DimsArg dims;
+    using Index = uint64_t;
 };
+
+// The arguments of one view of ND dimensions with fewer than 2^31 units, in 88 to 128 bytes where PackArgs has 608
+// (see SmallDims for what that saves).
+template <int ND>
+struct OneViewArgs {
+    char* base;      // the view's first element
+    char* packed;
+    uint32_t total, nchunks, shift;
+    uint32_t wg0, per_xcd, nwg;
+    uint32_t stream_stores;
+    uint32_t nrows;
+    FastDiv32 pieces_div;
+    SmallDims<ND> dims;
+    using Index = uint32_t;
+    OneViewArgs(const PackArgs& a, uint32_t unit)
+        : base(a.base + a.offset[0] * unit), packed(a.packed[0]), total((uint32_t)a.total), nchunks((uint32_t)a.nchunks), shift(a.shift),
+          wg0((uint32_t)a.wg0), per_xcd((uint32_t)a.per_xcd), nwg((uint32_t)a.nwg), stream_stores(a.stream_stores), nrows((uint32_t)a.nrows),
+          pieces_div(a.pieces_div), dims(a.dims) {}
+};
+template <int ND> __device__ __forceinline__ void tile_and_view(const OneViewArgs<ND>&, uint32_t wg, uint32_t* tile, uint32_t* v) {
+    *tile = wg;
+    *v = 0;
+}
+__device__ __forceinline__ char* packed_of(const PackArgs& a, uint32_t v) { return a.packed[v]; }
+template <int ND> __device__ __forceinline__ char* packed_of(const OneViewArgs<ND>& a, uint32_t) { return a.packed; }
+__device__ __forceinline__ char* strided_of(const PackArgs& a, uint32_t v, uint32_t unit) { return a.base + a.offset[v] * unit; }
+template <int ND> __device__ __forceinline__ char* strided_of(const OneViewArgs<ND>& a, uint32_t, uint32_t) { return a.base; }
 
 // The view index is the fastest-varying part of the workgroup id, so that workgroups running side by side work on the
 // same rows of neighbouring views (for column blocks of one tensor: neighbouring segments of the same rows).  No 64-bit
@@ -74,8 +104,8 @@ __device__ __forceinline__ void move_unit(char* strided, char* packed) {
 
 // One chunk moved unit by unit, with every unit tested against the view's extent: the ragged first
 // and last chunk of a view, and chunks that no vector form applies to.
-template <int U, bool PACK, bool WIDE, int NDIM>
-__device__ __forceinline__ void move_chunk_by_units(const PackArgs& a, char* strided, char* packed, uint64_t chunk) {
+template <int U, bool PACK, bool WIDE, int NDIM, typename Args>
+__device__ __forceinline__ void move_chunk_by_units(const Args& a, char* strided, char* packed, uint64_t chunk) {
     constexpr int VU = 16 / U;
     const uint64_t tb = chunk * VU;
     for (int j = 0; j < VU; ++j) {
@@ -92,35 +122,36 @@ __device__ __forceinline__ void move_chunk_by_units(const PackArgs& a, char* str
 // workgroup (back to back, pack / unpack: 0.5 MiB in rows of 1 KiB 3.04 / 2.92 us -> 2.65 / 2.66, 4 MiB 3.25 / 3.21 -> 2.75 /
 // 2.84, 2 MiB of attention heads 3.17 / 3.10 -> 2.47 / 2.61, 7 MiB in rows of 1200 bytes 4.02 / 4.59 -> 3.55 / 3.66), and at
 // 117 MiB eight chunks per lane reach 0.73 of peak where one reaches 0.76.
-template <int U, bool PACK, bool WIDE, int NDIM>
-__global__ __launch_bounds__(kPackThreads) void slice_copy_kernel(PackArgs a) {
+template <int U, bool PACK, bool WIDE, int NDIM, typename Args>
+__global__ __launch_bounds__(kPackThreads) void slice_copy_kernel(Args a) {
     constexpr int VU = 16 / U;  // units per chunk
-    uint64_t wg = a.wg0 + blockIdx.x;
+    using Index = typename Args::Index;
+    Index wg = a.wg0 + blockIdx.x;
     if (a.per_xcd != 0) {  // each XCD on a contiguous share: see the note above copy_views
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    uint64_t tile;
+    Index tile;
     uint32_t v;
     tile_and_view(a, wg, &tile, &v);
-    char* __restrict__ packed = a.packed[v];
-    char* __restrict__ strided = a.base + a.offset[v] * U;
-    const uint64_t c = tile * kPackThreads + threadIdx.x;
+    char* __restrict__ packed = packed_of(a, v);
+    char* __restrict__ strided = strided_of(a, v, U);
+    const Index c = tile * kPackThreads + threadIdx.x;
     if (c >= a.nchunks) return;
-    const uint64_t tb = c * VU;           // position counted from the aligned-down start
-    const uint64_t first = tb - a.shift;  // first packed unit of the chunk; wraps for a ragged chunk 0, which is not a vector
+    const Index tb = c * VU;           // position counted from the aligned-down start
+    const Index first = tb - a.shift;  // first packed unit of the chunk; wraps for a ragged chunk 0, which is not a vector
     if (tb >= a.shift && first + VU <= a.total) {
         uint64_t col;
         const uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
-        if (col + VU <= a.dims.run) {
+        if (col + VU <= run_of(a.dims)) {
             // Stores to 16-byte aligned addresses go out write-through (column blocks of 3584-byte runs: pack 0.77 -> 0.79 of
             // peak; 128-byte runs of a [B,H,S,D] -> [B,S,H,D] permute: 0.69 -> 0.77); unaligned ones do not
             // (a row pitch that is only 2-byte aligned: unpack 0.74 -> 0.71), nor do the
             // flat bucket pack and the fp8 accumulate, which all lose 1-2 points with it.
             if constexpr (PACK) {
-                store16_writethrough(packed + first * U, load16_unaligned(strided + loc * U));
+                store16_writethrough(packed + (uint64_t)first * U, load16_unaligned(strided + loc * U));
             } else {
-                const uint4 data = load16_aligned(packed + first * U);
+                const uint4 data = load16_aligned(packed + (uint64_t)first * U);
                 if constexpr (U == 16) {
                     if (a.stream_stores) store16_unaligned(strided + loc * U, data);  // wave-uniform
                     else store16_writethrough(strided + loc * U, data);
@@ -151,21 +182,22 @@ __global__ __launch_bounds__(kPackThreads) void slice_copy_kernel(PackArgs a) {
 // Needs rows of at least one chunk; the ragged first and last chunk of a view still go unit by unit.
 constexpr int kRaggedUnroll = 1;  // measured: 1 chunk per lane 0.75, 2 0.73, 4 0.72, 8 0.72 of peak (fp32 rows of 1791)
 
-template <int U, bool PACK, bool WIDE, int NDIM>
-__global__ __launch_bounds__(kPackThreads) void slice_copy_ragged_kernel(PackArgs a) {
+template <int U, bool PACK, bool WIDE, int NDIM, typename Args>
+__global__ __launch_bounds__(kPackThreads) void slice_copy_ragged_kernel(Args a) {
     constexpr int VU = 16 / U;
     constexpr int UN = kRaggedUnroll;
-    uint64_t wg = a.wg0 + blockIdx.x;
+    using Index = typename Args::Index;
+    Index wg = a.wg0 + blockIdx.x;
     if (a.per_xcd != 0) {  // each XCD on a contiguous share: see the note above copy_views
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    uint64_t tile;
+    Index tile;
     uint32_t v;
     tile_and_view(a, wg, &tile, &v);
-    char* __restrict__ packed = a.packed[v];
-    char* __restrict__ strided = a.base + a.offset[v] * U;
-    const uint64_t c0 = tile * (kPackThreads * UN) + threadIdx.x;
+    char* __restrict__ packed = packed_of(a, v);
+    char* __restrict__ strided = strided_of(a, v, U);
+    const Index c0 = tile * (kPackThreads * UN) + threadIdx.x;
     // what idle lanes load: the aligned vector that holds the first byte of the side that is read
     const char* const idle = reinterpret_cast<const char*>((uintptr_t)(PACK ? strided : packed) & ~(uintptr_t)15);
     uint64_t pa[UN], sa[UN], pb[UN], sb[UN];  // packed / strided unit index of vector A and vector B
@@ -173,16 +205,16 @@ __global__ __launch_bounds__(kPackThreads) void slice_copy_ragged_kernel(PackArg
     bool any_b = false;
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
-        const uint64_t c = c0 + (uint64_t)i * kPackThreads;
-        const uint64_t tb = c * VU;
-        const uint64_t first = tb - a.shift;
+        const Index c = c0 + i * kPackThreads;
+        const Index tb = c * VU;
+        const Index first = tb - a.shift;
         pa[i] = sa[i] = pb[i] = sb[i] = 0;
         do_a[i] = do_b[i] = edge[i] = false;
         if (c < a.nchunks) {
             if (tb >= a.shift && first + VU <= a.total) {
                 uint64_t col;
                 const uint64_t loc = decode<WIDE, NDIM>(a.dims, first, &col);
-                const uint64_t rem = a.dims.run - col;  // units of this row from `first` on
+                const uint64_t rem = run_of(a.dims) - col;  // units of this row from `first` on
                 do_a[i] = true;
                 if (rem >= VU) {
                     pa[i] = first;
@@ -249,18 +281,19 @@ __global__ __launch_bounds__(kPackThreads) void slice_copy_ragged_kernel(PackArg
 // sizes (u8 rows of 1788 0.41-0.44 -> 0.54-0.58, of 3580 0.59-0.63 -> 0.66-0.80, 82 MB 0.64 -> 0.76; eight bf16 column
 // blocks of 1790 in one launch, 59 MB together, 0.70 -> 0.76); larger ones stream (117 MB in eight views 0.72 against
 // 0.70 write-through, one view of 117 MB 0.71 against 0.66, of 235 MB 0.76 against 0.66).
-template <int U, bool WIDE, int NDIM>
-__global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackArgs a) {
-    uint64_t wg = a.wg0 + blockIdx.x;
+template <int U, bool WIDE, int NDIM, typename Args>
+__global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(Args a) {
+    using Index = typename Args::Index;
+    Index wg = a.wg0 + blockIdx.x;
     if (a.per_xcd != 0) {  // each XCD on a contiguous share: see the note above copy_views
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    uint64_t tile;
+    Index tile;
     uint32_t v;
     tile_and_view(a, wg, &tile, &v);
-    const uint64_t task = tile * (kPackThreads / 8) + (threadIdx.x >> 3);  // one line of one row
-    uint64_t r;                                                             // row of the view, in iteration order
+    const Index task = tile * (kPackThreads / 8) + (threadIdx.x >> 3);  // one line of one row
+    Index r;                                                                // row of the view, in iteration order
     uint32_t line;
     if constexpr (WIDE) {
         r = task / a.pieces;
@@ -274,10 +307,10 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
     const bool live = r < a.nrows;
     if (!live) r = 0;
     uint64_t col;
-    const uint64_t loc = decode<WIDE, NDIM>(a.dims, r * a.dims.run, &col);  // first unit of the row; col == 0
-    char* __restrict__ row = a.base + (a.offset[v] + loc) * U;
-    const char* __restrict__ prow = a.packed[v] + r * a.dims.run * U;       // the row in the packed image
-    const int64_t run_bytes = (int64_t)(a.dims.run * U);                    // at least 16
+    const uint64_t loc = decode<WIDE, NDIM>(a.dims, r * run_of(a.dims), &col);  // first unit of the row; col == 0
+    char* __restrict__ row = strided_of(a, v, U) + loc * U;
+    const char* __restrict__ prow = packed_of(a, v) + (uint64_t)r * run_of(a.dims) * U;       // the row in the packed image
+    const int64_t run_bytes = (int64_t)((uint64_t)run_of(a.dims) * U);                    // at least 16
     const int64_t lead = (int64_t)((uintptr_t)row & 127u);                  // the row starts `lead` bytes into its first line
     const int64_t at = (int64_t)line * 128 + (int64_t)(threadIdx.x & 7u) * 16 - lead;  // this lane's vector, relative to the row
     const bool active = live && at + 16 > 0 && at < run_bytes;
@@ -315,22 +348,23 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(PackAr
 // ones do not (u8 k=2 26.6 -> 28.5), nor do 8-byte units (bf16 rows of 1400 bytes packing 10.4 -> 11.0, of 3080 bytes 19.1 ->
 // 20.1), nor do rows under 256 bytes of 2- and 4-byte units packing 32 MiB and more (60 MB in rows of 20 / 44 / 136 bytes 35.4 /
 // 32.8 / 30.2, plain mapping 33.2 / 31.5 / 29.1; 16 MB in rows of 72 bytes 8.7, plain 9.9).
-template <int U, bool PACK, int NDIM, bool RUN1, bool STREAM>
-__global__ __launch_bounds__(kPackThreads) void slice_units_kernel(PackArgs a) {
+template <int U, bool PACK, int NDIM, bool RUN1, bool STREAM, typename Args>
+__global__ __launch_bounds__(kPackThreads) void slice_units_kernel(Args a) {
     using T = typename UnitType<U>::type;
     using M = typename UnitType<U>::mem;  // the strided side may be less aligned than the unit
     constexpr int VU = 16 / U;
     __shared__ __attribute__((aligned(16))) T buf[kPackThreads * VU];
-    uint64_t wg = a.wg0 + blockIdx.x;
+    using Index = typename Args::Index;
+    Index wg = a.wg0 + blockIdx.x;
     if (a.per_xcd != 0) {  // each XCD on a contiguous share: see the note above copy_views
         wg = (wg & 7) * a.per_xcd + (wg >> 3);
         if (wg >= a.nwg) return;
     }
-    uint64_t tile;
+    Index tile;
     uint32_t v;
     tile_and_view(a, wg, &tile, &v);
-    char* __restrict__ packed = a.packed[v];
-    M* __restrict__ strided = reinterpret_cast<M*>(a.base) + a.offset[v];
+    char* __restrict__ packed = packed_of(a, v);
+    M* __restrict__ strided = reinterpret_cast<M*>(strided_of(a, v, U));
     const uint32_t total = (uint32_t)a.total;
     const uint32_t pos0 = (uint32_t)tile * (kPackThreads * VU);  // position of the tile, counted from the aligned-down start
     const uint32_t mine = pos0 + threadIdx.x * VU;               // and of this lane's vector of the packed side
@@ -787,17 +821,24 @@ __global__ __launch_bounds__(THREADS) void flat_copy_kernel(FlatArgs a) {
 
 enum CopyForm { kWholeChunks, kRaggedRows, kShortRuns, kGatherUnits, kUnpackLines };
 
+// launch(args) with the arguments of one view in their short form (see OneViewArgs).
+template <int ND, typename F>
+static void with_args(const PackArgs& a, uint32_t unit, F&& launch) {
+    if (a.nviews == 1) launch(OneViewArgs<ND>(a, unit));
+    else launch(a);
+}
+
 template <int U, bool PACK>
 static void launch_whole_chunks(bool wide, int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
     const dim3 block(kPackThreads);
     if (wide) {
-        MHIP_LAUNCH((slice_copy_kernel<U, PACK, true, -1>), grid, block, 0, stream, a);
+        MHIP_LAUNCH((slice_copy_kernel<U, PACK, true, -1, PackArgs>), grid, block, 0, stream, a);
         return;
     }
     switch (ndim) {  // the common shapes get a decode without loops
-        case 1: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 1>), grid, block, 0, stream, a); break;
-        case 2: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 2>), grid, block, 0, stream, a); break;
-        default: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, -1>), grid, block, 0, stream, a); break;
+        case 1: with_args<1>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 1, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+        case 2: with_args<2>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, 2, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+        default: MHIP_LAUNCH((slice_copy_kernel<U, PACK, false, -1, PackArgs>), grid, block, 0, stream, a); break;
     }
 }
 
@@ -805,10 +846,10 @@ template <int U, bool PACK, bool RUN1, bool STREAM>
 static void launch_units(int ndim, dim3 grid, hipStream_t stream, const PackArgs& a) {
     const dim3 block(kPackThreads);
     switch (ndim) {
-        case 1: MHIP_LAUNCH((slice_units_kernel<U, PACK, 1, RUN1, STREAM>), grid, block, 0, stream, a); break;
-        case 2: MHIP_LAUNCH((slice_units_kernel<U, PACK, 2, RUN1, STREAM>), grid, block, 0, stream, a); break;
-        case 3: MHIP_LAUNCH((slice_units_kernel<U, PACK, 3, RUN1, STREAM>), grid, block, 0, stream, a); break;
-        default: MHIP_LAUNCH((slice_units_kernel<U, PACK, -1, RUN1, STREAM>), grid, block, 0, stream, a); break;
+        case 1: with_args<1>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_units_kernel<U, PACK, 1, RUN1, STREAM, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+        case 2: with_args<2>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_units_kernel<U, PACK, 2, RUN1, STREAM, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+        case 3: with_args<3>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_units_kernel<U, PACK, 3, RUN1, STREAM, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+        default: MHIP_LAUNCH((slice_units_kernel<U, PACK, -1, RUN1, STREAM, PackArgs>), grid, block, 0, stream, a); break;
     }
 }
 
@@ -818,13 +859,13 @@ static void launch_slice_copy_u(bool wide, CopyForm form, int ndim, dim3 grid, h
     if (form == kUnpackLines) {
         if constexpr (!PACK) {
             if (wide) {
-                MHIP_LAUNCH((slice_unpack_lines_kernel<U, true, -1>), grid, block, 0, stream, a);
+                MHIP_LAUNCH((slice_unpack_lines_kernel<U, true, -1, PackArgs>), grid, block, 0, stream, a);
                 return;
             }
             switch (ndim) {
-                case 1: MHIP_LAUNCH((slice_unpack_lines_kernel<U, false, 1>), grid, block, 0, stream, a); break;
-                case 2: MHIP_LAUNCH((slice_unpack_lines_kernel<U, false, 2>), grid, block, 0, stream, a); break;
-                default: MHIP_LAUNCH((slice_unpack_lines_kernel<U, false, -1>), grid, block, 0, stream, a); break;
+                case 1: with_args<1>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_unpack_lines_kernel<U, false, 1, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+                case 2: with_args<2>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_unpack_lines_kernel<U, false, 2, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+                default: MHIP_LAUNCH((slice_unpack_lines_kernel<U, false, -1, PackArgs>), grid, block, 0, stream, a); break;
             }
         }
         return;
@@ -847,13 +888,13 @@ static void launch_slice_copy_u(bool wide, CopyForm form, int ndim, dim3 grid, h
         }
         if (form == kRaggedRows) {
             if (wide) {
-                MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, true, -1>), grid, block, 0, stream, a);
+                MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, true, -1, PackArgs>), grid, block, 0, stream, a);
                 return;
             }
             switch (ndim) {
-                case 1: MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, false, 1>), grid, block, 0, stream, a); break;
-                case 2: MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, false, 2>), grid, block, 0, stream, a); break;
-                default: MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, false, -1>), grid, block, 0, stream, a); break;
+                case 1: with_args<1>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, false, 1, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+                case 2: with_args<2>(a, U, [&](const auto& args) { MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, false, 2, std::decay_t<decltype(args)>>), grid, block, 0, stream, args); }); break;
+                default: MHIP_LAUNCH((slice_copy_ragged_kernel<U, PACK, false, -1, PackArgs>), grid, block, 0, stream, a); break;
             }
             return;
         }

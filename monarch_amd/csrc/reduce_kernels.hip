@@ -14,16 +14,35 @@ namespace mhip {
 constexpr int kMaxInputs = 64;
 constexpr int kMaxOutputs = 16;
 
-struct ReduceArgs {
+template <int N>
+struct ReduceArgsOf {
     void* out;
-    const void* in[kMaxInputs];
+    const void* in[N];
     uint64_t numel;
     uint32_t n;
     float scale;   // 1/n when n is a power of two and op is Avg (exact), else 0
     float divisor; // n as a float
     uint32_t xcd_contiguous;  // kMap*: which chunk a workgroup takes, see inputs_alias()
     uint32_t op;              // MHIP_OP_*, read by the kGeneric kernels only
+    uint32_t grid;            // workgroups
 };
+using ReduceArgs = ReduceArgsOf<kMaxInputs>;
+
+// The same for a kernel of N inputs: a launch of 64 pointers costs more than one of N (see SmallDims).
+template <int N>
+static ReduceArgsOf<N> first_inputs(const ReduceArgs& a) {
+    ReduceArgsOf<N> b;
+    b.out = a.out;
+    for (int r = 0; r < N; ++r) b.in[r] = a.in[r];
+    b.numel = a.numel;
+    b.n = a.n;
+    b.scale = a.scale;
+    b.divisor = a.divisor;
+    b.xcd_contiguous = a.xcd_contiguous;
+    b.op = a.op;
+    b.grid = a.grid;
+    return b;
+}
 
 // How a kernel combines: Sum and Avg (the hot ops) are compiled as plain adds; Prod / Max / Min share one
 // instantiation per type that switches on the (wave-uniform) op in the arguments.
@@ -234,24 +253,24 @@ static bool inputs_alias(const void* const* in, uint32_t n) {
 
 enum : uint32_t { kMapPlain = 0, kMapEighths = 1, kMapRotated = 2 };
 
-__device__ __forceinline__ uint32_t xcd_rotated_block() {
-    if (blockIdx.x >= (gridDim.x & ~7u)) return blockIdx.x;  // the last, partial group of 8 keeps its order
+__device__ __forceinline__ uint32_t xcd_rotated_block(uint32_t grid) {
+    if (blockIdx.x >= (grid & ~7u)) return blockIdx.x;  // the last, partial group of 8 keeps its order
     return (blockIdx.x & ~7u) | ((blockIdx.x + (blockIdx.x >> 3)) & 7u);
 }
 
-__device__ __forceinline__ uint32_t xcd_contiguous_block() {
-    const uint32_t per = gridDim.x / 8;  // blocks past the last whole group of 8 keep their index
+__device__ __forceinline__ uint32_t xcd_contiguous_block(uint32_t grid) {
+    const uint32_t per = grid / 8;  // blocks past the last whole group of 8 keep their index
     return blockIdx.x < per * 8 ? (blockIdx.x & 7u) * per + (blockIdx.x >> 3) : blockIdx.x;
 }
 
 template <typename T, int N, int MODE>
-__global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceArgs a) {
+__global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceArgsOf<(N > 0 ? N : kMaxInputs)> a) {
     using VT = Vec<T>;
     using acc_t = typename VT::acc_t;
     constexpr int V = VT::V;
     const uint64_t nvec = a.numel / V;
-    const uint64_t stride = (uint64_t)gridDim.x * kReduceThreads;
-    const uint32_t bid = a.xcd_contiguous == kMapRotated ? xcd_rotated_block() : a.xcd_contiguous ? xcd_contiguous_block() : blockIdx.x;
+    const uint64_t stride = (uint64_t)a.grid * kReduceThreads;
+    const uint32_t bid = a.xcd_contiguous == kMapRotated ? xcd_rotated_block(a.grid) : a.xcd_contiguous ? xcd_contiguous_block(a.grid) : blockIdx.x;
     for (uint64_t v = (uint64_t)bid * kReduceThreads + threadIdx.x; v < nvec; v += stride) {
         acc_t acc[V];
         if constexpr (N > 0) {
@@ -317,6 +336,7 @@ struct ScatterArgs {
     float divisor;
     uint32_t xcd_contiguous;           // see inputs_alias()
     uint32_t op;                       // MHIP_OP_*, read by the kGeneric kernels only
+    uint32_t grid;                     // workgroups
     DimsArg out_dims;                  // packed output index -> reduced-tensor index
     DimsArg in_dims;                   // reduced-tensor index -> input memory
 };
@@ -335,10 +355,10 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_scatter_kernel(ScatterA
     // (Rotating k by the tile number, so that an output is not pinned to one XCD, was
     // measured and does not help: -6% on flat chunks, +0.5% on column blocks.)
     const uint32_t nk = a.n_out;
-    const uint32_t bid = a.xcd_contiguous ? xcd_contiguous_block() : blockIdx.x;
+    const uint32_t bid = a.xcd_contiguous ? xcd_contiguous_block(a.grid) : blockIdx.x;
     const uint64_t tile0 = bid / nk;
     const uint32_t k = bid % nk;
-    const uint64_t stride = (uint64_t)(gridDim.x / nk) * kReduceThreads;
+    const uint64_t stride = (uint64_t)(a.grid / nk) * kReduceThreads;
     for (uint64_t t = tile0 * kReduceThreads + threadIdx.x; t < a.total; t += stride) {
         uint64_t col;
         const uint64_t i = a.out_offset[k] + decode<WIDE, D>(a.out_dims, t, &col);
@@ -389,11 +409,11 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_scatter_ragged_kernel(S
     constexpr int V = VT::V;
     constexpr int ES = 16 / V;
     const uint32_t nk = a.n_out;
-    const uint32_t bid = a.xcd_contiguous ? xcd_contiguous_block() : blockIdx.x;
+    const uint32_t bid = a.xcd_contiguous ? xcd_contiguous_block(a.grid) : blockIdx.x;
     const uint64_t tile0 = bid / nk;
     const uint32_t k = bid % nk;
     const uint64_t nchunks = (a.total + V - 1) / V;
-    const uint64_t stride = (uint64_t)(gridDim.x / nk) * kReduceThreads;
+    const uint64_t stride = (uint64_t)(a.grid / nk) * kReduceThreads;
     char* __restrict__ out = static_cast<char*>(a.outs[k]);
 
     auto one_element = [&](uint64_t t) {  // output element t of output k, all inputs, element loads
@@ -538,20 +558,21 @@ static void avg_factors(uint32_t n, int op, float* scale, float* divisor) {
 }
 
 template <typename T, int MODE>
-static void launch_reduce_n(const ReduceArgs& a, hipStream_t s) {
-    const dim3 grid(grid_for(a.numel / Vec<T>::V)), block(kReduceThreads);
+static void launch_reduce_n(ReduceArgs a, hipStream_t s) {
+    a.grid = grid_for(a.numel / Vec<T>::V);
+    const dim3 grid(a.grid), block(kReduceThreads);
     if constexpr (MODE == kGeneric) {
         MHIP_LAUNCH((reduce_kernel<T, 0, MODE>), grid, block, 0, s, a);
     } else {
         switch (a.n) {
-            case 1: MHIP_LAUNCH((reduce_kernel<T, 1, MODE>), grid, block, 0, s, a); break;
-            case 2: MHIP_LAUNCH((reduce_kernel<T, 2, MODE>), grid, block, 0, s, a); break;
-            case 3: MHIP_LAUNCH((reduce_kernel<T, 3, MODE>), grid, block, 0, s, a); break;
-            case 4: MHIP_LAUNCH((reduce_kernel<T, 4, MODE>), grid, block, 0, s, a); break;
-            case 5: MHIP_LAUNCH((reduce_kernel<T, 5, MODE>), grid, block, 0, s, a); break;
-            case 6: MHIP_LAUNCH((reduce_kernel<T, 6, MODE>), grid, block, 0, s, a); break;
-            case 7: MHIP_LAUNCH((reduce_kernel<T, 7, MODE>), grid, block, 0, s, a); break;
-            case 8: MHIP_LAUNCH((reduce_kernel<T, 8, MODE>), grid, block, 0, s, a); break;
+            case 1: MHIP_LAUNCH((reduce_kernel<T, 1, MODE>), grid, block, 0, s, first_inputs<1>(a)); break;
+            case 2: MHIP_LAUNCH((reduce_kernel<T, 2, MODE>), grid, block, 0, s, first_inputs<2>(a)); break;
+            case 3: MHIP_LAUNCH((reduce_kernel<T, 3, MODE>), grid, block, 0, s, first_inputs<3>(a)); break;
+            case 4: MHIP_LAUNCH((reduce_kernel<T, 4, MODE>), grid, block, 0, s, first_inputs<4>(a)); break;
+            case 5: MHIP_LAUNCH((reduce_kernel<T, 5, MODE>), grid, block, 0, s, first_inputs<5>(a)); break;
+            case 6: MHIP_LAUNCH((reduce_kernel<T, 6, MODE>), grid, block, 0, s, first_inputs<6>(a)); break;
+            case 7: MHIP_LAUNCH((reduce_kernel<T, 7, MODE>), grid, block, 0, s, first_inputs<7>(a)); break;
+            case 8: MHIP_LAUNCH((reduce_kernel<T, 8, MODE>), grid, block, 0, s, first_inputs<8>(a)); break;
             default: MHIP_LAUNCH((reduce_kernel<T, 0, MODE>), grid, block, 0, s, a); break;
         }
     }
@@ -766,6 +787,7 @@ int mhip_reduce_scatter(void* const* outs, const mhip_slice_t* out_views, uint32
         uint64_t tiles = grid_for(ragged ? (a.total + V - 1) / V : a.total);
         while (tiles > 1 && tiles * nbatch > max_workgroups(kReduceThreads)) tiles = (tiles + 1) / 2;  // grid-stride takes over
         dim3 grid((uint32_t)(tiles * nbatch));
+        a.grid = grid.x;
         a.op = (uint32_t)op;
         switch (dtype) {
             case MHIP_DTYPE_F32: launch_scatter<float>(a, grid, vec, ragged, op, wide, d, hs); break;

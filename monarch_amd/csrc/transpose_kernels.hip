@@ -45,6 +45,7 @@ struct TransArgs {
     uint32_t outer_size[kMaxCanonDims];
     FastDiv32 outer_div[kMaxCanonDims];
     uint64_t outer_stride[kMaxCanonDims];
+    uint32_t grid;            // workgroups, slice_transpose_kernel
     uint32_t one_inner;       // consecutive q lie mem_pitch elements apart: one dimension after c
     uint32_t mem_pitch;
     // the walk (walk_tile): tiles per batch, tiles per block, c-groups, tiles along a block's side, tiles along q and along c
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(kThreads) void slice_transpose_kernel(TransArgs a) 
     T* __restrict__ packed = reinterpret_cast<T*>(a.packed);
     const uint64_t per_batch = (uint64_t)a.cgroups * ((a.qtiles + a.group - 1) / a.group) * a.group * a.group;
 
-    for (uint64_t tile_id = blockIdx.x; tile_id < a.ntiles; tile_id += gridDim.x) {
+    for (uint64_t tile_id = blockIdx.x; tile_id < a.ntiles; tile_id += a.grid) {
         const uint64_t b = tile_id / per_batch;
         const uint32_t in_batch = (uint32_t)(tile_id - b * per_batch);
         const uint32_t gsz = a.group * a.group;
@@ -983,8 +984,8 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     }
     if (unit != 16) return false;
     const uint64_t cap = max_workgroups(kThreads);  // grid-stride kernel
-    MHIP_LAUNCH((slice_transpose_kernel<uint4, 32, PACK>), dim3((uint32_t)(a.ntiles < cap ? a.ntiles : cap)), dim3(kThreads), 0,
-                       stream, a);
+    a.grid = (uint32_t)(a.ntiles < cap ? a.ntiles : cap);
+    MHIP_LAUNCH((slice_transpose_kernel<uint4, 32, PACK>), dim3(a.grid), dim3(kThreads), 0, stream, a);
     *rc = launch_status();
     return true;
 }

@@ -885,6 +885,33 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
         assert torch.equal(back.cpu(), ref), (shape, dtype)
 
 
+@pytest.mark.parametrize("nviews", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("row,step", [(1, 2), (3, 1), (64, 1), (65, 1), (200, 3), (1024, 1)])
+def test_views_of_one_to_four_dimensions_alone_and_two_in_a_launch(row, step, dtype, nviews):
+    # a launch for one view passes its arguments in another form than one for several, for each number of dimensions
+    g = torch.Generator(device=DEV).manual_seed(row)
+    width = 2 * row * step + 3 * step  # a Slice's strides are multiples of the next one
+    x = torch.randint(0, 100, (5, 3, 7, width), device=DEV, generator=g).to(dtype)
+    for dims in (1, 2, 3, 4):
+        y = x if dims == 4 else x[0] if dims == 3 else x[0, :, 0] if dims == 2 else x[0, 0, 0]
+        part = (lambda t: t[::2, ..., :row * step:step], lambda t: t[1::2, ..., row * step:2 * row * step:step])[:nviews]
+        if dims == 1:
+            part = (lambda t: t[:row * step:step], lambda t: t[row * step:2 * row * step:step])[:nviews]
+        views = [Slice.of_tensor(p(y)) for p in part]
+        bufs = staging.pack_many(y, views)
+        sync()
+        for p, b in zip(part, bufs):
+            assert torch.equal(b, p(y).contiguous().flatten()), dims
+        back, want = torch.full_like(x, 7), torch.full_like(x, 7)
+        sub, ref = (t if dims == 4 else t[0] if dims == 3 else t[0, :, 0] if dims == 2 else t[0, 0, 0] for t in (back, want))
+        staging.unpack_many(sub, views, bufs)
+        for p in part:
+            p(ref).copy_(p(y))
+        sync()
+        assert torch.equal(back, want), dims
+
+
 @pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
 @pytest.mark.parametrize("tiles", [399, 400, 512, 513])
 def test_transposes_with_a_short_side_in_tiles_that_are_resident_at_once(dtype, tiles):
