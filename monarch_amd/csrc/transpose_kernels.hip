@@ -719,7 +719,7 @@ static void launch_tiles(const TransForm& f, dim3 grid, hipStream_t stream, cons
     if (f.lines) {
         switch (f.unit) {
             case 1: MHIP_LAUNCH((slice_transpose_lines_kernel<uint8_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
-            case 2: MHIP_LAUNCH((slice_transpose_lines_kernel<uint16_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
+            case 2: MHIP_LAUNCH((slice_transpose_lines_kernel<uint16_t, 1024, PACK, ONE>), grid, dim3(1024), 0, stream, a); break;
             case 4: MHIP_LAUNCH((slice_transpose_lines_kernel<uint32_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
             default: MHIP_LAUNCH((slice_transpose_lines_kernel<uint64_t, 256, PACK, ONE>), grid, dim3(256), 0, stream, a); break;
         }
@@ -918,8 +918,13 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // never lower than 8 on the shapes of the walk table.
     a.group = big ? (unit == 2 ? 4 : 8) : (unit == 4 || unit == 8) ? 16 : unit == 2 ? 8 : 4;
     // the kernel with line-aligned windows re-reads rows of the tile before it along the written rows, and finds them
-    // in L2 sooner with smaller blocks: 4-byte elements 8200^2 0.66 / 0.65 -> 0.68 / 0.67, 8-byte 0.67 -> 0.69
-    if (lines && unit >= 4) a.group = 4;
+    // in L2 sooner with smaller blocks: 4-byte elements 8200^2 0.66 / 0.65 -> 0.68 / 0.67, 8-byte 0.67 -> 0.69.  2-byte elements in
+    // blocks of 2 (and 1024 lanes, half the passes per lane) against 8 (and 512), random sides from 1500 to 16000, pack /
+    // unpack, over buffers that no cache holds: 20 to 40 MiB 0.916 / 0.896 of the time, 40 to 80 MiB 0.96 / 0.935, 80 to 160 MiB
+    // 0.99 / 0.97, single shapes 0.78 to 1.09 (5000 x 7000 32.3 / 32.7 -> 31.7 / 31.7 us); blocks of 4 are up to 2 % behind, 1024
+    // lanes alone gain 1 %.  With fewer than 8 tiles along a side such blocks leave XCDs with whole rows of padding: 300 x
+    // 50001 17.5 / 18.5 us in blocks of 8, 20.9 / 22.1 in blocks of 2.
+    if (lines) a.group = unit != 2 ? 4 : a.ctiles >= 8 && a.qtiles >= 8 ? 2 : 8;
     // Where few tiles lie along one side, whole blocks are mostly padding, workgroups that are launched and retired without a
     // tile: blocks are halved while those are more than 0.7 of the tiles (fp32 [65536, 256], 4 tiles by 1024, blocks of
     // 16 / 4: 32.3 / 21.5 us, f64 [65536, 128] 37.5 / 21.4).  Less padding costs less than smaller blocks do (fp32 [144, 116508],
@@ -973,7 +978,7 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
         a.qtiles_div = FastDiv32(a.qtiles);
         a.ctiles_div = FastDiv32(a.ctiles);
         const uint64_t nblocks = 8 * ((a.ntiles + 7) / 8);  // one tile per workgroup, eight XCD ranges
-        const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big ? 1024 : 512;
+        const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big || (lines && unit == 2) ? 1024 : 512;
         *rc = launch_in_pieces(nblocks, lanes, 8, [&](uint64_t wg0, uint32_t count) {
             a.wg0 = wg0;
             const TransForm form{unit, lines, big, stream_loads, lanes};

@@ -885,6 +885,21 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
         assert torch.equal(back.cpu(), ref), (shape, dtype)
 
 
+@pytest.mark.parametrize("shape", [(895, 7403), (897, 7403), (1021, 6603), (1027, 6603), (3, 1000, 2201)])
+def test_transposes_of_two_byte_elements_with_few_tiles_along_a_side(shape):
+    # rows that are not whole lines, on both sides of the eight tiles of 128 elements at which the order of the tiles changes
+    g = torch.Generator(device=DEV).manual_seed(shape[-1])
+    for turned in (False, True):
+        x = torch.randint(-2**15, 2**15, shape[:-2] + shape[:-3:-1] if turned else shape, dtype=torch.int16, device=DEV, generator=g)
+        s = Slice.of_tensor(x.transpose(-1, -2))
+        out = staging.pack(x, s)
+        back = torch.zeros_like(x)
+        staging.unpack(back, s, out)
+        sync()
+        assert torch.equal(out, x.transpose(-1, -2).contiguous().flatten())
+        assert torch.equal(back, x)
+
+
 @pytest.mark.parametrize("nviews", [1, 2])
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("row,step", [(1, 2), (3, 1), (64, 1), (65, 1), (200, 3), (1024, 1)])
