@@ -730,7 +730,7 @@ static void launch_tiles(const TransForm& f, dim3 grid, hipStream_t stream, cons
             case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a); break;
             case 2:
                 if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
-                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a);
+                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 256, true>), grid, dim3(1024), 0, stream, a);
                 break;
             case 4:
                 if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
@@ -748,7 +748,7 @@ static void launch_tiles(const TransForm& f, dim3 grid, hipStream_t stream, cons
         case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
         case 2:
             if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
-            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a);
+            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE>), grid, dim3(1024), 0, stream, a);
             break;
         case 4:
             if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
@@ -924,7 +924,15 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // 0.99 / 0.97, single shapes 0.78 to 1.09 (5000 x 7000 32.3 / 32.7 -> 31.7 / 31.7 us); blocks of 4 are up to 2 % behind, 1024
     // lanes alone gain 1 %.  With fewer than 8 tiles along a side such blocks leave XCDs with whole rows of padding: 300 x
     // 50001 17.5 / 18.5 us in blocks of 8, 20.9 / 22.1 in blocks of 2.
-    if (lines) a.group = unit != 2 ? 4 : a.ctiles >= 8 && a.qtiles >= 8 ? 2 : 8;
+    const bool many_tiles = a.ctiles >= 8 && a.qtiles >= 8;
+    if (lines) a.group = unit != 2 ? 4 : many_tiles ? 2 : 8;
+    // Rows of whole lines: blocks of 2 for 2-byte elements (with 1024 lanes), and for 4- and 8-byte elements up to 80 MB, against
+    // 8 / 16 / 16 (and 512 lanes), random sides, pack and unpack, over buffers that no cache holds / that the Infinity Cache
+    // holds: 2 bytes 0.94 / 0.965 of the time, 4 bytes 0.955 / 0.94, 8 bytes 0.97 / 0.955, single shapes 0.80 to 1.06; 2-byte 7168 x 8192
+    // 51 -> 45 us, 4 x 4096^2 48 -> 46.5.  Above 80 MB 4- and 8-byte elements do better with 16 (f32 3520 x 11840 63 and 66.8 us, f64
+    // 4064 x 4416 51 and 65).  An odd number of blocks along a side of few tiles leaves every other workgroup of the last
+    // block without a tile: 3, 5 and 7 tiles lose 5 to 15 %.
+    if (!lines && !big && many_tiles && (unit == 2 || ((unit == 4 || unit == 8) && nbatch * Sc * Q * unit <= 80000000))) a.group = 2;
     // Where few tiles lie along one side, whole blocks are mostly padding, workgroups that are launched and retired without a
     // tile: blocks are halved while those are more than 0.7 of the tiles (fp32 [65536, 256], 4 tiles by 1024, blocks of
     // 16 / 4: 32.3 / 21.5 us, f64 [65536, 128] 37.5 / 21.4).  Less padding costs less than smaller blocks do (fp32 [144, 116508],
@@ -978,7 +986,7 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
         a.qtiles_div = FastDiv32(a.qtiles);
         a.ctiles_div = FastDiv32(a.ctiles);
         const uint64_t nblocks = 8 * ((a.ntiles + 7) / 8);  // one tile per workgroup, eight XCD ranges
-        const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big || (lines && unit == 2) ? 1024 : 512;
+        const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big || unit == 2 ? 1024 : 512;
         *rc = launch_in_pieces(nblocks, lanes, 8, [&](uint64_t wg0, uint32_t count) {
             a.wg0 = wg0;
             const TransForm form{unit, lines, big, stream_loads, lanes};

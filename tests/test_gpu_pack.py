@@ -900,6 +900,24 @@ def test_transposes_of_two_byte_elements_with_few_tiles_along_a_side(shape):
         assert torch.equal(back, x)
 
 
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int32, torch.int64])
+@pytest.mark.parametrize("tiles,mbytes", [(7, 13), (8, 13), (9, 13), (8, 80), (8, 81)])
+def test_transposes_of_whole_lines_on_both_sides_of_the_block_rule(dtype, tiles, mbytes):
+    # blocks of two tiles from eight tiles of 256 bytes along both sides and, for 4- and 8-byte elements, up to 80 MB
+    es = torch.empty(0, dtype=dtype).element_size()
+    n, lines = tiles * 256 // es, 128 // es
+    m = mbytes * 1000000 // es // n // lines * lines
+    x = torch.randint(-100, 100, (m, n), dtype=dtype, device=DEV, generator=torch.Generator(device=DEV).manual_seed(tiles))
+    for y in (x, x.view(n, m)):
+        s = Slice.of_tensor(y.t())
+        out = staging.pack(y, s)
+        back = torch.zeros_like(y)
+        staging.unpack(back, s, out)
+        sync()
+        assert torch.equal(out, y.t().contiguous().flatten())
+        assert torch.equal(back, y)
+
+
 @pytest.mark.parametrize("nviews", [1, 2])
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("row,step", [(1, 2), (3, 1), (64, 1), (65, 1), (200, 3), (1024, 1)])
