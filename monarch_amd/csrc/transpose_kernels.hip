@@ -913,7 +913,7 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // Tiles are walked in group x group blocks, and a block is about what one XCD runs at a time
     // (8 workgroups per CU of 4-byte tiles, 4 of 2-byte tiles), so that the eight XCDs each stream
     // runs of group * 256 bytes on both sides.  Measured at 8192^2 fp32 pack: group 1 0.47, 4 0.52,
-    // 16 0.65 of peak; 2-byte elements do best at 8.
+    // 16 0.65 of peak; 2-byte elements do best at 8 of 4 to 16 (blocks of 2, further down, win where they are taken).
     // 1-byte elements (256 x 256 tiles, two workgroups per CU) do best at 4: 8200^2 0.40 -> 0.47, 5000 x 7000 0.51 -> 0.57,
     // never lower than 8 on the shapes of the walk table.
     a.group = big ? (unit == 2 ? 4 : 8) : (unit == 4 || unit == 8) ? 16 : unit == 2 ? 8 : 4;
