@@ -23,7 +23,7 @@
 
 namespace {
 
-constexpr long kNotTaken = -1;
+constexpr long kNotTaken = LONG_MIN;  // no status (a C int), no negated one and no count
 constexpr Py_ssize_t kMaxItems = 64;  // tensors or views of one call; longer lists are left to the general path
 
 PyTypeObject* g_slice_type = nullptr;  // monarch_amd.ndslice.Slice

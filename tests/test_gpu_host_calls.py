@@ -3,7 +3,7 @@ for every call that one of them refuses.  A tensor subclass takes the general pa
 import pytest
 import torch
 
-from monarch_amd import Slice, fp8, staging
+from monarch_amd import MhipError, Slice, fp8, staging
 from monarch_amd import reduce as R
 from monarch_amd._native import host
 from monarch_amd.staging import RDMABuffer
@@ -46,6 +46,22 @@ def test_calls_that_are_not_on_plain_tensors_are_left_alone():
     assert host.tensor_addresses([x], (4).to_bytes(8, "little"), x) is None
     with pytest.raises(TypeError):
         host.slice_copy(True)
+
+
+@pytest.mark.parametrize("status", [1, 2, 719, 10201])
+def test_transfers_that_fail_are_not_posted_again(monkeypatch, status):
+    # minus a status (a C int) is none of a count, a status and the mark of a call that was left alone
+    assert host.NOT_TAKEN < -(1 << 31)
+
+    class Failing:
+        NOT_TAKEN = host.NOT_TAKEN
+        transfer_many = staticmethod(lambda *args: -status)
+
+    monkeypatch.setattr(staging, "host", Failing)
+    monkeypatch.setattr(staging, "lib", lambda: pytest.fail("posted a second time"))
+    with pytest.raises(MhipError) as e:
+        staging.transfer_many([16], [32], [8])
+    assert e.value.status == status
 
 
 def _filled(n, dtype=torch.float32, seed=0):
