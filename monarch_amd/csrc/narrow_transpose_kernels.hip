@@ -235,6 +235,9 @@ void slice_transpose_narrow_kernel(std::conditional_t<ONE, NarrowOneArgs, Narrow
     }
 }
 
+// Returned instead of a status for a view of too many tiles: the caller leaves the view to another kernel.
+constexpr int kTooManyTiles = -1;
+
 // WB and RB: bytes of a written and of a read row of the tile
 template <typename T, bool PACK, int WB, int RB, bool LATE = false>
 static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
@@ -247,8 +250,11 @@ static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     a.nv_div = FastDiv32(nv);
     a.row_step = kLanes / nv;
     a.vec_step = kLanes % nv;
-    // fewer than kFastDivLimit: a tile moves 256 bytes at least, and no GPU holds 2^31 times that (see try_narrow_transpose)
-    a.ntiles = (uint32_t)(nbatch * ti_count * tj_count);
+    // The kernel's tile numbers, up to 7 past the last one, are dividends of FastDiv32.  A tile holds 128 bytes at least (8 x 8
+    // elements of 2 bytes), so a view of 256 GiB can have more of them.
+    const uint64_t ntiles = nbatch * ti_count * tj_count;
+    if (ntiles >= kFastDivLimit - 8) return kTooManyTiles;
+    a.ntiles = (uint32_t)ntiles;
     a.per_xcd = (a.ntiles + 7) / 8;
     a.per_batch_div = FastDiv32(ti_count * tj_count);
     a.i_fast = ti_count < tj_count;
@@ -362,7 +368,6 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
     const uint64_t Sc = c.dims[cd].size, bytes = nbatch * Sc * Q * unit;
     const uint64_t short_side = (Sc < Q ? Sc : Q) * unit;
     if (unit > 8 || short_side < 16) return false;
-    if (bytes / 256 >= kFastDivLimit) return false;  // every tile holds at least 16 x 16 bytes: tile numbers stay below 2^31
     if (short_side > 512 && bytes > (unit == 1 ? 40ull << 20 : 12ull << 20)) return false;
     NarrowArgs a{};
     uint64_t written = PACK ? (uint64_t)(uintptr_t)packed | (uint64_t)Q * unit : (uint64_t)(uintptr_t)(base + c.offset * unit);
@@ -399,7 +404,7 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
         case 4: *rc = launch_narrow_tile<uint32_t, PACK>(a, nbatch, stream); break;
         default: *rc = launch_narrow_tile<uint64_t, PACK>(a, nbatch, stream); break;
     }
-    return true;
+    return *rc != kTooManyTiles;
 }
 
 template bool try_narrow_transpose<true>(char*, char*, const CanonSlice&, int, uint64_t, uint32_t, uint32_t, hipStream_t, int*);

@@ -977,7 +977,7 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     if (vec) choose_walk(&a, unit, nbatch);
     a.ntiles = a.walk == kWalkBlocked ? nbatch * a.cgroups * a.qgroups * a.group * a.group : nbatch * (uint64_t)a.qtiles * a.ctiles;
     if (vec) {
-        // tile numbers fit the 32-bit divisions of walk_tile: 2^31 tiles of 16 KiB and more would be 32 TiB
+        // tile numbers fit the 32-bit divisions of walk_tile: 2^31 tiles of 8 KiB (8-byte elements) and more would be 16 TiB
         if (a.ntiles >= kFastDivLimit - 8) return false;
         a.per_batch_div = FastDiv32(a.walk == kWalkBlocked ? a.cgroups * a.qgroups * a.group * a.group : a.qtiles * a.ctiles);
         a.block_div = FastDiv32(a.group * a.group);

@@ -1,0 +1,47 @@
+"""Which kernels a copy launches, without a GPU: tests/c_abi/launches.c links the library and takes the place of
+``hipLaunchKernel``, so that sizes no GPU holds can be asked for."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIMIT = (1 << 31) - 1  # dividends of the kernels' divisions by multiplication stay below this
+
+
+@pytest.fixture(scope="module")
+def launches(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("launches") / "launches")
+    lib = os.path.join(ROOT, "monarch_amd")
+    subprocess.check_call(["gcc", "-std=gnu11", "-O1", "-Wall", "-Wextra", "-Werror", "-rdynamic", "-I", os.path.join(ROOT, "include"),
+                           os.path.join(ROOT, "tests", "c_abi", "launches.c"), "-o", exe, "-L", lib, "-lmonarch_hip", "-Wl,-rpath," + lib, "-ldl"])
+
+    def run(pack, size, sizes, strides):
+        line = " ".join(str(x) for x in (int(pack), size, 0, len(sizes), *sizes, *strides))
+        out = subprocess.run([exe], input=line + "\n", capture_output=True, text=True, check=True, timeout=60).stdout.split()
+        assert out[0] == "0", out
+        return [(int(out[k]), out[k + 1]) for k in range(1, len(out), 2)]
+    return run
+
+
+@pytest.mark.parametrize("pack", [True, False])
+@pytest.mark.parametrize("size,a,b", [(2, 8, 8), (2, 8, 9), (2, 9, 8), (1, 16, 16), (1, 16, 17), (4, 8, 8), (4, 4 * 33, 8), (8, 8, 17), (2, 65, 8), (2, 8, 65),
+                                      (2, 520, 8)])
+def test_tile_numbers_of_small_matrices_fit_their_divisions(launches, pack, size, a, b):
+    # [n1, n2, a, b] -> [n1, n2, b, a] with a gap after every n2 matrices, up to 2^32 tiles and more: the transposing kernel of small
+    # matrices is launched with fewer workgroups than its divisions take, whatever its tile; beyond that another kernel is
+    def narrow(n):
+        n1 = 1 << 12
+        n2 = -(-n // n1)
+        got = launches(pack, size, [n1, n2, b, a], [(n2 + 1) * a * b, a * b, 1, b])
+        assert got
+        return n1 * n2, sum(wg for wg, name in got if "slice_transpose_narrow_kernel" in name)
+
+    n, wgs = narrow(1 << 24)
+    per_matrix = round(wgs / n)
+    assert per_matrix >= 1 and wgs >= n * per_matrix
+    n, wgs = narrow((LIMIT - (1 << 20)) // per_matrix)
+    assert n * per_matrix <= wgs < LIMIT
+    for tiles in (LIMIT - 7, LIMIT + 2, 3 << 30, (1 << 32) - (1 << 13), 1 << 32, (1 << 32) + 100, 3 << 32):
+        n, wgs = narrow(-(-tiles // per_matrix))
+        assert n * per_matrix >= LIMIT - 8 and wgs == 0, tiles
