@@ -21,6 +21,6 @@ except ImportError as e:
 
     class _NotBuilt:
         def __getattr__(self, name):
-            raise MonarchHipNotBuilt(f"the native host path is missing ({_reason}): build it with `make -C monarch_amd/csrc`")
+            raise MonarchHipNotBuilt(f"the native host path is missing ({_reason}): build it with `python -m monarch_amd.build`")
 
     host = _NotBuilt()

@@ -1,4 +1,5 @@
-"""Builds ``libmonarch_hip.so`` in-tree with hipcc for gfx950 (cross-compiles without a GPU)."""
+"""Builds ``libmonarch_hip.so`` in-tree with hipcc for gfx950 (cross-compiles without a GPU) and, for the running interpreter
+and its PyTorch, the native host path beside it."""
 from __future__ import annotations
 
 import os
@@ -9,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 def build(force: bool = True, jobs: int = 8) -> str:
-    cmd = ["make", "-C", os.path.join(HERE, "csrc"), f"-j{jobs}"]
+    cmd = ["make", "-C", os.path.join(HERE, "csrc"), f"-j{jobs}", "all", "python", f"PYTHON={sys.executable}"]
     if force:
         cmd.append("-B")
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
