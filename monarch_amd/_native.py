@@ -5,22 +5,29 @@ Every function of ``host`` returns the library's status, or ``NOT_TAKEN`` for a 
 that does not pass a check; the Python code behind it then runs as it would without it.
 
 The extension is loaded by the first call, not by an import, and ``lib()`` before it: the library reads its environment while it
-is loaded.  Without the extension that call raises ``MonarchHipNotBuilt``, as without the library.
+is loaded, and a missing library is an error.  The extension is linked to the ``libmonarch_hip.so`` beside it; where ``lib()`` is
+another one (``_lib.LIB_PATH``), every call is left alone and takes the ctypes path.
 """
 from __future__ import annotations
+
+import os
 
 import torch  # noqa: F401  (its libraries have to be in the process before the extension that uses them)
 
 from . import _lib
 from .ndslice import Slice
 
-_NAMES = ("slice_copy", "slice_copy_many", "rdma_copy", "transfer_many", "reduce", "stack", "reduce_scatter", "flat_copy", "quantize_bucket",
-          "dequant_accumulate_bucket", "tensor_addresses", "NOT_TAKEN")
+NOT_TAKEN = -(1 << 63)
+_CALLS = ("slice_copy", "slice_copy_many", "rdma_copy", "transfer_many", "reduce", "stack", "reduce_scatter", "flat_copy", "quantize_bucket",
+          "dequant_accumulate_bucket")
 
 
 def extension():
-    """The extension module."""
-    _lib.lib()
+    """The extension module, or None where calls have to take the ctypes path."""
+    beside = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmonarch_hip.so")
+    loaded = _lib.lib()._name
+    if not os.path.exists(beside) or not os.path.samefile(loaded, beside):
+        return None
     try:
         from . import _host_calls
     except ImportError as e:
@@ -33,11 +40,16 @@ class _Host:
     """The extension's functions, once one of them has been asked for."""
 
     def __getattr__(self, name):
-        if name not in _NAMES:
+        if name not in _CALLS and name not in ("tensor_addresses", "NOT_TAKEN"):
             raise AttributeError(name)
         ext = extension()
-        self.__dict__.update((n, getattr(ext, n)) for n in _NAMES)
-        return self.__dict__[name]
+        if ext is not None:
+            found = {n: getattr(ext, n) for n in (*_CALLS, "tensor_addresses", "NOT_TAKEN")}
+        else:
+            found = {n: lambda *args: NOT_TAKEN for n in _CALLS}
+            found.update(tensor_addresses=lambda *args: None, NOT_TAKEN=NOT_TAKEN)
+        self.__dict__.update(found)
+        return found[name]
 
 
 host = _Host()

@@ -1,8 +1,11 @@
-"""When the native host path and the library behind it are loaded.  Each case in a process of its own,
+"""When the native host path and the library behind it are loaded, and which library it is.  Each case in a process of its own,
 on the CPU: calls on CPU tensors end in the checks behind the native path."""
 import os
+import shutil
 import subprocess
 import sys
+
+from monarch_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 COMMON = f"""
@@ -42,4 +45,16 @@ s = Slice(offset=0, sizes=[8], strides=[1])
 _lib._lib, _lib.LIB_PATH = None, {str(tmp_path / "libmonarch_hip.so")!r}
 for call, args in ((staging.pack, (x, s, x)), (staging.unpack, (x, s, x)), (R.all_reduce, (x, [x], 0)), (staging.transfer_many, ([1], [1], [1]))):
     assert error(call, *args).startswith("MonarchHipNotBuilt"), call
+""")
+
+
+def test_calls_of_another_library_do_not_reach_the_one_beside_the_extension(tmp_path):
+    other = str(tmp_path / "libmonarch_hip.so")
+    shutil.copy(_lib.LIB_PATH, other)
+    run(f"""
+_lib.LIB_PATH = {other!r}
+s = Slice(offset=0, sizes=[8], strides=[1])
+assert error(staging.pack, x, s, x) == "MhipError InvalidDevice" and error(R.all_reduce, x, [x], 0) == "MhipError InvalidDevice"
+assert set(mapped("libmonarch_hip")) == {{{other!r}}} and not mapped("_host_calls")
+assert staging.host.slice_copy(True, x, s, x) == staging.host.NOT_TAKEN and staging.host.tensor_addresses([x], b"", x) is None
 """)
