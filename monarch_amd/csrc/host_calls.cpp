@@ -14,6 +14,7 @@
 
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <climits>
 #include <cstdint>
@@ -481,6 +482,9 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, g_met
 PyMODINIT_FUNC PyInit__host_calls() {
     g_addr_name = PyUnicode_InternFromString("_addr");
     PyObject* m = g_addr_name != nullptr ? PyModule_Create(&g_module) : nullptr;
-    if (m != nullptr) PyModule_AddIntConstant(m, "NOT_TAKEN", kNotTaken);
+    if (m != nullptr) {
+        PyModule_AddIntConstant(m, "NOT_TAKEN", kNotTaken);
+        PyModule_AddStringConstant(m, "TORCH_VERSION", TORCH_VERSION);  // whose layouts the checks read; monarch_amd/_native.py compares it
+    }
     return m;
 }

@@ -58,3 +58,16 @@ assert error(staging.pack, x, s, x) == "MhipError InvalidDevice" and error(R.all
 assert set(mapped("libmonarch_hip")) == {{{other!r}}} and not mapped("_host_calls")
 assert staging.host.slice_copy(True, x, s, x) == staging.host.NOT_TAKEN and staging.host.tensor_addresses([x], b"", x) is None
 """)
+
+
+def test_without_the_extension_calls_take_the_ctypes_path():
+    for state in ("sys.modules['monarch_amd._host_calls'] = None", "from monarch_amd import _host_calls; _host_calls.TORCH_VERSION = '1.2.3'"):
+        err = run(f"""
+{state}
+s = Slice(offset=0, sizes=[8], strides=[1])
+for _ in range(2):
+    for call, args in ((staging.pack, (x, s, x)), (staging.unpack, (x, s, x)), (R.all_reduce, (x, [x], 0)), (fp8.quantize, (x,))):
+        assert error(call, *args) == "MhipError InvalidDevice", call
+assert staging.host.slice_copy(True, x, s, x) == staging.host.NOT_TAKEN
+""")
+        assert err.count("no native host path") == 1
