@@ -730,7 +730,8 @@ static void launch_tiles(const TransForm& f, dim3 grid, hipStream_t stream, cons
             case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a); break;
             case 2:
                 if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
-                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 256, true>), grid, dim3(1024), 0, stream, a);
+                else if (f.lanes == 1024) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 256, true>), grid, dim3(1024), 0, stream, a);
+                else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, ONE, 256, true>), grid, dim3(512), 0, stream, a);
                 break;
             case 4:
                 if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, ONE, 512, true>), grid, dim3(1024), 0, stream, a);
@@ -748,7 +749,8 @@ static void launch_tiles(const TransForm& f, dim3 grid, hipStream_t stream, cons
         case 1: MHIP_LAUNCH((slice_transpose_vec_kernel<uint8_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a); break;
         case 2:
             if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
-            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE>), grid, dim3(1024), 0, stream, a);
+            else if (f.lanes == 1024) MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 1024, PACK, ONE>), grid, dim3(1024), 0, stream, a);
+            else MHIP_LAUNCH((slice_transpose_vec_kernel<uint16_t, 512, PACK, ONE>), grid, dim3(512), 0, stream, a);
             break;
         case 4:
             if (f.big) MHIP_LAUNCH((slice_transpose_vec_kernel<uint32_t, 1024, PACK, ONE, 512>), grid, dim3(1024), 0, stream, a);
@@ -931,7 +933,9 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
     // holds: 2 bytes 0.94 / 0.965 of the time, 4 bytes 0.955 / 0.94, 8 bytes 0.97 / 0.955, single shapes 0.80 to 1.06; 2-byte 7168 x 8192
     // 51 -> 45 us, 4 x 4096^2 48 -> 46.5.  Above 80 MB 4- and 8-byte elements do better with 16 (f32 3520 x 11840 63 and 66.8 us, f64
     // 4064 x 4416 51 and 65).  An odd number of blocks along a side of few tiles leaves every other workgroup of the last
-    // block without a tile: 3, 5 and 7 tiles lose 5 to 15 %.
+    // block without a tile: 3, 5 and 7 tiles lose 5 to 15 %.  Nor do 1024 lanes pay there for 2-byte elements: 3 to 7 tiles by 78 to
+    // 410, 92 calls, against 512 lanes 1.03 of the time between cached buffers (up to 1.14, 52480 x 640 24.5 / 21.7 us) and 0.96 beyond
+    // the caches.  (With windows 1024 lanes do better at any number of tiles: 0.975 and 0.98.)
     if (!lines && !big && many_tiles && (unit == 2 || ((unit == 4 || unit == 8) && nbatch * Sc * Q * unit <= 80000000))) a.group = 2;
     // Where few tiles lie along one side, whole blocks are mostly padding, workgroups that are launched and retired without a
     // tile: blocks are halved while those are more than 0.7 of the tiles (fp32 [65536, 256], 4 tiles by 1024, blocks of
@@ -986,7 +990,7 @@ bool try_transpose_copy(char* base, char* packed, const CanonSlice& c, uint32_t 
         a.qtiles_div = FastDiv32(a.qtiles);
         a.ctiles_div = FastDiv32(a.ctiles);
         const uint64_t nblocks = 8 * ((a.ntiles + 7) / 8);  // one tile per workgroup, eight XCD ranges
-        const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big || unit == 2 ? 1024 : 512;
+        const uint32_t lanes = unit == 8 ? (big ? big8_lanes : 256) : big || (unit == 2 && (lines || many_tiles)) ? 1024 : 512;
         *rc = launch_in_pieces(nblocks, lanes, 8, [&](uint64_t wg0, uint32_t count) {
             a.wg0 = wg0;
             const TransForm form{unit, lines, big, stream_loads, lanes};

@@ -45,3 +45,17 @@ def test_tile_numbers_of_small_matrices_fit_their_divisions(launches, pack, size
     for tiles in (LIMIT - 7, LIMIT + 2, 3 << 30, (1 << 32) - (1 << 13), 1 << 32, (1 << 32) + 100, 3 << 32):
         n, wgs = narrow(-(-tiles // per_matrix))
         assert n * per_matrix >= LIMIT - 8 and wgs == 0, tiles
+
+
+@pytest.mark.parametrize("pack", [True, False])
+def test_lanes_of_two_byte_transposes_follow_the_number_of_tiles(launches, pack):
+    # tiles of 128 x 128 elements whose written rows are whole lines: 1024 lanes from eight tiles along both sides on, else 512; rows
+    # that are not whole lines always 1024
+    def kernel(rows, cols):
+        got = launches(pack, 2, [cols, rows], [1, cols])
+        return got[0][1]
+
+    for tiles, lanes in ((5, 512), (7, 512), (8, 1024), (9, 1024)):
+        for rows, cols in ((tiles * 128, 20096), (20096, tiles * 128)):
+            assert f"slice_transpose_vec_kernelItLi{lanes}E" in kernel(rows, cols), (rows, cols)
+        assert "slice_transpose_lines_kernelItLi1024E" in (kernel(tiles * 128 - 20, 20096) if pack else kernel(20096, tiles * 128 - 20))
