@@ -238,8 +238,9 @@ void slice_transpose_narrow_kernel(std::conditional_t<ONE, NarrowOneArgs, Narrow
 // Returned instead of a status for a view of too many tiles: the caller leaves the view to another kernel.
 constexpr int kTooManyTiles = -1;
 
-// WB and RB: bytes of a written and of a read row of the tile
-template <typename T, bool PACK, int WB, int RB, bool LATE = false>
+// WB and RB: bytes of a written and of a read row of the tile; GENERAL: addresses by the general form for every view (see
+// launch_narrow_tile)
+template <typename T, bool PACK, int WB, int RB, bool LATE = false, bool GENERAL = false>
 static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     constexpr uint32_t ES = sizeof(T), E = 16 / ES, TI = WB / ES, TJ = RB / ES;
     constexpr int kBytes = TI * TJ * ES, kLanes = kBytes >= 32768 ? 512 : kBytes >= 8192 ? 256 : 128;
@@ -264,9 +265,14 @@ static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
     a.batch_stride = a.n_outer == 1 ? a.outer_stride[0] : 0;
     return launch_in_pieces((uint64_t)a.per_xcd * 8, kLanes, 8, [&](uint64_t wg0, uint32_t count) {
         a.wg0 = (uint32_t)wg0;
-        const NarrowOneArgs& small = a;
-        if (one) MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, true, LATE>), dim3(count), dim3(kLanes), 0, stream, small);
-        else MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, false, LATE>), dim3(count), dim3(kLanes), 0, stream, a);
+        if constexpr (!GENERAL) {
+            if (one) {
+                const NarrowOneArgs& small = a;
+                MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, true, LATE>), dim3(count), dim3(kLanes), 0, stream, small);
+                return;
+            }
+        }
+        MHIP_LAUNCH((slice_transpose_narrow_kernel<T, kLanes, PACK, TI, TJ, false, LATE>), dim3(count), dim3(kLanes), 0, stream, a);
     });
 }
 
@@ -317,7 +323,11 @@ static uint32_t narrow_tile_bytes(uint64_t bytes) {
 // 3.1 / 3.3 and 2.9 / 2.9, 640^2 3.1 / 3.2 and 3.3 / 3.1, 887^2 4.8 / 5.1 and 4.0 / 3.9, 1145^2 6.7 / 6.5 and 5.8 / 5.7, where the
 // tiles of transpose_kernels.hip take 6.0 / 6.0; [3584, 16, 16] 4.5 / 4.4 and 6.5 / 6.4).
 // Byte matrices of 12 to 23 MiB collect all columns of a tile before they store the first (LATE): warm 0.95 of the time it took
-// with 64-bit tile numbers where the other order takes 1.05, cold 0.98 and 1.11; up to 12 MiB 0.92 and 0.82.
+// with 64-bit tile numbers where the other order takes 1.05, cold 0.98 and 1.11; up to 12 MiB 0.92 and 0.82.  From 12 MiB on they
+// also keep the general form of addresses (GENERAL): its arithmetic spaces the stores, which in the short form leave in bursts
+// that some shapes pay for.  Against 64-bit tile numbers, random shapes, short form / general, warm and cold: 20 to 23 MiB mean
+// 0.977 / 0.954 and 0.989 / 0.953, slowest 1.007 / 0.999 and 1.052 / 0.997; 23 to 40 MiB 0.977 / 0.976 and 0.977 / 0.968, slowest
+// 1.139 / 1.042 and 1.087 / 0.998 ([1672, 15051] unpack 11.8 -> 13.4 us short, 12.1 general).
 // Batches of matrices that fit 128 x 128 bytes keep that tile at any size: u8 [78125, 16, 16] 94 / 95 us, in tiles of 1024 x 64 of
 // which one matrix fills little 335 / 333; bf16 [39062, 16, 16] 45 / 46 and 97 / 98, [8544, 64, 64] 23.2 / 23.3 and 30.2 / 31.3.
 template <typename T, bool PACK>
@@ -327,8 +337,8 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
     const uint64_t bytes = nbatch * ib * jb / ES;
     if constexpr (ES == 1)
         if (ib > 512 && jb > 512 && bytes > (12ull << 20)) {
-            if (bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256>(a, nbatch, stream);
-            return launch_narrow<T, PACK, 128, 128, true>(a, nbatch, stream);
+            if (bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256, false, true>(a, nbatch, stream);
+            return launch_narrow<T, PACK, 128, 128, true, true>(a, nbatch, stream);
         }
     if (bytes >= (16ull << 20) && (ib <= 512 || jb <= 512) && (ib > 128 || jb > 128)) {  // a long side to fill the tile with
         const bool short_j = jb <= ib;

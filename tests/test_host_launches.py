@@ -59,3 +59,18 @@ def test_lanes_of_two_byte_transposes_follow_the_number_of_tiles(launches, pack)
         for rows, cols in ((tiles * 128, 20096), (20096, tiles * 128)):
             assert f"slice_transpose_vec_kernelItLi{lanes}E" in kernel(rows, cols), (rows, cols)
         assert "slice_transpose_lines_kernelItLi1024E" in (kernel(tiles * 128 - 20, 20096) if pack else kernel(20096, tiles * 128 - 20))
+
+
+@pytest.mark.parametrize("pack", [True, False])
+def test_byte_matrices_of_12_to_40_mib_take_the_general_addresses(launches, pack):
+    # smaller ones the short form; it is the parameter before the last
+    def forms(rows, cols):
+        return {name.split("slice_transpose_narrow_kernelI")[1].split("EEEv")[0] for _, name in launches(pack, 1, [cols, rows], [1, cols])
+                if "slice_transpose_narrow_kernel" in name}
+
+    p = int(pack)
+    assert forms(3001, 4001) == {f"hLi256ELb{p}ELi128ELi128ELb1ELb0"}
+    assert forms(3301, 4001) == {f"hLi256ELb{p}ELi128ELi128ELb0ELb1"}
+    assert forms(1672, 15051) == {f"hLi512ELb{p}ELi256ELi256ELb0ELb0"}
+    assert forms(6301, 6501) == {f"hLi512ELb{p}ELi256ELi256ELb0ELb0"}
+    assert not forms(6501, 6501)
