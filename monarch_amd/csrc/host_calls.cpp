@@ -122,18 +122,20 @@ bool fits(const at::Tensor& base, const mhip_slice_t& s, const at::Tensor& buffe
     return buffer.device() == base.device() && bytes_of(buffer) == nbytes;
 }
 
-// Holds the objects of a list while the library runs without the interpreter's lock.
+// Holds objects of lists, tensors and Slices, while the library runs without the interpreter's lock: another thread may take
+// them out of the list meanwhile, and the library reads a Slice's memory and launches on a tensor's.  (The arguments themselves
+// are held by the caller.)
 class Held {
 public:
     ~Held() {
         for (Py_ssize_t i = 0; i < n_; ++i) Py_DECREF(at_[i]);
     }
-    void add(PyObject* o) {
+    PyObject* add(PyObject* o) {
         Py_INCREF(o);
-        at_[n_++] = o;
+        return at_[n_++] = o;
     }
 private:
-    PyObject* at_[2 * kMaxItems + 1];
+    PyObject* at_[3 * kMaxItems];  // a call has three lists at most
     Py_ssize_t n_ = 0;
 };
 
@@ -186,12 +188,11 @@ long slice_copy_many(PyObject* const* a) {
     void* ptrs[kMaxItems];
     Held held;
     for (Py_ssize_t i = 0; i < views.n; ++i) {
-        const mhip_slice_t* s = slice_of(views.at[i]);
-        const at::Tensor* buffer = plain_contiguous(buffers.at[i]);
+        const mhip_slice_t* s = slice_of(held.add(views.at[i]));
+        const at::Tensor* buffer = plain_contiguous(held.add(buffers.at[i]));
         if (s == nullptr || buffer == nullptr || !fits(*base, *s, *buffer)) return kNotTaken;
         slices[i] = *s;
         ptrs[i] = buffer->data_ptr();
-        held.add(views.at[i]);
     }
     void* mem = base->storage().mutable_data();
     const uint32_t n = (uint32_t)views.n, size = (uint32_t)base->itemsize();
@@ -239,10 +240,10 @@ long transfer_many(PyObject* const* a) {
 // ---- reductions ----
 
 // The members of a group: contiguous tensors of one type and size.
-bool members(const Items& group, c10::ScalarType type, int64_t numel, const void** ptrs) {
+bool members(const Items& group, c10::ScalarType type, int64_t numel, const void** ptrs, Held* held) {
     if (!group.few()) return false;
     for (Py_ssize_t i = 0; i < group.n; ++i) {
-        const at::Tensor* t = plain_contiguous(group.at[i]);
+        const at::Tensor* t = plain_contiguous(held->add(group.at[i]));
         if (t == nullptr || t->scalar_type() != type || t->numel() != numel) return false;
         ptrs[i] = t->data_ptr();
     }
@@ -255,9 +256,10 @@ long reduce(PyObject* const* a) {
     const Items group(a[1]);
     uint64_t op;
     const void* ptrs[kMaxItems];
+    Held held;
     if (out == nullptr || !to_u64(a[2], &op) || op > INT_MAX) return kNotTaken;
     const int code = reduce_code(*out);
-    if (code < 0 || !members(group, out->scalar_type(), out->numel(), ptrs)) return kNotTaken;
+    if (code < 0 || !members(group, out->scalar_type(), out->numel(), ptrs, &held)) return kNotTaken;
     void* dst = out->data_ptr();
     const uint64_t numel = (uint64_t)out->numel();
     const mhip_stream_t stream = current_stream();
@@ -269,9 +271,10 @@ long stack(PyObject* const* a) {
     const at::Tensor* out = plain_contiguous(a[0]);
     const Items group(a[1]);
     const void* ptrs[kMaxItems];
+    Held held;
     if (out == nullptr || !group.few() || out->numel() % group.n != 0) return kNotTaken;
     const int64_t numel = out->numel() / group.n;
-    if (!members(group, out->scalar_type(), numel, ptrs)) return kNotTaken;
+    if (!members(group, out->scalar_type(), numel, ptrs, &held)) return kNotTaken;
     void* dst = out->data_ptr();
     const uint32_t size = (uint32_t)out->itemsize();
     const mhip_stream_t stream = current_stream();
@@ -290,22 +293,20 @@ long reduce_scatter(PyObject* const* a) {
     Held held;
     int code = -1;
     for (Py_ssize_t i = 0; i < outs.n; ++i) {
-        const at::Tensor* t = plain_contiguous(outs.at[i]);
-        const mhip_slice_t* s = slice_of(views.at[i]);
+        const at::Tensor* t = plain_contiguous(held.add(outs.at[i]));
+        const mhip_slice_t* s = slice_of(held.add(views.at[i]));
         uint64_t len, hi;
         if (t == nullptr || s == nullptr || !extent(*s, &len, &hi) || (uint64_t)t->numel() != len) return kNotTaken;
         if (i == 0) code = reduce_code(*t);
         slices[i] = *s;
         dst[i] = t->data_ptr();
-        held.add(views.at[i]);
     }
     if (code < 0) return kNotTaken;
     for (Py_ssize_t i = 0; i < group.n; ++i) {
-        const at::Tensor* t = plain(group.at[i]);
+        const at::Tensor* t = plain(held.add(group.at[i]));
         if (t == nullptr) return kNotTaken;
         src[i] = t->data_ptr();
     }
-    held.add(a[3]);
     const mhip_stream_t stream = current_stream();
     return unlocked([&] {
         return mhip_reduce_scatter(dst, slices, (uint32_t)outs.n, src, in_view, 0, (uint32_t)group.n, code, (int)op, stream);
@@ -389,10 +390,11 @@ long dequant_accumulate_bucket(PyObject* const* a) {
     if (!bucket_of(a[0], a[1], a[2], a[3], &b) || !qs.few() || qs.n != ss.n) return kNotTaken;
     const uint8_t* q[kMaxItems];
     const float* scales[kMaxItems];
+    Held held;
     for (Py_ssize_t i = 0; i < qs.n; ++i) {
         void* qp;
         float* sp;
-        if (!payload(qs.at[i], ss.at[i], b, &qp, &sp)) return kNotTaken;
+        if (!payload(held.add(qs.at[i]), held.add(ss.at[i]), b, &qp, &sp)) return kNotTaken;
         q[i] = static_cast<const uint8_t*>(qp);
         scales[i] = sp;
     }

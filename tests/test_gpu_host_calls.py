@@ -1,5 +1,10 @@
 """The native host path (csrc/host_calls.cpp) against the general Python path behind it: the same bytes, and the same error
 for every call that one of them refuses.  A tensor subclass takes the general path, whatever else the call looks like."""
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -243,3 +248,12 @@ def test_the_current_stream_is_the_one_that_is_used():
     for t in threads:
         t.join()
     assert all(torch.equal(o, x[::2]) for o in outs)
+
+
+@pytest.mark.gpu
+def test_tensors_of_a_call_are_held_while_the_library_runs(tmp_path):
+    here = os.path.dirname(os.path.abspath(__file__))
+    shutil.copy(host.slice_copy.__self__.__file__, tmp_path)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", os.path.join(here, "c_abi", "held_library.c"), "-o", str(tmp_path / "libmonarch_hip.so")])
+    p = subprocess.run([sys.executable, os.path.join(here, "host_calls_held.py"), str(tmp_path)], capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0 and p.stdout.endswith("host_calls_held ok\n"), p.stdout + p.stderr[-2000:]
