@@ -73,6 +73,12 @@ __device__ __forceinline__ char* packed_of(const PackArgs& a, uint32_t v) { retu
 template <int ND> __device__ __forceinline__ char* packed_of(const OneViewArgs<ND>& a, uint32_t) { return a.packed; }
 __device__ __forceinline__ char* strided_of(const PackArgs& a, uint32_t v, uint32_t unit) { return a.base + a.offset[v] * unit; }
 template <int ND> __device__ __forceinline__ char* strided_of(const OneViewArgs<ND>& a, uint32_t, uint32_t) { return a.base; }
+// The same in units M, and `loc` units further on.  (As bytes, cast to M afterwards, the compiler waits for offset[v] before it decodes
+// the first unit: packs of two views in rows of 136 to 3080 bytes take 2.5 to 5 % longer, 32 MB in rows of 264 bytes 13.8 -> 14.5 us.)
+template <typename M> __device__ __forceinline__ M* strided_units_of(const PackArgs& a, uint32_t v) { return reinterpret_cast<M*>(a.base) + a.offset[v]; }
+template <typename M, int ND> __device__ __forceinline__ M* strided_units_of(const OneViewArgs<ND>& a, uint32_t) { return reinterpret_cast<M*>(a.base); }
+__device__ __forceinline__ char* strided_at(const PackArgs& a, uint32_t v, uint32_t unit, uint64_t loc) { return a.base + (a.offset[v] + loc) * unit; }
+template <int ND> __device__ __forceinline__ char* strided_at(const OneViewArgs<ND>& a, uint32_t, uint32_t unit, uint64_t loc) { return a.base + loc * unit; }
 
 // The view index is the fastest-varying part of the workgroup id, so that workgroups running side by side work on the
 // same rows of neighbouring views (for column blocks of one tensor: neighbouring segments of the same rows).  No 64-bit
@@ -308,7 +314,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_unpack_lines_kernel(Args a
     if (!live) r = 0;
     uint64_t col;
     const uint64_t loc = decode<WIDE, NDIM>(a.dims, r * run_of(a.dims), &col);  // first unit of the row; col == 0
-    char* __restrict__ row = strided_of(a, v, U) + loc * U;
+    char* __restrict__ row = strided_at(a, v, U, loc);
     const char* __restrict__ prow = packed_of(a, v) + (uint64_t)r * run_of(a.dims) * U;       // the row in the packed image
     const int64_t run_bytes = (int64_t)((uint64_t)run_of(a.dims) * U);                    // at least 16
     const int64_t lead = (int64_t)((uintptr_t)row & 127u);                  // the row starts `lead` bytes into its first line
@@ -364,7 +370,7 @@ __global__ __launch_bounds__(kPackThreads) void slice_units_kernel(Args a) {
     uint32_t v;
     tile_and_view(a, wg, &tile, &v);
     char* __restrict__ packed = packed_of(a, v);
-    M* __restrict__ strided = reinterpret_cast<M*>(strided_of(a, v, U));
+    M* __restrict__ strided = strided_units_of<M>(a, v);
     const uint32_t total = (uint32_t)a.total;
     const uint32_t pos0 = (uint32_t)tile * (kPackThreads * VU);  // position of the tile, counted from the aligned-down start
     const uint32_t mine = pos0 + threadIdx.x * VU;               // and of this lane's vector of the packed side
