@@ -322,12 +322,14 @@ static uint32_t narrow_tile_bytes(uint64_t bytes) {
 // 4 MiB and more whose sides are both longer than 512 bytes take 256 x 256 bytes (f64 pack / unpack, 128 x 128 and 256 x 256: 627^2
 // 3.1 / 3.3 and 2.9 / 2.9, 640^2 3.1 / 3.2 and 3.3 / 3.1, 887^2 4.8 / 5.1 and 4.0 / 3.9, 1145^2 6.7 / 6.5 and 5.8 / 5.7, where the
 // tiles of transpose_kernels.hip take 6.0 / 6.0; [3584, 16, 16] 4.5 / 4.4 and 6.5 / 6.4).
-// Byte matrices of 12 to 23 MiB collect all columns of a tile before they store the first (LATE): warm 0.95 of the time it took
-// with 64-bit tile numbers where the other order takes 1.05, cold 0.98 and 1.11; up to 12 MiB 0.92 and 0.82.  From 12 MiB on they
-// also keep the general form of addresses (GENERAL): its arithmetic spaces the stores, which in the short form leave in bursts
-// that some shapes pay for.  Against 64-bit tile numbers, random shapes, short form / general, warm and cold: 20 to 23 MiB mean
-// 0.977 / 0.954 and 0.989 / 0.953, slowest 1.007 / 0.999 and 1.052 / 0.997; 23 to 40 MiB 0.977 / 0.976 and 0.977 / 0.968, slowest
-// 1.139 / 1.042 and 1.087 / 0.998 ([1672, 15051] unpack 11.8 -> 13.4 us short, 12.1 general).
+// Byte matrices of more than 768 tiles (three on each of 256 CUs) and up to 23 MiB collect all columns of a tile before they store the
+// first (LATE) and keep the general form of addresses (GENERAL), whose arithmetic spaces the stores: in the short form they leave
+// in bursts, which pays while all tiles are in flight together and makes some shapes pay beyond.  Against 64-bit tile numbers,
+// random shapes, warm and cold: up to 768 tiles the short form takes 0.85 and 0.84 of the time, 0.93 at most (LATE and GENERAL 0.96,
+// 1.04 at most); 769 to 1000 tiles 0.985, but 1.05 to 1.20 on single shapes ([2049, 6001] unpack 8.6 -> 9.9 us), with LATE and
+// GENERAL 0.955, 0.976 at most; 20 to 23 MiB LATE alone 0.98 and 0.99, 1.05 at most, both 0.96, 1.02 at most.  Above 23 MiB, tiles of
+// 256 x 256 and GENERAL alone: 0.976 and 0.968, 1.04 at most, where the short form takes 0.977 with single shapes at 1.14 and 1.09
+// ([1672, 15051] unpack 11.8 -> 13.4 us, general 12.1).
 // Batches of matrices that fit 128 x 128 bytes keep that tile at any size: u8 [78125, 16, 16] 94 / 95 us, in tiles of 1024 x 64 of
 // which one matrix fills little 335 / 333; bf16 [39062, 16, 16] 45 / 46 and 97 / 98, [8544, 64, 64] 23.2 / 23.3 and 30.2 / 31.3.
 template <typename T, bool PACK>
@@ -336,9 +338,9 @@ static int launch_narrow_tile(NarrowArgs& a, uint64_t nbatch, hipStream_t stream
     const uint64_t ib = (uint64_t)(PACK ? a.Q : a.Sc) * ES, jb = (uint64_t)(PACK ? a.Sc : a.Q) * ES;
     const uint64_t bytes = nbatch * ib * jb / ES;
     if constexpr (ES == 1)
-        if (ib > 512 && jb > 512 && bytes > (12ull << 20)) {
+        if (ib > 512 && jb > 512) {
             if (bytes > (23ull << 20)) return launch_narrow<T, PACK, 256, 256, false, true>(a, nbatch, stream);
-            return launch_narrow<T, PACK, 128, 128, true, true>(a, nbatch, stream);
+            if (nbatch * ((ib + 127) / 128) * ((jb + 127) / 128) > 768) return launch_narrow<T, PACK, 128, 128, true, true>(a, nbatch, stream);
         }
     if (bytes >= (16ull << 20) && (ib <= 512 || jb <= 512) && (ib > 128 || jb > 128)) {  // a long side to fill the tile with
         const bool short_j = jb <= ib;

@@ -885,6 +885,20 @@ def test_transposes_with_a_short_side_and_small_ones(dtype):
         assert torch.equal(back.cpu(), ref), (shape, dtype)
 
 
+@pytest.mark.parametrize("shape", [(3072, 4096), (3001, 4001), (3073, 4001), (1025, 11001), (2, 1025, 5500), (2, 2049, 3001), (4801, 5001), (4923, 4923)])
+def test_byte_transposes_on_both_sides_of_768_tiles_and_23_mib(shape):
+    g = torch.Generator(device=DEV).manual_seed(shape[-1])
+    for turned in (False, True):
+        x = torch.randint(0, 256, shape[:-2] + shape[:-3:-1] if turned else shape, dtype=torch.uint8, device=DEV, generator=g)
+        s = Slice.of_tensor(x.transpose(-1, -2))
+        out = staging.pack(x, s)
+        back = torch.zeros_like(x)
+        staging.unpack(back, s, out)
+        sync()
+        assert torch.equal(out, x.transpose(-1, -2).contiguous().flatten())
+        assert torch.equal(back, x)
+
+
 @pytest.mark.parametrize("shape", [(895, 7403), (897, 7403), (1021, 6603), (1027, 6603), (3, 1000, 2201)])
 def test_transposes_of_two_byte_elements_with_few_tiles_along_a_side(shape):
     # rows that are not whole lines, on both sides of the eight tiles of 128 elements at which the order of the tiles changes

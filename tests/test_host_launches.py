@@ -62,15 +62,18 @@ def test_lanes_of_two_byte_transposes_follow_the_number_of_tiles(launches, pack)
 
 
 @pytest.mark.parametrize("pack", [True, False])
-def test_byte_matrices_of_12_to_40_mib_take_the_general_addresses(launches, pack):
-    # smaller ones the short form; it is the parameter before the last
+def test_byte_matrices_of_many_tiles_take_the_general_addresses(launches, pack):
+    # up to 768 tiles of 128 x 128 the short form (the parameter before the last), above it the general one and the columns of a
+    # tile before its first store (the last one), above 23 MiB the general one in tiles of 256 x 256
     def forms(rows, cols):
         return {name.split("slice_transpose_narrow_kernelI")[1].split("EEEv")[0] for _, name in launches(pack, 1, [cols, rows], [1, cols])
                 if "slice_transpose_narrow_kernel" in name}
 
     p = int(pack)
-    assert forms(3001, 4001) == {f"hLi256ELb{p}ELi128ELi128ELb1ELb0"}
-    assert forms(3301, 4001) == {f"hLi256ELb{p}ELi128ELi128ELb0ELb1"}
-    assert forms(1672, 15051) == {f"hLi512ELb{p}ELi256ELi256ELb0ELb0"}
-    assert forms(6301, 6501) == {f"hLi512ELb{p}ELi256ELi256ELb0ELb0"}
+    for rows, cols in ((600, 600), (3001, 4001), (2047, 6101), (6141, 2001)):
+        assert forms(rows, cols) == {f"hLi256ELb{p}ELi128ELi128ELb1ELb0"}
+    for rows, cols in ((3073, 4001), (1025, 11001), (2049, 6001), (3301, 4001), (4801, 5001)):
+        assert forms(rows, cols) == {f"hLi256ELb{p}ELi128ELi128ELb0ELb1"}
+    for rows, cols in ((1672, 15051), (6301, 6501)):
+        assert forms(rows, cols) == {f"hLi512ELb{p}ELi256ELi256ELb0ELb0"}
     assert not forms(6501, 6501)
