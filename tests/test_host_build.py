@@ -1,5 +1,6 @@
 """What the Makefile and the package's build step build, and for whom.  No GPU; nothing is compiled here."""
 import os
+import struct
 import subprocess
 import sys
 import sysconfig
@@ -41,3 +42,12 @@ def test_the_extension_is_built_for_the_interpreter_that_builds_it(monkeypatch):
 def test_an_interpreter_without_pytorch_is_named():
     p = plan("python", "PYTHON=/bin/false")
     assert p.returncode != 0 and "/bin/false is no Python with PyTorch" in p.stderr
+
+
+def test_the_extension_has_no_thread_local_data():
+    # it would slow down every thread-local access of a thread, a launch's among them, where the library was loaded first
+    with open(_native.host.slice_copy.__self__.__file__, "rb") as f:
+        elf = f.read()
+    start, size, count = struct.unpack_from("<Q", elf, 32)[0], *struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, start + k * size)[0] for k in range(count)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
