@@ -909,7 +909,10 @@ SWEEP_HEADERS = {
 further on); `packed fastest` / `memory fastest`: plain row-major walks; `diagonal`: consecutive workgroups step one
 tile along both axes.  The selection rule (`choose_walk` in `monarch_amd/csrc/transpose_kernels.hip`): 1/2/4-byte
 elements whose row pitches are multiples of 4 KiB on both sides take the diagonal walk, everything else the blocked
-walk (block 4 for 1-byte, 8 for 2-byte, 16 for 4/8-byte elements; 8 with the 512-byte-row tiles of 4- and 8-byte elements, 4 with that of 2-byte elements).  Every walk
+walk.  Its blocks are 4 x 4 tiles for 1-byte elements.  Tiles of 512-byte rows: 4 for 2-byte, 8 for 4- and 8-byte elements.  Rows of whole
+lines: 2 for 2-byte elements and for 4- and 8-byte elements up to 80 MB, where at least eight tiles lie along both sides, otherwise 8
+for 2-byte and 16 for 4- and 8-byte elements.  Written rows that start inside lines: 4 for 4- and 8-byte elements, 2 for 2-byte elements
+(8 with fewer than eight tiles along a side).  Blocks are halved while they are mostly padding.  Every walk
 runs with the cache policy the library picks for the element size.""",
     "transpose_policies": "# Transposing pack / unpack: A/B of the cache policies of its loads and stores (MI355X)\n\n"
     + _SWEEP_COMMON.format(which="transpose_policies", file="transpose_cache_policy_ab.md") + """\

@@ -10,8 +10,8 @@
 // over q and j over the memory-contiguous dimension c; unpacking, the other way round.  HBM-bound: 2 bytes of traffic
 // per byte moved.  Both sides move 16-byte vectors whatever the extents: the last vector of a row is moved back so that it
 // ends where the row ends.  bf16 [64, 4096, 64] -> [64, 64, 4096] (33.6 MB), pack / unpack: 95.8 / 104 us with the tiles
-// that fill a quarter of their lanes, 13.1 / 13.0 us here (5.1 / 5.2 TB/s); head dim 80: 98 / 82 -> 16.9 / 19.2,
-// 32: 94 / 81 -> 8.0 / 7.6; u8 head dim 128: 222 / 303 -> 12.9 / 13.8; bf16 1024^2: 3.3 / 3.4 -> 2.4 / 2.4.
+// that fill a quarter of their lanes, 10.9 / 11.0 us here (6.1 TB/s); head dim 80: 98 / 82 -> 15.6 / 17.7,
+// 32: 94 / 81 -> 6.5 / 6.6; u8 head dim 128: 222 / 303 -> 11.0 / 11.9; bf16 1024^2: 3.3 / 3.4 -> 2.2 / 2.2.
 //
 // Most launches are one or two rounds of workgroups, so what a wavefront issues before its first load and between its loads
 // and its stores is not hidden: tile numbers are decoded by multiplication (FastDiv32; the compiler's 64-bit divisions were
@@ -278,14 +278,15 @@ static int launch_narrow(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
 
 // The same with tiles that are longer along the long side (the written rows where LONG_I, else the read rows), where that
 // pays.  It does in two cases:
-//   * 400 to 512 tiles of 64 KiB (two fit a CU's LDS): all of them are resident at once, so the part first reads everything and
-//     then writes everything, in pieces of 1 KiB and more, and no write gets between the reads.  2- and 4-byte elements, packing /
-//     unpacking, one tile of 32 or 16 KiB -> 64 KiB, us: bf16 [64, 4096, 64] 15.6 / 14.9 -> 13.1 / 13.1, [56, 4096, 64] 13.9 / 13.7 ->
-//     12.1 / 11.2, [256, 1024, 64] 16.0 / 14.9 -> 13.1 / 15.0, f32 [262144, 32] 16.2 / 12.3 -> 11.1 / 10.8.  With fewer or more of them
-//     the part runs out of step again and large tiles lose: [32, 4096, 64] 8.1 / 7.5 -> 8.8 / 8.4, [96, 4001, 64] 21.7 / 20.2 ->
-//     22.4 / 22.1.  (Kernels with NarrowArgs; with NarrowOneArgs and registers for two tiles per CU the first is 12.3 / 12.6.)
-//   * 4-byte elements from 28 MiB on: tiles of 32 KiB instead of 16 (f32 [64, 4096, 32] 18.0 / 14.3 -> 15.2 / 14.5, [1 M, 16] 28.0 /
-//     25.8 -> 24.7 / 23.2; sides of 64 to 256 bytes, 33 to 100 MiB, 0.89 to 0.99 x; 17 MiB up to 1.1 x).
+//   * 400 to 512 tiles of 64 KiB (two fit a CU's LDS; the numbers stand for the 256 CUs of the whole part, on fewer the choice only
+//     costs time): all of them are resident at once, so the part first reads everything and then writes everything, in pieces of
+//     1 KiB and more, and no write gets between the reads.  2- and 4-byte elements, packing / unpacking, small tiles -> 64 KiB, us:
+//     bf16 [64, 4096, 64] 13.4 / 12.9 -> 10.9 / 11.0, [56, 4096, 64] 12.4 / 13.1 -> 10.1 / 10.1, [256, 1024, 64] 13.9 / 12.7 -> 11.0 /
+//     11.6, f32 [262144, 32] 14.1 / 12.5 -> 11.2 / 10.9.  With more of them the part runs out of step again and large tiles lose
+//     ([96, 4001, 64] 19.2 / 18.0 -> 20.8 / 20.0); with half as many they are within 4 % either way ([32, 4096, 64] 6.5 / 6.5 -> 6.3 / 6.4;
+//     the first line was measured at 8.1 / 7.5 and 8.8 / 8.4, with addresses in 64 bits).
+//   * 4-byte elements from 28 MiB on: tiles of 32 KiB instead of 16 ([1 M, 16] 28.0 / 25.8 -> 24.7 / 23.2 and others 0.89 to 0.99 x
+//     with addresses in 64 bits, 17 MiB up to 1.1 x; with the present ones 24.6 / 23.6 -> 24.8 / 23.1, nothing more than 4 % either way).
 constexpr uint64_t kResidentTilesMin = 400, kResidentTilesMax = 512;
 template <typename T, bool PACK, int WB, int RB, bool LONG_I>
 static int launch_narrow_long(NarrowArgs& a, uint64_t nbatch, hipStream_t stream) {
@@ -405,10 +406,10 @@ bool try_narrow_transpose(char* base, char* packed, const CanonSlice& c, int cd,
     a.packed = packed;
     a.Sc = (uint32_t)Sc;
     a.Q = Q;
-    // Written rows that start on half cache lines are stored write-through (33.6 MB of keys 14.8 us against 16.5 through
-    // the cache, unpacked rows of 64 bytes 7.6 against 8.5); others go through the cache, which combines what neighbouring
-    // tiles share (rows of 4001 bf16 15.9 against 18.9, unpacked rows of 160 bytes 19.2 against 19.9), unless the launch
-    // is small enough to be bound by latency (bf16 1500^2 3.5 against 3.7).
+    // Written rows that start on half cache lines are stored write-through (33.6 MB of keys 10.9 us against 12.3 through the
+    // cache, unpacked rows of 64 bytes 6.6 against 7.7); others go through the cache, which combines what neighbouring
+    // tiles share (rows of 4001 bf16 19.1 against 21.0, unpacked rows of 160 bytes 17.7 against 18.4), unless the launch
+    // is small enough to be bound by latency (bf16 1500^2 3.1 against 3.2).
     a.write_through = (written & 63u) == 0 || bytes <= (8ull << 20);
     switch (unit) {
         case 1: *rc = launch_narrow_tile<uint8_t, PACK>(a, nbatch, stream); break;
